@@ -36,7 +36,7 @@
 extern "C" {
 #endif
 
-#define CLUSTEN_ABI_VERSION 4
+#define CLUSTEN_ABI_VERSION 5
 
 /* Element type of every floating-point tensor of a call.  The reference dispatches
  * double / float / half (AT_DISPATCH_FLOATING_TYPES_AND_HALF, clustenqk_cuda_kernel.cu:78);
@@ -613,6 +613,41 @@ int clusten_merge_centres(const float* pos, const float* min_dist, const void* l
  * counterpart in the reference's extension modules. */
 int clusten_merge_rows(const void* const* src, void* const* dst, const int* row_bytes, int count,
                        const int64_t* centre, int64_t B, int N, int n_out, clusten_stream stream);
+
+/* ---- transformer blocks over token rows (optional) --------------------------------------------- */
+
+/* Weight matrices in the order the two block kernels below read them, for token rows of C channels (C in
+ * {32,64,128,256,512}, else CLUSTEN_ERR_BAD_DIMS): src fp32 (n,k) row-major, or (k,n) with `transposed`, whose transpose
+ * is packed then; dst n * k elements of dtype (F32, F16, BF16), 16-byte aligned.  n and k are multiples of C.  All `count`
+ * items are packed by one launch per eight.  No counterpart in the reference's extension modules. */
+typedef struct {
+    const float* src;
+    void* dst;
+    int32_t n, k, transposed, reserved;
+} clusten_pack_item;
+int clusten_block_pack(const clusten_pack_item* items, int count, int C, int dtype, clusten_stream stream);
+
+/* out = LayerNorm(x) W^T + bias: `norm1` and the q / kv projections of a block (models/aff_transformer.py:219, 103-106).
+ *   x (rows,C) of x_dtype (F32 or dtype); norm_w, norm_b fp32 (C); w: (N,C) packed for width C as dtype; bias0 fp32 (C):
+ *   the first C output channels' bias, bias1 fp32 (N-C): the others' (may be NULL when N == C); out (rows,N) of dtype.
+ *   normed (rows,C) of dtype and stats (rows,2) fp32 - mean and 1/deviation of every row - are written when not NULL.
+ * The norm is computed in fp32 and rounded to dtype, sums are fp32, biases are rounded to dtype.  N a multiple of C. */
+int clusten_norm_linear_forward(const void* x, int x_dtype, const float* norm_w, const float* norm_b, float eps,
+                                const void* w, const float* bias0, const float* bias1, void* out, void* normed,
+                                float* stats, int64_t rows, int C, int N, int dtype, clusten_stream stream);
+
+/* The block behind its attention (models/aff_transformer.py:157-158, 230-232, 181-196):
+ *   x1 = x + s (attn Wp^T + bp),   out = x1 + s (gelu(LayerNorm(x1) W1^T + b1) W2^T + b2)
+ *   attn (rows,C) of dtype; x, out (rows,C) of x_dtype (F32 or dtype); wp (C,C), w1 (H,C), w2 (C,H) packed for width C;
+ *   norm_w, norm_b, bp, b1, b2 fp32; H a multiple of C.  scale: fp32, one factor per image of rows_per_image rows (s;
+ *   rounded to dtype), or NULL for 1.  For a backward pass, all or none of: x1 (rows,C) of x_dtype, normed (rows,C) of dtype
+ *   = LayerNorm(x1), hidden (rows,H) of dtype = the sum ahead of the GELU, stats (rows,2) fp32.
+ * Intermediates are rounded to dtype (x1 to x_dtype) where separate layers would store them; sums are fp32. */
+int clusten_block_tail_forward(const void* attn, const void* x, int x_dtype, const void* wp, const float* bp,
+                               const float* norm_w, const float* norm_b, float eps, const void* w1, const float* b1,
+                               const void* w2, const float* b2, void* out, const float* scale, int rows_per_image,
+                               void* x1, void* normed, void* hidden, float* stats, int64_t rows, int C, int H, int dtype,
+                               clusten_stream stream);
 
 /* ---- producer of the neighbourhood lists (optional) ------------------------------------------- */
 

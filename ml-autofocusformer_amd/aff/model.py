@@ -57,7 +57,11 @@ def default_ops():
                            neighbour_lists_supported=_native.neighbour_lists_supported,
                            gather_rows=_native.gather_rows, gather_rows_supported=_native.gather_rows_supported,
                            merge_centres=_native.merge_centres, merge_centres_supported=_native.merge_centres_supported,
-                           merge_rows=_native.merge_rows, merge_rows_supported=_native.merge_rows_supported)
+                           merge_rows=_native.merge_rows, merge_rows_supported=_native.merge_rows_supported,
+                           block_pack=_native.block_pack, block_supported=_native.block_supported,
+                           norm_linear=_native.norm_linear, block_tail=_native.block_tail,
+                           block_stands_for=(("linear", _native.linear), ("layer_norm", _native.layer_norm),
+                                             ("add_layer_norm", _native.add_layer_norm)))
 
 
 def _cast_params(lin, dt):
@@ -321,14 +325,20 @@ class ClusterAttention(nn.Module):
     def forward(self, feat, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None):
         """`grid_lists`: (cluster_idx, pe_idx, cluster_mask) with a leading 1 instead of the batch size, when the
         lists are the same for every image (tokens of a regular grid); the one-kernel path reads those."""
-        b, n, c = feat.shape
+        q, kv = _linear_pair(self.q, self.kv, feat, self.ops)
+        out = self.attend(q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
+        return self.proj_drop(_linear(self.proj, out, self.ops))
+
+    def attend(self, q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None):
+        """The attention between its projections: q (b,n,c) and kv (b,n,2c) in, what the output projection reads (b,n,c)
+        out.  The query is not scaled yet; q and kv may be column ranges of one matrix."""
+        b, n, c = q.shape
         h = self.num_heads
         ch = c // h
         # inference: the neighbourhoods as (b,n,nnc) cluster numbers instead of the expanded (b,n,m*nnc) row lists
         numbered = cluster_idx is not None and not global_attn and not torch.is_grad_enabled()
         compact = numbered and getattr(self.ops, "qk_clusters", None) is not None
         sized = {} if self.cluster_size == 8 else {"cluster_size": self.cluster_size}
-        q, kv = _linear_pair(self.q, self.kv, feat, self.ops)
         kv = kv.view(b, n, h, 2, ch).permute(3, 0, 2, 1, 4)                                                 # (2,b,h,n,ch) view
         key, v = kv[0], kv[1]
         one_kernel = getattr(self.ops, "cluster_attention", None)
@@ -342,7 +352,7 @@ class ClusterAttention(nn.Module):
             out = one_kernel(q.view(b, n, h, ch).permute(0, 2, 1, 3), key, v, lists[0], self.bias_table(table),
                              lists[1], lists[2], self.blank_k, self.blank_v, scale=self.scale,
                              **({"plan": plan} if plan is not None else {}))
-            return self.proj_drop(_linear(self.proj, out, self.ops))
+            return out
         train_kernel = getattr(self.ops, "cluster_attention_backward", None)
         if (train_kernel is not None and torch.is_grad_enabled() and cluster_idx is not None and not global_attn
                 and self.cluster_size == 8 and grid_lists is not None and len(grid_lists) > 4 and not (self.training and self.attn_drop.p > 0)
@@ -353,7 +363,7 @@ class ClusterAttention(nn.Module):
             out = _ClusterAttention.apply(q.view(b, n, h, ch).permute(0, 2, 1, 3), key, v, bias, self.blank_k,
                                           self.blank_v, grid_lists[3], grid_lists[4], pe_idx, member_idx,
                                           self.scale, self.ops)
-            return self.proj_drop(_linear(self.proj, out, self.ops))
+            return out
         dense = getattr(self.ops, "dense_attention", None)
         if (global_attn and dense is not None and not torch.is_grad_enabled()
                 and not (self.training and self.attn_drop.p > 0)
@@ -361,7 +371,7 @@ class ClusterAttention(nn.Module):
             # inference on 16-bit data, every token attending to every token: one kernel as well
             out = dense(q.view(b, n, h, ch).permute(0, 2, 1, 3), key, v, self.bias_table(table), pe_idx,
                         self.blank_k, self.blank_v, scale=self.scale)
-            return self.proj_drop(_linear(self.proj, out, self.ops))
+            return out
         q = (q * self.scale).reshape(b, n, h, ch).permute(0, 2, 1, 3)                    # (b,h,n,ch) view
         if global_attn:
             attn = q @ key.transpose(-1, -2)                                             # (b,h,n,n)
@@ -401,8 +411,7 @@ class ClusterAttention(nn.Module):
         else:
             out = self.ops.av(attn, v, member_idx)                                       # (b,h,n,ch)
         out = out + blank * self.blank_v.reshape(1, h, 1, ch)
-        out = out.permute(0, 2, 1, 3).reshape(b, n, c)
-        return self.proj_drop(_linear(self.proj, out, self.ops))
+        return out.permute(0, 2, 1, 3).reshape(b, n, c)
 
 
 class ClusterTransformerBlock(nn.Module):
@@ -419,11 +428,52 @@ class ClusterTransformerBlock(nn.Module):
             self.gamma1 = nn.Parameter(layer_scale * torch.ones(dim))
             self.gamma2 = nn.Parameter(layer_scale * torch.ones(dim))
 
+    def _fused_dtype(self, feat):
+        """The type the block kernels work in, or None when the block runs layer by layer: with gradients, on widths or
+        types the kernels are not built for, with layer scale or an active dropout, and when the caller's `ops` has
+        another implementation of a layer they stand for."""
+        ops = self.attn.ops
+        if torch.is_grad_enabled() or self.layer_scale or getattr(ops, "block_tail", None) is None:
+            return None
+        if self.training and (self.mlp.drop.p > 0 or self.attn.proj_drop.p > 0 or not isinstance(self.drop_path, nn.Identity)):
+            return None
+        dt = torch.get_autocast_dtype("cuda") if feat.is_cuda and torch.is_autocast_enabled("cuda") else torch.float32
+        if not ops.block_supported(feat, dt, self.mlp.fc1.out_features) or self.norm1.weight.dtype != torch.float32:
+            return None
+        return dt if all(getattr(ops, name, None) is fn for name, fn in ops.block_stands_for) else None
+
+    def _packed(self, dt):
+        """(weights of the five Linear layers as the block kernels read them, byte offset of each), kept until one of
+        them changes."""
+        attn, mlp = self.attn, self.mlp
+        weights = (attn.q.weight, attn.kv.weight, attn.proj.weight, mlp.fc1.weight, mlp.fc2.weight)
+        key = (dt,) + tuple((w._version, w.data_ptr()) for w in weights)
+        cache = self.__dict__.get("_pack_cache")
+        if cache is None or cache[0] != key:
+            cache = (key, attn.ops.block_pack(attn.dim, dt, [(w.detach(), False) for w in weights]))
+            self.__dict__["_pack_cache"] = cache     # a plain attribute, as for the 16-bit copies of the single layers
+        return cache[1]
+
     def forward(self, feat, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None,
                 carry=None):
         """Returns (feat, branch): the block's output is feat + branch.  The addition is left to the caller, which
         hands `branch` to the next block as `carry` so that it can ride along with that block's first norm."""
         ops = self.attn.ops
+        dt = self._fused_dtype(feat)
+        if dt is not None:
+            # inference: three kernels - norm and projections, attention, everything behind it
+            if carry is not None:
+                feat = feat + carry
+            attn, mlp = self.attn, self.mlp
+            packed, at = self._packed(dt)
+            c = feat.shape[2]
+            qkv = ops.norm_linear(feat, self.norm1.weight, self.norm1.bias, self.norm1.eps, packed, at[0], attn.q.bias,
+                                  attn.kv.bias, 3 * c)
+            a = attn.attend(qkv[..., :c], qkv[..., c:], member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx,
+                            grid_lists)
+            a = a if a.dtype == dt else a.to(dt)
+            return ops.block_tail(a.contiguous(), feat, packed, at[2:], attn.proj.bias, self.norm2.weight, self.norm2.bias,
+                                  self.norm2.eps, mlp.fc1.bias, mlp.fc2.bias), None
         feat, x = _add_layer_norm(self.norm1, feat, carry, ops)
         a = self.attn(x, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
         feat, x = _add_layer_norm(self.norm2, feat, self.drop_path(self.gamma1 * a if self.layer_scale else a), ops)

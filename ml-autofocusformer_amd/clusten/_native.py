@@ -14,7 +14,7 @@ import torch
 
 _LIB_PATH = os.path.normpath(os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "lib", "libclusten_hip.so"))
 
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 _DTYPE_CODE = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2, torch.float64: 3}
 
@@ -29,6 +29,11 @@ class Strides(ctypes.Structure):
 
 class WfShape(ctypes.Structure):
     _fields_ = [(n, ctypes.c_int32) for n in ("B", "N", "Nout", "C", "M", "IC")]
+
+
+class PackItem(ctypes.Structure):
+    _fields_ = [("src", ctypes.c_void_p), ("dst", ctypes.c_void_p)] + [(n, ctypes.c_int32) for n in ("n", "k", "transposed",
+                                                                                                    "reserved")]
 
 
 _P = ctypes.c_void_p
@@ -113,6 +118,12 @@ _PROTOTYPES = {
     "clusten_scanline_rank_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int]),
     "clusten_scanline_rank": (ctypes.c_int, [_P, _P, _P, ctypes.c_size_t, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                             ctypes.c_int, ctypes.c_float, ctypes.c_float, _P]),
+    "clusten_block_pack": (ctypes.c_int, [ctypes.POINTER(PackItem), ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_norm_linear_forward": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, ctypes.c_float, _P, _P, _P, _P, _P, _P,
+                                                  ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_block_tail_forward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_float, _P, _P, _P, _P, _P,
+                                                 _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_int,
+                                                 ctypes.c_int, ctypes.c_int, _P]),
     "clusten_knn2d": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
 }
 
@@ -1585,3 +1596,93 @@ def knn2d(query: torch.Tensor, database: torch.Tensor, k: int, return_dist: bool
             _check(lib.clusten_knn2d(_ptr(query), _ptr(database), _ptr(idx), _ptr(dist), b, nq, n, k, _stream(device)),
                    "clusten_knn2d")
     return (idx, dist) if return_dist else idx
+
+
+_BLOCK_WIDTHS = (32, 64, 128, 256, 512)
+
+
+def block_supported(x: torch.Tensor, dtype: torch.dtype, hidden: int) -> bool:
+    """True when the block kernels (`norm_linear`, `block_tail`) take token rows `x` (..., C) for products in `dtype` and a
+    hidden layer of `hidden` channels: C of a built width, x fp32 or of `dtype`, hidden a multiple of C."""
+    return (x.is_cuda and x.shape[-1] in _BLOCK_WIDTHS and dtype in _DTYPE_CODES and x.dtype in (torch.float32, dtype)
+            and hidden % x.shape[-1] == 0 and x.is_contiguous())
+
+
+def block_pack(width: int, dtype: torch.dtype, weights):
+    """The matrices `weights` - (fp32 (n,k) tensor, transposed) pairs, n and k multiples of `width` - as the block kernels
+    of that width read them, one after the other in one tensor of `dtype`.  Returns (tensor, byte offset of each)."""
+    lib = load()
+    device = weights[0][0].device
+    total, offsets = 0, []
+    for w, _ in weights:
+        _require_cuda("weight", w, device)
+        if w.dim() != 2 or w.dtype != torch.float32 or not w.is_contiguous():
+            raise RuntimeError("weights must be contiguous fp32 matrices")
+        offsets.append(total)
+        total += w.numel()
+    out = torch.empty(total, dtype=dtype, device=device)
+    size = out.element_size()
+    items = (PackItem * len(weights))()
+    for it, (w, transposed), at in zip(items, weights, offsets):
+        n, k = w.shape
+        it.src, it.dst, it.transposed = w.data_ptr(), out.data_ptr() + at * size, int(bool(transposed))
+        it.n, it.k = (k, n) if transposed else (n, k)
+    with torch.cuda.device(device):
+        _check(lib.clusten_block_pack(items, len(weights), width, _DTYPE_CODES[dtype], _stream(device)), "clusten_block_pack")
+    return out, [at * size for at in offsets]
+
+
+def norm_linear(x: torch.Tensor, norm_w, norm_b, eps: float, packed: torch.Tensor, w_at: int, bias0, bias1, n_out: int):
+    """LayerNorm(x) @ W.T + bias over the last axis of x (..., C), in packed's dtype: W (n_out, C) at byte `w_at` of `packed`
+    (`block_pack`), bias0 fp32 (C,) for the first C outputs, bias1 for the others.  No autograd."""
+    lib = load()
+    _require_cuda("x", x)
+    device, c = x.device, x.shape[-1]
+    if not block_supported(x, packed.dtype, c):
+        raise RuntimeError("norm_linear takes contiguous rows of 32, 64, 128, 256 or 512 channels, fp32 or of the weights' dtype")
+    for t in (norm_w, norm_b, bias0, bias1):
+        if t.dtype != torch.float32 or not t.is_contiguous() or t.device != device:
+            raise RuntimeError("norm parameters and biases must be contiguous fp32 tensors on x's device")
+    if w_at + n_out * c * packed.element_size() > packed.numel() * packed.element_size() or bias0.numel() != c or \
+            bias1.numel() != n_out - c or norm_w.numel() != c or norm_b.numel() != c:
+        raise RuntimeError("norm_linear: weights, biases and norm must fit x and n_out")
+    out = torch.empty(x.shape[:-1] + (n_out,), dtype=packed.dtype, device=device)
+    if out.numel() == 0:
+        return out
+    with torch.cuda.device(device):
+        _check(lib.clusten_norm_linear_forward(x.data_ptr(), _DTYPE_CODES[x.dtype], norm_w.data_ptr(), norm_b.data_ptr(), eps,
+                                               packed.data_ptr() + w_at, bias0.data_ptr(), bias1.data_ptr(),
+                                               out.data_ptr(), None, None, x.numel() // c, c, n_out,
+                                               _DTYPE_CODES[packed.dtype], _stream(device)), "clusten_norm_linear_forward")
+    return out
+
+
+def block_tail(attn: torch.Tensor, x: torch.Tensor, packed: torch.Tensor, at, bias_p, norm_w, norm_b, eps: float, bias1,
+               bias2, scale=None):
+    """x1 = x + scale * (attn Wp^T + bp);  x1 + scale * (gelu(LayerNorm(x1) W1^T + b1) W2^T + b2) for token rows x (..., C):
+    everything of a transformer block behind its attention.  `at`: byte offsets of Wp, W1 and W2 in `packed`; the hidden
+    width is bias1's; `scale`: fp32 (B,) factors of the images (the first axis of x), or None.  No autograd."""
+    lib = load()
+    _require_cuda("x", x)
+    device, c, hidden = x.device, x.shape[-1], bias1.numel()
+    if not block_supported(x, packed.dtype, hidden) or attn.shape != x.shape or attn.dtype != packed.dtype or \
+            not attn.is_contiguous() or attn.device != device:
+        raise RuntimeError("block_tail takes contiguous rows of 32, 64, 128, 256 or 512 channels, attn of the weights' dtype")
+    for t in (bias_p, norm_w, norm_b, bias1, bias2):
+        if t.dtype != torch.float32 or not t.is_contiguous() or t.device != device or (t is not bias1 and t.numel() != c):
+            raise RuntimeError("norm parameters and biases must be contiguous fp32 tensors on x's device")
+    size = packed.element_size()
+    if at[0] + c * c * size > packed.numel() * size or max(at[1:]) + hidden * c * size > packed.numel() * size:
+        raise RuntimeError("block_tail: the packed weights do not hold three matrices of these sizes")
+    out = torch.empty_like(x)
+    if out.numel() == 0:
+        return out
+    with torch.cuda.device(device):
+        base = packed.data_ptr()
+        _check(lib.clusten_block_tail_forward(attn.data_ptr(), x.data_ptr(), _DTYPE_CODES[x.dtype], base + at[0],
+                                              bias_p.data_ptr(), norm_w.data_ptr(), norm_b.data_ptr(), eps, base + at[1],
+                                              bias1.data_ptr(), base + at[2], bias2.data_ptr(), out.data_ptr(),
+                                              None if scale is None else scale.data_ptr(), x.numel() // c // x.shape[0],
+                                              None, None, None, None, x.numel() // c, c, hidden,
+                                              _DTYPE_CODES[packed.dtype], _stream(device)), "clusten_block_tail_forward")
+    return out

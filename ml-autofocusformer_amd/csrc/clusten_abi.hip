@@ -13,6 +13,8 @@ inline int check_attn_call(const clusten_attn_shape& s, int dtype) {
     return check_attn_shape(s);
 }
 
+inline bool block_dtype_ok(int dtype) { return dtype == CLUSTEN_F32 || dtype == CLUSTEN_F16 || dtype == CLUSTEN_BF16; }
+
 inline clusten_strides contiguous_strides(const clusten_attn_shape& s) {
     clusten_strides r;
     r.n = s.C;
@@ -584,6 +586,58 @@ int clusten_knn2d(const float* query, const float* database, int64_t* idx, float
     if (B <= 0 || Nq <= 0 || N <= 0 || K < 1 || K > 8 || K > N) return CLUSTEN_ERR_BAD_DIMS;
     if ((int64_t)B * ((Nq + 255) / 256) >= ((int64_t)1 << 31)) return CLUSTEN_ERR_BAD_DIMS;
     return launch_knn2d(query, database, idx, dist, B, Nq, N, K, as_stream(stream));
+}
+
+int clusten_block_pack(const clusten_pack_item* items, int count, int C, int dtype, clusten_stream stream) {
+    if (!items) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (count <= 0 || !block_width_supported(C)) return CLUSTEN_ERR_BAD_DIMS;
+    for (int i = 0; i < count; ++i) {
+        const clusten_pack_item& it = items[i];
+        if (!it.src || !it.dst) return CLUSTEN_ERR_NULL_POINTER;
+        if (it.n <= 0 || it.k <= 0 || it.n % C != 0 || it.k % C != 0) return CLUSTEN_ERR_BAD_DIMS;
+        if (!aligned16(it.dst)) return CLUSTEN_ERR_UNALIGNED;
+    }
+    return launch_block_pack(items, count, C, dtype, as_stream(stream));
+}
+
+int clusten_norm_linear_forward(const void* x, int x_dtype, const float* norm_w, const float* norm_b, float eps,
+                                const void* w, const float* bias0, const float* bias1, void* out, void* normed,
+                                float* stats, int64_t rows, int C, int N, int dtype, clusten_stream stream) {
+    if (!x || !norm_w || !norm_b || !w || !bias0 || !out || (N > C && !bias1)) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype) || (x_dtype != dtype && x_dtype != CLUSTEN_F32)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (rows <= 0 || rows >= (int64_t)1 << 31 || !block_width_supported(C) || N <= 0 || N % C != 0) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(x) || !aligned16(norm_w) || !aligned16(norm_b) || !aligned16(w) || !aligned16(bias0) || !aligned16(bias1) ||
+        !aligned16(out) || !aligned16(normed) || (reinterpret_cast<uintptr_t>(stats) & 7)) {
+        return CLUSTEN_ERR_UNALIGNED;
+    }
+    NormLinearArgs a = {};
+    a.x = x, a.norm_w = norm_w, a.norm_b = norm_b, a.w = w, a.bias0 = bias0, a.bias1 = bias1, a.out = out, a.normed = normed;
+    a.stats = reinterpret_cast<float2*>(stats), a.rows = rows, a.chunks = N / C, a.eps = eps;
+    return launch_norm_linear(a, x_dtype, C, dtype, as_stream(stream));
+}
+
+int clusten_block_tail_forward(const void* attn, const void* x, int x_dtype, const void* wp, const float* bp,
+                               const float* norm_w, const float* norm_b, float eps, const void* w1, const float* b1,
+                               const void* w2, const float* b2, void* out, const float* scale, int rows_per_image,
+                               void* x1, void* normed, void* hidden, float* stats, int64_t rows, int C, int H, int dtype,
+                               clusten_stream stream) {
+    if (!attn || !x || !wp || !bp || !norm_w || !norm_b || !w1 || !b1 || !w2 || !b2 || !out) return CLUSTEN_ERR_NULL_POINTER;
+    const int kept = (x1 != nullptr) + (normed != nullptr) + (hidden != nullptr) + (stats != nullptr);
+    if (kept != 0 && kept != 4) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype) || (x_dtype != dtype && x_dtype != CLUSTEN_F32)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (rows <= 0 || rows >= (int64_t)1 << 31 || !block_width_supported(C) || H <= 0 || H % C != 0) return CLUSTEN_ERR_BAD_DIMS;
+    if (scale && (rows_per_image <= 0 || rows % rows_per_image != 0)) return CLUSTEN_ERR_BAD_DIMS;
+    const void* all[] = {attn, x, wp, bp, norm_w, norm_b, w1, b1, w2, b2, out, x1, normed, hidden};
+    for (const void* p : all) {
+        if (!aligned16(p)) return CLUSTEN_ERR_UNALIGNED;
+    }
+    if (reinterpret_cast<uintptr_t>(stats) & 7) return CLUSTEN_ERR_UNALIGNED;
+    BlockTailArgs a = {};
+    a.attn = attn, a.x = x, a.wp = wp, a.bp = bp, a.norm_w = norm_w, a.norm_b = norm_b, a.w1 = w1, a.b1 = b1, a.w2 = w2;
+    a.b2 = b2, a.out = out, a.scale = scale, a.rows_per_image = scale ? rows_per_image : 1, a.chunks = H / C, a.rows = rows;
+    a.eps = eps, a.x1 = x1, a.normed = normed, a.hidden = hidden, a.stats = reinterpret_cast<float2*>(stats);
+    return launch_block_tail(a, x_dtype, C, dtype, as_stream(stream));
 }
 
 }  // extern "C"

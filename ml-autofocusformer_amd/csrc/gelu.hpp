@@ -29,4 +29,33 @@ __device__ __forceinline__ float gelu_erf(float v) {
     return v * (v < 0.f ? half_erfc : 1.f - half_erfc);
 }
 
+// The same for results that are rounded to 16 bits, in two thirds of the instructions: Phi(-a) = exp2(Q(a)) with Q a
+// polynomial of degree 10 for log2 Phi(-a) on [0, 6.5] (minimax in log2, so the bound is relative: 1.3e-6 of Phi over the
+// whole range, fp32 evaluation included; half a unit in the last place of fp16 is 4.9e-4), and GELU(v) = max(v, 0) - a Phi(-a)
+// with a = |v|.  a stops at 6.5, where a Phi(-a) is 2.6e-10, below half of fp16's smallest number.  No reciprocal, no
+// select; a NaN stays one (`v_maximum3`).  One of the two transcendental instructions of the form above, which take four
+// times an ordinary one, goes with them.
+__device__ __forceinline__ float gelu_16bit(float v) {
+    const float a = fminf(fabsf(v), 6.5f);
+    float q = -8.44261482e-09f;
+    q = q * a + 3.01195427e-07f;
+    q = q * a - 4.53102646e-06f;
+    q = q * a + 3.56483971e-05f;
+    q = q * a - 0.000124659285f;
+    q = q * a - 0.000360930182f;
+    q = q * a + 0.00745342366f;
+    q = q * a - 0.0528455773f;
+    q = q * a - 0.459058428f;
+    q = q * a - 1.15112928f;
+    q = q * a - 0.999999368f;
+    return __builtin_elementwise_maximum(v, 0.f) - a * __builtin_amdgcn_exp2f(q);
+}
+
+// The GELU of a kernel whose results are stored as T.
+template <typename T>
+__device__ __forceinline__ float gelu_for(float v) {
+    if constexpr (sizeof(T) == 2) return gelu_16bit(v);
+    else return gelu_erf(v);
+}
+
 }  // namespace clusten

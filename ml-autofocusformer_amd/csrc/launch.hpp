@@ -244,6 +244,57 @@ int launch_scanline_rank(const float* pos, int64_t* ranking, void* workspace, in
 int launch_knn2d(const float* query, const float* database, int64_t* idx, float* dist, int B, int Nq, int N, int K,
                  hipStream_t stream);
 
+// ---- transformer blocks over token rows (token_block.hpp) -----------------------------------------------------------
+
+// out = LayerNorm(x) W^T + bias (norm_linear_impl.hpp) and the block behind its attention (block_tail_impl.hpp).
+//   T: the dtype of the call (weights as packed, results); S: the token stream's, fp32 or T.  C in {32,64,128,256,512}.
+struct NormLinearArgs {
+    const void* x;
+    const float* norm_w;
+    const float* norm_b;
+    const void* w;         // packed for width C
+    const float* bias0;    // first C output channels
+    const float* bias1;    // the others
+    void* out;             // (rows, N)
+    void* normed;          // (rows, C) of T, or null
+    float2* stats;         // (rows) mean and 1 / deviation, or null
+    int64_t rows;
+    int chunks;            // N / C
+    float eps;
+};
+struct BlockTailArgs {
+    const void* attn;      // (rows, C) of T
+    const void* x;         // (rows, C) of S
+    const void* wp;
+    const float* bp;
+    const float* norm_w;
+    const float* norm_b;
+    const void* w1;        // (H, C), packed for width C
+    const float* b1;
+    const void* w2;        // (C, H), packed for width C
+    const float* b2;
+    void* out;             // (rows, C) of S
+    const float* scale;    // per image, or null
+    int rows_per_image;
+    int chunks;            // H / C
+    int64_t rows;
+    float eps;
+    // what a backward pass wants to keep, each may be null
+    void* x1;              // (rows, C) of S
+    void* normed;          // (rows, C) of T
+    void* hidden;          // (rows, H) of T, ahead of the GELU
+    float2* stats;         // (rows)
+};
+bool block_width_supported(int C);
+// Tiles of 16 rows a workgroup takes (4, 2 or 1).
+int block_row_tiles(int elem_size, int C, int64_t rows);
+// dst = a weight matrix of fp32 in the order the block kernels of width C read it in, as dtype.  src is (n,k), or (k,n)
+//   when transposed (dst is then that of its transpose); n a multiple of the width's group, k of the fragment.
+int block_group_channels(int C);
+int launch_block_pack(const clusten_pack_item* items, int count, int C, int dtype, hipStream_t stream);
+int launch_norm_linear(const NormLinearArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);
+int launch_block_tail(const BlockTailArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);
+
 // Fill `count` fp32 / fp64 words with zero (a kernel, so that callers may capture it in a HIP graph).
 //   `only_if` (may be null): a device flag; the kernel does nothing when it points to zero.
 int launch_zero_f32(float* dst, size_t count, hipStream_t stream, const int32_t* only_if = nullptr);

@@ -1,0 +1,129 @@
+"""GPU parity of the block kernels (`clusten_norm_linear_forward`, `clusten_block_tail_forward`) against the layers they stand
+for (`norm1` + q / kv projections and proj + residual + `norm2` + MLP + residual, models/aff_transformer.py:103-106, 157-158,
+219-232), evaluated in fp32 from the same rounded operands with the intermediates rounded where the layers store them.
+
+Bar, max|x - ref| / max|ref|: 2e-3 fp16, 1e-2 bf16 (a handful of roundings of 2^-11 / 2^-8 on the way, those of the hidden
+layer averaged over its channels), 1e-5 fp32.
+"""
+import numpy as np
+import pytest
+import torch
+import torch.nn.functional as F
+
+from clusten import _native
+from oracle import clusten_oracle as oracle
+
+pytestmark = pytest.mark.gpu
+
+BAR = {torch.float16: 2e-3, torch.bfloat16: 1e-2, torch.float32: 1e-5}
+# fp32 and 16-bit token streams; row counts below a tile, across tiles, and enough for 2 and 4 tiles a workgroup
+CASES = [(torch.float16, torch.float16), (torch.float16, torch.float32), (torch.bfloat16, torch.bfloat16),
+         (torch.float32, torch.float32)]
+SHAPES = [(32, 64, 1), (32, 96, 70), (64, 192, 16), (64, 128, 16 * 1024 + 3), (128, 384, 33), (128, 128, 8192 + 17),
+          (256, 768, 49), (256, 512, 16 * 1024 + 1), (512, 1536, 15), (512, 1024, 8192 - 5)]
+
+
+class Block:
+    """Random parameters of one block on the device, and its weights packed."""
+
+    def __init__(self, c, hidden, dt, device, seed):
+        gen = torch.Generator().manual_seed(seed)
+
+        def draw(*shape, scale=1.0):
+            return (torch.randn(*shape, generator=gen) * scale).to(device)
+
+        self.c, self.hidden, self.dt = c, hidden, dt
+        self.w = [draw(c, c, scale=c ** -0.5), draw(2 * c, c, scale=c ** -0.5), draw(c, c, scale=c ** -0.5),
+                  draw(hidden, c, scale=c ** -0.5), draw(c, hidden, scale=hidden ** -0.5)]
+        self.b = [draw(t.shape[0], scale=0.3) for t in self.w]
+        self.norm = [1 + 0.2 * draw(c), 0.2 * draw(c), 1 + 0.2 * draw(c), 0.2 * draw(c)]
+        self.packed, self.at = _native.block_pack(c, dt, [(t, False) for t in self.w])
+
+    def rounded(self, t):
+        return t.to(self.dt).float()
+
+    def linear(self, x, i):
+        return self.rounded(F.linear(x, self.rounded(self.w[i]), self.rounded(self.b[i])))
+
+    def head(self, x):
+        y = self.rounded(F.layer_norm(x.float(), (self.c,), self.norm[0], self.norm[1]))
+        return torch.cat([self.linear(y, 0), self.linear(y, 1)], -1)
+
+    def tail(self, attn, x, scale=None):
+        s = 1.0 if scale is None else self.rounded(scale)[:, None, None]
+        x1 = (x.float() + self.rounded(self.linear(attn.float(), 2) * s)).to(x.dtype).float()
+        y = self.rounded(F.layer_norm(x1, (self.c,), self.norm[2], self.norm[3]))
+        h = self.rounded(F.gelu(F.linear(y, self.rounded(self.w[3]), self.rounded(self.b[3]))))
+        return x1 + self.rounded(self.linear(h, 4) * s)
+
+    def run_head(self, x):
+        return _native.norm_linear(x, self.norm[0], self.norm[1], 1e-5, self.packed, self.at[0], self.b[0], self.b[1],
+                                   3 * self.c)
+
+    def run_tail(self, attn, x, scale=None):
+        return _native.block_tail(attn, x, self.packed, self.at[2:], self.b[2], self.norm[2], self.norm[3], 1e-5, self.b[3],
+                                  self.b[4], scale)
+
+
+@pytest.mark.parametrize("dt,stream", CASES)
+@pytest.mark.parametrize("c,hidden,rows", SHAPES)
+def test_against_the_layers(device, dt, stream, c, hidden, rows):
+    block = Block(c, hidden, dt, device, c + rows)
+    gen = torch.Generator().manual_seed(rows)
+    x = (torch.randn(1, rows, c, generator=gen) * 2 + 0.5).to(device).to(stream)
+    attn = torch.randn(1, rows, c, generator=gen).to(device).to(dt)
+    got = block.run_head(x)
+    assert got.dtype == dt and got.shape == (1, rows, 3 * c)
+    assert oracle.rel_err(got.float(), block.head(x)) <= BAR[dt]
+    got = block.run_tail(attn, x)
+    assert got.dtype == stream and got.shape == x.shape
+    assert oracle.rel_err(got.float(), block.tail(attn, x)) <= BAR[dt]
+
+
+@pytest.mark.parametrize("dt,stream", CASES)
+def test_factors_of_the_images(device, dt, stream):
+    """Stochastic depth: a factor per image on both branches, 0 leaving the image's rows as they are."""
+    block = Block(64, 192, dt, device, 5)
+    gen = torch.Generator().manual_seed(6)
+    x = torch.randn(3, 37, 64, generator=gen).to(device).to(stream)
+    attn = torch.randn(3, 37, 64, generator=gen).to(device).to(dt)
+    scale = torch.tensor([1.25, 0.0, 1.25], device=device)
+    got = block.run_tail(attn, x, scale)
+    assert torch.equal(got[1], x[1])
+    assert oracle.rel_err(got.float(), block.tail(attn, x, scale)) <= BAR[dt]
+
+
+def test_gelu_of_every_fp16_number(device):
+    """With a norm of weight 0 the hidden layer is the norm's bias times the weights: identity weights bring every finite fp16
+    number to the GELU and its result to the output, at most one unit in the last place from the exactly rounded value."""
+    from scipy.special import ndtr
+    c, dt = 512, torch.float16
+    eye, zero = torch.eye(c, device=device), torch.zeros(c, device=device)
+    packed, at = _native.block_pack(c, dt, [(torch.zeros(c, c, device=device), False), (eye, False), (eye, False)])
+    values = np.arange(65536, dtype=np.uint16).view(np.float16)
+    values = values[np.isfinite(values)]
+    x = torch.zeros(1, 1, c, device=device, dtype=dt)
+    got = []
+    for v in np.split(values, len(values) // c):
+        bias = torch.from_numpy(v.astype(np.float32)).to(device)
+        got.append(_native.block_tail(x, x, packed, at, zero, zero, bias, 1e-5, zero, zero).reshape(-1))
+    got = torch.cat(got).cpu().numpy()
+    exact = (values.astype(np.float64) * ndtr(values.astype(np.float64))).astype(np.float16)
+    same_sign = np.signbit(got) == np.signbit(exact)
+    steps = np.abs(got.view(np.int16).astype(int) - exact.view(np.int16).astype(int))
+    assert ((steps <= 1) | ((got == 0) & (exact == 0))).all() and (same_sign | (got == 0)).all()
+    bias = torch.full((c,), float("nan"), device=device)
+    assert torch.isnan(_native.block_tail(x, x, packed, at, zero, zero, bias, 1e-5, zero, zero)).all()
+
+
+def test_what_is_refused(device):
+    block = Block(64, 192, torch.float16, device, 7)
+    x = torch.randn(2, 8, 64, device=device)
+    with pytest.raises(RuntimeError):
+        block.run_head(x.to(torch.bfloat16))                      # neither fp32 nor the weights' type
+    with pytest.raises(RuntimeError):
+        block.run_head(torch.randn(2, 8, 48, device=device))      # width without a kernel
+    with pytest.raises(RuntimeError):
+        block.run_tail(x, x)                                      # attn not of the weights' type
+    with pytest.raises(RuntimeError):
+        _native.block_pack(64, torch.float16, [(torch.randn(64, 40, device=device), False)])
