@@ -44,11 +44,24 @@ bool block_width_supported(int C) { return C == 32 || C == 64 || C == 128 || C =
 
 int block_group_channels(int C) { return C >= 128 ? 64 : 32; }
 
-int block_row_tiles(int elem_size, int C, int64_t rows) {
-    const int most = elem_size == 4 ? (C >= 512 ? 1 : 2) : (C >= 512 ? 2 : 4);
-    int tiles = most;
-    while (tiles > 1 && (rows + 16 * tiles - 1) / (16 * tiles) < 256) tiles /= 2;
-    return tiles;
+// 16-bit products are bound by the weights every workgroup streams from the L2 (0.9 MB at C = 256, H = 768): as many rows as
+// `most` allows, as long as half of the 256 compute units have a workgroup (tail, us with 4 / 2 / 1 tiles: 25 088 rows of 256
+// channels 44 / 54 / -, 9216 rows of 512 48 / 68 / 76, 6272 rows of 512 60 / 48 / 67, 1003 rows of 256 21 / 15 / 13).  fp32
+// products take sixteen times as long per weight and are bound by the compute unit that gets the most row tiles (9800 rows of
+// 256 channels: 129 us with 2 tiles, 307 workgroups, two of them on some units; 104 us with 1, 613, three on most).
+int block_row_tiles(int elem_size, int most, int64_t rows) {
+    int best = 1;
+    int64_t cost = 0;
+    for (int tiles = most; tiles >= 1; tiles /= 2) {
+        const int64_t groups = (rows + 16 * tiles - 1) / (16 * tiles);
+        if (elem_size == 2) {
+            if (groups >= 128 || tiles == 1) return tiles;
+        } else {
+            const int64_t here = (groups + 255) / 256 * tiles;
+            if (cost == 0 || here < cost) cost = here, best = tiles;
+        }
+    }
+    return best;
 }
 
 int launch_block_pack(const clusten_pack_item* items, int count, int C, int dtype, hipStream_t stream) {

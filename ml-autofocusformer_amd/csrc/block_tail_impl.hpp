@@ -28,6 +28,7 @@ template <typename T, typename S, int C, int TR>
 __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_kernel(BlockTailArgs a) {
     typedef BlockCfg<T, C> Cfg;
     constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, F = Cfg::kFrags, D = KS < 2 ? 1 : 2;
+    constexpr bool PARK = C > 64;
     __shared__ __attribute__((aligned(16))) Piece act[KS * TR * 64];
     __shared__ __attribute__((aligned(16))) Piece hid[KS * TR * 64];
     __shared__ float red[2 * WAVES * TR * 16];
@@ -66,8 +67,8 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
         F32x4 acc[NB][TR];
         bias_acc<T, NB, TR>(a.bp + wave * NB * 16, kq, acc);
         gemm_pass<T, TR, NB, KS, D>(wp, w1, lane * 16, wb, act + lane, acc);
-        // x1 waits for the end in the output buffer (every lane reads back what it wrote itself): its registers are worth
-        // more to the products between
+        // Wide rows: x1 waits for the end in the output buffer (every lane reads back what it wrote itself), its registers
+        // are worth more to the products between.  Up to 64 channels there are registers to spare and it is memory that counts.
 #pragma unroll
         for (int t = 0; t < TR; ++t) {
             const bool live = row0 + 16 * t + r16 < a.rows;
@@ -76,13 +77,22 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
                 float v[E];
                 results<NB, TR, E>(acc, f, t, v);
                 add_branch<T, S, E>(x[t][f], v, a.scale != nullptr, scale[t]);
-                if (live) store_values<S, E>(static_cast<S*>(a.out) + row[t] * C + ch0 + f * Cfg::kStep, x[t][f]);
+                if (PARK && live) store_values<S, E>(static_cast<S*>(a.out) + row[t] * C + ch0 + f * Cfg::kStep, x[t][f]);
                 if (live && a.x1) store_values<S, E>(static_cast<S*>(a.x1) + row[t] * C + ch0 + f * Cfg::kStep, x[t][f]);
             }
         }
     }
     float mean[TR], rstd[TR];
-    norm_to_fragments<T, C, TR>(a.norm_w, a.norm_b, a.eps, x, act, red, wave, lane, mean, rstd);
+    float y[TR][F][E];
+#pragma unroll
+    for (int t = 0; t < TR; ++t) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) y[t][f][e] = x[t][f][e];
+        }
+    }
+    norm_to_fragments<T, C, TR>(a.norm_w, a.norm_b, a.eps, y, act, red, wave, lane, mean, rstd);
     lds_barrier<WAVES>();
     if (a.x1) {
 #pragma unroll
@@ -125,7 +135,7 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
         gemm_pass<T, TR, NB, KS, D>(w2, w1, lane * 16, wb, hid + lane, acc2);
         w2 += (size_t)KS * NB * 64;
     }
-    {
+    if constexpr (PARK) {
         const S* rows[TR];
 #pragma unroll
         for (int t = 0; t < TR; ++t) rows[t] = static_cast<const S*>(a.out) + row[t] * C + ch0;
@@ -154,12 +164,17 @@ int launch_block_tail_tiles(const BlockTailArgs& a, hipStream_t stream) {
 
 template <typename T, typename S, int C>
 int launch_block_tail_width(const BlockTailArgs& a, hipStream_t stream) {
-    switch (block_row_tiles((int)sizeof(T), C, a.rows)) {
-        case 4:
-            if constexpr (sizeof(T) == 2) return launch_block_tail_tiles<T, S, C, 4>(a, stream);
-        case 2: return launch_block_tail_tiles<T, S, C, 2>(a, stream);
-        default: return launch_block_tail_tiles<T, S, C, 1>(a, stream);
+    // narrow rows are bound by memory and by their GELUs: more, smaller workgroups (2 tiles against 4: 98 against 110 us at
+    // 401 408 rows of 64 channels, 62 against 67 at 100 352 of 128); two fp32 tiles of 512 channels fill the LDS
+    constexpr int MOST = sizeof(T) == 4 ? (C > 256 ? 1 : 2) : (C > 128 ? 4 : 2);
+    const int tiles = block_row_tiles((int)sizeof(T), MOST, a.rows);
+    if constexpr (MOST >= 4) {
+        if (tiles == 4) return launch_block_tail_tiles<T, S, C, 4>(a, stream);
     }
+    if constexpr (MOST >= 2) {
+        if (tiles == 2) return launch_block_tail_tiles<T, S, C, 2>(a, stream);
+    }
+    return launch_block_tail_tiles<T, S, C, 1>(a, stream);
 }
 
 template <typename T, typename S>

@@ -286,8 +286,8 @@ struct BlockTailArgs {
     float2* stats;         // (rows)
 };
 bool block_width_supported(int C);
-// Tiles of 16 rows a workgroup takes (4, 2 or 1).
-int block_row_tiles(int elem_size, int C, int64_t rows);
+// Tiles of 16 rows a workgroup takes (4, 2 or 1, at most `most`).
+int block_row_tiles(int elem_size, int most, int64_t rows);
 // dst = a weight matrix of fp32 in the order the block kernels of width C read it in, as dtype.  src is (n,k), or (k,n)
 //   when transposed (dst is then that of its transpose); n a multiple of the width's group, k of the fragment.
 int block_group_channels(int C);

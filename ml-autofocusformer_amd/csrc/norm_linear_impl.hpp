@@ -31,19 +31,21 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void norm_linear_
         }
         load_rows<T, S, C, TR>(rows, x);
     }
-    const Piece* w = static_cast<const Piece*>(a.w) + (size_t)wave * KS * NB * 64;
+    // the workgroups of a row of the grid share the chunks of C output channels
+    const int first = a.chunks * blockIdx.y / gridDim.y, last = a.chunks * (blockIdx.y + 1) / gridDim.y;
+    const Piece* w = static_cast<const Piece*>(a.w) + ((size_t)first * WAVES + wave) * KS * NB * 64;
     Piece wb[D][NB];
     preload<NB, D>(w, lane * 16, wb);
     float mean[TR], rstd[TR];
     norm_to_fragments<T, C, TR>(a.norm_w, a.norm_b, a.eps, x, act, red, wave, lane, mean, rstd);
     lds_barrier<WAVES>();
-    if (a.stats && wave == 0 && kq == 0) {
+    if (a.stats && first == 0 && wave == 0 && kq == 0) {
 #pragma unroll
         for (int t = 0; t < TR; ++t) {
             if (row0 + 16 * t + r16 < a.rows) a.stats[row0 + 16 * t + r16] = float2{mean[t], rstd[t]};
         }
     }
-    if (a.normed) {
+    if (a.normed && first == 0) {
 #pragma unroll
         for (int t = 0; t < TR; ++t) {
             if (row0 + 16 * t + r16 < a.rows) {
@@ -55,10 +57,10 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void norm_linear_
             }
         }
     }
-    for (int chunk = 0; chunk < a.chunks; ++chunk) {
+    for (int chunk = first; chunk < last; ++chunk) {
         F32x4 acc[NB][TR];
         bias_acc<T, NB, TR>((chunk == 0 ? a.bias0 : a.bias1 + (size_t)(chunk - 1) * C) + wave * NB * 16, kq, acc);
-        const Piece* next = w + (chunk + 1 < a.chunks ? (size_t)WAVES * KS * NB * 64 : 0);
+        const Piece* next = w + (chunk + 1 < last ? (size_t)WAVES * KS * NB * 64 : 0);
         gemm_pass<T, TR, NB, KS, D>(w, next, lane * 16, wb, act + lane, acc);
         w = next;
 #pragma unroll
@@ -80,19 +82,26 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void norm_linear_
 template <typename T, typename S, int C, int TR>
 int launch_norm_linear_tiles(const NormLinearArgs& a, hipStream_t stream) {
     const int64_t groups = (a.rows + 16 * TR - 1) / (16 * TR);
-    hipLaunchKernelGGL((norm_linear_kernel<T, S, C, TR>), dim3((unsigned)groups), dim3(64 * BlockCfg<T, C>::kWaves), 0, stream,
+    // Few workgroups share the output chunks among them, each normalising its rows again: 17 -> 7 us for the 49 rows of 512
+    // channels of one image, 29 -> 27 us at 9216 rows of 512; at 25 088 rows of 256 (392 workgroups) 21.7 -> 23.5.  fp32
+    // products are long enough for it to pay up to a thousand (9800 rows of 256 channels, 613 workgroups: 50 -> 46 us).
+    const int split = groups < (sizeof(T) == 4 ? 1024 : 256) ? a.chunks : 1;
+    hipLaunchKernelGGL((norm_linear_kernel<T, S, C, TR>), dim3((unsigned)groups, (unsigned)split), dim3(64 * BlockCfg<T, C>::kWaves), 0, stream,
                        a);
     return launch_status();
 }
 
 template <typename T, typename S, int C>
 int launch_norm_linear_width(const NormLinearArgs& a, hipStream_t stream) {
-    switch (block_row_tiles((int)sizeof(T), C, a.rows)) {
-        case 4:
-            if constexpr (sizeof(T) == 2) return launch_norm_linear_tiles<T, S, C, 4>(a, stream);
-        case 2: return launch_norm_linear_tiles<T, S, C, 2>(a, stream);
-        default: return launch_norm_linear_tiles<T, S, C, 1>(a, stream);
+    constexpr int MOST = sizeof(T) == 4 ? 2 : 4;
+    const int tiles = block_row_tiles((int)sizeof(T), MOST, a.rows);
+    if constexpr (MOST >= 4) {
+        if (tiles == 4) return launch_norm_linear_tiles<T, S, C, 4>(a, stream);
     }
+    if constexpr (MOST >= 2) {
+        if (tiles == 2) return launch_norm_linear_tiles<T, S, C, 2>(a, stream);
+    }
+    return launch_norm_linear_tiles<T, S, C, 1>(a, stream);
 }
 
 template <typename T, typename S>
