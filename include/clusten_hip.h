@@ -649,6 +649,31 @@ int clusten_block_tail_forward(const void* attn, const void* x, int x_dtype, con
                                void* x1, void* normed, void* hidden, float* stats, int64_t rows, int C, int H, int dtype,
                                clusten_stream stream);
 
+/* `count` blocks one after the other (the inference forward of a stage's blocks, models/aff_transformer.py:488-490): per block
+ * clusten_norm_linear_forward, clusten_cluster_attention_forward_planned - or, when plan is NULL,
+ * clusten_dense_attention_forward with pe_idx (B,N,N), shape.M == shape.N <= 64 - and clusten_block_tail_forward, with the
+ * arguments and limits of those calls; x (B*N, H*C) of x_dtype is left as it is, out (same) may not overlap it.
+ *   blocks: `count` host structures of device pointers, weights packed for width H*C; bias_table (rows,H) of dtype;
+ *   blank_k, blank_v fp32 (H*C).  qkv (B*N, 3*H*C) and attn (B*N, H*C) of dtype: scratch.  hidden: channels of the hidden
+ *   layer, a multiple of H*C.  scale: of the query.  Enqueues 3 * count kernels on `stream`. */
+typedef struct {
+    const float *norm1_w, *norm1_b, *norm2_w, *norm2_b;
+    const void* w_qkv;
+    const float *b_q, *b_kv;
+    const void* w_proj;
+    const float* b_proj;
+    const void* w1;
+    const float* b1;
+    const void* w2;
+    const float* b2;
+    const void* bias_table;
+    const float *blank_k, *blank_v;
+    float eps1, eps2;
+} clusten_block;
+int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x, int x_dtype, void* out, void* qkv, void* attn,
+                           const void* plan, int lists_shared, const int64_t* pe_idx, clusten_attn_shape shape, int hidden,
+                           float scale, int dtype, clusten_stream stream);
+
 /* ---- producer of the neighbourhood lists (optional) ------------------------------------------- */
 
 /* K nearest neighbours of 2-D points inside each batch element: for query point q of batch element b,

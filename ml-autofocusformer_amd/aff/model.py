@@ -61,7 +61,11 @@ def default_ops():
                            block_pack=_native.block_pack, block_supported=_native.block_supported,
                            norm_linear=_native.norm_linear, block_tail=_native.block_tail,
                            block_stands_for=(("linear", _native.linear), ("layer_norm", _native.layer_norm),
-                                             ("add_layer_norm", _native.add_layer_norm)))
+                                             ("add_layer_norm", _native.add_layer_norm)),
+                           blocks_forward=_native.blocks_forward, block_params=_native.BlockParams,
+                           blocks_stand_for=(("cluster_attention", _native.cluster_attention),
+                                             ("dense_attention", _native.dense_attention),
+                                             ("norm_linear", _native.norm_linear), ("block_tail", _native.block_tail)))
 
 
 def _cast_params(lin, dt):
@@ -442,6 +446,18 @@ class ClusterTransformerBlock(nn.Module):
             return None
         return dt if all(getattr(ops, name, None) is fn for name, fn in ops.block_stands_for) else None
 
+    def tensors(self):
+        """The parameters of the block in one tuple, straight from the modules' tables: the look-ups of 30 blocks are a
+        visible part of a small forward's host time."""
+        m = self._modules
+        attn, mlp = m["attn"], m["mlp"]
+        n1, n2, a, ml, ap = m["norm1"]._parameters, m["norm2"]._parameters, attn._modules, mlp._modules, attn._parameters
+        q, kv, proj, pe = (a[k]._parameters for k in ("q", "kv", "proj", "pos_embed"))
+        f1, f2 = ml["fc1"]._parameters, ml["fc2"]._parameters
+        return (n1["weight"], n1["bias"], n2["weight"], n2["bias"], q["bias"], kv["bias"], proj["bias"], f1["bias"], f2["bias"],
+                ap["blank_k"], ap["blank_v"], q["weight"], kv["weight"], proj["weight"], f1["weight"], f2["weight"],
+                pe["weight"], pe["bias"])
+
     def _packed(self, dt):
         """(weights of the five Linear layers as the block kernels read them, byte offset of each), kept until one of
         them changes."""
@@ -640,6 +656,51 @@ class BasicLayer(nn.Module):
         ranking = self._grid_cache[key][1]
         return None if ranking is None else ranking[0, :, 0]
 
+    def _issue_blocks(self, feat, pe_idx, global_attn, table, lists):
+        """The stage's blocks through one call that issues all their kernels, or None when they go one by one: with
+        gradients, where a block would not take its three kernels (`_fused_dtype`), where the attention is not one kernel,
+        and when the caller's `ops` has another implementation of one of the pieces."""
+        ops = self.ops
+        first = self.blocks[0]
+        if getattr(ops, "blocks_forward", None) is None or torch.is_grad_enabled():
+            return None
+        dt = first._fused_dtype(feat)
+        b, n, c = feat.shape
+        h = first.attn.num_heads
+        if dt is None or c != 32 * h or any(getattr(ops, name, None) is not fn for name, fn in ops.blocks_stand_for):
+            return None
+        if self.training and any(blk._fused_dtype(feat) is None or blk.attn.attn_drop.p > 0 for blk in self.blocks):
+            return None
+        if global_attn:
+            if n > 64 or dt == torch.float32:
+                return None
+            plan = None
+        else:
+            plan = lists[3] if lists is not None and len(lists) > 3 else None
+            if plan is None or not (self.cluster_size == 8 or (self.cluster_size == 24 and dt != torch.float32)):
+                return None
+        tensors = [blk.tensors() for blk in self.blocks]
+        key = (dt, table.data_ptr(), table._version, table.dtype, [[(t._version, t.data_ptr()) for t in ts] for ts in tensors])
+        cache = self.__dict__.get("_issue_cache")
+        if cache is None or cache[0] != key:
+            if any(t.dtype != torch.float32 or not t.is_contiguous() or t.device != feat.device for ts in tensors for t in ts):
+                return None
+            params, held = (ops.block_params * len(tensors))(), [table]
+            for p, blk, ts in zip(params, self.blocks, tensors):
+                packed, at = blk._packed(dt)
+                bias = blk.attn.bias_table(table)
+                bias = bias.detach().to(dt).contiguous()
+                held += [packed, bias]
+                base = packed.data_ptr()
+                (p.norm1_w, p.norm1_b, p.norm2_w, p.norm2_b, p.b_q, p.b_kv, p.b_proj, p.b1, p.b2, p.blank_k,
+                 p.blank_v) = (t.data_ptr() for t in ts[:11])
+                p.w_qkv, p.w_proj, p.w1, p.w2 = (base + o for o in (at[0],) + tuple(at[2:]))
+                p.bias_table, p.eps1, p.eps2 = bias.data_ptr(), blk.norm1.eps, blk.norm2.eps
+            cache = (key, params, held)
+            self.__dict__["_issue_cache"] = cache     # a plain attribute, remade when a parameter changes
+        return ops.blocks_forward(cache[1], feat, h, first.mlp.fc1.out_features, dt, first.attn.scale, plan,
+                                  pe_idx if plan is None else None)
+
     def forward(self, pos, feat, h, w, on_grid, stride, table, radius, feat_ordered=False):
         """`feat_ordered`: the tokens already stand in the order `grid_order` gave (first stage only)."""
         b, n, d = pos.shape
@@ -700,7 +761,10 @@ class BasicLayer(nn.Module):
                 lists = grid_lists if grid_lists is not None else (cluster_idx, pe_idx, mask)
                 grid_lists = tuple(lists) + (planner(lists[0], lists[1], lists[2]), pairs)
         carry = None
-        for blk in self.blocks:
+        issued = self._issue_blocks(feat, pe_idx, global_attn, table, grid_lists)
+        if issued is not None:
+            feat = issued
+        for blk in self.blocks if issued is None else ():
             feat, carry = blk(feat, member_idx, mask, pe_idx, global_attn, table, cluster_idx, grid_lists, carry)
         learned_prob = None
         scorer = getattr(self.ops, "add_row_score", None)

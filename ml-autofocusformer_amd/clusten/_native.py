@@ -36,6 +36,13 @@ class PackItem(ctypes.Structure):
                                                                                                     "reserved")]
 
 
+class BlockParams(ctypes.Structure):
+    """clusten_block: the parameters of one transformer block (device pointers)."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("norm1_w", "norm1_b", "norm2_w", "norm2_b", "w_qkv", "b_q", "b_kv", "w_proj",
+                                                "b_proj", "w1", "b1", "w2", "b2", "bias_table", "blank_k", "blank_v")]
+                + [("eps1", ctypes.c_float), ("eps2", ctypes.c_float)])
+
+
 _P = ctypes.c_void_p
 _PROTOTYPES = {
     # name: (restype, argtypes)  — one entry per declaration in include/clusten_hip.h
@@ -124,6 +131,8 @@ _PROTOTYPES = {
     "clusten_block_tail_forward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_float, _P, _P, _P, _P, _P,
                                                  _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_int,
                                                  ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_blocks_forward": (ctypes.c_int, [ctypes.POINTER(BlockParams), ctypes.c_int, _P, ctypes.c_int, _P, _P, _P, _P,
+                                             ctypes.c_int, _P, AttnShape, ctypes.c_int, ctypes.c_float, ctypes.c_int, _P]),
     "clusten_knn2d": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
 }
 
@@ -194,12 +203,32 @@ def _strides(t: torch.Tensor) -> Strides:
     return Strides(t.stride(0), t.stride(1), t.stride(2))
 
 
-def _ptr(t) -> ctypes.c_void_p:
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
+def _ptr(t):
+    return t.data_ptr() if t is not None else None
 
 
-def _stream(device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device) -> int:
+    """The current stream of `device` as the handle the C ABI takes: the framework's raw getter, a tenth of the time of a
+    Stream object (a call of a small operator is host time: 3 us of its 17)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+class _Nothing:
+    __slots__ = ()
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NOTHING = _Nothing()
+
+
+def _on(device):
+    """`torch.cuda.device(device)`, which is only entered when `device` is not the current one."""
+    return _NOTHING if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def debug_indices() -> bool:
@@ -258,7 +287,7 @@ def qk_forward(query: torch.Tensor, key: torch.Tensor, nbhd_idx: torch.Tensor, _
     attn = torch.empty((shape.B, shape.H, shape.N, shape.M), dtype=query.dtype, device=device)
     if attn.numel() == 0:
         return attn
-    with torch.cuda.device(device):
+    with _on(device):
         fn = _entry or lib.clusten_qk_forward
         _check(fn(_ptr(query), _strides(query), _ptr(key), _strides(key), _ptr(idx), _ptr(attn), shape, code,
                   _stream(device)), "clusten_qk_forward")
@@ -283,7 +312,7 @@ def cluster_pairs(nbhd_idx: torch.Tensor, n_rows=None):
     idx = nbhd_idx.contiguous()
     device = idx.device
     block = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_cluster_pairs(_ptr(idx), _ptr(block), nbytes, B, rows, M, D, _stream(device)),
                "clusten_cluster_pairs")
     return block
@@ -305,7 +334,7 @@ def cluster_pairs_from_numbers(cluster_idx: torch.Tensor, n_rows=None):
     cidx = cluster_idx.contiguous()
     device = cidx.device
     block = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_cluster_pairs_from_numbers(_ptr(cidx), _ptr(block), nbytes, B, rows, nnc, D, _stream(device)),
                "clusten_cluster_pairs_from_numbers")
     return block
@@ -357,7 +386,7 @@ def scatter_rows_by_cluster(p: torch.Tensor, x: torch.Tensor, pair_lists: torch.
     if y.numel() == 0:
         return y
     shape = AttnShape(B, H, N, C, M)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_scatter_rows_by_cluster(_ptr(p), _ptr(x), _strides(x), _ptr(pair_lists), _ptr(y), shape,
                                                    code, _stream(device)),
                "clusten_scatter_rows_by_cluster")
@@ -388,7 +417,7 @@ def scatter_rows(p: torch.Tensor, x: torch.Tensor, nbhd_idx: torch.Tensor, pair_
             raise RuntimeError("scatter_rows: pair_lists does not belong to lists of this shape (cluster_pairs)")
     ws_bytes = lib.clusten_scatter_rows_workspace_bytes(shape, code)
     ws = _workspace(ws_bytes, device)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_scatter_rows(_ptr(p), _ptr(x), _strides(x), _ptr(idx), _ptr(pair_lists), _ptr(y), _ptr(ws),
                                         ws_bytes, shape, code, _stream(device)), "clusten_scatter_rows")
     return y
@@ -415,7 +444,7 @@ def qk_backward(d_attn: torch.Tensor, query: torch.Tensor, key: torch.Tensor, nb
         return d_query.zero_(), d_key.zero_()
     ws_bytes = lib.clusten_qk_backward_workspace_bytes(shape, code)
     ws = _workspace(ws_bytes, device)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_qk_backward(_ptr(d_attn), _ptr(query), _strides(query), _ptr(key), _strides(key), _ptr(idx),
                                        _ptr(d_query), _ptr(d_key), _ptr(ws), ws_bytes, shape, code, _stream(device)),
                "clusten_qk_backward")
@@ -444,7 +473,7 @@ def qk_backward_static(d_attn: torch.Tensor, query: torch.Tensor, key: torch.Ten
         raise RuntimeError("qk_backward_static copies nothing: d_attn and nbhd_idx contiguous, rows with channel stride 1")
     if d_query.numel() == 0 or shape.M == 0:
         raise RuntimeError("qk_backward_static: empty problem")
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_qk_backward_static(_ptr(d_attn), _ptr(query), _strides(query), _ptr(key), _strides(key),
                                               _ptr(idx), _ptr(d_query), _ptr(d_key), shape, code, _stream(device)),
                "clusten_qk_backward_static")
@@ -477,7 +506,7 @@ def av_forward(attn: torch.Tensor, v: torch.Tensor, nbhd_idx: torch.Tensor, toke
         return feat
     if shape.M == 0:
         return feat.zero_()
-    with torch.cuda.device(device):
+    with _on(device):
         fn = _entry or lib.clusten_av_forward
         _check(fn(_ptr(attn), _ptr(v), _strides(v), _ptr(idx), _ptr(feat), _strides(feat), shape, code, _stream(device)),
                "clusten_av_forward")
@@ -514,7 +543,7 @@ def av_forward_mixed(attn: torch.Tensor, v: torch.Tensor, nbhd_idx: torch.Tensor
         return feat
     if shape.M == 0:
         return feat.zero_()
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_av_forward_mixed(_ptr(attn), _ptr(v), _strides(v), _DTYPE_CODE[v.dtype], _ptr(idx), _ptr(feat),
                                             _strides(feat), shape, _stream(device)), "clusten_av_forward_mixed")
     return feat
@@ -539,7 +568,7 @@ def av_backward(d_feat: torch.Tensor, attn: torch.Tensor, v: torch.Tensor, nbhd_
         return d_attn.zero_(), d_v.zero_()
     ws_bytes = lib.clusten_av_backward_workspace_bytes(shape, code)
     ws = _workspace(ws_bytes, device)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_av_backward(_ptr(d_feat), _strides(d_feat), _ptr(attn), _ptr(v), _strides(v), _ptr(idx),
                                        _ptr(d_attn), _ptr(d_v), _ptr(ws), ws_bytes, shape, code, _stream(device)),
                "clusten_av_backward")
@@ -572,7 +601,7 @@ def wf_forward(weights: torch.Tensor, feat: torch.Tensor, nbhd_idx: torch.Tensor
         return out
     if shape.M == 0 or shape.N == 0:
         return out.zero_()
-    with torch.cuda.device(device):
+    with _on(device):
         fn = _entry or lib.clusten_wf_forward
         _check(fn(_ptr(weights), _ptr(feat), _ptr(idx), _ptr(out), shape, code, _stream(device)), "clusten_wf_forward")
     return out
@@ -600,7 +629,7 @@ def wf_forward_mixed(weights: torch.Tensor, feat: torch.Tensor, nbhd_idx: torch.
         return out
     if M == 0 or N == 0:
         return out.zero_()
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_wf_forward_mixed(_ptr(weights), _ptr(feat), _DTYPE_CODE[feat.dtype], _ptr(idx), _ptr(out), shape,
                                             _stream(device)), "clusten_wf_forward_mixed")
     return out
@@ -620,7 +649,7 @@ def wf_backward(d_feat_new: torch.Tensor, weights: torch.Tensor, feat: torch.Ten
         return d_weights.zero_(), d_feat.zero_()
     ws_bytes = lib.clusten_wf_backward_workspace_bytes(shape, code)
     ws = _workspace(ws_bytes, device)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_wf_backward(_ptr(d_feat_new), _ptr(weights), _ptr(feat), _ptr(idx), _ptr(d_weights),
                                        _ptr(d_feat), _ptr(ws), ws_bytes, shape, code, _stream(device)),
                "clusten_wf_backward")
@@ -642,7 +671,7 @@ def wf_backward_by_cluster(d_feat_new: torch.Tensor, weights: torch.Tensor, feat
     d_feat_new, weights, feat = d_feat_new.contiguous(), weights.contiguous(), feat.contiguous()
     d_weights = torch.empty_like(weights)
     d_feat = torch.empty_like(feat) if d_feat is None else d_feat
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_wf_backward_by_cluster(_ptr(d_feat_new), _ptr(weights), _ptr(feat), _ptr(idx), _ptr(pair_lists),
                                                   _ptr(d_weights), _ptr(d_feat), shape, code, _stream(device)),
                "clusten_wf_backward_by_cluster")
@@ -697,7 +726,7 @@ def qk_forward_clusters(query: torch.Tensor, key: torch.Tensor, cluster_idx: tor
     attn = torch.empty((B, H, N, shape.M), dtype=query.dtype, device=device)
     if attn.numel() == 0:
         return attn
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_qk_forward_clusters(_ptr(query), _strides(query), _ptr(key), _strides(key), _ptr(cidx),
                                                _ptr(attn), shape, _dtype_code(query, "query"), _stream(device)),
                "clusten_qk_forward_clusters")
@@ -721,7 +750,7 @@ def av_forward_clusters(attn: torch.Tensor, v: torch.Tensor, cluster_idx: torch.
     feat = torch.empty((B, H, N, C), dtype=attn.dtype, device=device)
     if feat.numel() == 0:
         return feat
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_av_forward_clusters(_ptr(attn), _ptr(v), _strides(v), _ptr(cidx), _ptr(feat), _strides(feat),
                                                shape, _dtype_code(attn, "attn"), _stream(device)),
                "clusten_av_forward_clusters")
@@ -783,7 +812,7 @@ def attn_softmax(attn: torch.Tensor, bias_table: torch.Tensor, pe_idx: torch.Ten
     if probs.numel() == 0:
         return probs, blank_prob
     shape = AttnShape(b, h, n, c, m)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_attn_softmax_forward(_ptr(attn), _ptr(bias_table), _ptr(pe_idx), _ptr(mask),
                                                 _ptr(blank_logit), _ptr(query), qs, _ptr(blank_key), _ptr(probs),
                                                 _ptr(blank_prob), shape, code, _stream(device)),
@@ -811,7 +840,7 @@ def attn_softmax_backward(probs: torch.Tensor, blank_prob: torch.Tensor, d_probs
     d_blank_logit = torch.empty(b, h, n, 1, dtype=torch.float32, device=device)
     if d_logit.numel() == 0:
         return d_logit, d_blank_logit
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_attn_softmax_backward(_ptr(probs), _ptr(blank_prob), _ptr(d_probs), _ptr(d_blank_prob),
                                                  _ptr(d_logit), _ptr(d_blank_logit), b * h * n, m,
                                                  _DTYPE_CODES[logit_dtype], _stream(device)),
@@ -851,7 +880,7 @@ def cluster_attention_plan(cluster_idx: torch.Tensor, pe_idx: torch.Tensor, mask
     nbytes = lib.clusten_cluster_attention_plan_bytes(lb, n, m)
     plan = torch.empty(nbytes, dtype=torch.uint8, device=device)
     if nbytes:
-        with torch.cuda.device(device):
+        with _on(device):
             _check(lib.clusten_cluster_attention_plan(_ptr(cidx), _ptr(pe_idx), _ptr(mask), _ptr(plan), nbytes, lb, n, m,
                                                       _stream(device)), "clusten_cluster_attention_plan")
     return plan
@@ -928,7 +957,7 @@ def cluster_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tenso
         if plan is None:
             raise RuntimeError("return_lse needs a plan")
         lse = torch.empty(b, h, n, dtype=torch.float32, device=device)
-        with torch.cuda.device(device):
+        with _on(device):
             _check(lib.clusten_cluster_attention_forward_train(_ptr(query), _strides(query), _ptr(key), _strides(key),
                                                                _ptr(value), _strides(value), _ptr(plan), _ptr(bias_table),
                                                                int(shared), _ptr(blank_key), _ptr(blank_value), _ptr(out),
@@ -937,7 +966,7 @@ def cluster_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tenso
                    "clusten_cluster_attention_forward_train")
         return out.reshape(b, n, h * c), lse
     if plan is not None:
-        with torch.cuda.device(device):
+        with _on(device):
             _check(lib.clusten_cluster_attention_forward_planned(_ptr(query), _strides(query), _ptr(key), _strides(key),
                                                                  _ptr(value), _strides(value), _ptr(plan), _ptr(bias_table),
                                                                  int(shared), _ptr(blank_key), _ptr(blank_value), _ptr(out),
@@ -945,7 +974,7 @@ def cluster_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tenso
                                                                  _stream(device)),
                    "clusten_cluster_attention_forward_planned")
         return out.reshape(b, n, h * c)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_cluster_attention_forward(_ptr(query), _strides(query), _ptr(key), _strides(key),
                                                      _ptr(value), _strides(value), _ptr(cidx), _ptr(bias_table),
                                                      _ptr(pe_idx), _ptr(mask), int(shared), _ptr(blank_key),
@@ -1007,7 +1036,7 @@ def cluster_attention_backward(query: torch.Tensor, key: torch.Tensor, value: to
     d_blank = torch.empty(b, h, n, dtype=torch.float32, device=device)
     if probs.numel() == 0:
         return d_query, probs, d_logit, blank_prob, d_blank
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_cluster_attention_backward(_ptr(query), _strides(query), _ptr(key), _strides(key), _ptr(value),
                                                       _strides(value), _ptr(g_view), _strides(g_view), _ptr(out_view),
                                                       _strides(out_view), _ptr(lse.contiguous()), _ptr(plan),
@@ -1063,7 +1092,7 @@ def dense_attention(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
         return out.reshape(b, n, h * c)
     out_view = out.permute(0, 2, 1, 3)                                   # (B,H,N,C) view of the (B,N,H,C) memory
     shape = AttnShape(b, h, n, c, n)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_dense_attention_forward(_ptr(query), _strides(query), _ptr(key), _strides(key), _ptr(value),
                                                    _strides(value), _ptr(bias_table), _ptr(pe_idx), _ptr(blank_key),
                                                    _ptr(blank_value), _ptr(out), _strides(out_view),
@@ -1116,7 +1145,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias, gelu: bool = False) -> t
     out = torch.empty(x.shape[:-1] + (nout,), dtype=x.dtype, device=device)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_linear_forward(_ptr(x2), x2.stride(0), _ptr(weight), _ptr(bias), _ptr(out), x2.shape[0], k,
                                           nout, int(bool(gelu)), code, _stream(device)),
                "clusten_linear_forward")
@@ -1158,7 +1187,7 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: f
     if out.numel() == 0:
         return out
     if order is None and pre_bias is None:
-        with torch.cuda.device(device):
+        with _on(device):
             _check(lib.clusten_layer_norm_forward(_ptr(x), _DTYPE_CODES[x.dtype], _ptr(weight), _ptr(bias), _ptr(out),
                                                   x.numel() // c, c,
                                                   ctypes.c_float(eps), _DTYPE_CODES[out_dtype], _stream(device)),
@@ -1176,7 +1205,7 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: f
         if pre_bias.numel() != c:
             raise RuntimeError("pre_bias must have as many elements as the last axis of x")
         pre_bias = pre_bias.detach().to(x.dtype).contiguous()
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_layer_norm_rows_forward(_ptr(x), _DTYPE_CODES[x.dtype], _ptr(order), group, _ptr(pre_bias),
                                                    _ptr(weight), _ptr(bias), _ptr(out), x.numel() // c, c,
                                                    ctypes.c_float(eps), _DTYPE_CODES[out_dtype], _stream(device)),
@@ -1209,7 +1238,7 @@ def channel_affine_gelu(x: torch.Tensor, scale: torch.Tensor, shift: torch.Tenso
     out = torch.empty_like(x)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_channel_affine_gelu_forward(_ptr(x), _ptr(scale), _ptr(shift), _ptr(out), b, c, h * w,
                                                        _DTYPE_CODES[x.dtype], _stream(device)),
                "clusten_channel_affine_gelu_forward")
@@ -1247,7 +1276,7 @@ def add_layer_norm(x: torch.Tensor, branch: torch.Tensor, weight: torch.Tensor, 
     out = torch.empty(x.shape, dtype=branch.dtype, device=device)
     if out.numel() == 0:
         return total, out
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_add_layer_norm_forward(_ptr(x), _DTYPE_CODES[x.dtype], _ptr(branch), _DTYPE_CODES[branch.dtype],
                                                   _ptr(total), _ptr(weight), _ptr(bias), _ptr(out), x.numel() // c, c,
                                                   ctypes.c_float(eps), _stream(device)),
@@ -1281,7 +1310,7 @@ def neighbour_lists(pos: torch.Tensor, nearest: torch.Tensor, m: int, radius: in
     cluster_idx = torch.empty(b, n, nnc, dtype=torch.int32, device=device)
     if member_idx.numel() == 0:
         return member_idx, mask, pe_idx, cluster_idx
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_neighbour_lists(_ptr(pos), _ptr(nearest), _ptr(member_idx), _ptr(mask), _ptr(pe_idx),
                                            _ptr(cluster_idx), b, n, nnc, m, int(radius), int(table_width),
                                            _stream(device)),
@@ -1329,7 +1358,7 @@ def add_row_score(x: torch.Tensor, branch, weight: torch.Tensor, bias):
     score = torch.empty(x.shape[:-1] + (1,), dtype=weight.dtype, device=device)
     if score.numel() == 0:
         return total, score
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_add_row_score_forward(_ptr(x), _DTYPE_CODES[x.dtype], _ptr(branch),
                                                  _ptr(total) if branch is not None else None, _ptr(weight), _ptr(bias),
                                                  _ptr(score), x.numel() // c, c, code, _stream(device)),
@@ -1358,7 +1387,7 @@ def bias_table_grad(d_logit: torch.Tensor, pe_idx: torch.Tensor, rows: int) -> t
     d_table = torch.zeros(rows, H, dtype=torch.float32, device=device)
     if d_logit.numel() == 0:
         return d_table
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_bias_table_grad(_ptr(d_logit), _ptr(pe_idx), _ptr(d_table), B, H, N, M, rows,
                                            _DTYPE_CODES[d_logit.dtype], _stream(device)),
                "clusten_bias_table_grad")
@@ -1396,7 +1425,7 @@ def merge_weights(table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: t
     out = torch.empty(b, n_out, m, table_weights.shape[1], dtype=torch.float32, device=device)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_merge_weights_forward(_ptr(table_weights), _ptr(pe_idx.contiguous()),
                                                  _ptr(nbhd_idx.contiguous()), _ptr(prob), _ptr(mask), _ptr(out), b, n,
                                                  n_out, m, table_weights.shape[1], _stream(device)),
@@ -1409,7 +1438,7 @@ def scanline_rank_supported(pos: torch.Tensor, rows: int, cols: int) -> bool:
     that one compute unit's LDS sorts (16384 tokens on an MI355X)."""
     if not (pos.is_cuda and pos.dim() == 3 and pos.shape[2] == 2 and pos.shape[1] > 0 and rows * cols >= 2):
         return False
-    with torch.cuda.device(pos.device):
+    with _on(pos.device):
         return pos.shape[1] <= load().clusten_scanline_rank_max_tokens()
 
 
@@ -1429,7 +1458,7 @@ def cluster_centres(pos: torch.Tensor, ranking: torch.Tensor, m: int):
     pos_sorted = torch.empty_like(pos)
     centres = torch.empty(b, k, 2, dtype=torch.float32, device=device)
     if pos.numel():
-        with torch.cuda.device(device):
+        with _on(device):
             _check(lib.clusten_cluster_centres(_ptr(pos), _ptr(ranking), _ptr(pos_sorted), _ptr(centres), b, n, m,
                                                _stream(device)), "clusten_cluster_centres")
     return pos_sorted, centres
@@ -1456,7 +1485,7 @@ def gather_rows(x: torch.Tensor, order: torch.Tensor) -> torch.Tensor:
     x = x.detach().contiguous()
     order = order.contiguous()
     out = torch.empty_like(x)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_gather_rows(_ptr(x), _ptr(order), _ptr(out), b, n, c * x.element_size(), int(shared),
                                        _stream(device)), "clusten_gather_rows")
     return out
@@ -1498,7 +1527,7 @@ def merge_centres(pos: torch.Tensor, min_dist, learned_prob, alpha: float, strid
         learned_prob = learned_prob.detach().contiguous()
         code = _DTYPE_CODES[learned_prob.dtype]
     centre = torch.empty(b, sample_num + (reserve_num if reserve_on else 0), dtype=torch.int64, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_merge_centres(_ptr(pos), _ptr(min_dist), _ptr(learned_prob), code, _ptr(centre), b, n,
                                          sample_num, reserve_num, int(bool(reserve_on)), ctypes.c_float(alpha),
                                          stride, _stream(device)), "clusten_merge_centres")
@@ -1542,7 +1571,7 @@ def merge_rows(centre: torch.Tensor, *tensors):
     srcs = (ctypes.c_void_p * k)(*[t.data_ptr() for t in src])
     dsts = (ctypes.c_void_p * k)(*[t.data_ptr() for t in dst])
     sizes = (ctypes.c_int * k)(*[t.shape[2] * t.element_size() for t in src])
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_merge_rows(srcs, dsts, sizes, k, _ptr(centre), b, n, n_out, _stream(device)),
                "clusten_merge_rows")
     return tuple(dst)
@@ -1563,7 +1592,7 @@ def scanline_rank(pos: torch.Tensor, rows: int, cols: int, cell_w: float, cell_h
         return ranking
     nbytes = lib.clusten_scanline_rank_workspace_bytes(b, n)
     workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_scanline_rank(_ptr(pos), _ptr(ranking), _ptr(workspace), nbytes, b, n, rows, cols,
                                          ctypes.c_float(cell_w), ctypes.c_float(cell_h), _stream(device)),
                "clusten_scanline_rank")
@@ -1592,7 +1621,7 @@ def knn2d(query: torch.Tensor, database: torch.Tensor, k: int, return_dist: bool
     idx = torch.empty(b, nq, k, dtype=torch.int64, device=device)
     dist = torch.empty(b, nq, k, dtype=torch.float32, device=device) if return_dist else None
     if idx.numel():
-        with torch.cuda.device(device):
+        with _on(device):
             _check(lib.clusten_knn2d(_ptr(query), _ptr(database), _ptr(idx), _ptr(dist), b, nq, n, k, _stream(device)),
                    "clusten_knn2d")
     return (idx, dist) if return_dist else idx
@@ -1627,7 +1656,7 @@ def block_pack(width: int, dtype: torch.dtype, weights):
         n, k = w.shape
         it.src, it.dst, it.transposed = w.data_ptr(), out.data_ptr() + at * size, int(bool(transposed))
         it.n, it.k = (k, n) if transposed else (n, k)
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_block_pack(items, len(weights), width, _DTYPE_CODES[dtype], _stream(device)), "clusten_block_pack")
     return out, [at * size for at in offsets]
 
@@ -1649,7 +1678,7 @@ def norm_linear(x: torch.Tensor, norm_w, norm_b, eps: float, packed: torch.Tenso
     out = torch.empty(x.shape[:-1] + (n_out,), dtype=packed.dtype, device=device)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(device):
+    with _on(device):
         _check(lib.clusten_norm_linear_forward(x.data_ptr(), _DTYPE_CODES[x.dtype], norm_w.data_ptr(), norm_b.data_ptr(), eps,
                                                packed.data_ptr() + w_at, bias0.data_ptr(), bias1.data_ptr(),
                                                out.data_ptr(), None, None, x.numel() // c, c, n_out,
@@ -1677,7 +1706,7 @@ def block_tail(attn: torch.Tensor, x: torch.Tensor, packed: torch.Tensor, at, bi
     out = torch.empty_like(x)
     if out.numel() == 0:
         return out
-    with torch.cuda.device(device):
+    with _on(device):
         base = packed.data_ptr()
         _check(lib.clusten_block_tail_forward(attn.data_ptr(), x.data_ptr(), _DTYPE_CODES[x.dtype], base + at[0],
                                               bias_p.data_ptr(), norm_w.data_ptr(), norm_b.data_ptr(), eps, base + at[1],
@@ -1685,4 +1714,42 @@ def block_tail(attn: torch.Tensor, x: torch.Tensor, packed: torch.Tensor, at, bi
                                               None if scale is None else scale.data_ptr(), x.numel() // c // x.shape[0],
                                               None, None, None, None, x.numel() // c, c, hidden,
                                               _DTYPE_CODES[packed.dtype], _stream(device)), "clusten_block_tail_forward")
+    return out
+
+
+def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torch.dtype, scale: float, plan=None, pe_idx=None):
+    """The transformer blocks of a stage one after the other, issued by one call: `params` is a ctypes array of BlockParams
+    (what it points at is the caller's to keep), x (B,N,C) the token rows with C = 32 * heads.  Local attention with the
+    lists `plan` was built from (`cluster_attention_plan`), or, with `pe_idx` (B,N,N) instead, attention over all N <= 64
+    tokens.  The same kernels as `norm_linear`, `cluster_attention` / `dense_attention` and `block_tail` block by block.  No
+    autograd: for inference."""
+    lib = load()
+    _require_cuda("x", x)
+    device = x.device
+    b, n, c = x.shape
+    if not block_supported(x, dtype, hidden) or c != 32 * heads:
+        raise RuntimeError("blocks_forward takes contiguous (B,N,32*heads) rows of a built width, fp32 or of the weights' dtype")
+    if plan is not None:
+        _require_cuda("plan", plan, device)
+        fits = [(lb, m) for m in (48, 144) for lb in (b, 1)
+                if plan.numel() == lib.clusten_cluster_attention_plan_bytes(lb, n, m)]
+        if plan.dtype != torch.uint8 or not fits:
+            raise RuntimeError("plan does not belong to lists of this shape")
+        lb, m = fits[0]
+    else:
+        _require_cuda("pe_idx", pe_idx, device)
+        if pe_idx.shape != (b, n, n) or pe_idx.dtype != torch.int64 or n > 64 or dtype == torch.float32:
+            raise RuntimeError("pe_idx must be int64 of shape (B,N,N), N <= 64, and the blocks fp16 / bf16")
+        pe_idx = pe_idx.contiguous()
+        lb, m = b, n
+    out = torch.empty_like(x)
+    if out.numel() == 0 or len(params) == 0:
+        return x
+    scratch = torch.empty(b * n * 4 * c, dtype=dtype, device=device)         # q | k, v rows and the attention's output
+    with _on(device):
+        at = scratch.data_ptr()
+        _check(lib.clusten_blocks_forward(params, len(params), x.data_ptr(), _DTYPE_CODES[x.dtype], out.data_ptr(), at,
+                                          at + b * n * 3 * c * scratch.element_size(), _ptr(plan), int(b != 1 and lb == 1),
+                                          _ptr(pe_idx), AttnShape(b, heads, n, 32, m), hidden, scale, _DTYPE_CODES[dtype],
+                                          _stream(device)), "clusten_blocks_forward")
     return out

@@ -640,4 +640,44 @@ int clusten_block_tail_forward(const void* attn, const void* x, int x_dtype, con
     return launch_block_tail(a, x_dtype, C, dtype, as_stream(stream));
 }
 
+int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x, int x_dtype, void* out, void* qkv, void* attn,
+                           const void* plan, int lists_shared, const int64_t* pe_idx, clusten_attn_shape shape, int hidden,
+                           float scale, int dtype, clusten_stream stream) {
+    if (!blocks || !x || !out || !qkv || !attn || (!plan && !pe_idx)) return CLUSTEN_ERR_NULL_POINTER;
+    if (count <= 0) return CLUSTEN_ERR_BAD_DIMS;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (int st = check_attn_shape(shape)) return st;
+    const int C = shape.H * shape.C;
+    const int64_t rows = (int64_t)shape.B * shape.N;
+    const size_t elem = dtype_size(dtype);
+    // q, k and v inside the rows of the projections' output: [q | head 0: k v | head 1: k v ...]
+    clusten_strides qs, kv, os;
+    qs.b = (int64_t)shape.N * 3 * C, qs.n = 3 * C, qs.h = shape.C;
+    kv = qs, kv.h = 2 * shape.C;
+    os.b = (int64_t)shape.N * C, os.n = C, os.h = shape.C;
+    char* q = static_cast<char*>(qkv);
+    char* k = q + (size_t)C * elem;
+    char* v = k + (size_t)shape.C * elem;
+    for (int i = 0; i < count; ++i) {
+        const clusten_block& b = blocks[i];
+        const void* in = i == 0 ? x : out;
+        if (int st = clusten_norm_linear_forward(in, x_dtype, b.norm1_w, b.norm1_b, b.eps1, b.w_qkv, b.b_q, b.b_kv, qkv, nullptr,
+                                                 nullptr, rows, C, 3 * C, dtype, stream)) {
+            return st;
+        }
+        const int st = plan ? clusten_cluster_attention_forward_planned(q, qs, k, kv, v, kv, plan, b.bias_table, lists_shared,
+                                                                        b.blank_k, b.blank_v, attn, os, scale, shape, dtype, stream)
+                            : clusten_dense_attention_forward(q, qs, k, kv, v, kv, b.bias_table, pe_idx, b.blank_k, b.blank_v,
+                                                              attn, os, scale, shape, dtype, stream);
+        if (st) return st;
+        // a workgroup of the tail reads its own rows only, all of them before it writes the first: in place from block 1 on
+        if (int st2 = clusten_block_tail_forward(attn, in, x_dtype, b.w_proj, b.b_proj, b.norm2_w, b.norm2_b, b.eps2, b.w1, b.b1,
+                                                 b.w2, b.b2, out, nullptr, 1, nullptr, nullptr, nullptr, nullptr, rows, C, hidden,
+                                                 dtype, stream)) {
+            return st2;
+        }
+    }
+    return CLUSTEN_OK;
+}
+
 }  // extern "C"

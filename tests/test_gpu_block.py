@@ -127,3 +127,30 @@ def test_what_is_refused(device):
         block.run_tail(x, x)                                      # attn not of the weights' type
     with pytest.raises(RuntimeError):
         _native.block_pack(64, torch.float16, [(torch.randn(64, 40, device=device), False)])
+
+
+@pytest.mark.parametrize("amp", [torch.float16, torch.bfloat16, None])
+def test_blocks_issued_by_one_call_equal_the_blocks_one_by_one(device, amp):
+    """Local stages with shared and with per-image lists, short last clusters and masks (196 tokens), and the global stage of
+    49 tokens: the same kernels on the same values, so bit for bit, and again after a parameter changed in place."""
+    from aff.model import aff_tiny, default_ops
+    torch.manual_seed(0)
+    net = aff_tiny().to(device).eval()
+    single_ops = default_ops()
+    del single_ops.blocks_forward
+    single = aff_tiny(ops=single_ops).to(device).eval()
+    single.load_state_dict(net.state_dict())
+    x = torch.randn(3, 3, 224, 224, generator=torch.Generator().manual_seed(1)).to(device)
+
+    def run(m):
+        with torch.no_grad(), torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+            return m(x)
+
+    first = run(net)
+    assert torch.isfinite(first).all() and torch.equal(first, run(single))
+    with torch.no_grad():
+        for m in (net, single):
+            m.layers[2].blocks[4].mlp.fc1.weight.mul_(1.5)
+            m.layers[1].blocks[0].attn.pos_embed.bias.add_(0.25)
+    second = run(net)
+    assert not torch.equal(first, second) and torch.equal(second, run(single))
