@@ -674,6 +674,21 @@ int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x
                            const void* plan, int lists_shared, const int64_t* pe_idx, clusten_attn_shape shape, int hidden,
                            float scale, int dtype, clusten_stream stream);
 
+/* Parameter gradients of Linear layers over the same `rows` token rows: d_weight (n,k) = d_y^T x and d_bias (n) = the column
+ * sums of d_y (d_bias NULL: none), fp32, written in full.  d_y (rows,n) and x (rows,k) of dtype (F32, F16, BF16) with row
+ * strides in elements; rows, bases and fp32 results on 16-byte boundaries; n and k multiples of 8; 1 <= count <= 8.  Sums are
+ * fp32 in a fixed order.  workspace: clusten_weight_grad_workspace_bytes(...) bytes of device memory (0: not supported).  The
+ * backward of the Linear layers of models/aff_transformer.py:103-106,157,181-196, which the reference leaves to autograd. */
+typedef struct {
+    const void *d_y, *x;
+    float *d_weight, *d_bias;
+    int64_t d_y_stride, x_stride;
+    int32_t n, k;
+} clusten_weight_grad_item;
+size_t clusten_weight_grad_workspace_bytes(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype);
+int clusten_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, void* workspace, size_t workspace_bytes,
+                        int dtype, clusten_stream stream);
+
 /* ---- producer of the neighbourhood lists (optional) ------------------------------------------- */
 
 /* K nearest neighbours of 2-D points inside each batch element: for query point q of batch element b,

@@ -25,6 +25,7 @@ from types import SimpleNamespace
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules import module as _module
 
 from .points import knn, space_filling_cluster
 
@@ -62,10 +63,59 @@ def default_ops():
                            norm_linear=_native.norm_linear, block_tail=_native.block_tail,
                            block_stands_for=(("linear", _native.linear), ("layer_norm", _native.layer_norm),
                                              ("add_layer_norm", _native.add_layer_norm)),
+                           weight_grad=_native.weight_grad, weight_grad_supported=_native.weight_grad_supported,
                            blocks_forward=_native.blocks_forward, block_params=_native.BlockParams,
                            blocks_stand_for=(("cluster_attention", _native.cluster_attention),
                                              ("dense_attention", _native.dense_attention),
                                              ("norm_linear", _native.norm_linear), ("block_tail", _native.block_tail)))
+
+
+class _Linear(torch.autograd.Function):
+    """`F.linear(x, weight, bias)` in x's dtype for parameters of any, with the parameters' gradients from the library's kernel:
+    both in one pass over the rows, in fp32 (not rounded to 16 bits on the way to fp32 parameters)."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, grad_kernel, supported):
+        ctx.save_for_backward(x, weight)
+        ctx.meta = (None if bias is None else bias.dtype, grad_kernel, supported)
+        return F.linear(x, weight.to(x.dtype), None if bias is None else bias.to(x.dtype))
+
+    @staticmethod
+    def backward(ctx, d_y):
+        x, weight = ctx.saved_tensors
+        bias_dtype, grad_kernel, supported = ctx.meta
+        need_x, need_w, need_b = ctx.needs_input_grad[:3]
+        d_x = d_y @ weight.to(x.dtype) if need_x else None
+        rows, x_rows = d_y.reshape(-1, d_y.shape[-1]), x.reshape(-1, x.shape[-1])
+        if need_w and not torch.is_grad_enabled():       # (a backward that is itself recorded stays with recorded operations)
+            if not supported(rows, x_rows):
+                rows = rows.contiguous()                 # e.g. the gradient of a column range
+            if supported(rows, x_rows):
+                (d_w, d_b), = grad_kernel([(rows, x_rows, need_b)])
+                return d_x, d_w.to(weight.dtype), None if d_b is None else d_b.to(bias_dtype), None, None
+        return (d_x, (rows.t() @ x_rows).to(weight.dtype) if need_w else None, rows.sum(0).to(bias_dtype) if need_b else None,
+                None, None)
+
+
+def _hooked(mod):
+    """True when calling `mod` runs more than its `forward`."""
+    return bool(mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
+                or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
+                or _module._global_backward_pre_hooks)
+
+
+def _train_linear(lin, x, ops):
+    """`lin(x)` of a training step: through `_Linear` for plain layers of a shape and type that the library's parameter
+    gradients take."""
+    w = lin.weight
+    if (getattr(ops, "weight_grad", None) is None or not x.is_cuda or type(lin) is not nn.Linear or _hooked(lin)
+            or not w.requires_grad or w.shape[0] % 8 or w.shape[1] % 8 or w.shape[0] * w.shape[1] >= 1 << 26 or x.numel() == 0):
+        return lin(x)
+    floats = (torch.float32, torch.float16, torch.bfloat16)
+    dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else w.dtype
+    if dt not in floats or x.dtype not in floats or w.dtype not in floats or (not torch.is_autocast_enabled("cuda") and x.dtype != dt):
+        return lin(x)
+    return _Linear.apply(x.to(dt), w, lin.bias, ops.weight_grad, ops.weight_grad_supported)
 
 
 def _cast_params(lin, dt):
@@ -85,7 +135,7 @@ def _linear(lin, x, ops=None, gelu=False):
     remade when the parameters change), and the small layers on many rows go through the library's kernel when
     `ops` has it."""
     if torch.is_grad_enabled() or not x.is_cuda or not torch.is_autocast_enabled("cuda"):
-        y = lin(x)
+        y = _train_linear(lin, x, ops) if torch.is_grad_enabled() else lin(x)
         return F.gelu(y) if gelu else y
     dt = torch.get_autocast_dtype("cuda")
     cache = _cast_params(lin, dt)
@@ -919,7 +969,7 @@ class AutoFocusFormer(nn.Module):
 
     def forward(self, x):
         x = self.forward_features(x)
-        return _linear(self.head, x) if isinstance(self.head, nn.Linear) else x
+        return _linear(self.head, x, self.ops) if isinstance(self.head, nn.Linear) else x
 
 
 def aff_tiny(**kw):

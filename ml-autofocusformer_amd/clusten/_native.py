@@ -36,6 +36,12 @@ class PackItem(ctypes.Structure):
                                                                                                     "reserved")]
 
 
+class WeightGradItem(ctypes.Structure):
+    """clusten_weight_grad_item: a Linear layer's operands and results (device pointers)."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("d_y", "x", "d_weight", "d_bias")]
+                + [(n, ctypes.c_int64) for n in ("d_y_stride", "x_stride")] + [(n, ctypes.c_int32) for n in ("n", "k")])
+
+
 class BlockParams(ctypes.Structure):
     """clusten_block: the parameters of one transformer block (device pointers)."""
     _fields_ = ([(n, ctypes.c_void_p) for n in ("norm1_w", "norm1_b", "norm2_w", "norm2_b", "w_qkv", "b_q", "b_kv", "w_proj",
@@ -128,6 +134,10 @@ _PROTOTYPES = {
     "clusten_block_pack": (ctypes.c_int, [ctypes.POINTER(PackItem), ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
     "clusten_norm_linear_forward": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, ctypes.c_float, _P, _P, _P, _P, _P, _P,
                                                   ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_weight_grad_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(WeightGradItem), ctypes.c_int, ctypes.c_int64,
+                                                              ctypes.c_int]),
+    "clusten_weight_grad": (ctypes.c_int, [ctypes.POINTER(WeightGradItem), ctypes.c_int, ctypes.c_int64, _P, ctypes.c_size_t,
+                                           ctypes.c_int, _P]),
     "clusten_block_tail_forward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_float, _P, _P, _P, _P, _P,
                                                  _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_int,
                                                  ctypes.c_int, ctypes.c_int, _P]),
@@ -1752,4 +1762,45 @@ def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torc
                                           at + b * n * 3 * c * scratch.element_size(), _ptr(plan), int(b != 1 and lb == 1),
                                           _ptr(pe_idx), AttnShape(b, heads, n, 32, m), hidden, scale, _DTYPE_CODES[dtype],
                                           _stream(device)), "clusten_blocks_forward")
+    return out
+
+
+_GRAD_DTYPES = (torch.float32, torch.float16, torch.bfloat16)
+
+
+def weight_grad_supported(d_y: torch.Tensor, x: torch.Tensor) -> bool:
+    """True when `weight_grad` takes token rows d_y (rows, n) and x (rows, k): CUDA tensors of one dtype, unit column stride,
+    n and k multiples of 8, rows on 16-byte boundaries."""
+    if not (d_y.is_cuda and d_y.device == x.device and d_y.dim() == 2 and x.dim() == 2 and d_y.dtype == x.dtype and d_y.dtype in _GRAD_DTYPES
+            and d_y.shape[0] == x.shape[0] and 0 < d_y.shape[0] < 1 << 31):
+        return False
+    for t in (d_y, x):
+        if t.shape[1] % 8 or not t.shape[1] or t.stride(1) != 1 or t.stride(0) < t.shape[1] or t.stride(0) >= 1 << 24 or \
+                t.stride(0) * t.element_size() % 16 or t.data_ptr() % 16:
+            return False
+    return d_y.shape[1] * x.shape[1] < 1 << 26
+
+
+def weight_grad(pairs):
+    """[(d_weight, d_bias)] of Linear layers over the same token rows: `pairs` of (d_y (rows, n), x (rows, k), with_bias), at
+    most eight, every one as `weight_grad_supported` says.  d_weight = d_y^T x (n, k) and d_bias = the column sums of d_y, fp32,
+    in two launches for all layers.  No autograd."""
+    lib = load()
+    items, out = (WeightGradItem * len(pairs))(), []
+    first = pairs[0][0]
+    device, rows, dtype = first.device, first.shape[0], first.dtype
+    for it, (d_y, x, with_bias) in zip(items, pairs):
+        if not weight_grad_supported(d_y, x) or d_y.shape[0] != rows or d_y.dtype != dtype or d_y.device != device:
+            raise RuntimeError("weight_grad: rows of one dtype and count, n and k multiples of 8, on 16-byte boundaries")
+        n, k = d_y.shape[1], x.shape[1]
+        d_w = torch.empty(n, k, dtype=torch.float32, device=device)
+        d_b = torch.empty(n, dtype=torch.float32, device=device) if with_bias else None
+        it.d_y, it.x, it.d_weight, it.d_bias = d_y.data_ptr(), x.data_ptr(), d_w.data_ptr(), _ptr(d_b)
+        it.d_y_stride, it.x_stride, it.n, it.k = d_y.stride(0), x.stride(0), n, k
+        out.append((d_w, d_b))
+    code = _DTYPE_CODES[dtype]
+    nbytes = lib.clusten_weight_grad_workspace_bytes(items, len(pairs), rows, code)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    with _on(device):
+        _check(lib.clusten_weight_grad(items, len(pairs), rows, work.data_ptr(), nbytes, code, _stream(device)), "clusten_weight_grad")
     return out

@@ -680,4 +680,39 @@ int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x
     return CLUSTEN_OK;
 }
 
+static int check_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype) {
+    if (!items) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (count < 1 || count > 8 || rows <= 0 || rows >= (int64_t)1 << 31) return CLUSTEN_ERR_BAD_DIMS;
+    for (int i = 0; i < count; ++i) {
+        const clusten_weight_grad_item& it = items[i];
+        if (it.n <= 0 || it.k <= 0 || it.n % 8 != 0 || it.k % 8 != 0 || (int64_t)it.n * it.k >= (int64_t)1 << 26 ||
+            it.d_y_stride < it.n || it.x_stride < it.k || it.d_y_stride >= (int64_t)1 << 24 || it.x_stride >= (int64_t)1 << 24) {
+            return CLUSTEN_ERR_BAD_DIMS;
+        }
+    }
+    return CLUSTEN_OK;
+}
+
+size_t clusten_weight_grad_workspace_bytes(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype) {
+    return check_weight_grad(items, count, rows, dtype) == CLUSTEN_OK ? weight_grad_workspace_bytes(items, count, rows, dtype) : 0;
+}
+
+int clusten_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, void* workspace, size_t workspace_bytes,
+                        int dtype, clusten_stream stream) {
+    if (int st = check_weight_grad(items, count, rows, dtype)) return st;
+    const int64_t elem = (int64_t)dtype_size(dtype);
+    for (int i = 0; i < count; ++i) {
+        const clusten_weight_grad_item& it = items[i];
+        if (!it.d_y || !it.x || !it.d_weight) return CLUSTEN_ERR_NULL_POINTER;
+        if (!aligned16(it.d_y) || !aligned16(it.x) || !aligned16(it.d_weight) || !aligned16(it.d_bias) ||
+            it.d_y_stride * elem % 16 != 0 || it.x_stride * elem % 16 != 0) {
+            return CLUSTEN_ERR_UNALIGNED;
+        }
+    }
+    if (!workspace || workspace_bytes < weight_grad_workspace_bytes(items, count, rows, dtype)) return CLUSTEN_ERR_WORKSPACE;
+    if (!aligned16(workspace)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_weight_grad(items, count, rows, static_cast<float*>(workspace), dtype, as_stream(stream));
+}
+
 }  // extern "C"

@@ -295,6 +295,10 @@ int launch_block_pack(const clusten_pack_item* items, int count, int C, int dtyp
 int launch_norm_linear(const NormLinearArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);
 int launch_block_tail(const BlockTailArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);
 
+// Parameter gradients of Linear layers over the same rows (weight_grad.hip).
+size_t weight_grad_workspace_bytes(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype);
+int launch_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, float* workspace, int dtype, hipStream_t stream);
+
 // Fill `count` fp32 / fp64 words with zero (a kernel, so that callers may capture it in a HIP graph).
 //   `only_if` (may be null): a device flag; the kernel does nothing when it points to zero.
 int launch_zero_f32(float* dst, size_t count, hipStream_t stream, const int32_t* only_if = nullptr);
