@@ -637,10 +637,10 @@ int clusten_norm_linear_forward(const void* x, int x_dtype, const float* norm_w,
                                 float* stats, int64_t rows, int C, int N, int dtype, clusten_stream stream);
 
 /* The block behind its attention (models/aff_transformer.py:157-158, 230-232, 181-196):
- *   x1 = x + s (attn Wp^T + bp),   out = x1 + s (gelu(LayerNorm(x1) W1^T + b1) W2^T + b2)
+ *   x1 = x + s1 (attn Wp^T + bp),  out = x1 + s2 (gelu(LayerNorm(x1) W1^T + b1) W2^T + b2)
  *   attn (rows,C) of dtype; x, out (rows,C) of x_dtype (F32 or dtype); wp (C,C), w1 (H,C), w2 (C,H) packed for width C;
- *   norm_w, norm_b, bp, b1, b2 fp32; H a multiple of C.  scale: fp32, one factor per image of rows_per_image rows (s;
- *   rounded to dtype), or NULL for 1.  For a backward pass, all or none of: x1 (rows,C) of x_dtype, normed (rows,C) of dtype
+ *   norm_w, norm_b, bp, b1, b2 fp32; H a multiple of C.  scale: fp32, one factor per image of rows_per_image rows
+ *   for s1, then one for s2 (rounded to dtype), or NULL for 1.  For a backward pass, all or none of: x1 (rows,C) of x_dtype, normed (rows,C) of dtype
  *   = LayerNorm(x1), hidden (rows,H) of dtype = the sum ahead of the GELU, stats (rows,2) fp32.
  * Intermediates are rounded to dtype (x1 to x_dtype) where separate layers would store them; sums are fp32. */
 int clusten_block_tail_forward(const void* attn, const void* x, int x_dtype, const void* wp, const float* bp,
@@ -688,6 +688,30 @@ typedef struct {
 size_t clusten_weight_grad_workspace_bytes(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype);
 int clusten_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, void* workspace, size_t workspace_bytes,
                         int dtype, clusten_stream stream);
+
+/* The backward of a block between its products, which the reference leaves to autograd.  Tensors are dense rows of C channels
+ * (C in {32,64,128,256,512}) of dtype F32, F16 or BF16 unless said otherwise, on 16-byte boundaries; sums are fp32 in a fixed
+ * order; workspace: clusten_row_sums_workspace_bytes(rows, C) bytes.
+ *   gelu: g = gelu(h), d_h = d_g gelu'(h); count a multiple of 8; d_h may be d_g.
+ *   norm: of y = LayerNorm(x), x of x_dtype (F32 or dtype) with stats (rows,2) as the forwards above keep them: d_x = d_res
+ *     + its gradient for d_y (d_res of x_dtype, or NULL), branch (of dtype, or NULL) = d_x times the factor of the row's image
+ *     (scale as above but one factor an image, or NULL), and the sums of the norm's parameters.
+ *   blank: d_blank_k (C) = scale * sum d_logit q, d_blank_v (C) = sum prob d_out; q rows q_stride elements apart (a multiple
+ *     of 8), d_logit and prob fp32 (B,H,N), C = H * channels of a head, which are a multiple of 8.
+ *   kv_columns: d_k, d_v (B,H,N,ch) into columns C .. 3C of d_qkv (B*N,3C), per head ch of scale * d_k, then ch of d_v.
+ *   table_linear: d_weight (n,k) = d^T x, d_bias = the column sums of d, for fp32 d (rows,n) and x (rows,k) of dtype, k <= 8. */
+size_t clusten_row_sums_workspace_bytes(int64_t rows, int C);
+int clusten_gelu_backward(const void* h, const void* d_g, void* g, void* d_h, int64_t count, int dtype, clusten_stream stream);
+int clusten_norm_backward(const void* d_y, const void* x, int x_dtype, const float* stats, const float* weight, const void* d_res,
+                          void* d_x, void* branch, const float* scale, int rows_per_image, float* d_weight, float* d_bias,
+                          void* workspace, size_t workspace_bytes, int64_t rows, int C, int dtype, clusten_stream stream);
+int clusten_blank_grad(const void* q, int q_stride, const void* d_out, const float* d_logit, const float* prob, float scale,
+                       float* d_blank_k, float* d_blank_v, void* workspace, size_t workspace_bytes, int B, int H, int N, int C,
+                       int dtype, clusten_stream stream);
+int clusten_kv_columns(const void* d_k, const void* d_v, void* d_qkv, float scale, int B, int H, int N, int ch, int dtype,
+                       clusten_stream stream);
+int clusten_table_linear_grad(const float* d, const void* x, float* d_weight, float* d_bias, int64_t rows, int n, int k, int dtype,
+                              clusten_stream stream);
 
 /* ---- producer of the neighbourhood lists (optional) ------------------------------------------- */
 

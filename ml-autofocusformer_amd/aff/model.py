@@ -64,6 +64,9 @@ def default_ops():
                            block_stands_for=(("linear", _native.linear), ("layer_norm", _native.layer_norm),
                                              ("add_layer_norm", _native.add_layer_norm)),
                            weight_grad=_native.weight_grad, weight_grad_supported=_native.weight_grad_supported,
+                           gelu_backward=_native.gelu_backward, norm_backward=_native.norm_backward,
+                           attention_columns_backward=_native.attention_columns_backward,
+                           table_linear_grad=_native.table_linear_grad,
                            blocks_forward=_native.blocks_forward, block_params=_native.BlockParams,
                            blocks_stand_for=(("cluster_attention", _native.cluster_attention),
                                              ("dense_attention", _native.dense_attention),
@@ -108,7 +111,7 @@ def _train_linear(lin, x, ops):
     """`lin(x)` of a training step: through `_Linear` for plain layers of a shape and type that the library's parameter
     gradients take."""
     w = lin.weight
-    if (getattr(ops, "weight_grad", None) is None or not x.is_cuda or type(lin) is not nn.Linear or _hooked(lin)
+    if (getattr(ops, "weight_grad", None) is None or not x.is_cuda or type(lin) is not nn.Linear or _hooked(lin) or _transformed()
             or not w.requires_grad or w.shape[0] % 8 or w.shape[1] % 8 or w.shape[0] * w.shape[1] >= 1 << 26 or x.numel() == 0):
         return lin(x)
     floats = (torch.float32, torch.float16, torch.bfloat16)
@@ -281,6 +284,155 @@ class _ClusterAttention(torch.autograd.Function):
                 d_bv.reshape(blank_v.shape).to(blank_v.dtype), None, None, None, None, None, None)
 
 
+def _recorded_backward(fn, ctx, tensors, grads):
+    """The gradients of `fn(*tensors)` by recorded operations, for a backward pass that is itself differentiated."""
+    needs = ctx.needs_input_grad[:len(tensors)]
+    with torch.enable_grad(), torch.autocast("cuda", enabled=False):
+        out = fn(*tensors)
+        out, grads = zip(*((o, g) for o, g in zip(out if isinstance(out, tuple) else (out,), grads) if o.requires_grad))
+        wanted = torch.autograd.grad(out, [t for t, need in zip(tensors, needs) if need], grads, create_graph=True, allow_unused=True)
+    wanted = iter(wanted)
+    return [next(wanted) if need else None for need in needs]
+
+
+class _NormLinearRows(torch.autograd.Function):
+    """`norm1` and the q / kv projections of a block as the inference kernel computes them, keeping the norm's result and
+    statistics.  Also hands x through: its other use is the residual addition, whose gradient then meets the norm's inside
+    the norm's backward kernel."""
+
+    @staticmethod
+    def forward(ctx, x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, eps, dt, ops):
+        c = x.shape[-1]
+        # packed in every forward, not kept: the weights of a training step are new ones
+        packed, at = ops.block_pack(c, dt, [(w_q, False), (w_kv, False)])
+        qkv, normed, stats = ops.norm_linear(x, norm_w, norm_b, eps, packed, at[0], b_q, b_kv, 3 * c, keep=True)
+        ctx.save_for_backward(x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, normed, stats, torch.cat([w_q, w_kv]).to(dt))
+        ctx.meta = (eps, dt, ops)
+        return qkv, x
+
+    @staticmethod
+    def backward(ctx, d_qkv, d_res):
+        x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, normed, stats, w = ctx.saved_tensors
+        eps, dt, ops = ctx.meta
+        c = x.shape[-1]
+        if torch.is_grad_enabled():
+            def layers(x, norm_w, norm_b, w_q, b_q, w_kv, b_kv):
+                y = F.layer_norm(x.float(), (c,), norm_w, norm_b, eps).to(dt)
+                return F.linear(y, torch.cat([w_q, w_kv]).to(dt), torch.cat([b_q, b_kv]).to(dt)), x
+            return (*_recorded_backward(layers, ctx, (x, norm_w, norm_b, w_q, b_q, w_kv, b_kv), (d_qkv, d_res)), None, None, None)
+        need = ctx.needs_input_grad
+        rows = d_qkv.reshape(-1, 3 * c)
+        flat = normed.view(-1, c)
+        grads = [None] * 7
+        if need[0] or need[1] or need[2]:
+            grads[0], _, grads[1], grads[2] = ops.norm_backward((rows @ w).view(x.shape), x, stats, norm_w, d_res.contiguous())
+        wanted = [(i, rows[:, cols], need[i + 1]) for i, cols in ((3, slice(0, c)), (5, slice(c, 3 * c))) if need[i] or need[i + 1]]
+        if wanted:
+            for (i, _, _), (grads[i], grads[i + 1]) in zip(wanted, ops.weight_grad([(d, flat, bias) for _, d, bias in wanted])):
+                pass
+        return (*(g if n else None for g, n in zip(grads, need)), None, None, None)
+
+
+class _BlockTail(torch.autograd.Function):
+    """A block behind its attention as the inference kernel computes it, keeping the rows between its two branches, their
+    norm and the hidden layer.  `scale`: (2, b) factors of stochastic depth, or None."""
+
+    @staticmethod
+    def forward(ctx, attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, eps, dt, ops):
+        weights = (w_p, w_1, w_2)
+        packed, at = ops.block_pack(x.shape[-1], dt, [(w, False) for w in weights])
+        out, x1, normed, hidden, stats = ops.block_tail(attn, x, packed, at, b_p, norm_w, norm_b, eps, b_1, b_2, scale, keep=True)
+        plain = torch.cat([w.reshape(-1) for w in weights]).to(dt)
+        ctx.save_for_backward(attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, x1, normed, hidden, stats, plain)
+        ctx.meta = (eps, dt, ops)
+        return out
+
+    @staticmethod
+    def backward(ctx, d_out):
+        attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, x1, normed, hidden, stats, plain = ctx.saved_tensors
+        eps, dt, ops = ctx.meta
+        b, c, h = x.shape[0], x.shape[-1], hidden.shape[-1]
+        if torch.is_grad_enabled():
+            def layers(attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2):
+                s = (1.0, 1.0) if scale is None else scale.to(dt).view(2, b, *(1,) * (x.dim() - 1))
+                x1 = x + (F.linear(attn, w_p.to(dt), b_p.to(dt)) * s[0]).to(x.dtype)
+                y = F.layer_norm(x1.float(), (c,), norm_w, norm_b, eps).to(dt)
+                y = F.gelu(F.linear(y, w_1.to(dt), b_1.to(dt)))
+                return x1 + (F.linear(y, w_2.to(dt), b_2.to(dt)) * s[1]).to(x.dtype)
+            return (*_recorded_backward(layers, ctx, (attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2), (d_out,)),
+                    None, None, None, None)
+        need = ctx.needs_input_grad
+        d_out = d_out.contiguous()
+        p16, one, two = plain[:c * c].view(c, c), plain[c * c:c * (c + h)].view(h, c), plain[c * (c + h):].view(c, h)
+        d_f = d_out.to(dt)
+        if scale is not None:
+            d_f = d_f * scale[1].to(dt).view(-1, *(1,) * (x.dim() - 1))
+        d_f = d_f.view(-1, c)
+        g, d_h = ops.gelu_backward(hidden.view(-1, h), d_f @ two)
+        grads = [None] * 10
+        separate = x.dtype != dt or scale is not None
+        grads[1], branch, grads[4], grads[5] = ops.norm_backward((d_h @ one).view(x.shape), x1, stats, norm_w, d_out, separate,
+                                                                 None if scale is None else scale[0])
+        branch = (branch if separate else grads[1]).view(-1, c)
+        if need[0]:
+            grads[0] = (branch @ p16).view(attn.shape)
+        wanted = [(i, d, y, need[i + 1]) for i, d, y in ((2, branch, attn.view(-1, c)), (6, d_h, normed.view(-1, c)), (8, d_f, g))
+                  if need[i] or need[i + 1]]
+        if wanted:
+            for (i, *_), (grads[i], grads[i + 1]) in zip(wanted, ops.weight_grad([item[1:] for item in wanted])):
+                pass
+        return (*(t if n else None for t, n in zip(grads, need)), None, None, None, None)
+
+
+class _ClusterAttentionRows(torch.autograd.Function):
+    """`_ClusterAttention` on the (b,n,3c) rows of the stacked projections, with the position bias' layer inside: the gradients
+    of q, k and v go into one tensor of that form, the blank token's and the bias layer's come from kernels of their own."""
+
+    @staticmethod
+    def forward(ctx, qkv, table, pe_w, pe_b, blank_k, blank_v, plan, pairs, pe_idx, member_idx, heads, scale, ops):
+        dt = qkv.dtype
+        table = table.to(dt)
+        bias = F.linear(table, pe_w.to(dt), pe_b.to(dt))
+        q, key, v = _columns(qkv, heads)
+        out, lse = ops.cluster_attention(q, key, v, None, bias, None, None, blank_k, blank_v, scale=scale, plan=plan,
+                                         return_lse=True)
+        ctx.save_for_backward(qkv, out, lse, bias, table, blank_k, blank_v, plan, pairs, pe_idx, member_idx)
+        ctx.meta = (heads, scale, pe_w.dtype, pe_b.dtype, ops)
+        return out
+
+    @staticmethod
+    def backward(ctx, d_out):
+        qkv, out, lse, bias, table, blank_k, blank_v, plan, pairs, pe_idx, member_idx = ctx.saved_tensors
+        heads, scale, w_dtype, b_dtype, ops = ctx.meta
+        q, key, v = _columns(qkv, heads)
+        d_out = d_out.to(qkv.dtype).contiguous()
+        d_qkv = torch.empty_like(qkv)
+        _, probs, d_logit, blank_prob, d_blank = ops.cluster_attention_backward(
+            q, key, v, d_out, out, lse, plan, bias, blank_k, blank_v, scale=scale, d_query=_columns(d_qkv, heads)[0])
+        b, h, n, ch = q.shape
+        d_v = ops.scatter_rows(probs, d_out.view(b, n, h, ch).permute(0, 2, 1, 3), member_idx, pairs)
+        d_k = ops.scatter_rows(d_logit, q, member_idx, pairs)
+        d_bk, d_bv = ops.attention_columns_backward(qkv, d_qkv, d_k, d_v, d_out, d_blank, blank_prob, scale)
+        d_w, d_b = ops.table_linear_grad(ops.bias_table_grad(d_logit, pe_idx, bias.shape[0]), table)
+        return (d_qkv, None, d_w.to(w_dtype), d_b.to(b_dtype), d_bk.reshape(blank_k.shape).to(blank_k.dtype),
+                d_bv.reshape(blank_v.shape).to(blank_v.dtype), None, None, None, None, None, None, None)
+
+
+def _columns(qkv, heads):
+    """(q, key, v), each (b,h,n,ch), of (b,n,3c) rows of stacked projections (views)."""
+    b, n, c3 = qkv.shape
+    c = c3 // 3
+    q = qkv[..., :c].view(b, n, heads, c // heads).permute(0, 2, 1, 3)
+    kv = qkv[..., c:].view(b, n, heads, 2, c // heads)
+    return q, kv[:, :, :, 0].permute(0, 2, 1, 3), kv[:, :, :, 1].permute(0, 2, 1, 3)
+
+
+def _transformed():
+    """True under forward-mode differentiation or a function transform (vmap, jvp, ...), which a custom Function without
+    rules for them does not take."""
+    return torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None
+
+
 def _position_bias(bias, pe_idx, ops):
     """(b, h, n, m) position bias of an attention layer: row pe_idx[b,i,j] of the (rows, h) table for every pair."""
     kernel = getattr(ops, "bias_table_grad", None)
@@ -335,9 +487,12 @@ class DropPath(nn.Module):
     def forward(self, x):
         if not self.training or self.p == 0.0:
             return x
+        return x * self.factors(x.shape[0], x.dtype, x.device).view((-1,) + (1,) * (x.dim() - 1))
+
+    def factors(self, samples, dtype, device):
+        """The factor of every sample: 0 with probability p, else 1 / (1 - p)."""
         keep = 1.0 - self.p
-        shape = (x.shape[0],) + (1,) * (x.dim() - 1)
-        return x * x.new_empty(shape).bernoulli_(keep).div_(keep)
+        return torch.empty(samples, dtype=dtype, device=device).bernoulli_(keep).div_(keep)
 
 
 class Mlp(nn.Module):
@@ -383,6 +538,25 @@ class ClusterAttention(nn.Module):
         out = self.attend(q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
         return self.proj_drop(_linear(self.proj, out, self.ops))
 
+    def _trains_in_one_kernel(self, q, global_attn, cluster_idx, grid_lists):
+        """True when the layer's training pass is the one-kernel attention; q: (b,n,c) rows of the queries."""
+        b, n, c = q.shape
+        h = self.num_heads
+        return (getattr(self.ops, "cluster_attention_backward", None) is not None and torch.is_grad_enabled()
+                and cluster_idx is not None and not global_attn and self.cluster_size == 8 and grid_lists is not None
+                and len(grid_lists) > 4 and not (self.training and self.attn_drop.p > 0)
+                and self.ops.cluster_attention_backward_supported(q.view(b, n, h, c // h).permute(0, 2, 1, 3), cluster_idx.shape[2]))
+
+    def attend_rows(self, qkv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None):
+        """`attend` of a training pass on the (b,n,3c) rows of the stacked projections."""
+        c = self.dim
+        pe = self.pos_embed
+        if self._trains_in_one_kernel(qkv[..., :c], global_attn, cluster_idx, grid_lists) and not table.requires_grad:
+            return _ClusterAttentionRows.apply(qkv, table, pe.weight, pe.bias, self.blank_k, self.blank_v, grid_lists[3],
+                                               grid_lists[4], pe_idx, member_idx, self.num_heads, self.scale, self.ops)
+        q, kv = qkv.split([c, 2 * c], dim=-1)
+        return self.attend(q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
+
     def attend(self, q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None):
         """The attention between its projections: q (b,n,c) and kv (b,n,2c) in, what the output projection reads (b,n,c)
         out.  The query is not scaled yet; q and kv may be column ranges of one matrix."""
@@ -393,8 +567,7 @@ class ClusterAttention(nn.Module):
         numbered = cluster_idx is not None and not global_attn and not torch.is_grad_enabled()
         compact = numbered and getattr(self.ops, "qk_clusters", None) is not None
         sized = {} if self.cluster_size == 8 else {"cluster_size": self.cluster_size}
-        kv = kv.view(b, n, h, 2, ch).permute(3, 0, 2, 1, 4)                                                 # (2,b,h,n,ch) view
-        key, v = kv[0], kv[1]
+        key, v = kv.view(b, n, h, 2, ch).permute(3, 0, 2, 1, 4).unbind(0)                                   # (b,h,n,ch) views
         one_kernel = getattr(self.ops, "cluster_attention", None)
         if (numbered and one_kernel is not None and not (self.training and self.attn_drop.p > 0)
                 and self.ops.cluster_attention_supported(q.view(b, n, h, ch).permute(0, 2, 1, 3), cluster_idx.shape[2],
@@ -407,11 +580,7 @@ class ClusterAttention(nn.Module):
                              lists[1], lists[2], self.blank_k, self.blank_v, scale=self.scale,
                              **({"plan": plan} if plan is not None else {}))
             return out
-        train_kernel = getattr(self.ops, "cluster_attention_backward", None)
-        if (train_kernel is not None and torch.is_grad_enabled() and cluster_idx is not None and not global_attn
-                and self.cluster_size == 8 and grid_lists is not None and len(grid_lists) > 4 and not (self.training and self.attn_drop.p > 0)
-                and self.ops.cluster_attention_backward_supported(q.view(b, n, h, ch).permute(0, 2, 1, 3),
-                                                                  cluster_idx.shape[2])):
+        if self._trains_in_one_kernel(q, global_attn, cluster_idx, grid_lists):
             # training: the same kernel forward, one kernel and four sums backward
             bias = self.bias_table(table)
             out = _ClusterAttention.apply(q.view(b, n, h, ch).permute(0, 2, 1, 3), key, v, bias, self.blank_k,
@@ -483,18 +652,41 @@ class ClusterTransformerBlock(nn.Module):
             self.gamma2 = nn.Parameter(layer_scale * torch.ones(dim))
 
     def _fused_dtype(self, feat):
-        """The type the block kernels work in, or None when the block runs layer by layer: with gradients, on widths or
-        types the kernels are not built for, with layer scale or an active dropout, and when the caller's `ops` has
-        another implementation of a layer they stand for."""
+        """The type the block kernels work in, or None when the block runs layer by layer: on widths or types the kernels
+        are not built for, with layer scale or an active dropout, with modules of other types or with hooks, and when the
+        caller's `ops` has another implementation of a layer they stand for."""
         ops = self.attn.ops
-        if torch.is_grad_enabled() or self.layer_scale or getattr(ops, "block_tail", None) is None:
+        if self.layer_scale or not feat.is_cuda or getattr(ops, "block_tail", None) is None or not self.plain():
             return None
-        if self.training and (self.mlp.drop.p > 0 or self.attn.proj_drop.p > 0 or not isinstance(self.drop_path, nn.Identity)):
+        grad = torch.is_grad_enabled()
+        if self.training and (self.mlp.drop.p > 0 or self.attn.proj_drop.p > 0
+                              or not (grad or isinstance(self.drop_path, nn.Identity))):
             return None
-        dt = torch.get_autocast_dtype("cuda") if feat.is_cuda and torch.is_autocast_enabled("cuda") else torch.float32
-        if not ops.block_supported(feat, dt, self.mlp.fc1.out_features) or self.norm1.weight.dtype != torch.float32:
+        dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else torch.float32
+        if (not ops.block_supported(feat, dt, self.mlp.fc1.out_features) or (grad and (_transformed() or feat.numel() == 0))
+                or not all(_kernel_parameter(t, feat) for t in self.tensors())):
             return None
         return dt if all(getattr(ops, name, None) is fn for name, fn in ops.block_stands_for) else None
+
+    def plain(self):
+        """True when calling the block's modules runs their own `forward` and nothing else."""
+        m = self._modules
+        attn, mlp = m["attn"], m["mlp"]
+        a, ml = attn._modules, mlp._modules
+        mods = (m["norm1"], attn, m["norm2"], mlp, a["q"], a["kv"], a["proj"], ml["fc1"], ml["fc2"], a["pos_embed"],
+                a["attn_drop"], a["proj_drop"], ml["drop"])
+        if tuple(map(type, mods)) != _BLOCK_TYPES or type(m["drop_path"]) not in (nn.Identity, DropPath):
+            return False
+        if not torch.is_grad_enabled():                    # hooks of backward passes have nothing to see
+            if _module._global_forward_hooks or _module._global_forward_pre_hooks:
+                return False
+            for mod in mods:
+                d = mod.__dict__
+                if d["_forward_hooks"] or d["_forward_pre_hooks"]:
+                    return False
+            d = m["drop_path"].__dict__
+            return not (d["_forward_hooks"] or d["_forward_pre_hooks"])
+        return not (any(map(_hooked, mods)) or _hooked(m["drop_path"]))
 
     def tensors(self):
         """The parameters of the block in one tuple, straight from the modules' tables: the look-ups of 30 blocks are a
@@ -525,7 +717,20 @@ class ClusterTransformerBlock(nn.Module):
         """Returns (feat, branch): the block's output is feat + branch.  The addition is left to the caller, which
         hands `branch` to the next block as `carry` so that it can ride along with that block's first norm."""
         ops = self.attn.ops
+        if carry is not None and torch.is_grad_enabled():
+            feat, carry = feat + carry, None
         dt = self._fused_dtype(feat)
+        if dt is not None and torch.is_grad_enabled():
+            # training: the same kernels, keeping what their backward reads
+            attn, mlp, norm1, norm2 = self.attn, self.mlp, self.norm1, self.norm2
+            qkv, feat = _NormLinearRows.apply(feat, norm1.weight, norm1.bias, attn.q.weight, attn.q.bias, attn.kv.weight,
+                                              attn.kv.bias, norm1.eps, dt, ops)
+            a = attn.attend_rows(qkv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
+            scale = None
+            if self.training and isinstance(self.drop_path, DropPath) and self.drop_path.p > 0:
+                scale = torch.stack([self.drop_path.factors(feat.shape[0], dt, feat.device) for _ in range(2)]).float()
+            return _BlockTail.apply(a.to(dt).contiguous(), feat, attn.proj.weight, attn.proj.bias, norm2.weight, norm2.bias,
+                                    mlp.fc1.weight, mlp.fc1.bias, mlp.fc2.weight, mlp.fc2.bias, scale, norm2.eps, dt, ops), None
         if dt is not None:
             # inference: three kernels - norm and projections, attention, everything behind it
             if carry is not None:
@@ -545,6 +750,16 @@ class ClusterTransformerBlock(nn.Module):
         feat, x = _add_layer_norm(self.norm2, feat, self.drop_path(self.gamma1 * a if self.layer_scale else a), ops)
         f = self.mlp(x)
         return feat, self.drop_path(self.gamma2 * f if self.layer_scale else f)
+
+
+_BLOCK_TYPES = (nn.LayerNorm, ClusterAttention, nn.LayerNorm, Mlp, nn.Linear, nn.Linear, nn.Linear, nn.Linear, nn.Linear,
+                nn.Linear, nn.Dropout, nn.Dropout, nn.Dropout)
+
+
+def _kernel_parameter(t, feat):
+    """True for a parameter the block kernels read in place."""
+    return (t is not None and t.dtype == torch.float32 and t.is_contiguous() and t.device == feat.device
+            and t.data_ptr() % 16 == 0)
 
 
 class ClusterMerging(nn.Module):
@@ -719,6 +934,9 @@ class BasicLayer(nn.Module):
         h = first.attn.num_heads
         if dt is None or c != 32 * h or any(getattr(ops, name, None) is not fn for name, fn in ops.blocks_stand_for):
             return None
+        if any(type(blk) is not ClusterTransformerBlock or blk._forward_hooks or blk._forward_pre_hooks or not blk.plain()
+               for blk in self.blocks):
+            return None
         if self.training and any(blk._fused_dtype(feat) is None or blk.attn.attn_drop.p > 0 for blk in self.blocks):
             return None
         if global_attn:
@@ -733,7 +951,7 @@ class BasicLayer(nn.Module):
         key = (dt, table.data_ptr(), table._version, table.dtype, [[(t._version, t.data_ptr()) for t in ts] for ts in tensors])
         cache = self.__dict__.get("_issue_cache")
         if cache is None or cache[0] != key:
-            if any(t.dtype != torch.float32 or not t.is_contiguous() or t.device != feat.device for ts in tensors for t in ts):
+            if not all(_kernel_parameter(t, feat) for ts in tensors for t in ts):
                 return None
             params, held = (ops.block_params * len(tensors))(), [table]
             for p, blk, ts in zip(params, self.blocks, tensors):

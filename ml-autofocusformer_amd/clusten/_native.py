@@ -138,6 +138,15 @@ _PROTOTYPES = {
                                                               ctypes.c_int]),
     "clusten_weight_grad": (ctypes.c_int, [ctypes.POINTER(WeightGradItem), ctypes.c_int, ctypes.c_int64, _P, ctypes.c_size_t,
                                            ctypes.c_int, _P]),
+    "clusten_row_sums_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
+    "clusten_gelu_backward": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, _P]),
+    "clusten_norm_backward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, ctypes.c_int, _P, _P, _P,
+                                            ctypes.c_size_t, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_blank_grad": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, ctypes.c_float, _P, _P, _P, ctypes.c_size_t, ctypes.c_int,
+                                         ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_kv_columns": (ctypes.c_int, [_P, _P, _P, ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                         ctypes.c_int, _P]),
+    "clusten_table_linear_grad": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
     "clusten_block_tail_forward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_float, _P, _P, _P, _P, _P,
                                                  _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_int,
                                                  ctypes.c_int, ctypes.c_int, _P]),
@@ -1004,12 +1013,12 @@ def cluster_attention_backward_supported(query: torch.Tensor, nnc: int) -> bool:
 
 def cluster_attention_backward(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, d_out: torch.Tensor,
                                out: torch.Tensor, lse: torch.Tensor, plan: torch.Tensor, bias_table: torch.Tensor,
-                               blank_key: torch.Tensor, blank_value: torch.Tensor, scale: float = 1.0):
+                               blank_key: torch.Tensor, blank_value: torch.Tensor, scale: float = 1.0, d_query=None):
     """The query-side half of the backward of `cluster_attention(..., plan=plan, return_lse=True)` in one kernel.
 
     query, key, value (B,H,N,32) fp32 / fp16 / bf16 as in the forward; out (B,N,H*32) its result, d_out the gradient of it,
     lse (B,H,N) fp32 from the forward.  Returns (d_query, probs, d_logit, blank_prob, d_blank_logit): d_query a
-    (B,H,N,32) view of (B,N,H,32) memory, probs and d_logit (B,H,N,48) of query's dtype, blank_prob and d_blank_logit
+    (B,H,N,32) view of (B,N,H,32) memory (or the caller's `d_query`, of query's dtype, rows on 16-byte boundaries), probs and d_logit (B,H,N,48) of query's dtype, blank_prob and d_blank_logit
     fp32 (B,H,N).  The other gradients are sums of these: d_value = scatter_rows_by_cluster(probs, d_out),
     d_key = scale * scatter_rows_by_cluster(d_logit, query), d_bias_table = bias_table_grad(d_logit, ...),
     d_blank_key = scale * sum d_blank_logit * query, d_blank_value = sum blank_prob * d_out."""
@@ -1039,7 +1048,10 @@ def cluster_attention_backward(query: torch.Tensor, key: torch.Tensor, value: to
     bias_table = bias_table.detach().to(dtype).contiguous()
     blank_key = blank_key.detach().reshape(h, c).float().contiguous()
     blank_value = blank_value.detach().reshape(h, c).float().contiguous()
-    d_query = torch.empty(b, n, h, c, dtype=dtype, device=device).permute(0, 2, 1, 3)
+    if d_query is None:
+        d_query = torch.empty(b, n, h, c, dtype=dtype, device=device).permute(0, 2, 1, 3)
+    elif d_query.shape != query.shape or d_query.dtype != dtype or d_query.device != device or _rows(d_query) is not d_query:
+        raise RuntimeError("d_query must be rows of query's shape, dtype and device")
     probs = torch.empty(b, h, n, m, dtype=dtype, device=device)
     d_logit = torch.empty(b, h, n, m, dtype=dtype, device=device)
     blank_prob = torch.empty(b, h, n, dtype=torch.float32, device=device)
@@ -1644,7 +1656,7 @@ def block_supported(x: torch.Tensor, dtype: torch.dtype, hidden: int) -> bool:
     """True when the block kernels (`norm_linear`, `block_tail`) take token rows `x` (..., C) for products in `dtype` and a
     hidden layer of `hidden` channels: C of a built width, x fp32 or of `dtype`, hidden a multiple of C."""
     return (x.is_cuda and x.shape[-1] in _BLOCK_WIDTHS and dtype in _DTYPE_CODES and x.dtype in (torch.float32, dtype)
-            and hidden % x.shape[-1] == 0 and x.is_contiguous())
+            and hidden % x.shape[-1] == 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
 
 
 def block_pack(width: int, dtype: torch.dtype, weights):
@@ -1671,9 +1683,11 @@ def block_pack(width: int, dtype: torch.dtype, weights):
     return out, [at * size for at in offsets]
 
 
-def norm_linear(x: torch.Tensor, norm_w, norm_b, eps: float, packed: torch.Tensor, w_at: int, bias0, bias1, n_out: int):
+def norm_linear(x: torch.Tensor, norm_w, norm_b, eps: float, packed: torch.Tensor, w_at: int, bias0, bias1, n_out: int,
+                keep=False):
     """LayerNorm(x) @ W.T + bias over the last axis of x (..., C), in packed's dtype: W (n_out, C) at byte `w_at` of `packed`
-    (`block_pack`), bias0 fp32 (C,) for the first C outputs, bias1 for the others.  No autograd."""
+    (`block_pack`), bias0 fp32 (C,) for the first C outputs, bias1 for the others.  With `keep`, (result, LayerNorm(x) in
+    packed's dtype, (rows, 2) fp32 statistics): what a backward pass reads.  No autograd."""
     lib = load()
     _require_cuda("x", x)
     device, c = x.device, x.shape[-1]
@@ -1686,21 +1700,25 @@ def norm_linear(x: torch.Tensor, norm_w, norm_b, eps: float, packed: torch.Tenso
             bias1.numel() != n_out - c or norm_w.numel() != c or norm_b.numel() != c:
         raise RuntimeError("norm_linear: weights, biases and norm must fit x and n_out")
     out = torch.empty(x.shape[:-1] + (n_out,), dtype=packed.dtype, device=device)
+    normed = torch.empty(x.shape, dtype=packed.dtype, device=device) if keep else None
+    stats = torch.empty(x.numel() // c, 2, dtype=torch.float32, device=device) if keep else None
     if out.numel() == 0:
-        return out
+        return (out, normed, stats) if keep else out
     with _on(device):
         _check(lib.clusten_norm_linear_forward(x.data_ptr(), _DTYPE_CODES[x.dtype], norm_w.data_ptr(), norm_b.data_ptr(), eps,
                                                packed.data_ptr() + w_at, bias0.data_ptr(), bias1.data_ptr(),
-                                               out.data_ptr(), None, None, x.numel() // c, c, n_out,
+                                               out.data_ptr(), _ptr(normed), _ptr(stats), x.numel() // c, c, n_out,
                                                _DTYPE_CODES[packed.dtype], _stream(device)), "clusten_norm_linear_forward")
-    return out
+    return (out, normed, stats) if keep else out
 
 
 def block_tail(attn: torch.Tensor, x: torch.Tensor, packed: torch.Tensor, at, bias_p, norm_w, norm_b, eps: float, bias1,
-               bias2, scale=None):
+               bias2, scale=None, keep=False):
     """x1 = x + scale * (attn Wp^T + bp);  x1 + scale * (gelu(LayerNorm(x1) W1^T + b1) W2^T + b2) for token rows x (..., C):
     everything of a transformer block behind its attention.  `at`: byte offsets of Wp, W1 and W2 in `packed`; the hidden
-    width is bias1's; `scale`: fp32 (B,) factors of the images (the first axis of x), or None.  No autograd."""
+    width is bias1's; `scale`: fp32 (B,) factors of the images (the first axis of x), or (2, B) for one of each branch, or
+    None.  With `keep`, (result, x1, LayerNorm(x1) in packed's dtype, the hidden layer ahead of its GELU, (rows, 2) fp32
+    statistics of the norm): what a backward pass reads.  No autograd."""
     lib = load()
     _require_cuda("x", x)
     device, c, hidden = x.device, x.shape[-1], bias1.numel()
@@ -1713,18 +1731,123 @@ def block_tail(attn: torch.Tensor, x: torch.Tensor, packed: torch.Tensor, at, bi
     size = packed.element_size()
     if at[0] + c * c * size > packed.numel() * size or max(at[1:]) + hidden * c * size > packed.numel() * size:
         raise RuntimeError("block_tail: the packed weights do not hold three matrices of these sizes")
+    if scale is not None:
+        if scale.dtype != torch.float32 or scale.device != device or tuple(scale.shape) not in ((x.shape[0],), (2, x.shape[0])):
+            raise RuntimeError("scale must be fp32 of shape (B,) or (2,B) on x's device")
+        scale = scale.expand(2, -1).contiguous()
     out = torch.empty_like(x)
+    kept = (None,) * 4
+    if keep:
+        kept = (torch.empty_like(x), torch.empty(x.shape, dtype=packed.dtype, device=device),
+                torch.empty(x.shape[:-1] + (hidden,), dtype=packed.dtype, device=device),
+                torch.empty(x.numel() // c, 2, dtype=torch.float32, device=device))
     if out.numel() == 0:
-        return out
+        return (out,) + kept if keep else out
     with _on(device):
         base = packed.data_ptr()
         _check(lib.clusten_block_tail_forward(attn.data_ptr(), x.data_ptr(), _DTYPE_CODES[x.dtype], base + at[0],
                                               bias_p.data_ptr(), norm_w.data_ptr(), norm_b.data_ptr(), eps, base + at[1],
                                               bias1.data_ptr(), base + at[2], bias2.data_ptr(), out.data_ptr(),
                                               None if scale is None else scale.data_ptr(), x.numel() // c // x.shape[0],
-                                              None, None, None, None, x.numel() // c, c, hidden,
+                                              *map(_ptr, kept), x.numel() // c, c, hidden,
                                               _DTYPE_CODES[packed.dtype], _stream(device)), "clusten_block_tail_forward")
-    return out
+    return (out,) + kept if keep else out
+
+
+def _row_sums(rows: int, c: int, device):
+    """Workspace of the row sums and the two (C,) results."""
+    nbytes = load().clusten_row_sums_workspace_bytes(rows, c)
+    return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes, torch.empty(2, c, dtype=torch.float32, device=device)
+
+
+def _block_rows(dtype, c, *tensors):
+    """Raises unless every tensor is None or dense CUDA rows of c channels, dtype (or any of them), on 16-byte boundaries."""
+    for t in tensors:
+        if t is not None and (not t.is_cuda or not t.is_contiguous() or t.shape[-1] != c or t.data_ptr() % 16
+                              or t.dtype not in dtype or t.device != tensors[0].device or t.numel() != tensors[0].numel()):
+            raise RuntimeError("contiguous rows of one shape, of the call's dtype and device, are required")
+
+
+def gelu_backward(hidden: torch.Tensor, d_g: torch.Tensor):
+    """(gelu(hidden), d_g * gelu'(hidden)), the exact GELU; d_g is overwritten with the second.  No autograd."""
+    _block_rows((hidden.dtype,), hidden.shape[-1], hidden, d_g)
+    if hidden.dtype not in _DTYPE_CODES or hidden.numel() % 8:
+        raise RuntimeError("gelu_backward takes fp32, fp16 or bf16 tensors of a multiple of 8 values")
+    g = torch.empty_like(hidden)
+    if g.numel():
+        with _on(g.device):
+            _check(load().clusten_gelu_backward(hidden.data_ptr(), d_g.data_ptr(), g.data_ptr(), d_g.data_ptr(), g.numel(),
+                                                _DTYPE_CODES[g.dtype], _stream(g.device)), "clusten_gelu_backward")
+    return g, d_g
+
+
+def norm_backward(d_y: torch.Tensor, x: torch.Tensor, stats: torch.Tensor, weight: torch.Tensor, d_res=None, branch=False, scale=None):
+    """Backward of y = LayerNorm(x) with statistics `stats` (`norm_linear(..., keep=True)`): (d_x, branch, d_weight, d_bias)
+    with d_x = d_res + the gradient through the norm, of x's dtype, and, with `branch`, a copy of it in d_y's dtype times the
+    images' factors `scale` (fp32 (B,), B the first axis of x; None: 1).  No autograd."""
+    c = x.shape[-1]
+    _block_rows((d_y.dtype,), c, d_y)
+    _block_rows((x.dtype,), c, x, d_res)
+    rows = x.numel() // c
+    if (x.dtype not in (torch.float32, d_y.dtype) or d_y.dtype not in _DTYPE_CODES or d_y.numel() != x.numel()
+            or c not in _BLOCK_WIDTHS or stats.numel() != 2 * rows or stats.dtype != torch.float32 or not stats.is_contiguous()
+            or weight.dtype != torch.float32 or not weight.is_contiguous() or weight.numel() != c):
+        raise RuntimeError("norm_backward: x fp32 or of d_y's dtype, fp32 statistics and weight, a width of the block kernels")
+    if scale is not None and (scale.dtype != torch.float32 or not scale.is_contiguous() or tuple(scale.shape) != (x.shape[0],)):
+        raise RuntimeError("scale must be contiguous fp32 of shape (B,)")
+    d_x = torch.empty_like(x)
+    out = torch.empty_like(d_y) if branch else None
+    if rows == 0:
+        zero = torch.zeros(2, c, device=x.device)
+        return d_x, out, zero[0], zero[1]
+    ws, nbytes, sums = _row_sums(rows, c, x.device)
+    with _on(x.device):
+        at = sums.data_ptr()
+        _check(load().clusten_norm_backward(d_y.data_ptr(), x.data_ptr(), _DTYPE_CODES[x.dtype], stats.data_ptr(), weight.data_ptr(),
+                                            _ptr(d_res), d_x.data_ptr(), _ptr(out), _ptr(scale), rows // x.shape[0], at, at + 4 * c,
+                                            ws.data_ptr(), nbytes, rows, c, _DTYPE_CODES[d_y.dtype], _stream(x.device)),
+               "clusten_norm_backward")
+    return d_x, out, sums[0], sums[1]
+
+
+def attention_columns_backward(qkv: torch.Tensor, d_qkv: torch.Tensor, d_k: torch.Tensor, d_v: torch.Tensor, d_out: torch.Tensor,
+                               d_blank: torch.Tensor, blank_prob: torch.Tensor, scale: float):
+    """What is left of an attention layer's backward behind its scatters: scale * d_k and d_v (B,H,N,ch) into the key / value
+    columns of d_qkv (B,N,3C), and the blank token's gradients (scale * sum d_blank q, sum blank_prob d_out), each (C,) fp32."""
+    lib = load()
+    b, n, c3 = qkv.shape
+    c, h = c3 // 3, d_k.shape[1]
+    ch = c // h
+    _block_rows((qkv.dtype,), c3, qkv, d_qkv)
+    _block_rows((qkv.dtype,), ch, d_k, d_v)
+    _block_rows((qkv.dtype,), c, d_out)
+    if (c not in _BLOCK_WIDTHS or ch % 8 or tuple(d_k.shape) != (b, h, n, ch) or d_out.numel() != b * n * c
+            or any(t.dtype != torch.float32 or not t.is_contiguous() or tuple(t.shape) != (b, h, n) for t in (d_blank, blank_prob))):
+        raise RuntimeError("attention_columns_backward: tensors do not belong to one attention layer")
+    if d_k.numel() == 0:
+        return torch.zeros(c, device=qkv.device), torch.zeros(c, device=qkv.device)
+    ws, nbytes, sums = _row_sums(b * n, c, qkv.device)
+    code = _DTYPE_CODES[qkv.dtype]
+    with _on(qkv.device):
+        at, stream = sums.data_ptr(), _stream(qkv.device)
+        _check(lib.clusten_kv_columns(d_k.data_ptr(), d_v.data_ptr(), d_qkv.data_ptr(), scale, b, h, n, ch, code, stream),
+               "clusten_kv_columns")
+        _check(lib.clusten_blank_grad(qkv.data_ptr(), c3, d_out.data_ptr(), d_blank.data_ptr(), blank_prob.data_ptr(), scale, at,
+                                      at + 4 * c, ws.data_ptr(), nbytes, b, h, n, c, code, stream), "clusten_blank_grad")
+    return sums[0], sums[1]
+
+
+def table_linear_grad(d: torch.Tensor, x: torch.Tensor):
+    """(d^T x, column sums of d) for fp32 d (rows, n) and x (rows, k), k <= 8: the parameter gradients of a position bias layer."""
+    if not (d.is_cuda and d.device == x.device and d.dtype == torch.float32 and x.dtype in _DTYPE_CODES and d.is_contiguous()
+            and x.is_contiguous() and d.dim() == 2 and x.dim() == 2 and d.shape[0] == x.shape[0] and 0 < x.shape[1] <= 8):
+        raise RuntimeError("table_linear_grad: contiguous fp32 d (rows,n) and x (rows,k), k <= 8")
+    n, k = d.shape[1], x.shape[1]
+    d_w, d_b = torch.empty(n, k, device=d.device), torch.empty(n, device=d.device)
+    with _on(d.device):
+        _check(load().clusten_table_linear_grad(d.data_ptr(), x.data_ptr(), d_w.data_ptr(), d_b.data_ptr(), d.shape[0], n, k,
+                                                _DTYPE_CODES[x.dtype], _stream(d.device)), "clusten_table_linear_grad")
+    return d_w, d_b
 
 
 def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torch.dtype, scale: float, plan=None, pe_idx=None):

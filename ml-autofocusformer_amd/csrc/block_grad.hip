@@ -1,0 +1,351 @@
+// What the backward pass of a transformer block does between its products: the gradient of the GELU, of a layer norm with the
+// residual addition ahead of it, of the blank token, of the position bias' small Linear layer, and the order of the key and
+// value gradients.  The products themselves are plain ones.
+//
+// All of them stream rows of C channels once and are bound by that.  A lane takes 8 consecutive channels (16 bytes of 16-bit
+// data), C / 8 lanes a row, so that a wave holds 512 / C whole rows and row sums are a few lane exchanges; column sums stay in
+// the lane's registers over all rows it takes, and every workgroup writes one partial row that `column_sums_kernel` adds up in
+// a fixed order.  No counterpart in the reference, which leaves all of it to autograd.
+#include "common.hpp"
+#include "gelu.hpp"
+#include "launch.hpp"
+
+namespace clusten {
+namespace {
+
+constexpr int kRowThreads = 256;
+
+template <typename T>
+__device__ __forceinline__ void load8(const T* p, float (&x)[8]) {
+    constexpr int PER = 16 / (int)sizeof(T);
+#pragma unroll
+    for (int o = 0; o < 8; o += PER) {
+        float v[PER];
+        VecIO<T, PER>::unpack(*reinterpret_cast<const Piece*>(p + o), v);
+#pragma unroll
+        for (int e = 0; e < PER; ++e) x[o + e] = v[e];
+    }
+}
+template <typename T>
+__device__ __forceinline__ void store8(T* p, const float (&x)[8]) {
+    constexpr int PER = 16 / (int)sizeof(T);
+#pragma unroll
+    for (int o = 0; o < 8; o += PER) {
+        float v[PER];
+#pragma unroll
+        for (int e = 0; e < PER; ++e) v[e] = x[o + e];
+        *reinterpret_cast<Piece*>(p + o) = VecIO<T, PER>::pack(v);
+    }
+}
+
+// Phi(v): from the polynomial of `gelu_16bit` (relative bound 1.3e-6 of Phi(-|v|)) for results of 16 bits, from erfc otherwise.
+template <typename T>
+__device__ __forceinline__ float normal_cdf(float v) {
+    if constexpr (sizeof(T) == 2) {
+        const float tail = normal_tail_16bit(fminf(fabsf(v), 6.5f));
+        return v < 0.f ? tail : 1.f - tail;
+    } else {
+        return 0.5f * erfcf(-0.70710678118654752440f * v);
+    }
+}
+
+// g = gelu(h) and d_h = d_g gelu'(h), gelu'(v) = Phi(v) + v phi(v): the activation is made again rather than kept.
+template <typename T>
+__global__ __launch_bounds__(256) void gelu_backward_kernel(const T* __restrict__ h, const T* d_g, T* __restrict__ g, T* d_h, int64_t pieces) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= pieces) return;
+    float v[8], d[8], y[8];
+    load8(h + i * 8, v);
+    load8(d_g + i * 8, d);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        y[e] = gelu_for<T>(v[e]);
+        d[e] *= normal_cdf<T>(v[e]) + v[e] * 0.39894228040143267794f * __expf(-0.5f * v[e] * v[e]);
+    }
+    store8(g + i * 8, y);
+    store8(d_h + i * 8, d);
+}
+
+// The partial sums of a workgroup's rows: lane groups that hold the same channels are added up in LDS.
+template <int C>
+__device__ __forceinline__ void store_partials(const float (&a)[8], const float (&b)[8], float* __restrict__ partial) {
+    constexpr int LANES = C / 8, SLOTS = kRowThreads / LANES;
+    __shared__ float sums[SLOTS * C];
+#pragma unroll
+    for (int which = 0; which < 2; ++which) {
+        if (which) __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sums[threadIdx.x * 8 + e] = which ? b[e] : a[e];
+        __syncthreads();
+        for (int c = threadIdx.x; c < C; c += kRowThreads) {
+            float s = 0.f;
+            for (int k = 0; k < SLOTS; ++k) s += sums[k * C + c];
+            partial[(int64_t)blockIdx.x * 2 * C + which * C + c] = s;
+        }
+    }
+}
+
+struct NormGrad {
+    const void* d_y;          // (rows, C) of T: gradient of the norm's result
+    const void* x;            // (rows, C) of S
+    const float2* stats;      // mean, 1 / deviation
+    const float* weight;
+    const void* d_res;        // (rows, C) of S, or null
+    void* d_x;                // (rows, C) of S
+    void* branch;             // (rows, C) of T: d_x times the image's factor, or null
+    const float* scale;       // (images), or null
+    float* partial;           // (workgroups, 2 C)
+    int64_t rows;
+    int rows_per_image;
+};
+
+// d_x = d_res + rstd (g - mean(g) - xhat mean(g xhat)), g = d_y weight; sums of d_y xhat and d_y over the rows.
+template <typename T, typename S, int C>
+__global__ __launch_bounds__(kRowThreads) void norm_backward_kernel(NormGrad a) {
+    constexpr int LANES = C / 8, ROWS = kRowThreads / LANES;
+    const int c = (threadIdx.x % LANES) * 8;
+    float w[8], dw[8] = {}, db[8] = {};
+    load8(a.weight + c, w);
+    const int64_t step = (int64_t)gridDim.x * ROWS;
+    for (int64_t base = (int64_t)blockIdx.x * ROWS; base < a.rows; base += step) {
+        const int64_t row = base + threadIdx.x / LANES;
+        const bool live = row < a.rows;
+        const int64_t at = min(row, a.rows - 1) * C + c;
+        float x[8], d[8], r[8] = {};
+        load8(static_cast<const S*>(a.x) + at, x);
+        load8(static_cast<const T*>(a.d_y) + at, d);
+        if (a.d_res) load8(static_cast<const S*>(a.d_res) + at, r);
+        const float2 st = a.stats[min(row, a.rows - 1)];
+        float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            x[e] = (x[e] - st.x) * st.y;
+            if (live) dw[e] += d[e] * x[e], db[e] += d[e];
+            d[e] *= w[e];
+            s1 += d[e];
+            s2 += d[e] * x[e];
+        }
+#pragma unroll
+        for (int o = 1; o < LANES; o <<= 1) {
+            s1 += __shfl_xor(s1, o);
+            s2 += __shfl_xor(s2, o);
+        }
+        s1 *= 1.f / C, s2 *= 1.f / C;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) r[e] += st.y * (d[e] - s1 - x[e] * s2);
+        if (!live) continue;
+        store8(static_cast<S*>(a.d_x) + at, r);
+        if (a.branch) {
+            const float f = a.scale ? a.scale[(uint32_t)row / (uint32_t)a.rows_per_image] : 1.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) r[e] = to_acc(from_acc<S>(r[e])) * f;
+            store8(static_cast<T*>(a.branch) + at, r);
+        }
+    }
+    store_partials<C>(dw, db, a.partial);
+}
+
+struct BlankGrad {
+    const void* q;            // rows of C channels, q_stride apart
+    const void* d_out;        // (rows, C)
+    const float* d_logit;     // (B, H, N)
+    const float* prob;        // (B, H, N)
+    float* partial;
+    int64_t rows;
+    int q_stride, heads, tokens;
+};
+
+// Sums over the rows of d_logit q and prob d_out, each head's channels with its own factor.
+template <typename T, int C>
+__global__ __launch_bounds__(kRowThreads) void blank_grad_kernel(BlankGrad a) {
+    constexpr int LANES = C / 8, ROWS = kRowThreads / LANES;
+    const int c = (threadIdx.x % LANES) * 8, head = c / (C / a.heads);
+    float dk[8] = {}, dv[8] = {};
+    for (int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / LANES; row < a.rows; row += (int64_t)gridDim.x * ROWS) {
+        const uint32_t image = (uint32_t)row / (uint32_t)a.tokens, token = (uint32_t)row - image * (uint32_t)a.tokens;
+        const int64_t f = ((int64_t)image * a.heads + head) * a.tokens + token;
+        const float fk = a.d_logit[f], fv = a.prob[f];
+        float q[8], g[8];
+        load8(static_cast<const T*>(a.q) + row * a.q_stride + c, q);
+        load8(static_cast<const T*>(a.d_out) + row * C + c, g);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dk[e] += fk * q[e], dv[e] += fv * g[e];
+    }
+    store_partials<C>(dk, dv, a.partial);
+}
+
+// Sums of `groups` partial rows of 2 C values: 16 threads a column, each 64 columns wide workgroup on its own.
+__global__ __launch_bounds__(1024) void column_sums_kernel(const float* __restrict__ partial, int groups, int C, float scale0, float* __restrict__ out0,
+                                                           float* __restrict__ out1) {
+    __shared__ float sums[16][64];
+    const int col = blockIdx.x * 64 + (threadIdx.x & 63), slice = threadIdx.x >> 6;
+    float s = 0.f;
+#pragma unroll 8
+    for (int g = slice; g < groups; g += 16) s += partial[(int64_t)g * 2 * C + col];
+    sums[slice][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (slice == 0) {
+        for (int k = 1; k < 16; ++k) s += sums[k][threadIdx.x];
+        if (col < C) out0[col] = s * scale0;
+        else out1[col - C] = s;
+    }
+}
+
+// d_k and d_v (B, H, N, ch) into the key / value columns of d_qkv (B N, 3 H ch): per head ch of d_k times scale, ch of d_v.
+template <typename T>
+__global__ __launch_bounds__(256) void kv_columns_kernel(const T* __restrict__ d_k, const T* __restrict__ d_v, T* __restrict__ out, float scale,
+                                                         int64_t pieces, int heads, int tokens, int ch) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;      // (row, head, k or v, piece of 8 channels)
+    if (i >= pieces) return;
+    const int per = ch / 8, p = (int)(i % per), is_v = (int)(i / per) & 1;
+    const int64_t rest = i / (2 * per), row = rest / heads;
+    const int head = (int)(rest % heads);
+    const int64_t image = row / tokens, token = row % tokens;
+    float v[8];
+    load8((is_v ? d_v : d_k) + ((image * heads + head) * tokens + token) * ch + p * 8, v);
+    if (!is_v) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] *= scale;
+    }
+    store8(out + row * 3 * heads * ch + heads * ch + (head * 2 + is_v) * ch + p * 8, v);
+}
+
+// d_weight (heads, k) = d^T x and d_bias (heads) for the few columns of a position bias layer: one workgroup a head.  The
+// library's product for this form walks the 12 000 rows in one or two workgroups (90 us).
+constexpr int kTableCols = 8;
+template <typename T>
+__global__ __launch_bounds__(1024) void table_linear_grad_kernel(const float* __restrict__ d, const T* __restrict__ x, float* __restrict__ d_w,
+                                                                 float* __restrict__ d_b, int64_t rows, int heads, int k) {
+    __shared__ float sums[16][kTableCols + 1];
+    const int head = blockIdx.x;
+    float s[kTableCols + 1] = {};
+    for (int64_t r = threadIdx.x; r < rows; r += 1024) {
+        const float g = d[r * heads + head];
+#pragma unroll
+        for (int j = 0; j < kTableCols; ++j) {
+            if (j < k) s[j] += g * to_acc(x[r * k + j]);
+        }
+        s[kTableCols] += g;
+    }
+#pragma unroll
+    for (int j = 0; j <= kTableCols; ++j) {
+        for (int o = 32; o > 0; o >>= 1) s[j] += __shfl_xor(s[j], o);
+        if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6][j] = s[j];
+    }
+    __syncthreads();
+    if (threadIdx.x <= kTableCols) {
+        float t = 0.f;
+        for (int w = 0; w < 16; ++w) t += sums[w][threadIdx.x];
+        if (threadIdx.x == kTableCols) d_b[head] = t;
+        else if ((int)threadIdx.x < k) d_w[head * k + threadIdx.x] = t;
+    }
+}
+
+// Workgroups for `rows` rows of C channels: four to six a compute unit are enough to keep the memory busy, and every one
+// costs a partial row.
+int row_groups(int64_t rows, int C) {
+    const int64_t per = kRowThreads / (C / 8);
+    return (int)min((rows + per - 1) / per, (int64_t)1024);
+}
+
+template <typename T, typename S>
+int norm_backward_width(const NormGrad& a, int C, int groups, hipStream_t stream) {
+    switch (C) {
+        case 32: hipLaunchKernelGGL((norm_backward_kernel<T, S, 32>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        case 64: hipLaunchKernelGGL((norm_backward_kernel<T, S, 64>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        case 128: hipLaunchKernelGGL((norm_backward_kernel<T, S, 128>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        case 256: hipLaunchKernelGGL((norm_backward_kernel<T, S, 256>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        case 512: hipLaunchKernelGGL((norm_backward_kernel<T, S, 512>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        default: return CLUSTEN_ERR_BAD_DIMS;
+    }
+    return launch_status();
+}
+
+template <typename T>
+int blank_grad_width(const BlankGrad& a, int C, int groups, hipStream_t stream) {
+    switch (C) {
+        case 32: hipLaunchKernelGGL((blank_grad_kernel<T, 32>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        case 64: hipLaunchKernelGGL((blank_grad_kernel<T, 64>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        case 128: hipLaunchKernelGGL((blank_grad_kernel<T, 128>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        case 256: hipLaunchKernelGGL((blank_grad_kernel<T, 256>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        case 512: hipLaunchKernelGGL((blank_grad_kernel<T, 512>), dim3(groups), dim3(kRowThreads), 0, stream, a); break;
+        default: return CLUSTEN_ERR_BAD_DIMS;
+    }
+    return launch_status();
+}
+
+int launch_column_sums(const float* partial, int groups, int C, float scale0, float* out0, float* out1, hipStream_t stream) {
+    hipLaunchKernelGGL(column_sums_kernel, dim3(2 * C / 64), dim3(1024), 0, stream, partial, groups, C, scale0, out0, out1);
+    return launch_status();
+}
+
+}  // namespace
+
+size_t row_sums_workspace_bytes(int64_t rows, int C) { return (size_t)row_groups(rows, C) * 2 * C * sizeof(float); }
+
+int launch_gelu_backward(const void* h, const void* d_g, void* g, void* d_h, int64_t count, int dtype, hipStream_t stream) {
+    const int64_t pieces = count / 8;
+    const dim3 grid((unsigned)((pieces + 255) / 256));
+    if (dtype == CLUSTEN_F16) {
+        hipLaunchKernelGGL((gelu_backward_kernel<f16_t>), grid, dim3(256), 0, stream, static_cast<const f16_t*>(h), static_cast<const f16_t*>(d_g),
+                           static_cast<f16_t*>(g), static_cast<f16_t*>(d_h), pieces);
+    } else if (dtype == CLUSTEN_BF16) {
+        hipLaunchKernelGGL((gelu_backward_kernel<bf16_t>), grid, dim3(256), 0, stream, static_cast<const bf16_t*>(h), static_cast<const bf16_t*>(d_g),
+                           static_cast<bf16_t*>(g), static_cast<bf16_t*>(d_h), pieces);
+    } else {
+        hipLaunchKernelGGL((gelu_backward_kernel<float>), grid, dim3(256), 0, stream, static_cast<const float*>(h), static_cast<const float*>(d_g),
+                           static_cast<float*>(g), static_cast<float*>(d_h), pieces);
+    }
+    return launch_status();
+}
+
+int launch_norm_backward(const void* d_y, const void* x, int x_dtype, const float* stats, const float* weight, const void* d_res, void* d_x,
+                         void* branch, const float* scale, int rows_per_image, float* d_weight, float* d_bias, float* workspace, int64_t rows, int C,
+                         int dtype, hipStream_t stream) {
+    const NormGrad a = {d_y, x, reinterpret_cast<const float2*>(stats), weight, d_res, d_x, branch, scale, workspace, rows, rows_per_image};
+    const int groups = row_groups(rows, C);
+    int st;
+    if (dtype == CLUSTEN_F32) st = norm_backward_width<float, float>(a, C, groups, stream);
+    else if (dtype == CLUSTEN_F16) st = x_dtype == CLUSTEN_F32 ? norm_backward_width<f16_t, float>(a, C, groups, stream)
+                                                                : norm_backward_width<f16_t, f16_t>(a, C, groups, stream);
+    else st = x_dtype == CLUSTEN_F32 ? norm_backward_width<bf16_t, float>(a, C, groups, stream) : norm_backward_width<bf16_t, bf16_t>(a, C, groups, stream);
+    return st ? st : launch_column_sums(workspace, groups, C, 1.f, d_weight, d_bias, stream);
+}
+
+int launch_blank_grad(const void* q, int q_stride, const void* d_out, const float* d_logit, const float* prob, float scale, float* d_blank_k,
+                      float* d_blank_v, float* workspace, int B, int H, int N, int C, int dtype, hipStream_t stream) {
+    const BlankGrad a = {q, d_out, d_logit, prob, workspace, (int64_t)B * N, q_stride, H, N};
+    const int groups = row_groups(a.rows, C);
+    const int st = dtype == CLUSTEN_F32 ? blank_grad_width<float>(a, C, groups, stream)
+                   : dtype == CLUSTEN_F16 ? blank_grad_width<f16_t>(a, C, groups, stream) : blank_grad_width<bf16_t>(a, C, groups, stream);
+    return st ? st : launch_column_sums(workspace, groups, C, scale, d_blank_k, d_blank_v, stream);
+}
+
+int launch_kv_columns(const void* d_k, const void* d_v, void* d_qkv, float scale, int B, int H, int N, int ch, int dtype, hipStream_t stream) {
+    const int64_t pieces = (int64_t)B * N * H * 2 * (ch / 8);
+    const dim3 grid((unsigned)((pieces + 255) / 256));
+    if (dtype == CLUSTEN_F16) {
+        hipLaunchKernelGGL((kv_columns_kernel<f16_t>), grid, dim3(256), 0, stream, static_cast<const f16_t*>(d_k), static_cast<const f16_t*>(d_v),
+                           static_cast<f16_t*>(d_qkv), scale, pieces, H, N, ch);
+    } else if (dtype == CLUSTEN_BF16) {
+        hipLaunchKernelGGL((kv_columns_kernel<bf16_t>), grid, dim3(256), 0, stream, static_cast<const bf16_t*>(d_k), static_cast<const bf16_t*>(d_v),
+                           static_cast<bf16_t*>(d_qkv), scale, pieces, H, N, ch);
+    } else {
+        hipLaunchKernelGGL((kv_columns_kernel<float>), grid, dim3(256), 0, stream, static_cast<const float*>(d_k), static_cast<const float*>(d_v),
+                           static_cast<float*>(d_qkv), scale, pieces, H, N, ch);
+    }
+    return launch_status();
+}
+
+int launch_table_linear_grad(const float* d, const void* x, float* d_w, float* d_b, int64_t rows, int heads, int k, int dtype, hipStream_t stream) {
+    if (dtype == CLUSTEN_F16) {
+        hipLaunchKernelGGL((table_linear_grad_kernel<f16_t>), dim3(heads), dim3(1024), 0, stream, d, static_cast<const f16_t*>(x), d_w, d_b, rows, heads, k);
+    } else if (dtype == CLUSTEN_BF16) {
+        hipLaunchKernelGGL((table_linear_grad_kernel<bf16_t>), dim3(heads), dim3(1024), 0, stream, d, static_cast<const bf16_t*>(x), d_w, d_b, rows, heads, k);
+    } else {
+        hipLaunchKernelGGL((table_linear_grad_kernel<float>), dim3(heads), dim3(1024), 0, stream, d, static_cast<const float*>(x), d_w, d_b, rows, heads, k);
+    }
+    return launch_status();
+}
+
+}  // namespace clusten

@@ -1,8 +1,8 @@
 // block_tail: everything of a transformer block behind its attention, in one kernel over token rows of C channels:
-//   x1 = x + s (attn Wp^T + bp)        out = x1 + s (gelu(LayerNorm(x1) W1^T + b1) W2^T + b2)
+//   x1 = x + s1 (attn Wp^T + bp)       out = x1 + s2 (gelu(LayerNorm(x1) W1^T + b1) W2^T + b2)
 //
-// The reference model's `proj`, residual, `norm2`, MLP and residual (models/aff_transformer.py:157-158, 230-232, 181-196; s
-// is the per-sample factor of stochastic depth, 1 without it).  As separate kernels - three products, an addition with the
+// The reference model's `proj`, residual, `norm2`, MLP and residual (models/aff_transformer.py:157-158, 230-232, 181-196; s1 and
+// s2 are the per-sample factors of stochastic depth, 1 without it).  As separate kernels - three products, an addition with the
 // norm, a GELU - the rows cross memory nine times and the hidden layer (2 to 3 C channels) four times; here a workgroup
 // takes R rows from the attention's output to the block's output with the hidden layer in LDS, C channels of it at a time.  Every intermediate is rounded to the storage type
 // where the separate kernels stored it.  It has no counterpart in the reference's extension modules.
@@ -45,6 +45,10 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
         const int64_t r = min(row0 + 16 * t + r16, a.rows - 1);
         CLUSTEN_LDS_DMA16(static_cast<const T*>(a.attn) + r * C + s * Cfg::kStep + kq * E, act + (size_t)i * 64);
     }
+    const auto factors = [&](const float* of, float (&scale)[TR]) {
+#pragma unroll
+        for (int t = 0; t < TR; ++t) scale[t] = of ? to_acc(from_acc<T>(of[(uint32_t)row[t] / (uint32_t)a.rows_per_image])) : 1.f;
+    };
     float x[TR][F][E];
     {
         const S* rows[TR];
@@ -58,8 +62,7 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
     Piece wb[D][NB];
     preload<NB, D>(wp, lane * 16, wb);
     float scale[TR];
-#pragma unroll
-    for (int t = 0; t < TR; ++t) scale[t] = a.scale ? to_acc(from_acc<T>(a.scale[(uint32_t)row[t] / (uint32_t)a.rows_per_image])) : 1.f;
+    factors(a.scale, scale);
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     lds_barrier<WAVES>();
 
@@ -135,6 +138,7 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
         gemm_pass<T, TR, NB, KS, D>(w2, w1, lane * 16, wb, hid + lane, acc2);
         w2 += (size_t)KS * NB * 64;
     }
+    if (a.scale) factors(a.scale + a.rows / a.rows_per_image, scale);
     if constexpr (PARK) {
         const S* rows[TR];
 #pragma unroll

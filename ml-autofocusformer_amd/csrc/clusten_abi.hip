@@ -680,6 +680,66 @@ int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x
     return CLUSTEN_OK;
 }
 
+size_t clusten_row_sums_workspace_bytes(int64_t rows, int C) {
+    return rows > 0 && rows < (int64_t)1 << 31 && block_width_supported(C) ? row_sums_workspace_bytes(rows, C) : 0;
+}
+
+int clusten_gelu_backward(const void* h, const void* d_g, void* g, void* d_h, int64_t count, int dtype, clusten_stream stream) {
+    if (!h || !d_g || !g || !d_h) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (count <= 0 || count % 8 != 0 || count >= (int64_t)1 << 40) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(h) || !aligned16(d_g) || !aligned16(g) || !aligned16(d_h)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_gelu_backward(h, d_g, g, d_h, count, dtype, as_stream(stream));
+}
+
+int clusten_norm_backward(const void* d_y, const void* x, int x_dtype, const float* stats, const float* weight, const void* d_res,
+                          void* d_x, void* branch, const float* scale, int rows_per_image, float* d_weight, float* d_bias,
+                          void* workspace, size_t workspace_bytes, int64_t rows, int C, int dtype, clusten_stream stream) {
+    if (!d_y || !x || !stats || !weight || !d_x || !d_weight || !d_bias || !workspace) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype) || (x_dtype != dtype && x_dtype != CLUSTEN_F32)) return CLUSTEN_ERR_BAD_DTYPE;
+    const size_t need = clusten_row_sums_workspace_bytes(rows, C);
+    if (need == 0 || (scale && (rows_per_image <= 0 || rows % rows_per_image != 0))) return CLUSTEN_ERR_BAD_DIMS;
+    if (workspace_bytes < need) return CLUSTEN_ERR_TOO_LARGE;
+    const void* all[] = {d_y, x, weight, d_res, d_x, branch, workspace};
+    for (const void* p : all) {
+        if (!aligned16(p)) return CLUSTEN_ERR_UNALIGNED;
+    }
+    if (reinterpret_cast<uintptr_t>(stats) & 7) return CLUSTEN_ERR_UNALIGNED;
+    return launch_norm_backward(d_y, x, x_dtype, stats, weight, d_res, d_x, branch, scale, scale ? rows_per_image : 1, d_weight, d_bias,
+                                static_cast<float*>(workspace), rows, C, dtype, as_stream(stream));
+}
+
+int clusten_blank_grad(const void* q, int q_stride, const void* d_out, const float* d_logit, const float* prob, float scale,
+                       float* d_blank_k, float* d_blank_v, void* workspace, size_t workspace_bytes, int B, int H, int N, int C,
+                       int dtype, clusten_stream stream) {
+    if (!q || !d_out || !d_logit || !prob || !d_blank_k || !d_blank_v || !workspace) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (B <= 0 || N <= 0 || H <= 0 || C <= 0 || C % H != 0 || C / H % 8 != 0 || q_stride < C || q_stride % 8 != 0) return CLUSTEN_ERR_BAD_DIMS;
+    const size_t need = clusten_row_sums_workspace_bytes((int64_t)B * N, C);
+    if (need == 0) return CLUSTEN_ERR_BAD_DIMS;
+    if (workspace_bytes < need) return CLUSTEN_ERR_TOO_LARGE;
+    if (!aligned16(q) || !aligned16(d_out) || !aligned16(workspace)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_blank_grad(q, q_stride, d_out, d_logit, prob, scale, d_blank_k, d_blank_v, static_cast<float*>(workspace), B, H, N, C, dtype,
+                             as_stream(stream));
+}
+
+int clusten_kv_columns(const void* d_k, const void* d_v, void* d_qkv, float scale, int B, int H, int N, int ch, int dtype,
+                       clusten_stream stream) {
+    if (!d_k || !d_v || !d_qkv) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (B <= 0 || H <= 0 || N <= 0 || ch <= 0 || ch % 8 != 0 || (int64_t)B * N >= (int64_t)1 << 31 || (int64_t)H * ch > 1 << 16) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(d_k) || !aligned16(d_v) || !aligned16(d_qkv)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_kv_columns(d_k, d_v, d_qkv, scale, B, H, N, ch, dtype, as_stream(stream));
+}
+
+int clusten_table_linear_grad(const float* d, const void* x, float* d_weight, float* d_bias, int64_t rows, int n, int k, int dtype,
+                              clusten_stream stream) {
+    if (!d || !x || !d_weight || !d_bias) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (rows <= 0 || n <= 0 || n > 1024 || k <= 0 || k > 8) return CLUSTEN_ERR_BAD_DIMS;
+    return launch_table_linear_grad(d, x, d_weight, d_bias, rows, n, k, dtype, as_stream(stream));
+}
+
 static int check_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype) {
     if (!items) return CLUSTEN_ERR_NULL_POINTER;
     if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;

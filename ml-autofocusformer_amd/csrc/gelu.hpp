@@ -35,8 +35,7 @@ __device__ __forceinline__ float gelu_erf(float v) {
 // with a = |v|.  a stops at 6.5, where a Phi(-a) is 2.6e-10, below half of fp16's smallest number.  No reciprocal, no
 // select; a NaN stays one (`v_maximum3`).  One of the two transcendental instructions of the form above, which take four
 // times an ordinary one, goes with them.
-__device__ __forceinline__ float gelu_16bit(float v) {
-    const float a = fminf(fabsf(v), 6.5f);
+__device__ __forceinline__ float normal_tail_16bit(float a) {       // Phi(-a), 0 <= a <= 6.5
     float q = -8.44261482e-09f;
     q = q * a + 3.01195427e-07f;
     q = q * a - 4.53102646e-06f;
@@ -48,7 +47,11 @@ __device__ __forceinline__ float gelu_16bit(float v) {
     q = q * a - 0.459058428f;
     q = q * a - 1.15112928f;
     q = q * a - 0.999999368f;
-    return __builtin_elementwise_maximum(v, 0.f) - a * __builtin_amdgcn_exp2f(q);
+    return __builtin_amdgcn_exp2f(q);
+}
+__device__ __forceinline__ float gelu_16bit(float v) {
+    const float a = fminf(fabsf(v), 6.5f);
+    return __builtin_elementwise_maximum(v, 0.f) - a * normal_tail_16bit(a);
 }
 
 // The GELU of a kernel whose results are stored as T.

@@ -274,7 +274,7 @@ struct BlockTailArgs {
     const void* w2;        // (C, H), packed for width C
     const float* b2;
     void* out;             // (rows, C) of S
-    const float* scale;    // per image, or null
+    const float* scale;    // (2, images): each image's factor of the attention's branch, then of the MLP's, or null
     int rows_per_image;
     int chunks;            // H / C
     int64_t rows;
@@ -298,6 +298,17 @@ int launch_block_tail(const BlockTailArgs& a, int x_dtype, int C, int dtype, hip
 // Parameter gradients of Linear layers over the same rows (weight_grad.hip).
 size_t weight_grad_workspace_bytes(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype);
 int launch_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, float* workspace, int dtype, hipStream_t stream);
+
+// Backward of a block between its products (block_grad.hip); arguments as in the C entry points.
+size_t row_sums_workspace_bytes(int64_t rows, int C);
+int launch_gelu_backward(const void* h, const void* d_g, void* g, void* d_h, int64_t count, int dtype, hipStream_t stream);
+int launch_norm_backward(const void* d_y, const void* x, int x_dtype, const float* stats, const float* weight, const void* d_res, void* d_x,
+                         void* branch, const float* scale, int rows_per_image, float* d_weight, float* d_bias, float* workspace, int64_t rows, int C,
+                         int dtype, hipStream_t stream);
+int launch_blank_grad(const void* q, int q_stride, const void* d_out, const float* d_logit, const float* prob, float scale, float* d_blank_k,
+                      float* d_blank_v, float* workspace, int B, int H, int N, int C, int dtype, hipStream_t stream);
+int launch_kv_columns(const void* d_k, const void* d_v, void* d_qkv, float scale, int B, int H, int N, int ch, int dtype, hipStream_t stream);
+int launch_table_linear_grad(const float* d, const void* x, float* d_w, float* d_b, int64_t rows, int heads, int k, int dtype, hipStream_t stream);
 
 // Fill `count` fp32 / fp64 words with zero (a kernel, so that callers may capture it in a HIP graph).
 //   `only_if` (may be null): a device flag; the kernel does nothing when it points to zero.

@@ -1,0 +1,200 @@
+"""GPU parity of a block's backward: the kernels between its products (`clusten_gelu_backward`, `clusten_norm_backward`,
+`clusten_kv_columns`, `clusten_blank_grad`, `clusten_table_linear_grad`) against float64, and training passes of whole models
+through the block kernels against the same models layer by layer (models/aff_transformer.py:181-232).
+
+Bars of the kernels, max|got - ref| / max|ref|: results stored in 16 bits half a unit in the last place and a little for the
+fp32 arithmetic ahead of it, 6e-4 fp16 and 5e-3 bf16; fp32 results 2e-6, sums over the rows 1e-5 (fp32 sums of up to 2e4 terms in
+some hundred partial sums).
+"""
+from types import SimpleNamespace
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from aff.model import AutoFocusFormer, ClusterTransformerBlock, default_ops
+from clusten import _native
+
+pytestmark = pytest.mark.gpu
+
+BAR = {torch.float16: 6e-4, torch.bfloat16: 5e-3, torch.float32: 2e-6}
+DTYPES = list(BAR)
+
+
+def close(got, ref, bar):
+    ref = ref.double()
+    assert got.shape == ref.shape
+    assert (got.double() - ref).abs().max() <= bar * ref.abs().max().clamp(min=1e-30)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("count", [8, 2040, 2056, 100_000])
+def test_gelu_backward(device, dt, count):
+    gen = torch.Generator(device).manual_seed(count)
+    h = (3 * torch.randn(count, generator=gen, device=device)).to(dt)
+    d = torch.randn(count, generator=gen, device=device).to(dt)
+    x = h.double().requires_grad_(True)
+    ref = F.gelu(x)
+    ref_d, = torch.autograd.grad(ref, x, d.double())
+    g, d_h = _native.gelu_backward(h, d.clone())
+    close(g, ref.detach(), BAR[dt])
+    close(d_h, ref_d, BAR[dt])
+
+
+@pytest.mark.parametrize("dt,stream", [(torch.float16, torch.float16), (torch.float16, torch.float32),
+                                       (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("c,b,n", [(32, 1, 1), (32, 3, 1021), (64, 2, 16 * 1024 + 3), (128, 3, 333), (256, 1, 7), (512, 2, 2051)])
+def test_norm_backward(device, dt, stream, c, b, n):
+    gen = torch.Generator(device).manual_seed(c + n)
+
+    def draw(*shape):
+        return torch.randn(*shape, generator=gen, device=device)
+
+    x, d_y, d_res = (1 + 2 * draw(b, n, c)).to(stream), draw(b, n, c).to(dt), draw(b, n, c).to(stream)
+    w, scale = 1 + 0.2 * draw(c), torch.tensor([1.25, 0.0, 2.0][:b], device=device)
+    x64 = x.double().requires_grad_(True)
+    w64, b64 = w.double().requires_grad_(True), torch.zeros(c, device=device, dtype=torch.float64, requires_grad=True)
+    ref = torch.autograd.grad(F.layer_norm(x64, (c,), w64, b64), (x64, w64, b64), d_y.double())
+    mean = x.double().mean(-1)
+    stats = torch.stack([mean, (x.double().var(-1, unbiased=False) + 1e-5).rsqrt()], -1).float().reshape(-1, 2).contiguous()
+    d_x, branch, d_w, d_b = _native.norm_backward(d_y, x, stats, w, d_res, True, scale)
+    close(d_x, ref[0] + d_res.double(), BAR[stream])
+    close(branch, d_x.double() * scale.double().view(b, 1, 1), BAR[dt])
+    close(d_w, ref[1], 1e-5)
+    close(d_b, ref[2], 1e-5)
+    d_x, branch, _, _ = _native.norm_backward(d_y, x, stats, w)
+    close(d_x, ref[0], BAR[stream])
+    assert branch is None
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("b,h,n,ch", [(1, 1, 1, 32), (2, 2, 777, 32), (3, 4, 100, 8), (2, 16, 259, 32)])
+def test_attention_columns(device, dt, b, h, n, ch):
+    gen = torch.Generator(device).manual_seed(n)
+    c = h * ch
+
+    def draw(*shape):
+        return torch.randn(*shape, generator=gen, device=device)
+
+    qkv, d_out, d_k, d_v = draw(b, n, 3 * c).to(dt), draw(b, n, c).to(dt), draw(b, h, n, ch).to(dt), draw(b, h, n, ch).to(dt)
+    d_blank, prob = draw(b, h, n), draw(b, h, n)
+    d_qkv = torch.full((b, n, 3 * c), 7.0, device=device, dtype=dt)
+    d_bk, d_bv = _native.attention_columns_backward(qkv, d_qkv, d_k, d_v, d_out, d_blank, prob, 0.3)
+    kv = torch.stack([0.3 * d_k.double(), d_v.double()], 3).permute(0, 2, 1, 3, 4).reshape(b, n, 2 * c)
+    assert (d_qkv[..., :c] == 7.0).all()
+    close(d_qkv[..., c:], kv, BAR[dt])
+    q = qkv[..., :c].double().view(b, n, h, ch)
+    close(d_bk, 0.3 * (d_blank.double().permute(0, 2, 1)[..., None] * q).sum((0, 1)).reshape(-1), 1e-5)
+    close(d_bv, (prob.double().permute(0, 2, 1)[..., None] * d_out.double().view(b, n, h, ch)).sum((0, 1)).reshape(-1), 1e-5)
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("rows,n,k", [(1, 1, 1), (1023, 3, 5), (12321, 16, 5), (1025, 2, 8)])
+def test_table_linear_grad(device, dt, rows, n, k):
+    gen = torch.Generator(device).manual_seed(rows)
+    d, x = torch.randn(rows, n, generator=gen, device=device), torch.randn(rows, k, generator=gen, device=device).to(dt)
+    d_w, d_b = _native.table_linear_grad(d, x)
+    close(d_w, d.double().t() @ x.double(), 1e-5)
+    close(d_b, d.double().sum(0), 1e-5)
+
+
+def build(ops, device, drop_path=0.0):
+    torch.manual_seed(5)
+    kw = dict(img_size=96, embed_dim=(32, 64, 128, 256), num_heads=(1, 2, 4, 8), depths=(1, 2, 2, 1), mlp_ratio=2.0,
+              cluster_size=8, nbhd_size=(48, 48, 48, 48), num_classes=40, drop_path_rate=drop_path)
+    return AutoFocusFormer(ops=ops, **kw).to(device)
+
+
+def step(net, dt, device, seed=3):
+    gen = torch.Generator(device).manual_seed(seed)
+    images = torch.randn(3, 3, 96, 96, generator=gen, device=device)
+    labels = torch.randint(40, (3,), generator=gen, device=device)
+    torch.manual_seed(9)
+    with torch.autocast("cuda", dtype=torch.float16 if dt == torch.float32 else dt, enabled=dt != torch.float32):
+        logits = net(images)
+        loss = F.cross_entropy(logits.float(), labels)
+    net.zero_grad(set_to_none=True)
+    (loss * (1.0 if dt == torch.float32 else 1024.0)).backward()
+    return logits.detach(), {name: p.grad for name, p in net.named_parameters()}
+
+
+def norm_error(got, ref):
+    return float((got.double() - ref.double()).norm() / ref.double().norm().clamp(min=1e-30))
+
+
+# A gradient by two orders of the same roundings: fp32 sums of up to 1700 tokens; in fp16 some ten roundings of 2^-11 of each of
+# up to six blocks, and a third of a unit more where sums over few tokens cancel (biases of the key projection: exactly zero).
+@pytest.mark.parametrize("dt,bar", [(torch.float32, 2e-4), (torch.float16, 4e-2)])
+@pytest.mark.parametrize("drop_path", [0.0, 0.4])
+def test_training_step_layer_by_layer(device, dt, bar, drop_path):
+    ops = default_ops()
+    layered = SimpleNamespace(**{**vars(ops), "block_tail": None})
+    got, got_grads = step(build(ops, device, drop_path).train(), dt, device)
+    ref, ref_grads = step(build(layered, device, drop_path).train(), dt, device)
+    assert norm_error(got, ref) < bar
+    everything = torch.cat([g.reshape(-1) for g in got_grads.values()])
+    assert norm_error(everything, torch.cat([g.reshape(-1) for g in ref_grads.values()])) < bar
+    for name, g in ref_grads.items():
+        assert got_grads[name].dtype == g.dtype and (norm_error(got_grads[name], g) < bar or "bias" in name), name
+
+
+def dense_block(device, ops=None, c=64, h=2):
+    torch.manual_seed(2)
+    blk = ClusterTransformerBlock(c, h, ops=ops or default_ops()).to(device)
+    feat = torch.randn(2, 36, c, device=device)
+    table = torch.randn(121, 5, device=device)
+    pe_idx = torch.randint(121, (2, 36, 36), device=device)
+    return blk, feat, lambda x: blk(x, None, None, pe_idx, True, table)
+
+
+def test_second_derivatives_and_frozen_parameters(device):
+    blk, feat, call = dense_block(device)
+    ref_blk, _, ref_call = dense_block(device, SimpleNamespace(**{**vars(default_ops()), "block_tail": None}))
+
+    def penalty(call, blk):
+        x = feat.clone().requires_grad_(True)
+        out, branch = call(x)
+        out = out if branch is None else out + branch
+        g, = torch.autograd.grad(out.square().sum(), x, create_graph=True)
+        return torch.autograd.grad(g.square().sum(), [x, blk.mlp.fc1.weight, blk.attn.q.weight])
+
+    for got, ref in zip(penalty(call, blk), penalty(ref_call, ref_blk)):
+        assert norm_error(got, ref) < 1e-4
+    for p in blk.parameters():
+        p.requires_grad_(False)
+    blk.norm2.weight.requires_grad_(True)
+    blk.mlp.fc2.bias.requires_grad_(True)
+    out, _ = call(feat)
+    out.square().sum().backward()
+    assert blk.norm2.weight.grad is not None and blk.mlp.fc2.bias.grad is not None and blk.attn.q.weight.grad is None
+
+
+def test_hooks_and_replaced_layers_are_called(device):
+    """Modules with hooks or of other types run as modules, with gradients and without."""
+    for grad in (True, False):
+        blk, feat, call = dense_block(device)
+        with torch.set_grad_enabled(grad):
+            plain, branch = call(feat)
+            assert branch is None                                   # the block kernels ran
+            seen = []
+            handle = blk.mlp.register_forward_hook(lambda *a: seen.append(1))
+            out, branch = call(feat)
+            assert seen and norm_error(out + branch, plain) < 1e-5
+            handle.remove()
+
+            class Doubled(torch.nn.Linear):
+                def forward(self, x):
+                    return 2 * super().forward(x)
+
+            twice = Doubled(64, 64).to(device)
+            twice.load_state_dict(blk.attn.proj.state_dict())
+            blk.attn.proj = twice
+            out, branch = call(feat)
+            assert branch is not None and norm_error(out + branch, plain) > 1e-2
+
+
+def test_forward_mode(device):
+    blk, feat, call = dense_block(device)
+    with torch.autograd.forward_ad.dual_level():
+        out, branch = call(torch.autograd.forward_ad.make_dual(feat, torch.ones_like(feat)))
+        assert torch.autograd.forward_ad.unpack_dual(out + branch).tangent is not None
