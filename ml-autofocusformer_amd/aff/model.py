@@ -707,10 +707,17 @@ class ClusterTransformerBlock(nn.Module):
         weights = (attn.q.weight, attn.kv.weight, attn.proj.weight, mlp.fc1.weight, mlp.fc2.weight)
         key = (dt,) + tuple((w._version, w.data_ptr()) for w in weights)
         cache = self.__dict__.get("_pack_cache")
-        if cache is None or cache[0] != key:
-            cache = (key, attn.ops.block_pack(attn.dim, dt, [(w.detach(), False) for w in weights]))
+        if cache is None or cache.key != key:
+            weights = [w.detach() for w in weights]
+            cache = _Kept(key, attn.ops.block_pack(attn.dim, dt, [(w, False) for w in weights]), weights)
             self.__dict__["_pack_cache"] = cache     # a plain attribute, as for the 16-bit copies of the single layers
-        return cache[1]
+        return cache.value
+
+    def fits(self, c, hidden, heads):
+        """True when every parameter has the shape of a block of c channels with `hidden` hidden ones and `heads` heads."""
+        want = 5 * [(c,)] + [(2 * c,), (c,), (hidden,)] + 3 * [(c,)] + [(c, c), (2 * c, c), (c, c), (hidden, c), (c, hidden),
+                                                                     (heads, 5), (heads,)]
+        return [tuple(t.shape) for t in self.tensors()] == want
 
     def forward(self, feat, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None,
                 carry=None):
@@ -754,6 +761,20 @@ class ClusterTransformerBlock(nn.Module):
 
 _BLOCK_TYPES = (nn.LayerNorm, ClusterAttention, nn.LayerNorm, Mlp, nn.Linear, nn.Linear, nn.Linear, nn.Linear, nn.Linear,
                 nn.Linear, nn.Dropout, nn.Dropout, nn.Dropout)
+
+
+class _Kept:
+    """What a module keeps between forwards under a key of addresses and versions.  `held` are the tensors behind these
+    addresses: as long as they are held no other tensor can come to lie there.  Copies and pickles of the module start
+    without it, as `value` may hold device addresses."""
+
+    __slots__ = ("key", "value", "held")
+
+    def __init__(self, key, value, held):
+        self.key, self.value, self.held = key, value, held
+
+    def __reduce__(self):
+        return type(None), ()
 
 
 def _kernel_parameter(t, feat):
@@ -934,8 +955,8 @@ class BasicLayer(nn.Module):
         h = first.attn.num_heads
         if dt is None or c != 32 * h or any(getattr(ops, name, None) is not fn for name, fn in ops.blocks_stand_for):
             return None
-        if any(type(blk) is not ClusterTransformerBlock or blk._forward_hooks or blk._forward_pre_hooks or not blk.plain()
-               for blk in self.blocks):
+        if any(type(blk) is not ClusterTransformerBlock or blk._forward_hooks or blk._forward_pre_hooks or blk.layer_scale
+               or not blk.plain() for blk in self.blocks):
             return None
         if self.training and any(blk._fused_dtype(feat) is None or blk.attn.attn_drop.p > 0 for blk in self.blocks):
             return None
@@ -948,12 +969,17 @@ class BasicLayer(nn.Module):
             if plan is None or not (self.cluster_size == 8 or (self.cluster_size == 24 and dt != torch.float32)):
                 return None
         tensors = [blk.tensors() for blk in self.blocks]
-        key = (dt, table.data_ptr(), table._version, table.dtype, [[(t._version, t.data_ptr()) for t in ts] for ts in tensors])
+        hidden, scale = first.mlp.fc1.out_features, first.attn.scale
+        key = (dt, table.data_ptr(), table._version, table.dtype, hidden,
+               [[(t._version, t.data_ptr()) for t in ts] for ts in tensors],
+               [(blk._modules["norm1"].eps, blk._modules["norm2"].eps, blk._modules["attn"].scale) for blk in self.blocks])
         cache = self.__dict__.get("_issue_cache")
-        if cache is None or cache[0] != key:
-            if not all(_kernel_parameter(t, feat) for ts in tensors for t in ts):
+        if cache is None or cache.key != key:
+            # the call has one width, hidden layer, number of heads and scale for all blocks
+            if not all(blk.fits(c, hidden, h) and blk.attn.num_heads == h and blk.attn.scale == scale
+                       and all(_kernel_parameter(t, feat) for t in ts) for blk, ts in zip(self.blocks, tensors)):
                 return None
-            params, held = (ops.block_params * len(tensors))(), [table]
+            params, held = (ops.block_params * len(tensors))(), [table] + [t.detach() for ts in tensors for t in ts]
             for p, blk, ts in zip(params, self.blocks, tensors):
                 packed, at = blk._packed(dt)
                 bias = blk.attn.bias_table(table)
@@ -964,9 +990,9 @@ class BasicLayer(nn.Module):
                  p.blank_v) = (t.data_ptr() for t in ts[:11])
                 p.w_qkv, p.w_proj, p.w1, p.w2 = (base + o for o in (at[0],) + tuple(at[2:]))
                 p.bias_table, p.eps1, p.eps2 = bias.data_ptr(), blk.norm1.eps, blk.norm2.eps
-            cache = (key, params, held)
+            cache = _Kept(key, params, held)
             self.__dict__["_issue_cache"] = cache     # a plain attribute, remade when a parameter changes
-        return ops.blocks_forward(cache[1], feat, h, first.mlp.fc1.out_features, dt, first.attn.scale, plan,
+        return ops.blocks_forward(cache.value, feat, h, hidden, dt, scale, plan,
                                   pe_idx if plan is None else None)
 
     def forward(self, pos, feat, h, w, on_grid, stride, table, radius, feat_ordered=False):

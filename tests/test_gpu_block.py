@@ -154,3 +154,37 @@ def test_blocks_issued_by_one_call_equal_the_blocks_one_by_one(device, amp):
             m.layers[1].blocks[0].attn.pos_embed.bias.add_(0.25)
     second = run(net)
     assert not torch.equal(first, second) and torch.equal(second, run(single))
+
+
+def test_models_copied_and_changed_after_a_forward(device):
+    """A model is copied and pickled after a forward that kept packed weights and addresses, new parameters in the place of old
+    ones are seen, and a block with another hidden width keeps its stage off the call that has one width for all."""
+    import copy
+    import io
+    from aff.model import Mlp, aff_tiny
+    torch.manual_seed(0)
+    net = aff_tiny().to(device).eval()
+    x = torch.randn(2, 3, 224, 224, generator=torch.Generator().manual_seed(1)).to(device)
+
+    def run(m):
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+            return m(x)
+
+    first = run(net)
+    assert torch.equal(first, run(copy.deepcopy(net)))
+    torch.save(net.layers[2].blocks[0].__dict__.get("_pack_cache"), io.BytesIO())
+    torch.save(net.layers[2].__dict__.get("_issue_cache"), io.BytesIO())
+    fc1 = net.layers[2].blocks[4].mlp.fc1
+    for factor in (1.5, 0.5):
+        value = (fc1.weight.detach() * factor).cpu()
+        fc1.weight = None                                        # its memory may be what the next one gets
+        fc1.weight = torch.nn.Parameter(value.to(device))
+        fresh = aff_tiny().to(device).eval()
+        fresh.load_state_dict(net.state_dict())
+        assert torch.equal(run(net), run(fresh))
+    blk = net.layers[2].blocks[3]
+    blk.mlp = Mlp(256, 256, ops=blk.mlp.ops).to(device).eval()    # narrower than the other blocks'
+    out = run(net)
+    calls = []
+    blk.register_forward_hook(lambda *_: calls.append(1))        # with a hook every block is called by itself
+    assert torch.equal(out, run(net)) and calls
