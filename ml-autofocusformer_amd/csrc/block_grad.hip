@@ -38,17 +38,6 @@ __device__ __forceinline__ void store8(T* p, const float (&x)[8]) {
     }
 }
 
-// Phi(v): from the polynomial of `gelu_16bit` (relative bound 1.3e-6 of Phi(-|v|)) for results of 16 bits, from erfc otherwise.
-template <typename T>
-__device__ __forceinline__ float normal_cdf(float v) {
-    if constexpr (sizeof(T) == 2) {
-        const float tail = normal_tail_16bit(fminf(fabsf(v), 6.5f));
-        return v < 0.f ? tail : 1.f - tail;
-    } else {
-        return 0.5f * erfcf(-0.70710678118654752440f * v);
-    }
-}
-
 // g = gelu(h) and d_h = d_g gelu'(h), gelu'(v) = Phi(v) + v phi(v): the activation is made again rather than kept.
 template <typename T>
 __global__ __launch_bounds__(256) void gelu_backward_kernel(const T* __restrict__ h, const T* d_g, T* __restrict__ g, T* d_h, int64_t pieces) {
@@ -59,8 +48,9 @@ __global__ __launch_bounds__(256) void gelu_backward_kernel(const T* __restrict_
     load8(d_g + i * 8, d);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        y[e] = gelu_for<T>(v[e]);
-        d[e] *= normal_cdf<T>(v[e]) + v[e] * 0.39894228040143267794f * __expf(-0.5f * v[e] * v[e]);
+        y[e] = gelu_erf(v[e]);
+        const float cdf = sizeof(T) == 2 ? normal_cdf(v[e]) : 0.5f * erfcf(-0.70710678118654752440f * v[e]);
+        d[e] *= cdf + v[e] * 0.39894228040143267794f * __expf(-0.5f * v[e] * v[e]);
     }
     store8(g + i * 8, y);
     store8(d_h + i * 8, d);

@@ -41,6 +41,19 @@ def test_gelu_backward(device, dt, count):
     close(d_h, ref_d, BAR[dt])
 
 
+def test_gelu_backward_in_the_tail(device):
+    """Where the derivative is small its relative error is that of rounding it to bf16, 2^-8, and a little: fp32 arithmetic with an
+    exponent of up to 72 leaves 1e-5."""
+    h = torch.linspace(-12, -1.5, 4096, device=device).to(torch.bfloat16)
+    x = h.double()
+    cdf = 0.5 * torch.erfc(-x * 0.5 ** 0.5)
+    ref = cdf + x * torch.exp(-0.5 * x * x) / (2 * torch.pi) ** 0.5
+    g, d_h = _native.gelu_backward(h, torch.ones_like(h))
+    assert ((d_h.double() - ref).abs() <= (2 ** -8 + 2e-5) * ref.abs()).all()
+    ref = x * cdf
+    assert ((g.double() - ref).abs() <= (2 ** -8 + 2e-5) * ref.abs()).all()
+
+
 @pytest.mark.parametrize("dt,stream", [(torch.float16, torch.float16), (torch.float16, torch.float32),
                                        (torch.bfloat16, torch.float32), (torch.float32, torch.float32)])
 @pytest.mark.parametrize("c,b,n", [(32, 1, 1), (32, 3, 1021), (64, 2, 16 * 1024 + 3), (128, 3, 333), (256, 1, 7), (512, 2, 2051)])
