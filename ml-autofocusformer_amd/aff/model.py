@@ -59,7 +59,7 @@ def default_ops():
                            gather_rows=_native.gather_rows, gather_rows_supported=_native.gather_rows_supported,
                            merge_centres=_native.merge_centres, merge_centres_supported=_native.merge_centres_supported,
                            merge_rows=_native.merge_rows, merge_rows_supported=_native.merge_rows_supported,
-                           block_pack=_native.block_pack, block_supported=_native.block_supported,
+                           block_pack=_native.block_pack, block_layout=_native.BlockLayout, block_supported=_native.block_supported,
                            norm_linear=_native.norm_linear, block_tail=_native.block_tail,
                            block_stands_for=(("linear", _native.linear), ("layer_norm", _native.layer_norm),
                                              ("add_layer_norm", _native.add_layer_norm)),
@@ -701,10 +701,14 @@ class ClusterTransformerBlock(nn.Module):
                 pe["weight"], pe["bias"])
 
     def _packed(self, dt):
-        """(weights of the five Linear layers as the block kernels read them, byte offset of each), kept until one of
-        them changes."""
+        """(weights of the five Linear layers as the block kernels read them, byte offset of each).  16-bit ones are kept until a
+        weight changes, like the 16-bit copies of single layers.  fp32 ones are laid out anew in every forward: without
+        mixed precision a forward reads the parameters as they are, also after a write that leaves no trace in the key
+        (through `p.data`, or by a replayed recording)."""
         attn, mlp = self.attn, self.mlp
         weights = (attn.q.weight, attn.kv.weight, attn.proj.weight, mlp.fc1.weight, mlp.fc2.weight)
+        if dt == torch.float32:
+            return attn.ops.block_pack(attn.dim, dt, [(w.detach(), False) for w in weights])
         key = (dt,) + tuple((w._version, w.data_ptr()) for w in weights)
         cache = self.__dict__.get("_pack_cache")
         if cache is None or cache.key != key:
@@ -953,7 +957,8 @@ class BasicLayer(nn.Module):
         dt = first._fused_dtype(feat)
         b, n, c = feat.shape
         h = first.attn.num_heads
-        if dt is None or c != 32 * h or any(getattr(ops, name, None) is not fn for name, fn in ops.blocks_stand_for):
+        if dt is None or c != 32 * h or any(getattr(ops, name, None) is not fn for name, fn in ops.blocks_stand_for) or (
+                dt == torch.float32 and getattr(ops, "block_layout", None) is None):
             return None
         if any(type(blk) is not ClusterTransformerBlock or blk._forward_hooks or blk._forward_pre_hooks or blk.layer_scale
                or not blk.plain() for blk in self.blocks):
@@ -981,19 +986,31 @@ class BasicLayer(nn.Module):
                 return None
             params, held = (ops.block_params * len(tensors))(), [table] + [t.detach() for ts in tensors for t in ts]
             for p, blk, ts in zip(params, self.blocks, tensors):
-                packed, at = blk._packed(dt)
                 bias = blk.attn.bias_table(table)
                 bias = bias.detach().to(dt).contiguous()
-                held += [packed, bias]
-                base = packed.data_ptr()
+                held.append(bias)
+                if dt != torch.float32:
+                    packed, at = blk._packed(dt)
+                    held.append(packed)
+                    p.w_qkv, p.w_proj, p.w1, p.w2 = (packed.data_ptr() + o for o in (at[0],) + tuple(at[2:]))
                 (p.norm1_w, p.norm1_b, p.norm2_w, p.norm2_b, p.b_q, p.b_kv, p.b_proj, p.b1, p.b2, p.blank_k,
                  p.blank_v) = (t.data_ptr() for t in ts[:11])
-                p.w_qkv, p.w_proj, p.w1, p.w2 = (base + o for o in (at[0],) + tuple(at[2:]))
                 p.bias_table, p.eps1, p.eps2 = bias.data_ptr(), blk.norm1.eps, blk.norm2.eps
-            cache = _Kept(key, params, held)
+            layout = None
+            if dt == torch.float32:
+                layout = ops.block_layout([w.detach() for ts in tensors for w in ts[11:16]])
+            cache = _Kept(key, (params, layout), held)
             self.__dict__["_issue_cache"] = cache     # a plain attribute, remade when a parameter changes
-        return ops.blocks_forward(cache.value, feat, h, hidden, dt, scale, plan,
-                                  pe_idx if plan is None else None)
+        params, layout = cache.value
+        packed = None
+        if layout is not None:
+            # fp32: the weights as they are now (`_packed`), for this call only
+            packed = layout.pack(c, dt)
+            params = type(params).from_buffer_copy(params)
+            at = layout.addresses(packed)
+            for i, p in enumerate(params):
+                p.w_qkv, _, p.w_proj, p.w1, p.w2 = at[5 * i:5 * i + 5]
+        return ops.blocks_forward(params, feat, h, hidden, dt, scale, plan, pe_idx if plan is None else None)
 
     def forward(self, pos, feat, h, w, on_grid, stride, table, radius, feat_ordered=False):
         """`feat_ordered`: the tokens already stand in the order `grid_order` gave (first stage only)."""

@@ -1659,28 +1659,51 @@ def block_supported(x: torch.Tensor, dtype: torch.dtype, hidden: int) -> bool:
             and hidden % x.shape[-1] == 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
 
 
+class BlockLayout:
+    """The order in which fp32 matrices - (n,k) tensors, or (tensor, transposed) pairs - lie in one tensor of packed weights, with
+    what `clusten_block_pack` is told of them: prepared once for weights that are packed more than once.  It holds their
+    addresses, not the weights."""
+
+    __slots__ = ("device", "count", "offsets", "items")
+
+    def __init__(self, weights):
+        weights = [w if isinstance(w, tuple) else (w, False) for w in weights]
+        self.device = weights[0][0].device
+        self.items = (PackItem * len(weights))()
+        self.offsets, total = [], 0
+        for it, (w, transposed) in zip(self.items, weights):
+            _require_cuda("weight", w, self.device)
+            if w.dim() != 2 or w.dtype != torch.float32 or not w.is_contiguous():
+                raise RuntimeError("weights must be contiguous fp32 matrices")
+            self.offsets.append(total)
+            total += w.numel()
+            it.src, it.transposed = w.data_ptr(), int(bool(transposed))
+            it.n, it.k = reversed(w.shape) if transposed else w.shape
+        self.count = total
+
+    def addresses(self, packed):
+        """Device address of each matrix in `packed`."""
+        base, size = packed.data_ptr(), packed.element_size()
+        return [base + at * size for at in self.offsets]
+
+    def pack(self, width: int, dtype: torch.dtype) -> torch.Tensor:
+        """The matrices, n and k multiples of `width`, as the block kernels of that width read them."""
+        out = torch.empty(self.count, dtype=dtype, device=self.device)
+        items = type(self.items).from_buffer_copy(self.items)        # callers may share the layout between threads
+        for it, dst in zip(items, self.addresses(out)):
+            it.dst = dst
+        with _on(self.device):
+            _check(load().clusten_block_pack(items, len(items), width, _DTYPE_CODES[dtype], _stream(self.device)),
+                   "clusten_block_pack")
+        return out
+
+
 def block_pack(width: int, dtype: torch.dtype, weights):
     """The matrices `weights` - (fp32 (n,k) tensor, transposed) pairs, n and k multiples of `width` - as the block kernels
     of that width read them, one after the other in one tensor of `dtype`.  Returns (tensor, byte offset of each)."""
-    lib = load()
-    device = weights[0][0].device
-    total, offsets = 0, []
-    for w, _ in weights:
-        _require_cuda("weight", w, device)
-        if w.dim() != 2 or w.dtype != torch.float32 or not w.is_contiguous():
-            raise RuntimeError("weights must be contiguous fp32 matrices")
-        offsets.append(total)
-        total += w.numel()
-    out = torch.empty(total, dtype=dtype, device=device)
-    size = out.element_size()
-    items = (PackItem * len(weights))()
-    for it, (w, transposed), at in zip(items, weights, offsets):
-        n, k = w.shape
-        it.src, it.dst, it.transposed = w.data_ptr(), out.data_ptr() + at * size, int(bool(transposed))
-        it.n, it.k = (k, n) if transposed else (n, k)
-    with _on(device):
-        _check(lib.clusten_block_pack(items, len(weights), width, _DTYPE_CODES[dtype], _stream(device)), "clusten_block_pack")
-    return out, [at * size for at in offsets]
+    layout = BlockLayout(weights)
+    out = layout.pack(width, dtype)
+    return out, [at * out.element_size() for at in layout.offsets]
 
 
 def norm_linear(x: torch.Tensor, norm_w, norm_b, eps: float, packed: torch.Tensor, w_at: int, bias0, bias1, n_out: int,

@@ -12,7 +12,8 @@ int launch_block_tail_f32(const BlockTailArgs& a, int C, hipStream_t stream);
 
 namespace {
 
-constexpr int kPackItems = 8;
+// matrices of a launch, 32 bytes of arguments each: the fp32 weights of a stage of 18 blocks are two launches in every forward
+constexpr int kPackItems = 64;
 struct PackItems {
     clusten_pack_item item[kPackItems];
 };

@@ -1,0 +1,58 @@
+"""What a model keeps between inference forwards - packed weights, 16-bit copies, tables, argument arrays - against models that
+have kept nothing: after writes that the keys cannot see, in recordings, and on other streams."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from aff.model import AutoFocusFormer, CapturedForward, default_ops
+
+pytestmark = pytest.mark.gpu
+
+# 576 and 144 tokens with local lists, 36 and 9 with global attention
+CFG = dict(img_size=96, embed_dim=(32, 64, 128, 256), num_heads=(1, 2, 4, 8), depths=(1, 2, 2, 1), mlp_ratio=2.0, cluster_size=8,
+           nbhd_size=(48, 48, 48, 48), num_classes=40)
+
+
+def build(device, ops=None, seed=5):
+    torch.manual_seed(seed)
+    return AutoFocusFormer(ops=ops or default_ops(), **CFG).to(device).eval()
+
+
+def images(device, b=3):
+    return torch.randn(b, 3, 96, 96, generator=torch.Generator().manual_seed(b)).to(device)
+
+
+def run(net, x, amp=None):
+    with torch.no_grad(), torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+        return net(x)
+
+
+def fresh_copy(net, device, ops=None):
+    other = build(device, ops, seed=6)
+    other.load_state_dict(net.state_dict())
+    return other
+
+
+def block_weights(net):
+    for layer in net.layers:
+        for blk in layer.blocks:
+            yield from (blk.attn.q.weight, blk.attn.kv.weight, blk.attn.proj.weight, blk.mlp.fc1.weight, blk.mlp.fc2.weight)
+
+
+@pytest.mark.parametrize("one_call", [True, False])
+def test_fp32_forwards_read_the_parameters_as_they_are(device, one_call):
+    """A write through `.data` leaves address and version as they were: forwards without mixed precision see it all the same,
+    with the blocks of a stage issued by one call and one by one, and so do replays of a recording."""
+    ops = default_ops() if one_call else SimpleNamespace(**{**vars(default_ops()), "blocks_forward": None})
+    net, x = build(device, ops), images(device)
+    first = run(net, x)
+    recorded = CapturedForward(net, x, autocast_dtype=None)
+    assert torch.equal(recorded(x), first)
+    for factor in (1.25, 0.5):
+        for w in block_weights(net):
+            w.data.mul_(factor)
+        want = run(fresh_copy(net, device, ops), x)
+        assert not torch.equal(want, first)
+        assert torch.equal(run(net, x), want)
+        assert torch.equal(recorded(x), want)
