@@ -20,6 +20,7 @@ neighbours use a sort of exact distances instead of an external library; the ope
 `self.ops`, so a test can run the very same modules on another implementation of the three functions.
 """
 import math
+import threading
 from types import SimpleNamespace
 
 import torch
@@ -121,15 +122,53 @@ def _train_linear(lin, x, ops):
     return _Linear.apply(x.to(dt), w, lin.bias, ops.weight_grad, ops.weight_grad_supported)
 
 
+_recording = threading.local()      # .reads: what the `CapturedForward` being made by this thread has read so far
+
+
+class _Kept:
+    """What a module keeps between forwards under a key of addresses and versions.  `held` are the tensors behind these
+    addresses: as long as they are held no other tensor can come to lie there.  Copies and pickles of the module start
+    without it, as `value` may hold device addresses."""
+
+    __slots__ = ("key", "value", "held")
+
+    def __init__(self, key, value, held):
+        self.key, self.value, self.held = key, value, held
+
+    def __reduce__(self):
+        return type(None), ()
+
+
+def _kept(table, slot, key, make, lasting=False):
+    """The `_Kept` in `table[slot]`, made by `make()` - (value, tensors to hold) - when there is none under `key`.
+
+    A recorded graph reads the addresses it was recorded with for as long as it is replayed, which a kept value does not
+    outlive its key for.  `CapturedForward` holds what its recording reads; any other recording computes it again as a part of
+    itself, but for what is `lasting` (never replaced while its owner lives).  What is made during a recording has no
+    contents until the first replay, so it is not kept."""
+    kept = table.get(slot)
+    hit = type(kept) is _Kept and kept.key == key
+    if torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing():
+        reads = getattr(_recording, "reads", None)
+        if not hit or not (lasting or reads is not None):
+            return _Kept(key, *make())
+        if reads is not None:
+            reads.append(kept)
+    elif not hit:
+        kept = table[slot] = _Kept(key, *make())     # in a module's __dict__: no parameter, no buffer, not in the state_dict
+    return kept
+
+
 def _cast_params(lin, dt):
-    """(key, weight, bias) of an nn.Linear in dtype `dt`, kept until the parameters change."""
-    key = (dt, lin.weight._version, lin.weight.data_ptr(),
-           None if lin.bias is None else (lin.bias._version, lin.bias.data_ptr()))
-    cache = lin.__dict__.get("_cast_cache")
-    if cache is None or cache[0] != key:
-        cache = (key, lin.weight.detach().to(dt), None if lin.bias is None else lin.bias.detach().to(dt))
-        lin.__dict__["_cast_cache"] = cache      # a plain attribute: no parameter, no buffer, not in the state_dict
-    return cache
+    """(weight, bias) of an nn.Linear in dtype `dt` as a `_Kept` value, remade when the parameters change."""
+    weight, bias = lin.weight, lin.bias
+    key = (dt, weight._version, weight.data_ptr(), None if bias is None else (bias._version, bias.data_ptr()))
+
+    def make():
+        held = [t.detach() for t in (weight, bias) if t is not None]
+        return (held[0].to(dt), None if bias is None else held[1].to(dt)), held
+
+    return _kept(lin.__dict__, "_cast_cache", key, make)
 
 
 def _linear(lin, x, ops=None, gelu=False):
@@ -141,12 +180,12 @@ def _linear(lin, x, ops=None, gelu=False):
         y = _train_linear(lin, x, ops) if torch.is_grad_enabled() else lin(x)
         return F.gelu(y) if gelu else y
     dt = torch.get_autocast_dtype("cuda")
-    cache = _cast_params(lin, dt)
+    weight, bias = _cast_params(lin, dt).value
     x = x if x.dtype == dt else x.to(dt)
     fn = getattr(ops, "linear", None)
-    if fn is not None and ops.linear_supported(x, cache[1], gelu):
-        return fn(x, cache[1], cache[2], gelu)
-    y = F.linear(x, cache[1], cache[2])
+    if fn is not None and ops.linear_supported(x, weight, gelu):
+        return fn(x, weight, bias, gelu)
+    y = F.linear(x, weight, bias)
     return F.gelu(y) if gelu else y
 
 
@@ -159,18 +198,16 @@ def _linear_pair(first, second, x, ops=None):
             or first.bias is None or second.bias is None):
         return _linear(first, x, ops), _linear(second, x, ops)
     dt = torch.get_autocast_dtype("cuda")
-    a, b = _cast_params(first, dt), _cast_params(second, dt)
+    kept = _cast_params(first, dt), _cast_params(second, dt)
+    a, b = (k.value for k in kept)
     x = x if x.dtype == dt else x.to(dt)
     fn = getattr(ops, "linear", None)
-    if fn is not None and ops.linear_supported(x, a[1], False) and ops.linear_supported(x, b[1], False):
-        return fn(x, a[1], a[2], False), fn(x, b[1], b[2], False)
-    key = (a[0], b[0])
-    cache = first.__dict__.get("_pair_cache")
-    if cache is None or cache[0] != key:
-        cache = (key, torch.cat([a[1], b[1]], 0), torch.cat([a[2], b[2]], 0))
-        first.__dict__["_pair_cache"] = cache    # a plain attribute, like _cast_cache
-    y = F.linear(x, cache[1], cache[2])
-    n_first = a[1].shape[0]
+    if fn is not None and ops.linear_supported(x, a[0], False) and ops.linear_supported(x, b[0], False):
+        return fn(x, *a, False), fn(x, *b, False)
+    weight, bias = _kept(first.__dict__, "_pair_cache", tuple(k.key for k in kept),
+                         lambda: ((torch.cat([a[0], b[0]], 0), torch.cat([a[1], b[1]], 0)), kept)).value
+    y = F.linear(x, weight, bias)
+    n_first = a[0].shape[0]
     return y[..., :n_first], y[..., n_first:]
 
 
@@ -455,11 +492,7 @@ def _table_function(owner, slot, module, table, compute):
         return compute()
     key = (tuple((q.data_ptr(), q._version) for q in module.parameters()), table.data_ptr(), table._version, table.dtype,
            _autocast_key())
-    hit = owner.__dict__.get(slot)
-    if hit is None or hit[0] != key:
-        hit = (key, compute(), table)         # the table is held, so that its address cannot be reused by another one
-        owner.__dict__[slot] = hit
-    return hit[1]
+    return _kept(owner.__dict__, slot, key, lambda: (compute(), [table] + [q.detach() for q in module.parameters()])).value
 
 
 def relative_position_table(img_size):
@@ -710,12 +743,12 @@ class ClusterTransformerBlock(nn.Module):
         if dt == torch.float32:
             return attn.ops.block_pack(attn.dim, dt, [(w.detach(), False) for w in weights])
         key = (dt,) + tuple((w._version, w.data_ptr()) for w in weights)
-        cache = self.__dict__.get("_pack_cache")
-        if cache is None or cache.key != key:
-            weights = [w.detach() for w in weights]
-            cache = _Kept(key, attn.ops.block_pack(attn.dim, dt, [(w, False) for w in weights]), weights)
-            self.__dict__["_pack_cache"] = cache     # a plain attribute, as for the 16-bit copies of the single layers
-        return cache.value
+
+        def make():
+            held = [w.detach() for w in weights]
+            return attn.ops.block_pack(attn.dim, dt, [(w, False) for w in held]), held
+
+        return _kept(self.__dict__, "_pack_cache", key, make).value
 
     def fits(self, c, hidden, heads):
         """True when every parameter has the shape of a block of c channels with `hidden` hidden ones and `heads` heads."""
@@ -765,20 +798,6 @@ class ClusterTransformerBlock(nn.Module):
 
 _BLOCK_TYPES = (nn.LayerNorm, ClusterAttention, nn.LayerNorm, Mlp, nn.Linear, nn.Linear, nn.Linear, nn.Linear, nn.Linear,
                 nn.Linear, nn.Dropout, nn.Dropout, nn.Dropout)
-
-
-class _Kept:
-    """What a module keeps between forwards under a key of addresses and versions.  `held` are the tensors behind these
-    addresses: as long as they are held no other tensor can come to lie there.  Copies and pickles of the module start
-    without it, as `value` may hold device addresses."""
-
-    __slots__ = ("key", "value", "held")
-
-    def __init__(self, key, value, held):
-        self.key, self.value, self.held = key, value, held
-
-    def __reduce__(self):
-        return type(None), ()
 
 
 def _kernel_parameter(t, feat):
@@ -934,6 +953,13 @@ class BasicLayer(nn.Module):
         cluster_idx = nearest.to(torch.int32).contiguous() if (ranking is not None and m in (8, 24)) else None
         return pos, ranking, member_idx, mask, pe_idx, cluster_idx
 
+    def _grid(self, key, make):
+        """What the lists of a full grid are made into, kept for good."""
+        return _kept(self._grid_cache, key, None, lambda: (make(), ()), lasting=True).value
+
+    def _grid_lists(self, key, pos1, h, w, radius):
+        return self._grid(key, lambda: self.neighbourhoods(pos1, h, w, radius, 2 * radius + 1))
+
     def grid_order(self, pos1, h, w, radius):
         """The order (n,) in which this stage, as the first one, takes the tokens of the full grid (`pos1`: the
         positions of one image), or None when it leaves them as they are; fills the stage's cache of grid lists."""
@@ -941,9 +967,7 @@ class BasicLayer(nn.Module):
         if self.nbhd_size >= n:
             return None
         key = (n, h, w, str(pos1.device))
-        if key not in self._grid_cache:
-            self._grid_cache[key] = self.neighbourhoods(pos1[:1], h, w, radius, 2 * radius + 1)
-        ranking = self._grid_cache[key][1]
+        ranking = self._grid_lists(key, pos1[:1], h, w, radius)[1]
         return None if ranking is None else ranking[0, :, 0]
 
     def _issue_blocks(self, feat, pe_idx, global_attn, table, lists):
@@ -975,16 +999,18 @@ class BasicLayer(nn.Module):
                 return None
         tensors = [blk.tensors() for blk in self.blocks]
         hidden, scale = first.mlp.fc1.out_features, first.attn.scale
-        key = (dt, table.data_ptr(), table._version, table.dtype, hidden,
+        key = (dt, table.data_ptr(), table._version, table.dtype, c, h, hidden,
                [[(t._version, t.data_ptr()) for t in ts] for ts in tensors],
-               [(blk._modules["norm1"].eps, blk._modules["norm2"].eps, blk._modules["attn"].scale) for blk in self.blocks])
-        cache = self.__dict__.get("_issue_cache")
-        if cache is None or cache.key != key:
+               [(blk._modules["norm1"].eps, blk._modules["norm2"].eps, blk._modules["attn"].scale, blk._modules["attn"].num_heads)
+                for blk in self.blocks])
+
+        def make():
+            held = [table] + [t.detach() for ts in tensors for t in ts]
             # the call has one width, hidden layer, number of heads and scale for all blocks
             if not all(blk.fits(c, hidden, h) and blk.attn.num_heads == h and blk.attn.scale == scale
                        and all(_kernel_parameter(t, feat) for t in ts) for blk, ts in zip(self.blocks, tensors)):
-                return None
-            params, held = (ops.block_params * len(tensors))(), [table] + [t.detach() for ts in tensors for t in ts]
+                return (None, None), held
+            params = (ops.block_params * len(tensors))()
             for p, blk, ts in zip(params, self.blocks, tensors):
                 bias = blk.attn.bias_table(table)
                 bias = bias.detach().to(dt).contiguous()
@@ -996,12 +1022,13 @@ class BasicLayer(nn.Module):
                 (p.norm1_w, p.norm1_b, p.norm2_w, p.norm2_b, p.b_q, p.b_kv, p.b_proj, p.b1, p.b2, p.blank_k,
                  p.blank_v) = (t.data_ptr() for t in ts[:11])
                 p.bias_table, p.eps1, p.eps2 = bias.data_ptr(), blk.norm1.eps, blk.norm2.eps
-            layout = None
-            if dt == torch.float32:
-                layout = ops.block_layout([w.detach() for ts in tensors for w in ts[11:16]])
-            cache = _Kept(key, (params, layout), held)
-            self.__dict__["_issue_cache"] = cache     # a plain attribute, remade when a parameter changes
-        params, layout = cache.value
+            layout = ops.block_layout([w.detach() for ts in tensors for w in ts[11:16]]) if dt == torch.float32 else None
+            return (params, layout), held
+
+        kept = _kept(self.__dict__, "_issue_cache", key, make)     # in this frame until the kernels are issued
+        params, layout = kept.value
+        if params is None:
+            return None
         packed = None
         if layout is not None:
             # fp32: the weights as they are now (`_packed`), for this call only
@@ -1026,23 +1053,18 @@ class BasicLayer(nn.Module):
             if on_grid:
                 # grid tokens are the same for every image: one image's lists serve the whole batch
                 key = (n, h, w, str(pos.device))
-                if key not in self._grid_cache:
-                    self._grid_cache[key] = self.neighbourhoods(pos[:1], h, w, radius, table_width)
-                pos1, ranking, member_idx, mask, pe_idx, cluster_idx = self._grid_cache[key]
-                if (key, b) not in self._grid_cache:   # the batch-sized copies the operators read
-                    self._grid_cache[(key, b)] = (member_idx.expand(b, -1, -1).contiguous(),
-                                                  pe_idx.expand(b, -1, -1).contiguous(),
-                                                  None if mask is None else mask.expand(b, -1, -1).contiguous(),
-                                                  None if cluster_idx is None else cluster_idx.expand(b, -1, -1).contiguous())
+                pos1, ranking, *lists = self._grid_lists(key, pos[:1], h, w, radius)
+                member_idx, mask, pe_idx, cluster_idx = lists
                 if cluster_idx is not None:
                     grid_lists = (cluster_idx, pe_idx, mask)           # one image's lists, for the one-kernel attention
                     planner = getattr(self.ops, "cluster_attention_plan", None)
                     if (planner is not None and not torch.is_grad_enabled() and cluster_idx.shape[2] == 6 and pe_idx.is_cuda
                             and (self.cluster_size == 8 or torch.is_autocast_enabled("cuda"))):
-                        if (key, "plan") not in self._grid_cache:      # what that kernel makes of them, kept with them
-                            self._grid_cache[(key, "plan")] = planner(cluster_idx, pe_idx, mask)
-                        grid_lists = grid_lists + (self._grid_cache[(key, "plan")],)
-                member_idx, pe_idx, mask, cluster_idx = self._grid_cache[(key, b)]
+                        # what that kernel makes of them, kept with them
+                        grid_lists = grid_lists + (self._grid((key, "plan"), lambda: planner(*grid_lists)),)
+                # the batch-sized copies the operators read
+                member_idx, mask, pe_idx, cluster_idx = self._grid(
+                    (key, b), lambda: [None if t is None else t.expand(b, -1, -1).contiguous() for t in lists])
                 pos = pos1.expand(b, -1, -1)
                 if ranking is not None and not feat_ordered:
                     feat = feat[:, ranking[0, :, 0]]
@@ -1082,7 +1104,7 @@ class BasicLayer(nn.Module):
         if (self.downsample is not None and scorer is not None and not torch.is_grad_enabled() and feat.is_cuda
                 and torch.is_autocast_enabled("cuda")):
             # inference: the last residual addition and the importance score of the tokens in one pass
-            _, w16, b16 = _cast_params(self.prob_net, torch.get_autocast_dtype("cuda"))
+            w16, b16 = _cast_params(self.prob_net, torch.get_autocast_dtype("cuda")).value
             if self.ops.add_row_score_supported(feat, carry, w16):
                 feat, learned_prob = scorer(feat, carry, w16, b16)
                 carry = None
@@ -1117,8 +1139,8 @@ class PatchEmbed(nn.Module):
         bn, conv = self.bn, self.proj1
         parts = [t for t in (bn.weight, bn.bias, bn.running_mean, bn.running_var, conv.bias) if t is not None]
         key = tuple((t.data_ptr(), t._version) for t in parts)
-        hit = self.__dict__.get("_bn_affine_cache")
-        if hit is None or hit[0] != key:
+
+        def make():
             scale = torch.rsqrt(bn.running_var.float() + bn.eps)
             if bn.weight is not None:
                 scale = scale * bn.weight.float()
@@ -1126,9 +1148,9 @@ class PatchEmbed(nn.Module):
             shift = shift * scale
             if bn.bias is not None:
                 shift = shift + bn.bias.float()
-            hit = (key, scale.detach(), shift.detach())
-            self.__dict__["_bn_affine_cache"] = hit
-        return hit[1], hit[2]
+            return (scale.detach(), shift.detach()), [t.detach() for t in parts]
+
+        return _kept(self.__dict__, "_bn_affine_cache", key, make).value
 
     def forward(self, x, token_order=None):
         """`token_order(pos_of_one_image, h, w)`, when given, returns the order (N,) in which the first stage wants
@@ -1218,11 +1240,8 @@ class AutoFocusFormer(nn.Module):
             # every block's position-embedding Linear would round the table to 16 bits again: one copy, kept
             dt = torch.get_autocast_dtype("cuda")
             key = (table.data_ptr(), table._version, dt)
-            hit = self.__dict__.get("_table_cast_cache")
-            if hit is None or hit[0] != key:
-                hit = (key, table.to(dt))
-                self.__dict__["_table_cast_cache"] = hit
-            table = hit[1]
+            full = table
+            table = _kept(self.__dict__, "_table_cast_cache", key, lambda: (full.to(dt), [full])).value
         for i, layer in enumerate(self.layers):
             pos, x = layer(pos, x, h, w, on_grid=(i == 0), stride=2 ** (i + 1), table=table, radius=self.radius,
                            feat_ordered=(i == 0 and ordered))
@@ -1244,14 +1263,16 @@ def aff_tiny(**kw):
 class CapturedForward:
     """One inference forward of `net` at a fixed input shape, recorded into a HIP graph and replayed.
 
-    A forward of the classifier is some 800 kernel launches of 5-100 us each; issued one by one from Python they
-    take as long on the host as on the GPU.  Replaying the recorded graph leaves one launch per forward.  The
+    A forward of AFF-Tiny is some 170 kernel launches of 5-100 us each; issued one by one from Python they take, for few
+    images, longer on the host than on the GPU.  Replaying the recorded graph leaves one launch per forward.  The
     model's forward has no host synchronisation and every kernel of the library takes the current stream and
     allocates through the framework, so the recording is the plain forward under `torch.cuda.graph`.
 
-    Replays read the parameters in place (their 16-bit copies are part of the recording: record again after the
-    weights change) and return the same output tensor every time: copy it before the next call if it must outlive
-    it.  `autocast_dtype=None` records without mixed precision.
+    Under mixed precision the 16-bit copies of the weights, and with either the tables made of parameters (position bias,
+    merge weights), are those of the time of recording, held by this object: record again after the weights change.
+    Everything else is read in place by every replay; with `autocast_dtype=None`, which records without mixed precision,
+    that is every weight matrix.  The same output tensor is returned every time: copy it before the next call if it
+    must outlive it.
     """
 
     def __init__(self, net, example, autocast_dtype=torch.float16, warmup=3):
@@ -1268,8 +1289,12 @@ class CapturedForward:
         torch.cuda.current_stream(example.device).wait_stream(side)
         torch.cuda.synchronize(example.device)
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
-            self.static_out = self._forward()
+        _recording.reads = self._reads = []      # the graph has their addresses
+        try:
+            with torch.cuda.graph(self.graph):
+                self.static_out = self._forward()
+        finally:
+            del _recording.reads
 
     def _forward(self):
         with torch.no_grad(), torch.autocast("cuda", dtype=self.autocast_dtype or torch.float16,

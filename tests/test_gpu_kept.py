@@ -56,3 +56,51 @@ def test_fp32_forwards_read_the_parameters_as_they_are(device, one_call):
         assert not torch.equal(want, first)
         assert torch.equal(run(net, x), want)
         assert torch.equal(recorded(x), want)
+
+
+def churn(net, x):
+    """What drops a kept value: forwards in other types, a changed weight; and memory for whoever asks for it, not zeros."""
+    for amp in (torch.bfloat16, None, torch.float16):
+        run(net, x, amp)
+    with torch.no_grad():
+        for w in block_weights(net):
+            w.mul_(1.5)
+    run(net, x, torch.float16)
+    run(net, x)
+    return [torch.full((1 << k,), float("nan"), device=x.device) for k in range(6, 22) for _ in range(8)]
+
+
+@pytest.mark.parametrize("amp", [torch.float16, torch.bfloat16])
+def test_recordings_outlive_what_the_model_keeps(device, amp):
+    """16-bit weights are part of a recording: its replays repeat bit for bit after forwards in other types and changes of the
+    weights have replaced what the model keeps."""
+    net, x = build(device), images(device)
+    recorded = CapturedForward(net, x, autocast_dtype=amp)
+    first = recorded(x).clone()
+    assert torch.equal(first, run(net, x, amp))
+    junk = churn(net, x)
+    for _ in range(3):
+        assert torch.equal(recorded(x), first)
+    del junk
+
+
+@pytest.mark.parametrize("amp", [torch.float16, None])
+def test_a_recording_of_the_callers_own(device, amp):
+    """Recorded by `torch.cuda.graph` itself, of a model that has kept nothing yet: forwards between recording and first replay
+    take nothing from it, and replays read the parameters as they are."""
+    x = images(device)
+    run(build(device, seed=7), x, amp)                           # library handles and kernel choices
+    net = build(device)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run(net, x, amp)
+    want = run(fresh_copy(net, device), x, amp)
+    assert torch.equal(run(net, x, amp), want)
+    graph.replay()
+    assert torch.equal(out, want)
+    junk = churn(net, x)
+    want = run(fresh_copy(net, device), x, amp)
+    for _ in range(3):
+        graph.replay()
+        assert torch.equal(out, want)
+    del junk
