@@ -128,19 +128,45 @@ _recording = threading.local()      # .reads: what the `CapturedForward` being m
 class _Kept:
     """What a module keeps between forwards under a key of addresses and versions.  `held` are the tensors behind these
     addresses: as long as they are held no other tensor can come to lie there.  Copies and pickles of the module start
-    without it, as `value` may hold device addresses."""
+    without it, as `value` may hold device addresses.
 
-    __slots__ = ("key", "value", "held")
+    A value is computed by the stream that was current then, and its memory belongs to that stream.  Another stream that
+    takes it up waits for it first, and is noted in its memory's list of users, so that the memory is not handed out
+    again before that stream is done."""
 
-    def __init__(self, key, value, held):
+    __slots__ = ("key", "value", "held", "made", "device", "ready", "streams")
+
+    def __init__(self, key, value, held, made=None):
         self.key, self.value, self.held = key, value, held
+        self.made = _tensors(value if made is None else made)
+        self.device = self.made[0].device if self.made and self.made[0].is_cuda else None
+        if self.device is not None:
+            stream = torch.cuda.current_stream(self.device)
+            self.streams = (stream.cuda_stream,)
+            self.ready = None if torch.cuda.is_current_stream_capturing() else stream.record_event()
+
+    def join(self):
+        """Makes the value usable on the current stream."""
+        if self.device is None or torch._C._cuda_getCurrentRawStream(self.device.index) in self.streams:
+            return
+        stream = torch.cuda.current_stream(self.device)
+        stream.wait_event(self.ready)
+        for t in self.made:
+            t.record_stream(stream)
+        self.streams += (stream.cuda_stream,)
 
     def __reduce__(self):
         return type(None), ()
 
 
+def _tensors(value):
+    """The tensors of a value: one, or a sequence that may hold other things as well."""
+    return [t for t in (value if isinstance(value, (tuple, list)) else (value,)) if isinstance(t, torch.Tensor)]
+
+
 def _kept(table, slot, key, make, lasting=False):
-    """The `_Kept` in `table[slot]`, made by `make()` - (value, tensors to hold) - when there is none under `key`.
+    """The `_Kept` in `table[slot]`, made by `make()` - (value, tensors to hold[, tensors computed for it, if they are not the
+    value]) - when there is none under `key`.
 
     A recorded graph reads the addresses it was recorded with for as long as it is replayed, which a kept value does not
     outlive its key for.  `CapturedForward` holds what its recording reads; any other recording computes it again as a part of
@@ -154,7 +180,9 @@ def _kept(table, slot, key, make, lasting=False):
             return _Kept(key, *make())
         if reads is not None:
             reads.append(kept)
-    elif not hit:
+    elif hit:
+        kept.join()
+    else:
         kept = table[slot] = _Kept(key, *make())     # in a module's __dict__: no parameter, no buffer, not in the state_dict
     return kept
 
@@ -1005,25 +1033,25 @@ class BasicLayer(nn.Module):
                 for blk in self.blocks])
 
         def make():
-            held = [table] + [t.detach() for ts in tensors for t in ts]
+            held, made = [table] + [t.detach() for ts in tensors for t in ts], []
             # the call has one width, hidden layer, number of heads and scale for all blocks
             if not all(blk.fits(c, hidden, h) and blk.attn.num_heads == h and blk.attn.scale == scale
                        and all(_kernel_parameter(t, feat) for t in ts) for blk, ts in zip(self.blocks, tensors)):
-                return (None, None), held
+                return (None, None), held, made
             params = (ops.block_params * len(tensors))()
             for p, blk, ts in zip(params, self.blocks, tensors):
                 bias = blk.attn.bias_table(table)
                 bias = bias.detach().to(dt).contiguous()
-                held.append(bias)
+                made.append(bias)
                 if dt != torch.float32:
                     packed, at = blk._packed(dt)
-                    held.append(packed)
+                    made.append(packed)
                     p.w_qkv, p.w_proj, p.w1, p.w2 = (packed.data_ptr() + o for o in (at[0],) + tuple(at[2:]))
                 (p.norm1_w, p.norm1_b, p.norm2_w, p.norm2_b, p.b_q, p.b_kv, p.b_proj, p.b1, p.b2, p.blank_k,
                  p.blank_v) = (t.data_ptr() for t in ts[:11])
                 p.bias_table, p.eps1, p.eps2 = bias.data_ptr(), blk.norm1.eps, blk.norm2.eps
             layout = ops.block_layout([w.detach() for ts in tensors for w in ts[11:16]]) if dt == torch.float32 else None
-            return (params, layout), held
+            return (params, layout), held, made
 
         kept = _kept(self.__dict__, "_issue_cache", key, make)     # in this frame until the kernels are issued
         params, layout = kept.value

@@ -104,3 +104,34 @@ def test_a_recording_of_the_callers_own(device, amp):
         graph.replay()
         assert torch.equal(out, want)
     del junk
+
+
+def delayed(stream):
+    """Makes `stream` start what comes next some 30 ms late."""
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(60_000_000)
+
+
+@pytest.mark.parametrize("amp", [torch.float16, None])
+def test_kept_values_on_other_streams(device, amp):
+    """What one stream is still to compute another one waits for, and what one stream is still to read is not overwritten when
+    another one drops it."""
+    x = images(device)
+    want = run(build(device), x, amp)
+    net, side = build(device), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    delayed(side)
+    with torch.cuda.stream(side):
+        first = run(net, x, amp)
+    second = run(net, x, amp)                                    # by the lists, tables and weights the other stream makes
+    torch.cuda.synchronize()
+    assert torch.equal(first, want) and torch.equal(second, want)
+    delayed(side)
+    with torch.cuda.stream(side):
+        third = run(net, x, amp)
+    for other in (torch.bfloat16, torch.float16, None):
+        run(net, x, other)
+    junk = [torch.full((1 << k,), float("nan"), device=device) for k in range(6, 22) for _ in range(8)]
+    torch.cuda.synchronize()
+    assert torch.equal(third, want)
+    del junk
