@@ -187,6 +187,16 @@ def _kept(table, slot, key, make, lasting=False):
     return kept
 
 
+class _Module(nn.Module):
+    """A module that drops what it and the modules in it keep, and with it the old parameters it holds, when it is moved or converted."""
+
+    def _apply(self, fn, recurse=True):
+        for mod in self.modules():
+            for slot in [name for name, value in mod.__dict__.items() if type(value) is _Kept]:
+                del mod.__dict__[slot]
+        return super()._apply(fn, recurse)
+
+
 def _cast_params(lin, dt):
     """(weight, bias) of an nn.Linear in dtype `dt` as a `_Kept` value, remade when the parameters change."""
     weight, bias = lin.weight, lin.bias
@@ -556,7 +566,7 @@ class DropPath(nn.Module):
         return torch.empty(samples, dtype=dtype, device=device).bernoulli_(keep).div_(keep)
 
 
-class Mlp(nn.Module):
+class Mlp(_Module):
     def __init__(self, dim, hidden, drop=0.0, ops=None):
         super().__init__()
         self.fc1 = nn.Linear(dim, hidden)
@@ -570,7 +580,7 @@ class Mlp(nn.Module):
         return self.drop(_linear(self.fc2, self.drop(hidden), self.ops))
 
 
-class ClusterAttention(nn.Module):
+class ClusterAttention(_Module):
     """Attention of every token over the members of its nearest clusters, plus one learned blank token."""
 
     def __init__(self, dim, num_heads, attn_drop=0.0, proj_drop=0.0, ops=None):
@@ -698,7 +708,7 @@ class ClusterAttention(nn.Module):
         return out.permute(0, 2, 1, 3).reshape(b, n, c)
 
 
-class ClusterTransformerBlock(nn.Module):
+class ClusterTransformerBlock(_Module):
     def __init__(self, dim, num_heads, mlp_ratio=2.0, drop=0.0, attn_drop=0.0, drop_path=0.0, layer_scale=0.0,
                  ops=None):
         super().__init__()
@@ -834,7 +844,7 @@ def _kernel_parameter(t, feat):
             and t.data_ptr() % 16 == 0)
 
 
-class ClusterMerging(nn.Module):
+class ClusterMerging(_Module):
     """Adaptive down-sampling: keeps ds_rate of the tokens and merges each one's neighbourhood into it."""
 
     INNER = 4
@@ -915,7 +925,7 @@ class ClusterMerging(nn.Module):
         return pos, _linear(self.linear, _layer_norm(self.norm, merged, self.ops, True), self.ops)
 
 
-class BasicLayer(nn.Module):
+class BasicLayer(_Module):
     """One stage: neighbourhood lists, `depth` blocks over them, optional merging into the next stage."""
 
     def __init__(self, dim, out_dim, cluster_size, nbhd_size, depth, num_heads, mlp_ratio, alpha=4.0, ds_rate=0.25,
@@ -1149,7 +1159,7 @@ class BasicLayer(nn.Module):
         return pos, feat
 
 
-class PatchEmbed(nn.Module):
+class PatchEmbed(_Module):
     """Two stride-2 3x3 convolutions (BatchNorm + GELU between them): one token per 4x4 pixels."""
 
     def __init__(self, in_chans=3, embed_dim=32, patch_norm=True, ops=None):
@@ -1222,7 +1232,7 @@ class PatchEmbed(nn.Module):
         return pos.expand(b, -1, -1).to(tokens.dtype), tokens, h, w, False
 
 
-class AutoFocusFormer(nn.Module):
+class AutoFocusFormer(_Module):
     """aff_transformer.py:560-670.  Defaults are the reference's; `aff_tiny()` gives configs/aff_tiny.yaml."""
 
     def __init__(self, in_chans=3, num_classes=1000, embed_dim=(32, 128, 256, 512), cluster_size=8,

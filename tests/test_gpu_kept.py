@@ -135,3 +135,20 @@ def test_kept_values_on_other_streams(device, amp):
     torch.cuda.synchronize()
     assert torch.equal(third, want)
     del junk
+
+
+@pytest.mark.parametrize("amp", [torch.float16, None])
+def test_a_model_that_leaves_takes_everything_along(device, amp):
+    """Moved to the CPU a model leaves nothing behind but the lists of its grid."""
+    x = images(device)
+    run(build(device, seed=7), x, amp)                           # library workspaces
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    net = build(device)
+    want = run(net, x, amp)
+    net.cpu()
+    grid = [t for layer in net.layers for kept in layer._grid_cache.values() for t in kept.made]
+    lists = sum({t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() + 512 for t in grid}.values())
+    # 512: allocations are rounded up; the result of the forward, the table of positions
+    assert torch.cuda.memory_allocated() - before <= lists + 512 * 2
+    assert torch.equal(run(net.to(device), x, amp), want)
