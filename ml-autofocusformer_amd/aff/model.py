@@ -566,6 +566,11 @@ class DropPath(nn.Module):
         return torch.empty(samples, dtype=dtype, device=device).bernoulli_(keep).div_(keep)
 
 
+def _drops(mod):
+    """True for a Dropout or DropPath that drops: by its own mode, which need not be that of the layer it is in."""
+    return mod.training and type(mod) is not nn.Identity and mod.p > 0
+
+
 class Mlp(_Module):
     def __init__(self, dim, hidden, drop=0.0, ops=None):
         super().__init__()
@@ -615,7 +620,7 @@ class ClusterAttention(_Module):
         h = self.num_heads
         return (getattr(self.ops, "cluster_attention_backward", None) is not None and torch.is_grad_enabled()
                 and cluster_idx is not None and not global_attn and self.cluster_size == 8 and grid_lists is not None
-                and len(grid_lists) > 4 and not (self.training and self.attn_drop.p > 0)
+                and len(grid_lists) > 4 and not _drops(self.attn_drop)
                 and self.ops.cluster_attention_backward_supported(q.view(b, n, h, c // h).permute(0, 2, 1, 3), cluster_idx.shape[2]))
 
     def attend_rows(self, qkv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None):
@@ -640,7 +645,7 @@ class ClusterAttention(_Module):
         sized = {} if self.cluster_size == 8 else {"cluster_size": self.cluster_size}
         key, v = kv.view(b, n, h, 2, ch).permute(3, 0, 2, 1, 4).unbind(0)                                   # (b,h,n,ch) views
         one_kernel = getattr(self.ops, "cluster_attention", None)
-        if (numbered and one_kernel is not None and not (self.training and self.attn_drop.p > 0)
+        if (numbered and one_kernel is not None and not _drops(self.attn_drop)
                 and self.ops.cluster_attention_supported(q.view(b, n, h, ch).permute(0, 2, 1, 3), cluster_idx.shape[2],
                                                          self.cluster_size)):
             # inference on 16-bit or fp32 data: scores, position bias, mask, blank token, softmax and the weighted sum
@@ -660,7 +665,7 @@ class ClusterAttention(_Module):
             return out
         dense = getattr(self.ops, "dense_attention", None)
         if (global_attn and dense is not None and not torch.is_grad_enabled()
-                and not (self.training and self.attn_drop.p > 0)
+                and not _drops(self.attn_drop)
                 and self.ops.dense_attention_supported(q.view(b, n, h, ch).permute(0, 2, 1, 3))):
             # inference on 16-bit data, every token attending to every token: one kernel as well
             out = dense(q.view(b, n, h, ch).permute(0, 2, 1, 3), key, v, self.bias_table(table), pe_idx,
@@ -678,7 +683,7 @@ class ClusterAttention(_Module):
         bias = self.bias_table(table)                                                     # (rows, h)
         fused = getattr(self.ops, "attn_softmax", None)
         if (fused is not None and not global_attn and not torch.is_grad_enabled()
-                and not (self.training and self.attn_drop.p > 0) and self.ops.attn_softmax_supported(attn, attn.shape[-1])):
+                and not _drops(self.attn_drop) and self.ops.attn_softmax_supported(attn, attn.shape[-1])):
             # inference: bias gather, mask, blank-token logit and softmax in one kernel
             attn, blank = fused(attn, bias, pe_idx, cluster_mask, query=q, blank_key=self.blank_k)
         else:
@@ -686,7 +691,7 @@ class ClusterAttention(_Module):
             if (fused is not None and getattr(self.ops, "attn_softmax_backward", None) is not None
                     and getattr(self.ops, "bias_table_grad", None) is not None and torch.is_grad_enabled()
                     and not global_attn and attn.is_cuda
-                    and not (self.training and self.attn_drop.p > 0)
+                    and not _drops(self.attn_drop)
                     and self.ops.attn_softmax_supported(attn, attn.shape[-1])):
                 # training: the same glue as one kernel forward and one backward
                 attn, blank = _AttnSoftmax.apply(attn, bias, pe_idx, cluster_mask, blank, self.ops)
@@ -730,8 +735,7 @@ class ClusterTransformerBlock(_Module):
         if self.layer_scale or not feat.is_cuda or getattr(ops, "block_tail", None) is None or not self.plain():
             return None
         grad = torch.is_grad_enabled()
-        if self.training and (self.mlp.drop.p > 0 or self.attn.proj_drop.p > 0
-                              or not (grad or isinstance(self.drop_path, nn.Identity))):
+        if _drops(self.mlp.drop) or _drops(self.attn.proj_drop) or (not grad and _drops(self.drop_path)):
             return None
         dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else torch.float32
         if (not ops.block_supported(feat, dt, self.mlp.fc1.out_features) or (grad and (_transformed() or feat.numel() == 0))
@@ -809,7 +813,7 @@ class ClusterTransformerBlock(_Module):
                                               attn.kv.bias, norm1.eps, dt, ops)
             a = attn.attend_rows(qkv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
             scale = None
-            if self.training and isinstance(self.drop_path, DropPath) and self.drop_path.p > 0:
+            if _drops(self.drop_path):
                 scale = torch.stack([self.drop_path.factors(feat.shape[0], dt, feat.device) for _ in range(2)]).float()
             return _BlockTail.apply(a.to(dt).contiguous(), feat, attn.proj.weight, attn.proj.bias, norm2.weight, norm2.bias,
                                     mlp.fc1.weight, mlp.fc1.bias, mlp.fc2.weight, mlp.fc2.bias, scale, norm2.eps, dt, ops), None
@@ -1025,7 +1029,8 @@ class BasicLayer(_Module):
         if any(type(blk) is not ClusterTransformerBlock or blk._forward_hooks or blk._forward_pre_hooks or blk.layer_scale
                or not blk.plain() for blk in self.blocks):
             return None
-        if self.training and any(blk._fused_dtype(feat) is None or blk.attn.attn_drop.p > 0 for blk in self.blocks):
+        if any(_drops(blk.attn.attn_drop) or _drops(blk.attn.proj_drop) or _drops(blk.mlp.drop) or _drops(blk.drop_path)
+               for blk in self.blocks):
             return None
         if global_attn:
             if n > 64 or dt == torch.float32:

@@ -193,3 +193,25 @@ def test_models_copied_and_changed_after_a_forward(device):
     calls = []
     blk.register_forward_hook(lambda *_: calls.append(1))        # with a hook every block is called by itself
     assert torch.equal(out, run(net)) and calls
+
+
+def test_stages_with_active_dropout_are_not_issued_by_one_call(device):
+    """Dropout in training mode somewhere in a model in eval mode drops."""
+    from aff.model import AutoFocusFormer, default_ops
+    torch.manual_seed(0)
+    net = AutoFocusFormer(img_size=96, embed_dim=(32, 64, 128, 256), num_heads=(1, 2, 4, 8), depths=(1, 2, 2, 1), mlp_ratio=2.0,
+                          nbhd_size=(48, 48, 48, 48), num_classes=40, drop_rate=0.5, attn_drop_rate=0.5, drop_path_rate=0.5,
+                          ops=default_ops()).to(device).eval()
+    x = torch.randn(2, 3, 96, 96, generator=torch.Generator().manual_seed(1)).to(device)
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16):
+            return net(x)
+
+    plain = run()
+    for name in ("mlp.drop", "attn.proj_drop", "attn.attn_drop", "drop_path"):
+        for stage in (1, 2):                                     # local and global attention; the stages' second blocks
+            net.layers[stage].blocks[1].get_submodule(name).train()
+            assert not torch.equal(run(), plain), (name, stage)
+            net.eval()
+            assert torch.equal(run(), plain)

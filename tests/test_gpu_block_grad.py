@@ -211,3 +211,30 @@ def test_forward_mode(device):
     with torch.autograd.forward_ad.dual_level():
         out, branch = call(torch.autograd.forward_ad.make_dual(feat, torch.ones_like(feat)))
         assert torch.autograd.forward_ad.unpack_dual(out + branch).tangent is not None
+
+
+@pytest.mark.parametrize("grad", [True, False])
+def test_dropout_follows_its_own_mode(device, grad):
+    """Dropout of a block in eval mode that is itself in training mode drops (Monte-Carlo dropout), and stochastic depth of a
+    training block that is itself in eval mode does not."""
+    torch.manual_seed(0)
+    blk = ClusterTransformerBlock(64, 2, drop=0.5, attn_drop=0.5, drop_path=0.9, ops=default_ops()).to(device).eval()
+    feat, table = torch.randn(8, 36, 64, device=device), torch.randn(121, 5, device=device)
+    pe_idx = torch.randint(121, (8, 36, 36), device=device)
+
+    def call():
+        with torch.set_grad_enabled(grad):
+            out, branch = blk(feat, None, None, pe_idx, True, table)
+            return (out if branch is None else out + branch).detach()
+
+    plain = call()
+    for name in ("mlp.drop", "attn.proj_drop", "attn.attn_drop"):
+        blk.get_submodule(name).train()
+        assert norm_error(call(), plain) > 1e-2, name
+        blk.eval()
+    blk.train()
+    for name in ("mlp.drop", "attn.proj_drop", "attn.attn_drop", "drop_path"):
+        blk.get_submodule(name).eval()
+    assert norm_error(call(), plain) < 1e-5
+    blk.drop_path.train()
+    assert norm_error(call(), plain) > 1e-2
