@@ -765,15 +765,21 @@ class ClusterTransformerBlock(_Module):
 
     def tensors(self):
         """The parameters of the block in one tuple, straight from the modules' tables: the look-ups of 30 blocks are a
-        visible part of a small forward's host time."""
+        visible part of a small forward's host time.  Where one is not in its table - replicas and wrappers set plain
+        attributes - all come by attribute."""
         m = self._modules
         attn, mlp = m["attn"], m["mlp"]
-        n1, n2, a, ml, ap = m["norm1"]._parameters, m["norm2"]._parameters, attn._modules, mlp._modules, attn._parameters
-        q, kv, proj, pe = (a[k]._parameters for k in ("q", "kv", "proj", "pos_embed"))
-        f1, f2 = ml["fc1"]._parameters, ml["fc2"]._parameters
-        return (n1["weight"], n1["bias"], n2["weight"], n2["bias"], q["bias"], kv["bias"], proj["bias"], f1["bias"], f2["bias"],
-                ap["blank_k"], ap["blank_v"], q["weight"], kv["weight"], proj["weight"], f1["weight"], f2["weight"],
-                pe["weight"], pe["bias"])
+        a, ml = attn._modules, mlp._modules
+        mods = m["norm1"], m["norm2"], a["q"], a["kv"], a["proj"], ml["fc1"], ml["fc2"], attn, a["pos_embed"]
+        n1, n2, q, kv, proj, f1, f2, ap, pe = (mod._parameters for mod in mods)
+        try:
+            return (n1["weight"], n1["bias"], n2["weight"], n2["bias"], q["bias"], kv["bias"], proj["bias"], f1["bias"], f2["bias"],
+                    ap["blank_k"], ap["blank_v"], q["weight"], kv["weight"], proj["weight"], f1["weight"], f2["weight"],
+                    pe["weight"], pe["bias"])
+        except KeyError:
+            n1, n2, q, kv, proj, f1, f2, ap, pe = mods
+            return (n1.weight, n1.bias, n2.weight, n2.bias, q.bias, kv.bias, proj.bias, f1.bias, f2.bias, ap.blank_k, ap.blank_v,
+                    q.weight, kv.weight, proj.weight, f1.weight, f2.weight, pe.weight, pe.bias)
 
     def _packed(self, dt):
         """(weights of the five Linear layers as the block kernels read them, byte offset of each).  16-bit ones are kept until a

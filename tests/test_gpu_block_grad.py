@@ -238,3 +238,18 @@ def test_dropout_follows_its_own_mode(device, grad):
     assert norm_error(call(), plain) < 1e-5
     blk.drop_path.train()
     assert norm_error(call(), plain) > 1e-2
+
+
+@pytest.mark.parametrize("grad", [True, False])
+def test_parameters_that_are_plain_attributes(device, grad):
+    """A replica, as `nn.DataParallel` makes them: no entries in the modules' tables of parameters."""
+    blk, feat, call = dense_block(device)
+    replica, = torch.nn.parallel.replicate(blk, [device])
+    args = (None, None, torch.randint(121, (2, 36, 36), device=device), True, torch.randn(121, 5, device=device))
+    assert not replica.norm1._parameters
+    with torch.set_grad_enabled(grad):
+        (want, _), (got, branch) = blk(feat, *args), replica(feat, *args)
+        assert branch is None and torch.equal(got, want)                # the block kernels, for the replica too
+        if grad:
+            got.square().sum().backward()
+            assert blk.mlp.fc1.weight.grad.norm() > 0 and blk.attn.blank_k.grad.norm() > 0
