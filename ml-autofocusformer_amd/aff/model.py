@@ -74,6 +74,19 @@ def default_ops():
                                              ("norm_linear", _native.norm_linear), ("block_tail", _native.block_tail)))
 
 
+def _by_kernels(*grads):
+    """True when a backward pass may hand its incoming gradients to kernels: it is not itself recorded, and they are no batch of
+    gradients (`is_grads_batched`), which has no memory to point at."""
+    if torch.is_grad_enabled():
+        return False
+    try:
+        for g in grads:
+            g.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
 class _Linear(torch.autograd.Function):
     """`F.linear(x, weight, bias)` in x's dtype for parameters of any, with the parameters' gradients from the library's kernel:
     both in one pass over the rows, in fp32 (not rounded to 16 bits on the way to fp32 parameters)."""
@@ -91,7 +104,7 @@ class _Linear(torch.autograd.Function):
         need_x, need_w, need_b = ctx.needs_input_grad[:3]
         d_x = d_y @ weight.to(x.dtype) if need_x else None
         rows, x_rows = d_y.reshape(-1, d_y.shape[-1]), x.reshape(-1, x.shape[-1])
-        if need_w and not torch.is_grad_enabled():       # (a backward that is itself recorded stays with recorded operations)
+        if need_w and _by_kernels(d_y):
             if not supported(rows, x_rows):
                 rows = rows.contiguous()                 # e.g. the gradient of a column range
             if supported(rows, x_rows):
@@ -301,6 +314,10 @@ class _PositionBias(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad):
         (pe_idx,) = ctx.saved_tensors
+        if not _by_kernels(grad):
+            rows = grad.permute(0, 2, 3, 1).reshape(-1, grad.shape[1])
+            table = torch.zeros(ctx.rows, grad.shape[1], dtype=torch.float32, device=grad.device)
+            return table.scatter_add(0, pe_idx.reshape(-1, 1).expand(-1, grad.shape[1]), rows.float()).to(ctx.dtype), None, None
         return ctx.grad_kernel(grad, pe_idx, ctx.rows).to(ctx.dtype), None, None
 
 
@@ -360,7 +377,7 @@ class _ClusterAttention(torch.autograd.Function):
 
 
 def _recorded_backward(fn, ctx, tensors, grads):
-    """The gradients of `fn(*tensors)` by recorded operations, for a backward pass that is itself differentiated."""
+    """The gradients of `fn(*tensors)` by recorded operations, for a backward pass that is itself differentiated or batched."""
     needs = ctx.needs_input_grad[:len(tensors)]
     with torch.enable_grad(), torch.autocast("cuda", enabled=False):
         out = fn(*tensors)
@@ -390,7 +407,7 @@ class _NormLinearRows(torch.autograd.Function):
         x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, normed, stats, w = ctx.saved_tensors
         eps, dt, ops = ctx.meta
         c = x.shape[-1]
-        if torch.is_grad_enabled():
+        if not _by_kernels(d_qkv, d_res):
             def layers(x, norm_w, norm_b, w_q, b_q, w_kv, b_kv):
                 y = F.layer_norm(x.float(), (c,), norm_w, norm_b, eps).to(dt)
                 return F.linear(y, torch.cat([w_q, w_kv]).to(dt), torch.cat([b_q, b_kv]).to(dt)), x
@@ -427,7 +444,7 @@ class _BlockTail(torch.autograd.Function):
         attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, x1, normed, hidden, stats, plain = ctx.saved_tensors
         eps, dt, ops = ctx.meta
         b, c, h = x.shape[0], x.shape[-1], hidden.shape[-1]
-        if torch.is_grad_enabled():
+        if not _by_kernels(d_out):
             def layers(attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2):
                 s = (1.0, 1.0) if scale is None else scale.to(dt).view(2, b, *(1,) * (x.dim() - 1))
                 x1 = x + (F.linear(attn, w_p.to(dt), b_p.to(dt)) * s[0]).to(x.dtype)

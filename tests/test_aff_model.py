@@ -924,3 +924,24 @@ def test_training_with_the_one_kernel_attention_matches_the_operator_path(device
         seen.add(f)
         stack.extend(nf for nf, _ in f.next_functions)
     assert any("_ClusterAttention" in type(f).__name__ for f in seen)
+
+
+def test_linear_layers_take_batched_gradients():
+    """`is_grads_batched` hands the backward pass of a training Linear a batch of gradients, which has no address."""
+    from aff.model import _Linear
+    asked = []
+
+    def supported(d_y, x):
+        asked.append(d_y.data_ptr())
+        return False
+
+    gen = torch.Generator().manual_seed(1)
+    x, w, b = (torch.randn(*shape, generator=gen, requires_grad=True) for shape in ((6, 8), (16, 8), (16,)))
+    batch = torch.randn(3, 6, 16, generator=gen)
+    got = torch.autograd.grad(_Linear.apply(x, w, b, None, supported), (x, w, b), batch, is_grads_batched=True)
+    want = torch.autograd.grad(torch.nn.functional.linear(x, w, b), (x, w, b), batch, is_grads_batched=True)
+    assert not asked
+    for g, ref in zip(got, want):
+        torch.testing.assert_close(g, ref)
+    torch.autograd.grad(_Linear.apply(x, w, b, None, supported), (x, w, b), batch[0])
+    assert asked

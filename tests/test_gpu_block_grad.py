@@ -253,3 +253,17 @@ def test_parameters_that_are_plain_attributes(device, grad):
         if grad:
             got.square().sum().backward()
             assert blk.mlp.fc1.weight.grad.norm() > 0 and blk.attn.blank_k.grad.norm() > 0
+
+
+def test_batched_gradients(device):
+    """`is_grads_batched` through a training block: each row as by itself."""
+    blk, feat, call = dense_block(device)
+    x = feat.clone().requires_grad_(True)
+    wanted = [x] + list(blk.parameters())
+    batch = torch.randn(3, *feat.shape, generator=torch.Generator(device).manual_seed(1), device=device)
+    out, branch = call(x)
+    assert branch is None                                            # the block kernels ran
+    got = torch.autograd.grad(out, wanted, batch, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for g, ref in zip(got, torch.autograd.grad(out, wanted, batch[i], retain_graph=True)):
+            assert norm_error(g[i], ref) < 1e-5
