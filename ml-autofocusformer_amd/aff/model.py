@@ -342,6 +342,32 @@ class _AttnSoftmax(torch.autograd.Function):
         return d_logit, d_bias, None, None, d_blank.to(blank_dtype), None
 
 
+def _recorded_backward(fn, ctx, tensors, grads):
+    """The gradients of `fn(*tensors)` by recorded operations, for a backward pass that is itself differentiated or batched."""
+    needs = ctx.needs_input_grad[:len(tensors)]
+    with torch.enable_grad(), torch.autocast("cuda", enabled=False):
+        out = fn(*tensors)
+        out, grads = zip(*((o, g) for o, g in zip(out if isinstance(out, tuple) else (out,), grads) if o.requires_grad))
+        wanted = torch.autograd.grad(out, [t for t, need in zip(tensors, needs) if need], grads, create_graph=True, allow_unused=True)
+    wanted = iter(wanted)
+    return [next(wanted) if need else None for need in needs]
+
+
+def _local_attention(q, key, v, bias, blank_k, blank_v, mask, pe_idx, member_idx, scale):
+    """The local attention of a block in recorded operations, fp32 inside: what the kernel computes (aff_transformer.py:120-155)."""
+    b, h, n, ch = q.shape
+    m = member_idx.shape[-1]
+    rows = member_idx.reshape(b, 1, n * m, 1).expand(-1, h, -1, ch)
+    dtype = q.dtype
+    q, key, v, bias, blank_k, blank_v = (t.float() for t in (q, key, v, bias, blank_k.reshape(1, h, 1, ch), blank_v.reshape(1, h, 1, ch)))
+    logits = (q.unsqueeze(3) * key.gather(2, rows).view(b, h, n, m, ch)).sum(-1) * scale + _table_rows(bias, pe_idx).permute(0, 3, 1, 2)
+    if mask is not None:
+        logits = logits + (1 - mask.reshape(b, 1, n, m)) * (-100)
+    probs = torch.softmax(torch.cat([logits, (q * blank_k).sum(-1, keepdim=True) * scale], dim=-1), dim=-1)
+    out = (probs[..., :-1, None] * v.gather(2, rows).view(b, h, n, m, ch)).sum(3) + probs[..., -1:] * blank_v
+    return out.permute(0, 2, 1, 3).reshape(b, n, h * ch).to(dtype)
+
+
 class _ClusterAttention(torch.autograd.Function):
     """The local attention of a block between its projections (aff_transformer.py:120-155) as one kernel forward and,
     backward, one kernel for the query side - the probabilities are recomputed from the softmax denominators the
@@ -352,17 +378,20 @@ class _ClusterAttention(torch.autograd.Function):
     are complete sums whatever `member_idx` holds."""
 
     @staticmethod
-    def forward(ctx, q, key, v, bias, blank_k, blank_v, plan, pairs, pe_idx, member_idx, scale, ops):
+    def forward(ctx, q, key, v, bias, blank_k, blank_v, plan, pairs, pe_idx, member_idx, mask, scale, ops):
         out, lse = ops.cluster_attention(q, key, v, None, bias, None, None, blank_k, blank_v, scale=scale, plan=plan,
                                          return_lse=True)
-        ctx.save_for_backward(q, key, v, out, lse, bias, blank_k, blank_v, plan, pairs, pe_idx, member_idx)
+        ctx.save_for_backward(q, key, v, out, lse, bias, blank_k, blank_v, plan, pairs, pe_idx, member_idx, mask)
         ctx.meta = (scale, ops)
         return out
 
     @staticmethod
     def backward(ctx, d_out):
-        q, key, v, out, lse, bias, blank_k, blank_v, plan, pairs, pe_idx, member_idx = ctx.saved_tensors
+        q, key, v, out, lse, bias, blank_k, blank_v, plan, pairs, pe_idx, member_idx, mask = ctx.saved_tensors
         scale, ops = ctx.meta
+        if not _by_kernels(d_out):
+            return (*_recorded_backward(lambda *t: _local_attention(*t, mask, pe_idx, member_idx, scale), ctx,
+                                        (q, key, v, bias, blank_k, blank_v), (d_out,)), *(None,) * 7)
         b, h, n, ch = q.shape
         d_q, probs, d_logit, blank_prob, d_blank = ops.cluster_attention_backward(
             q, key, v, d_out, out, lse, plan, bias, blank_k, blank_v, scale=scale)
@@ -373,18 +402,7 @@ class _ClusterAttention(torch.autograd.Function):
         d_bk = torch.einsum("bhn,bhnc->hc", d_blank, q.float()) * scale
         d_bv = torch.einsum("bhn,bhnc->hc", blank_prob, g.float())
         return (d_q, d_k.to(key.dtype), d_v.to(v.dtype), d_bias, d_bk.reshape(blank_k.shape).to(blank_k.dtype),
-                d_bv.reshape(blank_v.shape).to(blank_v.dtype), None, None, None, None, None, None)
-
-
-def _recorded_backward(fn, ctx, tensors, grads):
-    """The gradients of `fn(*tensors)` by recorded operations, for a backward pass that is itself differentiated or batched."""
-    needs = ctx.needs_input_grad[:len(tensors)]
-    with torch.enable_grad(), torch.autocast("cuda", enabled=False):
-        out = fn(*tensors)
-        out, grads = zip(*((o, g) for o, g in zip(out if isinstance(out, tuple) else (out,), grads) if o.requires_grad))
-        wanted = torch.autograd.grad(out, [t for t, need in zip(tensors, needs) if need], grads, create_graph=True, allow_unused=True)
-    wanted = iter(wanted)
-    return [next(wanted) if need else None for need in needs]
+                d_bv.reshape(blank_v.shape).to(blank_v.dtype), *(None,) * 7)
 
 
 class _NormLinearRows(torch.autograd.Function):
@@ -481,21 +499,26 @@ class _ClusterAttentionRows(torch.autograd.Function):
     of q, k and v go into one tensor of that form, the blank token's and the bias layer's come from kernels of their own."""
 
     @staticmethod
-    def forward(ctx, qkv, table, pe_w, pe_b, blank_k, blank_v, plan, pairs, pe_idx, member_idx, heads, scale, ops):
+    def forward(ctx, qkv, pe_w, pe_b, blank_k, blank_v, table, plan, pairs, pe_idx, member_idx, mask, heads, scale, ops):
         dt = qkv.dtype
         table = table.to(dt)
         bias = F.linear(table, pe_w.to(dt), pe_b.to(dt))
         q, key, v = _columns(qkv, heads)
         out, lse = ops.cluster_attention(q, key, v, None, bias, None, None, blank_k, blank_v, scale=scale, plan=plan,
                                          return_lse=True)
-        ctx.save_for_backward(qkv, out, lse, bias, table, blank_k, blank_v, plan, pairs, pe_idx, member_idx)
-        ctx.meta = (heads, scale, pe_w.dtype, pe_b.dtype, ops)
+        ctx.save_for_backward(qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, table, plan, pairs, pe_idx, member_idx, mask)
+        ctx.meta = (heads, scale, ops)
         return out
 
     @staticmethod
     def backward(ctx, d_out):
-        qkv, out, lse, bias, table, blank_k, blank_v, plan, pairs, pe_idx, member_idx = ctx.saved_tensors
-        heads, scale, w_dtype, b_dtype, ops = ctx.meta
+        qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, table, plan, pairs, pe_idx, member_idx, mask = ctx.saved_tensors
+        heads, scale, ops = ctx.meta
+        if not _by_kernels(d_out):
+            def layers(qkv, pe_w, pe_b, blank_k, blank_v):
+                bias = F.linear(table, pe_w.to(table.dtype), pe_b.to(table.dtype))
+                return _local_attention(*_columns(qkv, heads), bias, blank_k, blank_v, mask, pe_idx, member_idx, scale)
+            return (*_recorded_backward(layers, ctx, (qkv, pe_w, pe_b, blank_k, blank_v), (d_out,)), *(None,) * 9)
         q, key, v = _columns(qkv, heads)
         d_out = d_out.to(qkv.dtype).contiguous()
         d_qkv = torch.empty_like(qkv)
@@ -506,8 +529,8 @@ class _ClusterAttentionRows(torch.autograd.Function):
         d_k = ops.scatter_rows(d_logit, q, member_idx, pairs)
         d_bk, d_bv = ops.attention_columns_backward(qkv, d_qkv, d_k, d_v, d_out, d_blank, blank_prob, scale)
         d_w, d_b = ops.table_linear_grad(ops.bias_table_grad(d_logit, pe_idx, bias.shape[0]), table)
-        return (d_qkv, None, d_w.to(w_dtype), d_b.to(b_dtype), d_bk.reshape(blank_k.shape).to(blank_k.dtype),
-                d_bv.reshape(blank_v.shape).to(blank_v.dtype), None, None, None, None, None, None, None)
+        return (d_qkv, d_w.to(pe_w.dtype), d_b.to(pe_b.dtype), d_bk.reshape(blank_k.shape).to(blank_k.dtype),
+                d_bv.reshape(blank_v.shape).to(blank_v.dtype), *(None,) * 9)
 
 
 def _columns(qkv, heads):
@@ -645,8 +668,8 @@ class ClusterAttention(_Module):
         c = self.dim
         pe = self.pos_embed
         if self._trains_in_one_kernel(qkv[..., :c], global_attn, cluster_idx, grid_lists) and not table.requires_grad:
-            return _ClusterAttentionRows.apply(qkv, table, pe.weight, pe.bias, self.blank_k, self.blank_v, grid_lists[3],
-                                               grid_lists[4], pe_idx, member_idx, self.num_heads, self.scale, self.ops)
+            return _ClusterAttentionRows.apply(qkv, pe.weight, pe.bias, self.blank_k, self.blank_v, table, grid_lists[3],
+                                               grid_lists[4], pe_idx, member_idx, cluster_mask, self.num_heads, self.scale, self.ops)
         q, kv = qkv.split([c, 2 * c], dim=-1)
         return self.attend(q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
 
@@ -678,7 +701,7 @@ class ClusterAttention(_Module):
             bias = self.bias_table(table)
             out = _ClusterAttention.apply(q.view(b, n, h, ch).permute(0, 2, 1, 3), key, v, bias, self.blank_k,
                                           self.blank_v, grid_lists[3], grid_lists[4], pe_idx, member_idx,
-                                          self.scale, self.ops)
+                                          cluster_mask, self.scale, self.ops)
             return out
         dense = getattr(self.ops, "dense_attention", None)
         if (global_attn and dense is not None and not torch.is_grad_enabled()

@@ -12,7 +12,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from aff.model import AutoFocusFormer, ClusterTransformerBlock, default_ops
+from aff.model import AutoFocusFormer, BasicLayer, ClusterTransformerBlock, default_ops, relative_position_table
 from clusten import _native
 
 pytestmark = pytest.mark.gpu
@@ -132,6 +132,7 @@ def step(net, dt, device, seed=3):
 
 
 def norm_error(got, ref):
+    got, ref = got.detach(), ref.detach()
     return float((got.double() - ref.double()).norm() / ref.double().norm().clamp(min=1e-30))
 
 
@@ -267,3 +268,59 @@ def test_batched_gradients(device):
     for i in range(3):
         for g, ref in zip(got, torch.autograd.grad(out, wanted, batch[i], retain_graph=True)):
             assert norm_error(g[i], ref) < 1e-5
+
+
+def gathered(t, idx):
+    b, h, n, c = t.shape
+    m = idx.shape[-1]
+    return t.gather(2, idx.reshape(b, 1, n * m, 1).expand(-1, h, -1, c)).view(b, h, n, m, c)
+
+
+RECORDED = SimpleNamespace(qk=lambda q, k, idx: (q.unsqueeze(3) * gathered(k, idx)).sum(-1),
+                           av=lambda a, v, idx: (a.unsqueeze(-1) * gathered(v, idx)).sum(3), wf=None)
+
+
+def local_stage(device, ops):
+    """Two blocks on 100 tokens: a short last cluster, pad slots and a mask."""
+    torch.manual_seed(3)
+    stage = BasicLayer(64, None, 8, 48, 2, 2, 2.0, downsample=False, ops=ops).to(device)
+    ys, xs = torch.meshgrid(torch.arange(10.0), torch.arange(10.0), indexing="ij")
+    pos = torch.stack([xs, ys], 2).reshape(1, 100, 2).expand(2, -1, -1).to(device)
+    table, radius = relative_position_table(40)
+    feat = torch.randn(2, 100, 64, device=device)
+    table = table.to(device)
+    return stage, feat, lambda x: stage(pos, x, 10, 10, False, 2, table, radius)[1]
+
+
+# one Function for the attention's rows, and, where the block kernels are not there, one for its query, key and value
+@pytest.mark.parametrize("layered", [False, True])
+def test_second_derivatives_of_local_attention(device, layered):
+    """Against the same stage in operations that autograd records, all terms of every parameter; and a batch of gradients."""
+    ops = SimpleNamespace(**{**vars(default_ops()), **({"block_tail": None} if layered else {})})
+    results = []
+    for these in (ops, RECORDED):
+        stage, feat, call = local_stage(device, these)
+        x = feat.clone().requires_grad_(True)
+        out = call(x)
+        names = {type(f).__name__ for f in walk(out.grad_fn)}
+        assert ("_ClusterAttentionBackward" in names) == (layered and these is ops)
+        assert ("_ClusterAttentionRowsBackward" in names) == (not layered and these is ops)
+        wanted = [x] + list(stage.parameters())
+        first = torch.autograd.grad(out.square().sum(), wanted, create_graph=True)
+        second = torch.autograd.grad(sum(g.square().sum() for g in first), wanted)
+        batch = torch.randn(2, *out.shape, generator=torch.Generator(device).manual_seed(1), device=device)
+        batched = torch.autograd.grad(call(x), wanted, batch, is_grads_batched=True)
+        results.append((first, second, batched))
+    for kind, got, ref in zip(("first", "second", "batched"), *results):
+        for (name, _), g, r in zip([("x", None)] + list(stage.named_parameters()), got, ref):
+            assert norm_error(g, r) < 1e-4, (kind, name)
+
+
+def walk(node):
+    seen, todo = set(), [node]
+    while todo:
+        f = todo.pop()
+        if f is not None and f not in seen:
+            seen.add(f)
+            todo += [g for g, _ in f.next_functions]
+    return seen
