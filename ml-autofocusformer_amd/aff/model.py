@@ -115,8 +115,8 @@ class _Linear(torch.autograd.Function):
 
 
 def _hooked(mod):
-    """True when calling `mod` runs more than its `forward`."""
-    return bool(mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
+    """True when calling `mod` runs more than its class' `forward`, or another one that was set on the module itself."""
+    return bool("forward" in mod.__dict__ or mod._forward_hooks or mod._forward_pre_hooks or mod._backward_hooks or mod._backward_pre_hooks
                 or _module._global_forward_hooks or _module._global_forward_pre_hooks or _module._global_backward_hooks
                 or _module._global_backward_pre_hooks)
 
@@ -784,7 +784,7 @@ class ClusterTransformerBlock(_Module):
         return dt if all(getattr(ops, name, None) is fn for name, fn in ops.block_stands_for) else None
 
     def plain(self):
-        """True when calling the block's modules runs their own `forward` and nothing else."""
+        """True when calling the block's modules runs the `forward` of their classes and nothing else."""
         m = self._modules
         attn, mlp = m["attn"], m["mlp"]
         a, ml = attn._modules, mlp._modules
@@ -797,10 +797,10 @@ class ClusterTransformerBlock(_Module):
                 return False
             for mod in mods:
                 d = mod.__dict__
-                if d["_forward_hooks"] or d["_forward_pre_hooks"]:
+                if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
                     return False
             d = m["drop_path"].__dict__
-            return not (d["_forward_hooks"] or d["_forward_pre_hooks"])
+            return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d)
         return not (any(map(_hooked, mods)) or _hooked(m["drop_path"]))
 
     def tensors(self):
@@ -1072,8 +1072,8 @@ class BasicLayer(_Module):
         if dt is None or c != 32 * h or any(getattr(ops, name, None) is not fn for name, fn in ops.blocks_stand_for) or (
                 dt == torch.float32 and getattr(ops, "block_layout", None) is None):
             return None
-        if any(type(blk) is not ClusterTransformerBlock or blk._forward_hooks or blk._forward_pre_hooks or blk.layer_scale
-               or not blk.plain() for blk in self.blocks):
+        if any(type(blk) is not ClusterTransformerBlock or blk._forward_hooks or blk._forward_pre_hooks or "forward" in blk.__dict__
+               or blk.layer_scale or not blk.plain() for blk in self.blocks):
             return None
         if any(_drops(blk.attn.attn_drop) or _drops(blk.attn.proj_drop) or _drops(blk.mlp.drop) or _drops(blk.drop_path)
                for blk in self.blocks):

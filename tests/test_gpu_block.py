@@ -193,6 +193,11 @@ def test_models_copied_and_changed_after_a_forward(device):
     calls = []
     blk.register_forward_hook(lambda *_: calls.append(1))        # with a hook every block is called by itself
     assert torch.equal(out, run(net)) and calls
+    blk = net.layers[1].blocks[2]
+    blk.forward = lambda *a, f=blk.forward: (calls.clear(), f(*a))[1]
+    assert torch.equal(out, run(net)) and len(calls) == 1        # by the hooked block behind it only
+    blk.mlp.forward = lambda x, f=blk.mlp.forward: 0 * f(x)
+    assert not torch.equal(out, run(net))
 
 
 def test_stages_with_active_dropout_are_not_issued_by_one_call(device):

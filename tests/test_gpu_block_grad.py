@@ -196,6 +196,13 @@ def test_hooks_and_replaced_layers_are_called(device):
             assert seen and norm_error(out + branch, plain) < 1e-5
             handle.remove()
 
+            for name in ("mlp", "attn", "attn.proj", "mlp.drop") + (("norm1",) if grad else ()):    # a norm is a kernel in inference
+                mod = blk.get_submodule(name)                       # a forward of the module's own, as wrapping libraries set
+                mod.forward = lambda *a, f=mod.forward: 2 * f(*a)
+                out, branch = call(feat)
+                assert norm_error(out if branch is None else out + branch, plain) > 1e-2, name
+                del mod.forward
+
             class Doubled(torch.nn.Linear):
                 def forward(self, x):
                     return 2 * super().forward(x)
