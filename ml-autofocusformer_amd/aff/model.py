@@ -803,6 +803,18 @@ class ClusterTransformerBlock(_Module):
             return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d)
         return not (any(map(_hooked, mods)) or _hooked(m["drop_path"]))
 
+    def issued_with(self, ops, cluster_size):
+        """True when an inference forward of the block may be issued from outside: nothing but its own modules' forwards runs, they
+        use `ops` on clusters of that size, and nothing drops."""
+        d = self.__dict__
+        if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d or self.layer_scale or not self.plain():
+            return False
+        m = d["_modules"]
+        attn, mlp = m["attn"], m["mlp"]
+        a = attn._modules
+        return (attn.ops is ops and mlp.ops is ops and attn.cluster_size == cluster_size
+                and not (_drops(a["attn_drop"]) or _drops(a["proj_drop"]) or _drops(mlp._modules["drop"]) or _drops(m["drop_path"])))
+
     def tensors(self):
         """The parameters of the block in one tuple, straight from the modules' tables: the look-ups of 30 blocks are a
         visible part of a small forward's host time.  Where one is not in its table - replicas and wrappers set plain
@@ -1063,20 +1075,16 @@ class BasicLayer(_Module):
         gradients, where a block would not take its three kernels (`_fused_dtype`), where the attention is not one kernel,
         and when the caller's `ops` has another implementation of one of the pieces."""
         ops = self.ops
-        first = self.blocks[0]
-        if getattr(ops, "blocks_forward", None) is None or torch.is_grad_enabled():
+        if not feat.is_cuda or torch.is_grad_enabled() or getattr(ops, "blocks_forward", None) is None or not len(self.blocks):
             return None
+        if not all(type(blk) is ClusterTransformerBlock and blk.issued_with(ops, self.cluster_size) for blk in self.blocks):
+            return None
+        first = self.blocks[0]
         dt = first._fused_dtype(feat)
         b, n, c = feat.shape
         h = first.attn.num_heads
         if dt is None or c != 32 * h or any(getattr(ops, name, None) is not fn for name, fn in ops.blocks_stand_for) or (
                 dt == torch.float32 and getattr(ops, "block_layout", None) is None):
-            return None
-        if any(type(blk) is not ClusterTransformerBlock or blk._forward_hooks or blk._forward_pre_hooks or "forward" in blk.__dict__
-               or blk.layer_scale or not blk.plain() for blk in self.blocks):
-            return None
-        if any(_drops(blk.attn.attn_drop) or _drops(blk.attn.proj_drop) or _drops(blk.mlp.drop) or _drops(blk.drop_path)
-               for blk in self.blocks):
             return None
         if global_attn:
             if n > 64 or dt == torch.float32:
@@ -1087,6 +1095,8 @@ class BasicLayer(_Module):
             if plan is None or not (self.cluster_size == 8 or (self.cluster_size == 24 and dt != torch.float32)):
                 return None
         tensors = [blk.tensors() for blk in self.blocks]
+        if any(t is None for ts in tensors for t in ts):           # a layer without a bias, say
+            return None
         hidden, scale = first.mlp.fc1.out_features, first.attn.scale
         key = (dt, table.data_ptr(), table._version, table.dtype, c, h, hidden,
                [[(t._version, t.data_ptr()) for t in ts] for ts in tensors],

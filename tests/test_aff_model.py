@@ -945,3 +945,31 @@ def test_linear_layers_take_batched_gradients():
         torch.testing.assert_close(g, ref)
     torch.autograd.grad(_Linear.apply(x, w, b, None, supported), (x, w, b), batch[0])
     assert asked
+
+
+class Wrapped(torch.nn.Module):
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, *args):
+        return self.inner(*args)
+
+
+@pytest.mark.parametrize("grad", [True, False])
+def test_stages_without_blocks_and_with_wrapped_ones(grad):
+    """A stage of depth 0 hands its tokens to the merge; a block inside a module of the caller's is called through it.  Both also
+    where the operators come with a call for all blocks of a stage."""
+    from aff.model import AutoFocusFormer
+    ops = SimpleNamespace(**vars(oracle_ops()), blocks_forward=None, blocks_stand_for=())
+    ops.blocks_forward = lambda *a: pytest.fail("not for these stages")
+    torch.manual_seed(0)
+    kw = dict(img_size=64, embed_dim=(32, 64, 64, 64), num_heads=(1, 2, 2, 2), nbhd_size=(48, 48, 48, 48), num_classes=10, ops=ops)
+    x = torch.randn(1, 3, 64, 64)
+    with torch.set_grad_enabled(grad):
+        assert torch.isfinite(AutoFocusFormer(depths=(0, 1, 0, 1), **kw).eval()(x)).all()
+        net = AutoFocusFormer(depths=(1, 1, 1, 1), **kw).eval()
+        want = net(x)
+        for layer in net.layers:
+            layer.blocks[0] = Wrapped(layer.blocks[0])
+        assert torch.equal(net(x), want)

@@ -220,3 +220,32 @@ def test_stages_with_active_dropout_are_not_issued_by_one_call(device):
             assert not torch.equal(run(), plain), (name, stage)
             net.eval()
             assert torch.equal(run(), plain)
+
+
+@pytest.mark.parametrize("amp", [torch.float16, None])
+def test_stages_that_one_call_does_not_fit(device, amp):
+    """A later block without a bias, and one with operators of its own, go block by block; a stage without blocks has none."""
+    from types import SimpleNamespace
+    from aff.model import AutoFocusFormer, default_ops
+    cfg = dict(img_size=96, embed_dim=(32, 64, 128, 256), num_heads=(1, 2, 4, 8), mlp_ratio=2.0, nbhd_size=(48, 48, 48, 48),
+               num_classes=40)
+    x = torch.randn(2, 3, 96, 96, generator=torch.Generator().manual_seed(1)).to(device)
+
+    def run(net):
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, enabled=amp is not None):
+            return net(x)
+
+    torch.manual_seed(0)
+    net = AutoFocusFormer(depths=(1, 2, 2, 1), ops=default_ops(), **cfg).to(device).eval()
+    want = run(net)
+    calls = []
+    other = SimpleNamespace(**vars(default_ops()))
+    other.block_tail = lambda *a, f=other.block_tail, **kw: (calls.append(1), f(*a, **kw))[1]
+    blk = net.layers[1].blocks[1]
+    blk.attn.ops = blk.mlp.ops = other
+    assert torch.equal(run(net), want) and calls
+    net.layers[2].blocks[1].attn.proj.bias = None                # zeros so far
+    assert torch.isfinite(run(net)).all()
+    assert (run(net) - want).norm() <= (1e-5 if amp is None else 4e-3) * want.norm()
+    net = AutoFocusFormer(depths=(0, 1, 0, 1), ops=default_ops(), **cfg).to(device).eval()
+    assert torch.isfinite(run(net)).all()
