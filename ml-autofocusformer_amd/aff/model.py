@@ -19,6 +19,7 @@ are computed once and reused (the reference caches the clustering but repeats th
 neighbours use a sort of exact distances instead of an external library; the operators are reached through
 `self.ops`, so a test can run the very same modules on another implementation of the three functions.
 """
+import functools
 import math
 import threading
 from types import SimpleNamespace
@@ -72,6 +73,18 @@ def default_ops():
                            blocks_stand_for=(("cluster_attention", _native.cluster_attention),
                                              ("dense_attention", _native.dense_attention),
                                              ("norm_linear", _native.norm_linear), ("block_tail", _native.block_tail)))
+
+
+def _types_of_forward(backward):
+    """A `backward` that works in the types its forward kept, also when it is called under autocast (of another type, or after a
+    forward without it): its products would come back in another type than the kernels behind them are given."""
+    @functools.wraps(backward)
+    def outside(ctx, *grads):
+        if not torch.is_autocast_enabled("cuda"):
+            return backward(ctx, *grads)
+        with torch.autocast("cuda", enabled=False):
+            return backward(ctx, *grads)
+    return outside
 
 
 def _by_kernels(*grads):
@@ -421,6 +434,7 @@ class _NormLinearRows(torch.autograd.Function):
         return qkv, x
 
     @staticmethod
+    @_types_of_forward
     def backward(ctx, d_qkv, d_res):
         x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, normed, stats, w = ctx.saved_tensors
         eps, dt, ops = ctx.meta
@@ -458,6 +472,7 @@ class _BlockTail(torch.autograd.Function):
         return out
 
     @staticmethod
+    @_types_of_forward
     def backward(ctx, d_out):
         attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, x1, normed, hidden, stats, plain = ctx.saved_tensors
         eps, dt, ops = ctx.meta
@@ -511,6 +526,7 @@ class _ClusterAttentionRows(torch.autograd.Function):
         return out
 
     @staticmethod
+    @_types_of_forward
     def backward(ctx, d_out):
         qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, table, plan, pairs, pe_idx, member_idx, mask = ctx.saved_tensors
         heads, scale, ops = ctx.meta

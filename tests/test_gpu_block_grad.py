@@ -263,6 +263,23 @@ def test_parameters_that_are_plain_attributes(device, grad):
             assert blk.mlp.fc1.weight.grad.norm() > 0 and blk.attn.blank_k.grad.norm() > 0
 
 
+@pytest.mark.parametrize("forward,backward", [(None, torch.float16), (torch.bfloat16, torch.float16), (torch.float16, None)])
+def test_backward_under_another_autocast(device, forward, backward):
+    """The backward of a block computes in the types of its forward, wherever it is called."""
+    results = []
+    for amp in (forward, backward):
+        blk, feat, call = dense_block(device)
+        with torch.autocast("cuda", dtype=forward or torch.float16, enabled=forward is not None):
+            out, branch = call(feat)
+        assert branch is None
+        with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+            out.square().sum().backward()
+        results.append([p.grad for p in (blk.norm1.weight, blk.attn.q.weight, blk.mlp.fc1.weight, blk.mlp.fc2.bias)])
+    bar = 2e-2 if forward == torch.bfloat16 else 2e-3        # the attention between them is the framework's: its products follow autocast
+    for got, ref in zip(*results):
+        assert norm_error(got, ref) < bar
+
+
 def test_batched_gradients(device):
     """`is_grads_batched` through a training block: each row as by itself."""
     blk, feat, call = dense_block(device)
