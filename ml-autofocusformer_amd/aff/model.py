@@ -100,6 +100,13 @@ def _by_kernels(*grads):
     return True
 
 
+def _dense(t):
+    """`t` as rows the kernels read in place: contiguous and from a 16-byte boundary on, as a gradient that is part of a larger
+    buffer need not be."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 class _Linear(torch.autograd.Function):
     """`F.linear(x, weight, bias)` in x's dtype for parameters of any, with the parameters' gradients from the library's kernel:
     both in one pass over the rows, in fp32 (not rounded to 16 bits on the way to fp32 parameters)."""
@@ -445,11 +452,11 @@ class _NormLinearRows(torch.autograd.Function):
                 return F.linear(y, torch.cat([w_q, w_kv]).to(dt), torch.cat([b_q, b_kv]).to(dt)), x
             return (*_recorded_backward(layers, ctx, (x, norm_w, norm_b, w_q, b_q, w_kv, b_kv), (d_qkv, d_res)), None, None, None)
         need = ctx.needs_input_grad
-        rows = d_qkv.reshape(-1, 3 * c)
+        rows = _dense(d_qkv).view(-1, 3 * c)
         flat = normed.view(-1, c)
         grads = [None] * 7
         if need[0] or need[1] or need[2]:
-            grads[0], _, grads[1], grads[2] = ops.norm_backward((rows @ w).view(x.shape), x, stats, norm_w, d_res.contiguous())
+            grads[0], _, grads[1], grads[2] = ops.norm_backward((rows @ w).view(x.shape), x, stats, norm_w, _dense(d_res))
         wanted = [(i, rows[:, cols], need[i + 1]) for i, cols in ((3, slice(0, c)), (5, slice(c, 3 * c))) if need[i] or need[i + 1]]
         if wanted:
             for (i, _, _), (grads[i], grads[i + 1]) in zip(wanted, ops.weight_grad([(d, flat, bias) for _, d, bias in wanted])):
@@ -487,7 +494,7 @@ class _BlockTail(torch.autograd.Function):
             return (*_recorded_backward(layers, ctx, (attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2), (d_out,)),
                     None, None, None, None)
         need = ctx.needs_input_grad
-        d_out = d_out.contiguous()
+        d_out = _dense(d_out)
         p16, one, two = plain[:c * c].view(c, c), plain[c * c:c * (c + h)].view(h, c), plain[c * (c + h):].view(c, h)
         d_f = d_out.to(dt)
         if scale is not None:
@@ -536,7 +543,7 @@ class _ClusterAttentionRows(torch.autograd.Function):
                 return _local_attention(*_columns(qkv, heads), bias, blank_k, blank_v, mask, pe_idx, member_idx, scale)
             return (*_recorded_backward(layers, ctx, (qkv, pe_w, pe_b, blank_k, blank_v), (d_out,)), *(None,) * 9)
         q, key, v = _columns(qkv, heads)
-        d_out = d_out.to(qkv.dtype).contiguous()
+        d_out = _dense(d_out.to(qkv.dtype))
         d_qkv = torch.empty_like(qkv)
         _, probs, d_logit, blank_prob, d_blank = ops.cluster_attention_backward(
             q, key, v, d_out, out, lse, plan, bias, blank_k, blank_v, scale=scale, d_query=_columns(d_qkv, heads)[0])

@@ -280,6 +280,24 @@ def test_backward_under_another_autocast(device, forward, backward):
         assert norm_error(got, ref) < bar
 
 
+def test_gradients_that_are_parts_of_a_buffer(device):
+    """Incoming gradients off 16-byte boundaries, and expanded ones."""
+    blk, feat, call = dense_block(device)
+    _, stage_feat, stage = local_stage(device, default_ops())
+    for feat, f in ((feat, lambda x: call(x)[0]), (stage_feat, stage)):
+        x = feat.clone().requires_grad_(True)
+        out = f(x)
+        buffer = torch.randn(out.numel() + 1, generator=torch.Generator(device).manual_seed(1), device=device)
+        part = buffer[1:].view(out.shape)
+        got, = torch.autograd.grad(out, x, part, retain_graph=True)
+        want, = torch.autograd.grad(out, x, part.clone(), retain_graph=True)
+        assert torch.equal(got, want)
+        part = buffer[1].expand(out.shape)
+        got, = torch.autograd.grad(out, x, part, retain_graph=True)
+        want, = torch.autograd.grad(out, x, part.contiguous())
+        assert torch.equal(got, want)
+
+
 def test_batched_gradients(device):
     """`is_grads_batched` through a training block: each row as by itself."""
     blk, feat, call = dense_block(device)
