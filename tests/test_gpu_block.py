@@ -121,6 +121,18 @@ def test_gelu_of_every_16_bit_number(device, dt):
         assert torch.isnan(_native.block_tail(x, x, packed, at, zero, zero, bias, 1e-5, inf, zero)).all()
 
 
+@pytest.mark.parametrize("dt", list(BAR))
+@pytest.mark.parametrize("c,count", [(32, 1), (256, 70)])
+def test_packed_from_a_transpose(device, dt, c, count):
+    """A matrix given as its transpose is packed as the matrix; more of them than one launch takes."""
+    gen = torch.Generator().manual_seed(c)
+    weights = [torch.randn(2 * c if i % 2 else c, c, generator=gen).to(device) for i in range(count)]
+    want, at = _native.block_pack(c, dt, [(w, False) for w in weights])
+    got, at_t = _native.block_pack(c, dt, [(w.t().contiguous(), True) for w in weights])
+    assert at == at_t and torch.equal(got, want)
+    assert torch.equal(got.float().sort().values, torch.cat([w.reshape(-1) for w in weights]).to(dt).float().sort().values)
+
+
 def test_what_is_refused(device):
     block = Block(64, 192, torch.float16, device, 7)
     x = torch.randn(2, 8, 64, device=device)

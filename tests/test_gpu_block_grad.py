@@ -136,20 +136,29 @@ def norm_error(got, ref):
     return float((got.double() - ref.double()).norm() / ref.double().norm().clamp(min=1e-30))
 
 
-# A gradient by two orders of the same roundings: fp32 sums of up to 1700 tokens; in fp16 some ten roundings of 2^-11 of each of
-# up to six blocks, and a third of a unit more where sums over few tokens cancel (biases of the key projection: exactly zero).
-@pytest.mark.parametrize("dt,bar", [(torch.float32, 2e-4), (torch.float16, 4e-2)])
+# Two orders of the same sums and roundings: about four times the largest relative difference seen, of the logits and of all
+# gradients together (2.5e-7, 5.4e-4, 3.5e-3) and of a single parameter's (3.8e-6, 1.8e-3, 2.7e-2).
+BARS = {torch.float32: (1e-6, 1.5e-5), torch.float16: (2e-3, 8e-3), torch.bfloat16: (1.5e-2, 0.1)}
+# Gradients that are nearly nothing are measured by that of their layer's weight: a bias ahead of a BatchNorm (exactly 0), and
+# of the score that only weighs a token against its neighbours.
+CANCELS = ("patch_embed.proj1.bias", "prob_net.bias")
+
+
+@pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("drop_path", [0.0, 0.4])
-def test_training_step_layer_by_layer(device, dt, bar, drop_path):
+def test_training_step_layer_by_layer(device, dt, drop_path):
     ops = default_ops()
     layered = SimpleNamespace(**{**vars(ops), "block_tail": None})
     got, got_grads = step(build(ops, device, drop_path).train(), dt, device)
     ref, ref_grads = step(build(layered, device, drop_path).train(), dt, device)
-    assert norm_error(got, ref) < bar
+    together, single = BARS[dt]
+    assert norm_error(got, ref) < together
     everything = torch.cat([g.reshape(-1) for g in got_grads.values()])
-    assert norm_error(everything, torch.cat([g.reshape(-1) for g in ref_grads.values()])) < bar
+    assert norm_error(everything, torch.cat([g.reshape(-1) for g in ref_grads.values()])) < together
     for name, g in ref_grads.items():
-        assert got_grads[name].dtype == g.dtype and (norm_error(got_grads[name], g) < bar or "bias" in name), name
+        assert got_grads[name].dtype == g.dtype
+        by = ref_grads[name[:-4] + "weight"] if name.endswith(CANCELS) else g
+        assert (got_grads[name].double() - g.double()).norm() <= single * by.double().norm(), name
 
 
 def dense_block(device, ops=None, c=64, h=2):
