@@ -48,7 +48,7 @@ __global__ __launch_bounds__(256) void gelu_backward_kernel(const T* __restrict_
     load8(d_g + i * 8, d);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        y[e] = gelu_erf(v[e]);
+        y[e] = gelu_for<T>(v[e]);
         const float cdf = sizeof(T) == 2 ? normal_cdf(v[e]) : 0.5f * erfcf(-0.70710678118654752440f * v[e]);
         d[e] *= cdf + v[e] * 0.39894228040143267794f * __expf(-0.5f * v[e] * v[e]);
     }

@@ -129,7 +129,7 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
                     store_values<T, E>(static_cast<T*>(a.hidden) + (row[t] * a.chunks + chunk) * C + ch0 + f * Cfg::kStep, v);
                 }
 #pragma unroll
-                for (int e = 0; e < E; ++e) v[e] = gelu_erf(v[e]);
+                for (int e = 0; e < E; ++e) v[e] = gelu_for<T>(v[e]);
                 hid[((wave * F + f) * TR + t) * 64 + lane] = VecIO<T, E>::pack(v);
             }
         }

@@ -121,6 +121,20 @@ def test_gelu_of_every_16_bit_number(device, dt):
         assert torch.isnan(_native.block_tail(x, x, packed, at, zero, zero, bias, 1e-5, inf, zero)).all()
 
 
+def test_gelu_in_fp32(device):
+    """The erf formula in fp32 leaves the roundings of an error function, a sum and a product: 4.1e-8 of the result's root mean
+    square over normal numbers of deviation 0.3, in the forward kernel as in the one ahead of the backward's products."""
+    c = 512
+    eye, zero = torch.eye(c, device=device), torch.zeros(c, device=device)
+    packed, at = _native.block_pack(c, torch.float32, [(torch.zeros(c, c, device=device), False), (eye, False), (eye, False)])
+    v = 0.3 * torch.randn(64 * c, generator=torch.Generator(device).manual_seed(1), device=device)
+    x = torch.zeros(1, 1, c, device=device)
+    rows = [_native.block_tail(x, x, packed, at, zero, zero, part.contiguous(), 1e-5, zero, zero).reshape(-1) for part in v.split(c)]
+    exact = v.double() * 0.5 * torch.erfc(-v.double() * 0.5 ** 0.5)
+    for got in (torch.cat(rows), _native.gelu_backward(v, torch.ones_like(v))[0]):
+        assert (got.double() - exact).norm() <= 5e-8 * exact.norm()
+
+
 @pytest.mark.parametrize("dt", list(BAR))
 @pytest.mark.parametrize("c,count", [(32, 1), (256, 70)])
 def test_packed_from_a_transpose(device, dt, c, count):
