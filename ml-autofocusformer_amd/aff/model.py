@@ -21,6 +21,7 @@ neighbours use a sort of exact distances instead of an external library; the ope
 """
 import functools
 import math
+import operator
 import threading
 from types import SimpleNamespace
 
@@ -155,7 +156,8 @@ def _train_linear(lin, x, ops):
     return _Linear.apply(x.to(dt), w, lin.bias, ops.weight_grad, ops.weight_grad_supported)
 
 
-_recording = threading.local()      # .reads: what the `CapturedForward` being made by this thread has read so far
+# .reads: what the `CapturedForward` being made by this thread has read so far; .parts: what was kept for the value being made
+_thread = threading.local()
 
 
 class _Kept:
@@ -167,23 +169,21 @@ class _Kept:
     takes it up waits for it first, and is noted in its memory's list of users, so that the memory is not handed out
     again before that stream is done."""
 
-    __slots__ = ("key", "value", "held", "made", "device", "ready", "streams")
+    __slots__ = ("key", "value", "held", "made", "stream", "ready", "streams")
 
     def __init__(self, key, value, held, made=None):
         self.key, self.value, self.held = key, value, held
         self.made = _tensors(value if made is None else made)
-        self.device = self.made[0].device if self.made and self.made[0].is_cuda else None
-        if self.device is not None:
-            stream = torch.cuda.current_stream(self.device)
-            self.streams = (stream.cuda_stream,)
-            self.ready = None if torch.cuda.is_current_stream_capturing() else stream.record_event()
+        self.stream = torch.cuda.current_stream(self.made[0].device) if self.made and self.made[0].is_cuda else None
+        self.ready = None               # an event behind the computation; until there is one, the end of the stream
+        self.streams = () if self.stream is None else (self.stream.cuda_stream,)
 
     def join(self):
         """Makes the value usable on the current stream."""
-        if self.device is None or torch._C._cuda_getCurrentRawStream(self.device.index) in self.streams:
+        if self.stream is None or torch._C._cuda_getCurrentRawStream(self.stream.device_index) in self.streams:
             return
-        stream = torch.cuda.current_stream(self.device)
-        stream.wait_event(self.ready)
+        stream = torch.cuda.current_stream(self.stream.device)
+        stream.wait_event(self.ready or self.stream.record_event())
         for t in self.made:
             t.record_stream(stream)
         self.streams += (stream.cuda_stream,)
@@ -208,7 +208,7 @@ def _kept(table, slot, key, make, lasting=False):
     kept = table.get(slot)
     hit = type(kept) is _Kept and kept.key == key
     if torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing():
-        reads = getattr(_recording, "reads", None)
+        reads = getattr(_thread, "reads", None)
         if not hit or not (lasting or reads is not None):
             return _Kept(key, *make())
         if reads is not None:
@@ -216,8 +216,23 @@ def _kept(table, slot, key, make, lasting=False):
     elif hit:
         kept.join()
     else:
-        kept = table[slot] = _Kept(key, *make())     # in a module's __dict__: no parameter, no buffer, not in the state_dict
+        outer, _thread.parts = getattr(_thread, "parts", None), []
+        try:
+            kept = _Kept(key, *make())
+            parts = _thread.parts + [kept]
+        finally:
+            _thread.parts = outer
+        if outer is not None:
+            outer += parts                           # the event behind the whole will do for them: 10 us each
+        elif kept.stream is not None:
+            ready = kept.stream.record_event()
+            for part in parts:
+                part.ready = ready
+        table[slot] = kept                           # in a module's __dict__: no parameter, no buffer, not in the state_dict
     return kept
+
+
+_modules_of = operator.attrgetter("_modules")
 
 
 class _Module(nn.Module):
@@ -834,9 +849,13 @@ class ClusterTransformerBlock(_Module):
             return False
         m = d["_modules"]
         attn, mlp = m["attn"], m["mlp"]
+        if attn.ops is not ops or mlp.ops is not ops or attn.cluster_size != cluster_size:
+            return False
         a = attn._modules
-        return (attn.ops is ops and mlp.ops is ops and attn.cluster_size == cluster_size
-                and not (_drops(a["attn_drop"]) or _drops(a["proj_drop"]) or _drops(mlp._modules["drop"]) or _drops(m["drop_path"])))
+        for mod in (a["attn_drop"], a["proj_drop"], mlp._modules["drop"], m["drop_path"]):
+            if mod.training and _drops(mod):
+                return False
+        return True
 
     def tensors(self):
         """The parameters of the block in one tuple, straight from the modules' tables: the look-ups of 30 blocks are a
@@ -845,15 +864,16 @@ class ClusterTransformerBlock(_Module):
         m = self._modules
         attn, mlp = m["attn"], m["mlp"]
         a, ml = attn._modules, mlp._modules
-        mods = m["norm1"], m["norm2"], a["q"], a["kv"], a["proj"], ml["fc1"], ml["fc2"], attn, a["pos_embed"]
-        n1, n2, q, kv, proj, f1, f2, ap, pe = (mod._parameters for mod in mods)
         try:
+            n1, n2, ap = m["norm1"]._parameters, m["norm2"]._parameters, attn._parameters
+            q, kv, proj, pe = a["q"]._parameters, a["kv"]._parameters, a["proj"]._parameters, a["pos_embed"]._parameters
+            f1, f2 = ml["fc1"]._parameters, ml["fc2"]._parameters
             return (n1["weight"], n1["bias"], n2["weight"], n2["bias"], q["bias"], kv["bias"], proj["bias"], f1["bias"], f2["bias"],
                     ap["blank_k"], ap["blank_v"], q["weight"], kv["weight"], proj["weight"], f1["weight"], f2["weight"],
                     pe["weight"], pe["bias"])
         except KeyError:
-            n1, n2, q, kv, proj, f1, f2, ap, pe = mods
-            return (n1.weight, n1.bias, n2.weight, n2.bias, q.bias, kv.bias, proj.bias, f1.bias, f2.bias, ap.blank_k, ap.blank_v,
+            n1, n2, q, kv, proj, pe, f1, f2 = m["norm1"], m["norm2"], a["q"], a["kv"], a["proj"], a["pos_embed"], ml["fc1"], ml["fc2"]
+            return (n1.weight, n1.bias, n2.weight, n2.bias, q.bias, kv.bias, proj.bias, f1.bias, f2.bias, attn.blank_k, attn.blank_v,
                     q.weight, kv.weight, proj.weight, f1.weight, f2.weight, pe.weight, pe.bias)
 
     def _packed(self, dt):
@@ -1118,13 +1138,13 @@ class BasicLayer(_Module):
             if plan is None or not (self.cluster_size == 8 or (self.cluster_size == 24 and dt != torch.float32)):
                 return None
         tensors = [blk.tensors() for blk in self.blocks]
-        if any(t is None for ts in tensors for t in ts):           # a layer without a bias, say
-            return None
         hidden, scale = first.mlp.fc1.out_features, first.attn.scale
-        key = (dt, table.data_ptr(), table._version, table.dtype, c, h, hidden,
-               [[(t._version, t.data_ptr()) for t in ts] for ts in tensors],
-               [(blk._modules["norm1"].eps, blk._modules["norm2"].eps, blk._modules["attn"].scale, blk._modules["attn"].num_heads)
-                for blk in self.blocks])
+        try:
+            key = (dt, table.data_ptr(), table._version, table.dtype, c, h, hidden,
+                   [[(t._version, t.data_ptr()) for t in ts] for ts in tensors],
+                   [(m["norm1"].eps, m["norm2"].eps, m["attn"].scale, m["attn"].num_heads) for m in map(_modules_of, self.blocks)])
+        except AttributeError:                                     # a parameter is None, say the bias of a layer without one
+            return None
 
         def make():
             held, made = [table] + [t.detach() for ts in tensors for t in ts], []
@@ -1151,14 +1171,13 @@ class BasicLayer(_Module):
         params, layout = kept.value
         if params is None:
             return None
-        packed = None
         if layout is not None:
             # fp32: the weights as they are now (`_packed`), for this call only
-            packed = layout.pack(c, dt)
+            packed, at = layout.pack(c, dt)
+            base = packed.data_ptr()
             params = type(params).from_buffer_copy(params)
-            at = layout.addresses(packed)
             for i, p in enumerate(params):
-                p.w_qkv, _, p.w_proj, p.w1, p.w2 = at[5 * i:5 * i + 5]
+                p.w_qkv, _, p.w_proj, p.w1, p.w2 = (base + o for o in at[5 * i:5 * i + 5])
         return ops.blocks_forward(params, feat, h, hidden, dt, scale, plan, pe_idx if plan is None else None)
 
     def forward(self, pos, feat, h, w, on_grid, stride, table, radius, feat_ordered=False):
@@ -1390,8 +1409,8 @@ class CapturedForward:
     model's forward has no host synchronisation and every kernel of the library takes the current stream and
     allocates through the framework, so the recording is the plain forward under `torch.cuda.graph`.
 
-    Under mixed precision the 16-bit copies of the weights, and with either the tables made of parameters (position bias,
-    merge weights), are those of the time of recording, held by this object: record again after the weights change.
+    The tables made of parameters (position bias, merge weights) and, under mixed precision, the 16-bit copies of the weights and
+    the folded BatchNorm are those of the time of recording, held by this object: record again after the weights change.
     Everything else is read in place by every replay; with `autocast_dtype=None`, which records without mixed precision,
     that is every weight matrix.  The same output tensor is returned every time: copy it before the next call if it
     must outlive it.
@@ -1411,12 +1430,12 @@ class CapturedForward:
         torch.cuda.current_stream(example.device).wait_stream(side)
         torch.cuda.synchronize(example.device)
         self.graph = torch.cuda.CUDAGraph()
-        _recording.reads = self._reads = []      # the graph has their addresses
+        _thread.reads = self._reads = []      # the graph has their addresses
         try:
             with torch.cuda.graph(self.graph):
                 self.static_out = self._forward()
         finally:
-            del _recording.reads
+            del _thread.reads
 
     def _forward(self):
         with torch.no_grad(), torch.autocast("cuda", dtype=self.autocast_dtype or torch.float16,

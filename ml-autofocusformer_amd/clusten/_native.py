@@ -1659,51 +1659,55 @@ def block_supported(x: torch.Tensor, dtype: torch.dtype, hidden: int) -> bool:
             and hidden % x.shape[-1] == 0 and x.is_contiguous() and x.data_ptr() % 16 == 0)
 
 
-class BlockLayout:
-    """The order in which fp32 matrices - (n,k) tensors, or (tensor, transposed) pairs - lie in one tensor of packed weights, with
-    what `clusten_block_pack` is told of them: prepared once for weights that are packed more than once.  It holds their
-    addresses, not the weights."""
+def _pack_items(weights):
+    """((tensor, transposed) pairs as `clusten_block_pack` is told of them, but for where they go; place of each in elements; total)."""
+    device = weights[0][0].device
+    items, places, total = (PackItem * len(weights))(), [], 0
+    for it, (w, transposed) in zip(items, weights):
+        _require_cuda("weight", w, device)
+        if w.dim() != 2 or w.dtype != torch.float32 or not w.is_contiguous():
+            raise RuntimeError("weights must be contiguous fp32 matrices")
+        n, k = w.shape
+        it.src, it.transposed = w.data_ptr(), int(bool(transposed))
+        it.n, it.k = (k, n) if transposed else (n, k)
+        places.append(total)
+        total += w.numel()
+    return items, places, total
 
-    __slots__ = ("device", "count", "offsets", "items")
 
-    def __init__(self, weights):
-        weights = [w if isinstance(w, tuple) else (w, False) for w in weights]
-        self.device = weights[0][0].device
-        self.items = (PackItem * len(weights))()
-        self.offsets, total = [], 0
-        for it, (w, transposed) in zip(self.items, weights):
-            _require_cuda("weight", w, self.device)
-            if w.dim() != 2 or w.dtype != torch.float32 or not w.is_contiguous():
-                raise RuntimeError("weights must be contiguous fp32 matrices")
-            self.offsets.append(total)
-            total += w.numel()
-            it.src, it.transposed = w.data_ptr(), int(bool(transposed))
-            it.n, it.k = reversed(w.shape) if transposed else w.shape
-        self.count = total
-
-    def addresses(self, packed):
-        """Device address of each matrix in `packed`."""
-        base, size = packed.data_ptr(), packed.element_size()
-        return [base + at * size for at in self.offsets]
-
-    def pack(self, width: int, dtype: torch.dtype) -> torch.Tensor:
-        """The matrices, n and k multiples of `width`, as the block kernels of that width read them."""
-        out = torch.empty(self.count, dtype=dtype, device=self.device)
-        items = type(self.items).from_buffer_copy(self.items)        # callers may share the layout between threads
-        for it, dst in zip(items, self.addresses(out)):
-            it.dst = dst
-        with _on(self.device):
-            _check(load().clusten_block_pack(items, len(items), width, _DTYPE_CODES[dtype], _stream(self.device)),
-                   "clusten_block_pack")
-        return out
+def _pack_into(out, items, places, width):
+    """Packs `items` to their places in `out`; returns the byte offset of each."""
+    size, base, at = out.element_size(), out.data_ptr(), []
+    for it, place in zip(items, places):
+        at.append(place * size)
+        it.dst = base + place * size
+    with _on(out.device):
+        _check(load().clusten_block_pack(items, len(items), width, _DTYPE_CODES[out.dtype], _stream(out.device)), "clusten_block_pack")
+    return at
 
 
 def block_pack(width: int, dtype: torch.dtype, weights):
     """The matrices `weights` - (fp32 (n,k) tensor, transposed) pairs, n and k multiples of `width` - as the block kernels
     of that width read them, one after the other in one tensor of `dtype`.  Returns (tensor, byte offset of each)."""
-    layout = BlockLayout(weights)
-    out = layout.pack(width, dtype)
-    return out, [at * out.element_size() for at in layout.offsets]
+    items, places, total = _pack_items(weights)
+    out = torch.empty(total, dtype=dtype, device=weights[0][0].device)
+    return out, _pack_into(out, items, places, width)
+
+
+class BlockLayout:
+    """`block_pack` prepared once for (n,k) matrices that are packed again and again: what does not change from call to call.  It
+    has their addresses, and does not hold the matrices."""
+
+    __slots__ = ("device", "items", "places", "total")
+
+    def __init__(self, weights):
+        self.device = weights[0].device
+        self.items, self.places, self.total = _pack_items([(w, False) for w in weights])
+
+    def pack(self, width: int, dtype: torch.dtype):
+        out = torch.empty(self.total, dtype=dtype, device=self.device)
+        items = type(self.items).from_buffer_copy(self.items)        # threads may share the layout
+        return out, _pack_into(out, items, self.places, width)
 
 
 def norm_linear(x: torch.Tensor, norm_w, norm_b, eps: float, packed: torch.Tensor, w_at: int, bias0, bias1, n_out: int,
