@@ -4,8 +4,9 @@
 // The reference model's `proj`, residual, `norm2`, MLP and residual (models/aff_transformer.py:157-158, 230-232, 181-196; s1 and
 // s2 are the per-sample factors of stochastic depth, 1 without it).  As separate kernels - three products, an addition with the
 // norm, a GELU - the rows cross memory nine times and the hidden layer (2 to 3 C channels) four times; here a workgroup
-// takes R rows from the attention's output to the block's output with the hidden layer in LDS, C channels of it at a time.  Every intermediate is rounded to the storage type
-// where the separate kernels stored it.  It has no counterpart in the reference's extension modules.
+// takes R rows from the attention's output to the block's output with the hidden layer in LDS, C channels of it at a time.  Every
+// intermediate is rounded to the storage type where the separate kernels stored it, but for the hidden layer ahead of its GELU, which
+// is rounded only where a backward pass keeps it.  It has no counterpart in the reference's extension modules.
 #pragma once
 
 #include "gelu.hpp"
