@@ -421,6 +421,7 @@ class _ClusterAttention(torch.autograd.Function):
         return out
 
     @staticmethod
+    @_types_of_forward
     def backward(ctx, d_out):
         q, key, v, out, lse, bias, blank_k, blank_v, plan, pairs, pe_idx, member_idx, mask = ctx.saved_tensors
         scale, ops = ctx.meta

@@ -111,10 +111,12 @@ def test_table_linear_grad(device, dt, rows, n, k):
     close(d_b, d.double().sum(0), 1e-5)
 
 
-def build(ops, device, drop_path=0.0):
+def build(ops, device, drop_path=0.0, nbhd_size=(48, 48, 48, 48)):
+    """A model of as many stages as `nbhd_size` has, on 576, 144, 36 and 9 tokens."""
     torch.manual_seed(5)
-    kw = dict(img_size=96, embed_dim=(32, 64, 128, 256), num_heads=(1, 2, 4, 8), depths=(1, 2, 2, 1), mlp_ratio=2.0,
-              cluster_size=8, nbhd_size=(48, 48, 48, 48), num_classes=40, drop_path_rate=drop_path)
+    k = len(nbhd_size)
+    kw = dict(img_size=96, embed_dim=(32, 64, 128, 256)[:k], num_heads=(1, 2, 4, 8)[:k], depths=(1, 2, 2, 1)[:k], mlp_ratio=2.0,
+              cluster_size=8, nbhd_size=nbhd_size, num_classes=40, drop_path_rate=drop_path)
     return AutoFocusFormer(ops=ops, **kw).to(device)
 
 
@@ -149,8 +151,11 @@ CANCELS = ("patch_embed.proj1.bias", "prob_net.bias")
 def test_training_step_layer_by_layer(device, dt, drop_path):
     ops = default_ops()
     layered = SimpleNamespace(**{**vars(ops), "block_tail": None})
-    got, got_grads = step(build(ops, device, drop_path).train(), dt, device)
-    ref, ref_grads = step(build(layered, device, drop_path).train(), dt, device)
+    # in bf16 with local lists in every stage (the third: 24 of 36 tokens): the attention of a global one is the framework's batched
+    # products, which are not to be given transposed operands of that type
+    nbhd_size = (48, 48, 24) if dt == torch.bfloat16 else (48, 48, 48, 48)
+    got, got_grads = step(build(ops, device, drop_path, nbhd_size).train(), dt, device)
+    ref, ref_grads = step(build(layered, device, drop_path, nbhd_size).train(), dt, device)
     together, single = BARS[dt]
     assert norm_error(got, ref) < together
     everything = torch.cat([g.reshape(-1) for g in got_grads.values()])
@@ -272,21 +277,22 @@ def test_parameters_that_are_plain_attributes(device, grad):
             assert blk.mlp.fc1.weight.grad.norm() > 0 and blk.attn.blank_k.grad.norm() > 0
 
 
-@pytest.mark.parametrize("forward,backward", [(None, torch.float16), (torch.bfloat16, torch.float16), (torch.float16, None)])
-def test_backward_under_another_autocast(device, forward, backward):
-    """The backward of a block computes in the types of its forward, wherever it is called."""
+@pytest.mark.parametrize("layered", [False, True])
+@pytest.mark.parametrize("forward,backward", [(None, torch.float16), (torch.bfloat16, torch.float16), (torch.float16, torch.bfloat16),
+                                              (torch.float16, None)])
+def test_backward_under_another_autocast(device, forward, backward, layered):
+    """The backward of a block computes in the types of its forward, wherever it is called: the gradients are the same numbers."""
+    ops = SimpleNamespace(**{**vars(default_ops()), **({"block_tail": None} if layered else {})})
     results = []
     for amp in (forward, backward):
-        blk, feat, call = dense_block(device)
+        stage, feat, call = local_stage(device, ops)
         with torch.autocast("cuda", dtype=forward or torch.float16, enabled=forward is not None):
-            out, branch = call(feat)
-        assert branch is None
+            out = call(feat)
         with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
             out.square().sum().backward()
-        results.append([p.grad for p in (blk.norm1.weight, blk.attn.q.weight, blk.mlp.fc1.weight, blk.mlp.fc2.bias)])
-    bar = 2e-2 if forward == torch.bfloat16 else 2e-3        # the attention between them is the framework's: its products follow autocast
+        results.append([p.grad for p in stage.parameters()])
     for got, ref in zip(*results):
-        assert norm_error(got, ref) < bar
+        assert norm_error(got, ref) < (5e-2 if layered else 1e-6)    # layer by layer the products follow the region
 
 
 def test_gradients_that_are_parts_of_a_buffer(device):
