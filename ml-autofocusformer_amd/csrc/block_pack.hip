@@ -18,21 +18,21 @@ struct PackItems {
     clusten_pack_item item[kPackItems];
 };
 
-// One thread per 16-byte piece: piece (group, s, nb, lane) holds channels k = kStep s + kElems (lane / 16) .. of the output
-// channel that row lane % 16 of block nb stands for.
+// One thread per 16-byte piece: piece (group, s, nb, part, lane) holds channels k = 32 s + 8 (lane / 16) + E part .. of the
+// output channel that row lane % 16 of block nb stands for; fp32 pieces are two parts of four channels.
 template <typename T>
 __global__ __launch_bounds__(256) void block_pack_kernel(PackItems items, int NB) {
-    constexpr int E = 16 / (int)sizeof(T), STEP = 4 * E;
+    constexpr int E = 16 / (int)sizeof(T), PARTS = 8 / E;
     const clusten_pack_item it = items.item[blockIdx.y];
     const int64_t pieces = (int64_t)it.n * it.k / E;
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= pieces) return;
-    const int lane = (int)(i & 63), nb = (int)((i >> 6) % NB);
-    const int64_t rest = (i >> 6) / NB;
-    const int steps = it.k / STEP, s = (int)(rest % steps);
+    const int lane = (int)(i & 63), part = (int)((i >> 6) % PARTS), nb = (int)((i >> 6) / PARTS % NB);
+    const int64_t rest = (i >> 6) / (PARTS * NB);
+    const int steps = it.k / 32, s = (int)(rest % steps);
     const int64_t group = rest / steps;
-    const int64_t n = group * 16 * NB + weight_channel<T>(nb, lane & 15);
-    const int64_t k = (int64_t)s * STEP + E * (lane >> 4);
+    const int64_t n = group * 16 * NB + weight_channel(nb, lane & 15);
+    const int64_t k = (int64_t)s * 32 + 8 * (lane >> 4) + E * part;
     float v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = it.transposed ? it.src[(k + e) * it.n + n] : it.src[n * it.k + k + e];
@@ -43,30 +43,37 @@ __global__ __launch_bounds__(256) void block_pack_kernel(PackItems items, int NB
 
 bool block_width_supported(int C) { return C == 32 || C == 64 || C == 128 || C == 256 || C == 512; }
 
-int block_group_channels(int C) { return C >= 128 ? 64 : 32; }
-
 // 16-bit products are bound by the weights every workgroup streams from the L2 (0.9 MB at C = 256, H = 768): as many rows as
 // `most` allows, as long as half of the 256 compute units have a workgroup (tail, us with 4 / 2 / 1 tiles: 25 088 rows of 256
-// channels 44 / 54 / -, 9216 rows of 512 48 / 68 / 76, 6272 rows of 512 60 / 48 / 67, 1003 rows of 256 21 / 15 / 13).  fp32
-// products take sixteen times as long per weight and are bound by the compute unit that gets the most row tiles (9800 rows of
-// 256 channels: 129 us with 2 tiles, 307 workgroups, two of them on some units; 104 us with 1, 613, three on most).
-int block_row_tiles(int elem_size, int most, int64_t rows) {
-    int best = 1;
+// channels 44 / 54 / -, 9216 rows of 512 48 / 68 / 76, 6272 rows of 512 60 / 48 / 67, 1003 rows of 256 21 / 15 / 13).
+int block_row_tiles(int most, int64_t rows) {
+    int tiles = most;
+    while (tiles > 1 && (rows + 16 * tiles - 1) / (16 * tiles) < 128) tiles /= 2;
+    return tiles;
+}
+
+// fp32 weights are twice the bytes and are split next to the products: a workgroup's time is some w for the weights of a chunk of C
+// outputs and m a row tile for its products, w : m = 5 : 3 (784 rows of 256 channels: tail 33 / 44 / 57 us with 1 / 2 / 3 tiles,
+// norm_linear 16 / 20 / 24 / 30 with 1 .. 4), and a round of 256 workgroups, one a compute unit, takes as long as one.  What gives
+// the fewest rounds' time is taken.  Tail, us with 1 / 2 / 3 tiles: 9800 rows of 256 channels 99 / 93 / 61, 3136 rows 34 / 44 / 57;
+// norm_linear at 9800 rows 41 / 39 / 28 / 33 unsplit, 45 / 38 / 39 / 33 in three; 3136 rows 17 / 21 / 25 / 30 and 19 / 19 / 14 / 16;
+// 2450 rows of 512 50 / 64 / 88 and 42 / 30 / 39.
+BlockSplit block_split_f32(int most, int64_t rows, int chunks, bool may_split) {
+    BlockSplit best = {1, 1};
     int64_t cost = 0;
-    for (int tiles = most; tiles >= 1; tiles /= 2) {
+    for (int tiles = 1; tiles <= most; ++tiles) {
         const int64_t groups = (rows + 16 * tiles - 1) / (16 * tiles);
-        if (elem_size == 2) {
-            if (groups >= 128 || tiles == 1) return tiles;
-        } else {
-            const int64_t here = (groups + 255) / 256 * tiles;
-            if (cost == 0 || here < cost) cost = here, best = tiles;
+        for (int split = 1; split <= (may_split && groups <= 256 ? chunks : 1); ++split) {
+            // the norm ahead of the products is about as long as the weights of a chunk
+            const int64_t here = (groups * split + 255) / 256 * ((chunks + split - 1) / split * (5 + 3 * tiles) + 5);
+            if (cost == 0 || here < cost) cost = here, best = {tiles, split};
         }
     }
     return best;
 }
 
 int launch_block_pack(const clusten_pack_item* items, int count, int C, int dtype, hipStream_t stream) {
-    const int NB = block_group_channels(C) / 16;
+    const int NB = block_group(dtype == CLUSTEN_F32 ? 4 : 2, C) / 16;
     for (int at = 0; at < count; at += kPackItems) {
         PackItems p;
         const int here = min(kPackItems, count - at);

@@ -28,10 +28,11 @@ __device__ __forceinline__ void add_branch(float (&x)[E], const float (&branch)[
 template <typename T, typename S, int C, int TR>
 __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_kernel(BlockTailArgs a) {
     typedef BlockCfg<T, C> Cfg;
-    constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, F = Cfg::kFrags, D = KS < 2 ? 1 : 2;
+    constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, F = Cfg::kFrags, D = Cfg::kAhead;
     constexpr bool PARK = C > 64;
-    __shared__ __attribute__((aligned(16))) Piece act[KS * TR * 64];
-    __shared__ __attribute__((aligned(16))) Piece hid[KS * TR * 64];
+    constexpr int P = Cfg::kParts;
+    __shared__ __attribute__((aligned(16))) Piece act[KS * TR * P * 64];
+    __shared__ __attribute__((aligned(16))) Piece hid[KS * TR * P * 64];
     __shared__ float red[2 * WAVES * TR * 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
@@ -44,7 +45,14 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
     for (int i = wave; i < KS * TR; i += WAVES) {
         const int s = i / TR, t = i % TR;
         const int64_t r = min(row0 + 16 * t + r16, a.rows - 1);
-        CLUSTEN_LDS_DMA16(static_cast<const T*>(a.attn) + r * C + s * Cfg::kStep + kq * E, act + (size_t)i * 64);
+        const T* at = static_cast<const T*>(a.attn) + r * C + s * Cfg::kStep + kq * E;
+        if constexpr (P == 1) {
+            CLUSTEN_LDS_DMA16(at, act + (size_t)i * 64);
+        } else {
+            float v[E];
+            load_values<T, E>(at, v);
+            put_fragment<T>(act + (size_t)i * P * 64 + lane, v);
+        }
     }
     const auto factors = [&](const float* of, float (&scale)[TR]) {
 #pragma unroll
@@ -57,11 +65,12 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
         for (int t = 0; t < TR; ++t) rows[t] = static_cast<const S*>(a.x) + row[t] * C + ch0;
         load_rows<T, S, C, TR>(rows, x);
     }
-    const Piece* wp = static_cast<const Piece*>(a.wp) + (size_t)wave * KS * NB * 64;
-    const Piece* w1 = static_cast<const Piece*>(a.w1) + (size_t)wave * KS * NB * 64;
-    const Piece* w2 = static_cast<const Piece*>(a.w2) + (size_t)wave * a.chunks * KS * NB * 64;
-    Piece wb[D][NB];
-    preload<NB, D>(wp, lane * 16, wb);
+    constexpr size_t WEIGHTS = (size_t)KS * NB * 64 * Cfg::kRaw;       // of a wave's channels and C inputs
+    const Piece* wp = static_cast<const Piece*>(a.wp) + wave * WEIGHTS;
+    const Piece* w1 = static_cast<const Piece*>(a.w1) + wave * WEIGHTS;
+    const Piece* w2 = static_cast<const Piece*>(a.w2) + wave * a.chunks * WEIGHTS;
+    Piece wb[D][NB][Cfg::kRaw];
+    preload(wp, lane * 16, wb);
     float scale[TR];
     factors(a.scale, scale);
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
@@ -96,19 +105,17 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
             for (int e = 0; e < E; ++e) y[t][f][e] = x[t][f][e];
         }
     }
-    norm_to_fragments<T, C, TR>(a.norm_w, a.norm_b, a.eps, y, act, red, wave, lane, mean, rstd);
+    T* keep[TR];
+#pragma unroll
+    for (int t = 0; t < TR; ++t) {
+        keep[t] = a.x1 && row0 + 16 * t + r16 < a.rows ? static_cast<T*>(a.normed) + row[t] * C + ch0 : nullptr;
+    }
+    norm_to_fragments<T, C, TR>(a.norm_w, a.norm_b, a.eps, y, act, red, wave, lane, mean, rstd, keep);
     lds_barrier<WAVES>();
-    if (a.x1) {
+    if (a.x1 && wave == 0 && kq == 0) {
 #pragma unroll
         for (int t = 0; t < TR; ++t) {
-            if (row0 + 16 * t + r16 < a.rows) {
-                T* xn = static_cast<T*>(a.normed) + row[t] * C + ch0;
-#pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    *reinterpret_cast<Piece*>(xn + f * Cfg::kStep) = act[((wave * F + f) * TR + t) * 64 + lane];
-                }
-                if (wave == 0 && kq == 0) a.stats[row[t]] = float2{mean[t], rstd[t]};
-            }
+            if (row0 + 16 * t + r16 < a.rows) a.stats[row[t]] = float2{mean[t], rstd[t]};
         }
     }
 
@@ -131,13 +138,13 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_k
                 }
 #pragma unroll
                 for (int e = 0; e < E; ++e) v[e] = gelu_for<T>(v[e]);
-                hid[((wave * F + f) * TR + t) * 64 + lane] = VecIO<T, E>::pack(v);
+                put_fragment<T>(hid + ((wave * F + f) * TR + t) * P * 64 + lane, v);
             }
         }
         lds_barrier<WAVES>();
-        w1 += chunk + 1 < a.chunks ? (size_t)WAVES * KS * NB * 64 : 0;
+        w1 += chunk + 1 < a.chunks ? WAVES * WEIGHTS : 0;
         gemm_pass<T, TR, NB, KS, D>(w2, w1, lane * 16, wb, hid + lane, acc2);
-        w2 += (size_t)KS * NB * 64;
+        w2 += WEIGHTS;
     }
     if (a.scale) factors(a.scale + a.rows / a.rows_per_image, scale);
     if constexpr (PARK) {
@@ -169,12 +176,18 @@ int launch_block_tail_tiles(const BlockTailArgs& a, hipStream_t stream) {
 
 template <typename T, typename S, int C>
 int launch_block_tail_width(const BlockTailArgs& a, hipStream_t stream) {
-    // narrow rows are bound by memory and by their GELUs: more, smaller workgroups (2 tiles against 4: 98 against 110 us at
-    // 401 408 rows of 64 channels, 62 against 67 at 100 352 of 128); two fp32 tiles of 512 channels fill the LDS
-    constexpr int MOST = sizeof(T) == 4 ? (C > 256 ? 1 : 2) : (C > 128 ? 4 : 2);
-    const int tiles = block_row_tiles((int)sizeof(T), MOST, a.rows);
+    // narrow rows are bound by memory and by their GELUs: more, smaller workgroups (16 bits, 2 tiles against 4: 98 against 110 us at
+    // 401 408 rows of 64 channels, 62 against 67 at 100 352 of 128; fp32, 1 / 2 / 3 / 4 tiles: 98 / 84 / 87 / 105 at 156 800 rows of 64,
+    // 10.8 / 12.4 / 17 / 20 at 25 088 of 32); one fp32 tile of 512 channels, three of 256 fill the LDS.
+    // fp32 with three bf16 parts a value, against fp32 instructions: 9800 rows of 256 channels 111 -> 62 us, 39 200 of 128 115 -> 74,
+    // 156 800 of 64 110 -> 84, 2450 of 512 136 -> 112, bound by the weights from the L2 (20 us of the 62) and the products (36).
+    constexpr int MOST = sizeof(T) == 4 ? (C == 256 ? 3 : C == 64 || C == 128 ? 2 : 1) : (C > 128 ? 4 : 2);
+    const int tiles = sizeof(T) == 4 ? block_split_f32(MOST, a.rows, 1, false).tiles : block_row_tiles(MOST, a.rows);
     if constexpr (MOST >= 4) {
         if (tiles == 4) return launch_block_tail_tiles<T, S, C, 4>(a, stream);
+    }
+    if constexpr (MOST >= 3 && sizeof(T) == 4) {
+        if (tiles == 3) return launch_block_tail_tiles<T, S, C, 3>(a, stream);
     }
     if constexpr (MOST >= 2) {
         if (tiles == 2) return launch_block_tail_tiles<T, S, C, 2>(a, stream);

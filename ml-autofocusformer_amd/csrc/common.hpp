@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "../../include/clusten_hip.h"
 
 namespace clusten {
@@ -162,9 +164,16 @@ struct VecIO {
         constexpr int kWords = (VEC + kPerWord - 1) / kPerWord;
 #pragma unroll
         for (int k = 0; k < kWords; ++k) {
-            uint32_t w = storage_bits(from_acc<T>(x[k * kPerWord]));
-            if constexpr (kPerWord == 2 && VEC > 1) w |= storage_bits(from_acc<T>(x[k * kPerWord + 1])) << 16;
-            set_raw_word(r, k, w);
+            if constexpr (std::is_same<T, bf16_t>::value && VEC > 1) {
+                // a pair with one conversion instruction; bit by bit it took four
+                typedef float F2 __attribute__((ext_vector_type(2)));
+                typedef __bf16 B2 __attribute__((ext_vector_type(2)));
+                set_raw_word(r, k, __builtin_bit_cast(uint32_t, __builtin_convertvector((F2{x[2 * k], x[2 * k + 1]}), B2)));
+            } else {
+                uint32_t w = storage_bits(from_acc<T>(x[k * kPerWord]));
+                if constexpr (kPerWord == 2 && VEC > 1) w |= storage_bits(from_acc<T>(x[k * kPerWord + 1])) << 16;
+                set_raw_word(r, k, w);
+            }
         }
         return r;
     }

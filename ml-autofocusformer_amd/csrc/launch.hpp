@@ -286,11 +286,15 @@ struct BlockTailArgs {
     float2* stats;         // (rows)
 };
 bool block_width_supported(int C);
-// Tiles of 16 rows a workgroup takes (4, 2 or 1, at most `most`).
-int block_row_tiles(int elem_size, int most, int64_t rows);
+// Tiles of 16 rows a workgroup takes (4, 2 or 1, at most `most`): 16-bit products.
+int block_row_tiles(int most, int64_t rows);
+// The same for fp32 products (1 .. most), and over how many workgroups the chunks of C outputs are shared.
+struct BlockSplit {
+    int tiles, split;
+};
+BlockSplit block_split_f32(int most, int64_t rows, int chunks, bool may_split);
 // dst = a weight matrix of fp32 in the order the block kernels of width C read it in, as dtype.  src is (n,k), or (k,n)
-//   when transposed (dst is then that of its transpose); n a multiple of the width's group, k of the fragment.
-int block_group_channels(int C);
+//   when transposed (dst is then that of its transpose); n and k multiples of C.
 int launch_block_pack(const clusten_pack_item* items, int count, int C, int dtype, hipStream_t stream);
 int launch_norm_linear(const NormLinearArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);
 int launch_block_tail(const BlockTailArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);

@@ -14,8 +14,8 @@ namespace clusten {
 template <typename T, typename S, int C, int TR>
 __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void norm_linear_kernel(NormLinearArgs a) {
     typedef BlockCfg<T, C> Cfg;
-    constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, D = KS < 2 ? 1 : 2;
-    __shared__ __attribute__((aligned(16))) Piece act[KS * TR * 64];
+    constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, D = Cfg::kAhead;
+    __shared__ __attribute__((aligned(16))) Piece act[KS * TR * Cfg::kParts * 64];
     __shared__ float red[2 * WAVES * TR * 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, kq = lane >> 4;
@@ -33,11 +33,18 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void norm_linear_
     }
     // the workgroups of a row of the grid share the chunks of C output channels
     const int first = a.chunks * blockIdx.y / gridDim.y, last = a.chunks * (blockIdx.y + 1) / gridDim.y;
-    const Piece* w = static_cast<const Piece*>(a.w) + ((size_t)first * WAVES + wave) * KS * NB * 64;
-    Piece wb[D][NB];
-    preload<NB, D>(w, lane * 16, wb);
+    constexpr size_t WEIGHTS = (size_t)KS * NB * 64 * Cfg::kRaw;       // of a wave's channels
+    const Piece* w = static_cast<const Piece*>(a.w) + ((size_t)first * WAVES + wave) * WEIGHTS;
+    Piece wb[D][NB][Cfg::kRaw];
+    preload(w, lane * 16, wb);
     float mean[TR], rstd[TR];
-    norm_to_fragments<T, C, TR>(a.norm_w, a.norm_b, a.eps, x, act, red, wave, lane, mean, rstd);
+    T* keep[TR];
+#pragma unroll
+    for (int t = 0; t < TR; ++t) {
+        const int64_t row = row0 + 16 * t + r16;
+        keep[t] = a.normed && first == 0 && row < a.rows ? static_cast<T*>(a.normed) + row * C + ch0 : nullptr;
+    }
+    norm_to_fragments<T, C, TR>(a.norm_w, a.norm_b, a.eps, x, act, red, wave, lane, mean, rstd, keep);
     lds_barrier<WAVES>();
     if (a.stats && first == 0 && wave == 0 && kq == 0) {
 #pragma unroll
@@ -45,22 +52,10 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void norm_linear_
             if (row0 + 16 * t + r16 < a.rows) a.stats[row0 + 16 * t + r16] = float2{mean[t], rstd[t]};
         }
     }
-    if (a.normed && first == 0) {
-#pragma unroll
-        for (int t = 0; t < TR; ++t) {
-            if (row0 + 16 * t + r16 < a.rows) {
-                T* row = static_cast<T*>(a.normed) + (row0 + 16 * t + r16) * C + ch0;
-#pragma unroll
-                for (int f = 0; f < Cfg::kFrags; ++f) {
-                    *reinterpret_cast<Piece*>(row + f * Cfg::kStep) = act[((wave * Cfg::kFrags + f) * TR + t) * 64 + lane];
-                }
-            }
-        }
-    }
     for (int chunk = first; chunk < last; ++chunk) {
         F32x4 acc[NB][TR];
         bias_acc<T, NB, TR>((chunk == 0 ? a.bias0 : a.bias1 + (size_t)(chunk - 1) * C) + wave * NB * 16, kq, acc);
-        const Piece* next = w + (chunk + 1 < last ? (size_t)WAVES * KS * NB * 64 : 0);
+        const Piece* next = w + (chunk + 1 < last ? WAVES * WEIGHTS : 0);
         gemm_pass<T, TR, NB, KS, D>(w, next, lane * 16, wb, act + lane, acc);
         w = next;
 #pragma unroll
@@ -80,12 +75,8 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void norm_linear_
 }
 
 template <typename T, typename S, int C, int TR>
-int launch_norm_linear_tiles(const NormLinearArgs& a, hipStream_t stream) {
+int launch_norm_linear_tiles(const NormLinearArgs& a, int split, hipStream_t stream) {
     const int64_t groups = (a.rows + 16 * TR - 1) / (16 * TR);
-    // Few workgroups share the output chunks among them, each normalising its rows again: 17 -> 7 us for the 49 rows of 512
-    // channels of one image, 29 -> 27 us at 9216 rows of 512; at 25 088 rows of 256 (392 workgroups) 21.7 -> 23.5.  fp32
-    // products are long enough for it to pay up to a thousand (9800 rows of 256 channels, 613 workgroups: 50 -> 46 us).
-    const int split = groups < (sizeof(T) == 4 ? 1024 : 256) ? a.chunks : 1;
     hipLaunchKernelGGL((norm_linear_kernel<T, S, C, TR>), dim3((unsigned)groups, (unsigned)split), dim3(64 * BlockCfg<T, C>::kWaves), 0, stream,
                        a);
     return launch_status();
@@ -93,15 +84,26 @@ int launch_norm_linear_tiles(const NormLinearArgs& a, hipStream_t stream) {
 
 template <typename T, typename S, int C>
 int launch_norm_linear_width(const NormLinearArgs& a, hipStream_t stream) {
-    constexpr int MOST = sizeof(T) == 4 ? 2 : 4;
-    const int tiles = block_row_tiles((int)sizeof(T), MOST, a.rows);
+    // Up to 64 channels two fp32 tiles (25 088 rows of 64: 11 us, 13 with four).  fp32 with three bf16 parts a value, against fp32
+    // instructions: 9800 rows of 256 channels 51 -> 28 us, 39 200 of 128 48 -> 32, 156 800 of 64 58 -> 38, 2450 of 512 45 -> 30.
+    constexpr int MOST = sizeof(T) == 4 ? (C > 256 ? 3 : C > 64 ? 4 : 2) : 4;
+    BlockSplit cut;
+    if constexpr (sizeof(T) == 4) {
+        cut = block_split_f32(MOST, a.rows, a.chunks, true);
+    } else {
+        // Few workgroups share the output chunks among them, each normalising its rows again: 17 -> 7 us for the 49 rows of 512
+        // channels of one image, 29 -> 27 us at 9216 rows of 512; at 25 088 rows of 256 (392 workgroups) 21.7 -> 23.5.
+        cut.tiles = block_row_tiles(MOST, a.rows);
+        cut.split = (a.rows + 16 * cut.tiles - 1) / (16 * cut.tiles) < 256 ? a.chunks : 1;
+    }
     if constexpr (MOST >= 4) {
-        if (tiles == 4) return launch_norm_linear_tiles<T, S, C, 4>(a, stream);
+        if (cut.tiles == 4) return launch_norm_linear_tiles<T, S, C, 4>(a, cut.split, stream);
     }
-    if constexpr (MOST >= 2) {
-        if (tiles == 2) return launch_norm_linear_tiles<T, S, C, 2>(a, stream);
+    if constexpr (MOST >= 3 && sizeof(T) == 4) {
+        if (cut.tiles == 3) return launch_norm_linear_tiles<T, S, C, 3>(a, cut.split, stream);
     }
-    return launch_norm_linear_tiles<T, S, C, 1>(a, stream);
+    if (cut.tiles == 2) return launch_norm_linear_tiles<T, S, C, 2>(a, cut.split, stream);
+    return launch_norm_linear_tiles<T, S, C, 1>(a, cut.split, stream);
 }
 
 template <typename T, typename S>

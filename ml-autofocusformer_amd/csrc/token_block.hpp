@@ -8,7 +8,16 @@
 // says, it holds 16 bytes of consecutive channels of that row - which is a store, and which is also what the same lane
 // has to supply as B operand of the next product.  Results therefore go to the next product's activation buffer (or to
 // memory) as they are, and both ends of the buffer are conflict free: it is kept in fragment order,
-//   piece (s, t, lane) = channels s * kStep + kElems * kq .. of row 16 t + r16      (kStep = 64 bytes of a row).
+//   piece (s, t, lane) = channels s * kStep + kElems * kq .. of row 16 t + r16      (kStep = 32 channels).
+//
+// fp32 products run on the bf16 matrix instructions, every operand as the sum of three bf16 numbers (`split`): 24 bits, so that
+// nothing of an operand is lost.  The six products of parts that reach above 2^-24 of a term are summed in fp32, what is left out is
+// below 2^-25 of it.  Six instructions of 16 clocks then stand for eight fp32 ones of 32.  Activations are split once, on their way
+// into LDS (6 bytes a channel); weights stay fp32 in memory and are split by the one wave that reads them, next to the matrix
+// instructions of all its row tiles, in their shadow.  Against float64 the results are nearer than the fp32 instructions' (relative
+// 2-norm, norm_linear / block_tail, fp32 instructions -> parts): 1.56 / 1.69 -> 1.11 / 1.25e-7 at 64 channels, 2.14 / 2.34 ->
+// 1.65 / 1.87e-7 at 128, 2.93 / 3.30 -> 2.38 / 2.73e-7 at 256, 4.12 / 4.63 -> 3.42 / 3.92e-7 at 512.
+// An operand that is infinite makes its results NaN where fp32 arithmetic may give infinity; finite ones up to 3.38e38 are exact.
 #pragma once
 
 #include <type_traits>
@@ -18,26 +27,65 @@
 
 namespace clusten {
 
+// Output channels of a wave: what the weights of a width are grouped by.
+constexpr int block_group(int elem_size, int C) { return elem_size == 4 ? (C >= 512 ? 64 : 32) : (C >= 128 ? 64 : 32); }
+
 // What a width of C channels is cut into.  A wave has NB blocks of 16 output channels: with 4 blocks and 4 row tiles an
 // activation fragment read from LDS (1 KB) feeds 4 matrix instructions and a weight fragment another 4, half of the 128
-// bytes a clock the LDS delivers; narrow layers have too few blocks for that and are bound by memory anyway.
+// bytes a clock the LDS delivers; narrow layers have too few blocks for that and are bound by memory anyway.  In fp32 an activation
+// fragment of 3 KB feeds 6 instructions a block: 2 blocks are enough, and twice the waves split twice the weights at a time.
 template <typename T, int C>
 struct BlockCfg {
-    static constexpr int kElems = 16 / (int)sizeof(T);      // channels of a 16-byte piece
+    static constexpr int kElems = 8;                        // channels of a piece: what a lane brings to a matrix instruction
     static constexpr int kStep = 4 * kElems;                // channels of a fragment: one step of the contraction
-    static constexpr int kPair = sizeof(T) == 2 ? 2 : 1;    // 16-channel blocks of a fragment
-    static constexpr int NB = C >= 128 ? 4 : 2;             // blocks per wave
-    static constexpr int kFrags = NB / kPair;               // fragments of a wave's output channels
+    static constexpr int NB = block_group(sizeof(T), C) / 16;   // blocks per wave
+    static constexpr int kFrags = NB / 2;                   // fragments of a wave's output channels
     static constexpr int kWaves = C / 16 / NB;
     static constexpr int kSteps = C / kStep;
+    static constexpr int kAhead = sizeof(T) == 2 ? (kSteps < 2 ? 1 : 2) : (kSteps < 4 ? kSteps : 4);   // steps of weights on their way
+    static constexpr int kParts = sizeof(T) == 2 ? 1 : 3;   // pieces of an activation fragment a lane has
+    static constexpr int kRaw = (int)sizeof(T) / 2;         // pieces of a weight fragment a lane reads
     static_assert(C % (16 * NB) == 0, "whole waves");
 };
 
 // Output channel (within a wave's group) that row i of the instruction stands for in block nb.
+__device__ __forceinline__ int weight_channel(int nb, int i) { return 32 * (nb >> 1) + 8 * (i >> 2) + 4 * (nb & 1) + (i & 3); }
+
+// x = part[0] + part[1] + part[2] in bf16, each the rounding of what the ones before it leave.  Of x as rounded to fp32: without the
+// pragma the product that x may come from is fused into the first subtraction.
+__device__ __forceinline__ void split(const float (&x)[8], Piece (&part)[3]) {
+#pragma clang fp contract(off)
+    float left[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) left[e] = x[e];
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+        part[p] = VecIO<bf16_t, 8>::pack(left);
+        if (p < 2) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) left[e] -= piece_get<bf16_t>(part[p], e);
+        }
+    }
+}
+
+__device__ __forceinline__ void split_piece(const Piece (&raw)[2], Piece (&part)[3]) {
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(raw[e >> 2][e & 3]);
+    split(v, part);
+}
+
+// A lane's 8 channels into the activation buffer (`at`: its place in the fragment's first piece).
 template <typename T>
-__device__ __forceinline__ int weight_channel(int nb, int i) {
-    if (sizeof(T) == 4) return 16 * nb + i;
-    return 32 * (nb >> 1) + 8 * (i >> 2) + 4 * (nb & 1) + (i & 3);
+__device__ __forceinline__ void put_fragment(Piece* at, const float (&v)[8]) {
+    if constexpr (sizeof(T) == 2) {
+        *at = VecIO<T, 8>::pack(v);
+    } else {
+        Piece part[3];
+        split(v, part);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) at[p * 64] = part[p];
+    }
 }
 
 // Barrier of the workgroup that orders LDS traffic only: vector-memory operations (weights on their way) stay in flight.
@@ -55,47 +103,82 @@ __device__ __forceinline__ Piece weight_piece(const Piece* w, uint32_t lane16) {
     return *reinterpret_cast<const Piece*>(reinterpret_cast<const char*>(w) + lane16);
 }
 
-// acc[nb][t] += W X^T over KS steps.  `w` / `wnext`: this wave's weights, fragment (s, nb) at (s * NB + nb) * 64; wb holds
+// acc[nb][t] += W X^T over KS steps.  `w` / `wnext`: this wave's weights, fragment (s, nb) at (s * NB + nb) * 64 * kRaw; wb holds
 // the first D steps on entry and the first D steps of `wnext` on return, so that the weights of the next product travel
 // while this one's results are worked on.  `act`: the activation buffer at this lane's piece, read one step ahead.  The
 // scheduling barriers keep every load in the step that issues it: under register pressure the compiler otherwise moves the
 // weight loads down to their use and waits for each (the first version of the C = 256 block tail: 62 us instead of 40).
-template <typename T, int TR, int NB, int KS, int D>
+template <typename T, int TR, int NB, int KS, int D, int RAW = (int)sizeof(T) / 2>
 __device__ __forceinline__ void gemm_pass(const Piece* __restrict__ w, const Piece* __restrict__ wnext, uint32_t lane16,
-                                          Piece (&wb)[D][NB], const Piece* act, F32x4 (&acc)[NB][TR]) {
-    constexpr int U = KS < 2 ? 1 : 2;      // steps per turn: the registers of wb and a are named statically
+                                          Piece (&wb)[D][NB][RAW], const Piece* act, F32x4 (&acc)[NB][TR]) {
+    constexpr int U = KS < 2 ? 1 : D > 2 ? D : 2;      // steps per turn: the registers of wb and a are named statically
+    constexpr int P = sizeof(T) == 2 ? 1 : 3;
     static_assert(KS % U == 0 && U % D == 0, "whole turns of the weight registers");
-    Piece a[2][TR];
+    Piece a[2][TR][P];
 #pragma unroll
-    for (int t = 0; t < TR; ++t) a[0][t] = act[t * 64];
-#pragma unroll 4
+    for (int t = 0; t < TR; ++t) {
+#pragma unroll
+        for (int p = 0; p < P; ++p) a[0][t][p] = act[(t * P + p) * 64];
+    }
+    Piece part[2][3];                      // fp32: of the weight fragment at hand and of the next
+    if constexpr (P == 3) split_piece(wb[0][0], part[0]);
+#pragma unroll sizeof(T) == 2 ? 4 : 1
     for (int s0 = 0; s0 < KS; s0 += U) {
 #pragma unroll
         for (int d = 0; d < U; ++d) {
             const int s = s0 + d;
             if (s + 1 < KS) {
 #pragma unroll
-                for (int t = 0; t < TR; ++t) a[(d + 1) & 1][t] = act[((s + 1) * TR + t) * 64];
+                for (int t = 0; t < TR; ++t) {
+#pragma unroll
+                    for (int p = 0; p < P; ++p) a[(d + 1) & 1][t][p] = act[(((s + 1) * TR + t) * P + p) * 64];
+                }
             }
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
+                if constexpr (P == 1) {
 #pragma unroll
-                for (int t = 0; t < TR; ++t) acc[nb][t] = tile_mfma<T>(wb[d % D][nb], a[d & 1][t], acc[nb][t]);
+                    for (int t = 0; t < TR; ++t) acc[nb][t] = tile_mfma<T>(wb[d % D][nb][0], a[d & 1][t][0], acc[nb][t]);
+                } else {
+                    constexpr int last = NB - 1;
+                    const int at = (d * NB + nb) & 1;
+                    split_piece(wb[(d + (nb == last)) % D][nb == last ? 0 : nb + 1], part[at ^ 1]);
+#pragma unroll
+                    for (int sum = 2; sum >= 0; --sum) {       // the smallest products first
+#pragma unroll
+                        for (int p = sum; p >= 0; --p) {
+#pragma unroll
+                            for (int t = 0; t < TR; ++t) acc[nb][t] = tile_mfma<bf16_t>(part[at][p], a[d & 1][t][sum - p], acc[nb][t]);
+                        }
+                    }
+                    // the next fragment is split in the shadow of this one's products
+#pragma unroll
+                    for (int i = 0; i < 6 * TR; ++i) {
+                        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x2, (44 + 6 * TR - 1) / (6 * TR), 0);
+                    }
+                }
             }
-            const Piece* src = s + D < KS ? w + (size_t)(s + D) * NB * 64 : wnext + (size_t)(s + D - KS) * NB * 64;
+            const Piece* src = s + D < KS ? w + (size_t)(s + D) * NB * 64 * RAW : wnext + (size_t)(s + D - KS) * NB * 64 * RAW;
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) wb[d % D][nb] = weight_piece(src + nb * 64, lane16);
+            for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+                for (int r = 0; r < RAW; ++r) wb[d % D][nb][r] = weight_piece(src + (nb * RAW + r) * 64, lane16);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
 
-template <int NB, int D>
-__device__ __forceinline__ void preload(const Piece* __restrict__ w, uint32_t lane16, Piece (&wb)[D][NB]) {
+template <int NB, int D, int RAW>
+__device__ __forceinline__ void preload(const Piece* __restrict__ w, uint32_t lane16, Piece (&wb)[D][NB][RAW]) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
 #pragma unroll
-        for (int nb = 0; nb < NB; ++nb) wb[d][nb] = weight_piece(w + (d * NB + nb) * 64, lane16);
+        for (int nb = 0; nb < NB; ++nb) {
+#pragma unroll
+            for (int r = 0; r < RAW; ++r) wb[d][nb][r] = weight_piece(w + ((d * NB + nb) * RAW + r) * 64, lane16);
+        }
     }
     __builtin_amdgcn_sched_barrier(0);
 }
@@ -165,12 +248,13 @@ __device__ __forceinline__ void row_totals(float (&part)[TR], float* red, int wa
 }
 
 // Layer norm of the R rows held in `x` (mean, then centred squares, all fp32), written as fragments of T into `act`; x is
-// used up.  Every wave is past its reads of `act` when the first row total is complete.  mean / rstd: of the lane's rows.
+// used up.  Every wave is past its reads of `act` when the first row total is complete.  mean / rstd: of the lane's rows.  keep:
+// where the lane's rows of the result go in memory as well (from the lane's first channel on), or null.
 template <typename T, int C, int TR>
 __device__ __forceinline__ void norm_to_fragments(const float* __restrict__ weight, const float* __restrict__ bias, float eps,
                                                   float (&x)[TR][BlockCfg<T, C>::kFrags][BlockCfg<T, C>::kElems],
                                                   Piece* act, float* red, int wave, int lane, float (&mean)[TR],
-                                                  float (&rstd)[TR]) {
+                                                  float (&rstd)[TR], T* const (&keep)[TR]) {
     typedef BlockCfg<T, C> Cfg;
     constexpr int E = Cfg::kElems;
 #pragma unroll
@@ -211,7 +295,8 @@ __device__ __forceinline__ void norm_to_fragments(const float* __restrict__ weig
             float v[E];
 #pragma unroll
             for (int e = 0; e < E; ++e) v[e] = x[t][f][e] * rstd[t] * g[e] + b[e];
-            act[(s * TR + t) * 64 + lane] = VecIO<T, E>::pack(v);
+            put_fragment<T>(act + (s * TR + t) * Cfg::kParts * 64 + lane, v);
+            if (keep[t]) store_values<T, E>(keep[t] + f * Cfg::kStep, v);
         }
     }
 }
@@ -219,7 +304,7 @@ __device__ __forceinline__ void norm_to_fragments(const float* __restrict__ weig
 // Starts a product's sums at the bias of the output channels, as the storage type T holds it.  `bias`: the wave's first channel.
 template <typename T, int NB, int TR>
 __device__ __forceinline__ void bias_acc(const float* __restrict__ bias, int kq, F32x4 (&acc)[NB][TR]) {
-    constexpr int E = 16 / (int)sizeof(T), P = E / 4;
+    constexpr int E = 8, P = E / 4;
 #pragma unroll
     for (int f = 0; f < NB / P; ++f) {
         float b[E];

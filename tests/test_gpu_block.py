@@ -80,6 +80,29 @@ def test_against_the_layers(device, dt, stream, c, hidden, rows):
     assert oracle.rel_err(got.float(), block.tail(attn, x)) <= BAR[dt]
 
 
+@pytest.mark.parametrize("c,hidden,rows", [(32, 96, 17), (64, 192, 513), (64, 192, 25089), (128, 384, 4095), (128, 256, 6273),
+                                           (256, 768, 47), (256, 768, 784), (256, 768, 1569), (256, 768, 3137), (256, 768, 8193),
+                                           (256, 512, 12289), (512, 1536, 393), (512, 1024, 2450), (512, 512, 4097)])
+def test_fp32_against_float64(device, c, hidden, rows):
+    """fp32 products are sums over three bf16 parts of every operand, over 1 to 4 row tiles a workgroup, the outputs shared
+    among 1 to 3 of them: the parts hold all 24 bits, so what is left is the rounding of fp32 sums.  Relative 2-norm from
+    float64: fp32 instructions 4.6e-7 at 512 channels (the root of 512 + 1536 terms at some 2^-27 each), the parts 3.9e-7."""
+    block = Block(c, hidden, torch.float32, device, c + rows)
+    gen = torch.Generator().manual_seed(rows)
+    x = (torch.randn(1, rows, c, generator=gen) * 2 + 0.5).to(device)
+    x[0, -1] *= 1e-30                                            # far below and above the other rows
+    attn = torch.randn(1, rows, c, generator=gen).to(device)
+    attn[0, 0] *= 1e25
+    w, b, norm = ([t.double() for t in ts] for ts in (block.w, block.b, block.norm))
+    got, ref = block.run_head(x), F.layer_norm(x.double(), (c,), norm[0], norm[1])
+    ref = torch.cat([F.linear(ref, w[0], b[0]), F.linear(ref, w[1], b[1])], -1)
+    assert (got.double() - ref).norm() <= 5e-7 * ref.norm()
+    got, x1 = block.run_tail(attn, x), x.double() + F.linear(attn.double(), w[2], b[2])
+    ref = F.gelu(F.linear(F.layer_norm(x1, (c,), norm[2], norm[3]), w[3], b[3]))
+    ref = x1 + F.linear(ref, w[4], b[4])
+    assert ((got.double() - ref).norm(dim=-1) <= 8e-7 * ref.norm(dim=-1)).all()
+
+
 @pytest.mark.parametrize("dt,stream", CASES)
 def test_factors_of_the_images(device, dt, stream):
     """Stochastic depth: a factor per image on both branches, 0 leaving the image's rows as they are."""
