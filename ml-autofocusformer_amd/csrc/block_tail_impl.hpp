@@ -28,7 +28,7 @@ __device__ __forceinline__ void add_branch(float (&x)[E], const float (&branch)[
 template <typename T, typename S, int C, int TR>
 __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_kernel(BlockTailArgs a) {
     typedef BlockCfg<T, C> Cfg;
-    constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, F = Cfg::kFrags, D = Cfg::kAhead;
+    constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, F = Cfg::kFrags, D = Cfg::ahead(TR);
     constexpr bool PARK = C > 64;
     constexpr int P = Cfg::kParts;
     __shared__ __attribute__((aligned(16))) Piece act[KS * TR * P * 64];
@@ -179,8 +179,8 @@ int launch_block_tail_width(const BlockTailArgs& a, hipStream_t stream) {
     // narrow rows are bound by memory and by their GELUs: more, smaller workgroups (16 bits, 2 tiles against 4: 98 against 110 us at
     // 401 408 rows of 64 channels, 62 against 67 at 100 352 of 128; fp32, 1 / 2 / 3 / 4 tiles: 98 / 84 / 87 / 105 at 156 800 rows of 64,
     // 10.8 / 12.4 / 17 / 20 at 25 088 of 32); one fp32 tile of 512 channels, three of 256 fill the LDS.
-    // fp32 with three bf16 parts a value, against fp32 instructions: 9800 rows of 256 channels 111 -> 62 us, 39 200 of 128 115 -> 74,
-    // 156 800 of 64 110 -> 84, 2450 of 512 136 -> 112, bound by the weights from the L2 (20 us of the 62) and the products (36).
+    // fp32 with three bf16 parts a value, against fp32 instructions: 9800 rows of 256 channels 111 -> 68 us, 39 200 of 128 115 -> 74,
+    // 156 800 of 64 110 -> 86, 2450 of 512 136 -> 118, bound by the weights from the L2 (20 us of the 68) and the products (40).
     constexpr int MOST = sizeof(T) == 4 ? (C == 256 ? 3 : C == 64 || C == 128 ? 2 : 1) : (C > 128 ? 4 : 2);
     const int tiles = sizeof(T) == 4 ? block_split_f32(MOST, a.rows, 1, false).tiles : block_row_tiles(MOST, a.rows);
     if constexpr (MOST >= 4) {

@@ -14,7 +14,7 @@ namespace clusten {
 template <typename T, typename S, int C, int TR>
 __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void norm_linear_kernel(NormLinearArgs a) {
     typedef BlockCfg<T, C> Cfg;
-    constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, D = Cfg::kAhead;
+    constexpr int NB = Cfg::NB, KS = Cfg::kSteps, WAVES = Cfg::kWaves, E = Cfg::kElems, D = Cfg::ahead(TR);
     __shared__ __attribute__((aligned(16))) Piece act[KS * TR * Cfg::kParts * 64];
     __shared__ float red[2 * WAVES * TR * 16];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -85,8 +85,8 @@ int launch_norm_linear_tiles(const NormLinearArgs& a, int split, hipStream_t str
 template <typename T, typename S, int C>
 int launch_norm_linear_width(const NormLinearArgs& a, hipStream_t stream) {
     // Up to 64 channels two fp32 tiles (25 088 rows of 64: 11 us, 13 with four).  fp32 with three bf16 parts a value, against fp32
-    // instructions: 9800 rows of 256 channels 51 -> 28 us, 39 200 of 128 48 -> 32, 156 800 of 64 58 -> 38, 2450 of 512 45 -> 30.
-    constexpr int MOST = sizeof(T) == 4 ? (C > 256 ? 3 : C > 64 ? 4 : 2) : 4;
+    // instructions: 9800 rows of 256 channels 51 -> 34 us, 39 200 of 128 48 -> 35, 156 800 of 64 58 -> 38, 2450 of 512 45 -> 31.
+    constexpr int MOST = sizeof(T) == 4 ? (C > 256 || C <= 64 ? 2 : 4) : 4;
     BlockSplit cut;
     if constexpr (sizeof(T) == 4) {
         cut = block_split_f32(MOST, a.rows, a.chunks, true);

@@ -12,11 +12,14 @@
 //
 // fp32 products run on the bf16 matrix instructions, every operand as the sum of three bf16 numbers (`split`): 24 bits, so that
 // nothing of an operand is lost.  The six products of parts that reach above 2^-24 of a term are summed in fp32, what is left out is
-// below 2^-25 of it.  Six instructions of 16 clocks then stand for eight fp32 ones of 32.  Activations are split once, on their way
+// below 2^-25 of it.  The instructions round a sum down, by up to 2^-26 of it: six to a step on running sums shifted the mean of 33 000
+// rows' results by 3e-6 of their deviation.  The six of a step therefore start from zero, smallest first, and their sum is
+// added by a fp32 addition, which rounds to nearest; and every other step is summed negated and subtracted, so that what is left of
+// the shift cancels (1e-8 of a result's deviation without: invisible in a row, but not in sums over all rows).  Six instructions of 16 clocks then stand for eight fp32 ones of 32.  Activations are split once, on their way
 // into LDS (6 bytes a channel); weights stay fp32 in memory and are split by the one wave that reads them, next to the matrix
 // instructions of all its row tiles, in their shadow.  Against float64 the results are nearer than the fp32 instructions' (relative
-// 2-norm, norm_linear / block_tail, fp32 instructions -> parts): 1.56 / 1.69 -> 1.11 / 1.25e-7 at 64 channels, 2.14 / 2.34 ->
-// 1.65 / 1.87e-7 at 128, 2.93 / 3.30 -> 2.38 / 2.73e-7 at 256, 4.12 / 4.63 -> 3.42 / 3.92e-7 at 512.
+// 2-norm, norm_linear / block_tail, fp32 instructions -> parts): 1.56 / 1.69 -> 0.77 / 0.72e-7 at 64 channels, 2.14 / 2.34 ->
+// 0.83 / 0.79e-7 at 128, 2.93 / 3.30 -> 0.92 / 0.93e-7 at 256, 4.12 / 4.63 -> 1.07 / 1.13e-7 at 512.
 // An operand that is infinite makes its results NaN where fp32 arithmetic may give infinity; finite ones up to 3.38e38 are exact.
 #pragma once
 
@@ -42,7 +45,9 @@ struct BlockCfg {
     static constexpr int kFrags = NB / 2;                   // fragments of a wave's output channels
     static constexpr int kWaves = C / 16 / NB;
     static constexpr int kSteps = C / kStep;
-    static constexpr int kAhead = sizeof(T) == 2 ? (kSteps < 2 ? 1 : 2) : (kSteps < 4 ? kSteps : 4);   // steps of weights on their way
+    // Steps of weights on their way: as many as the registers of TR row tiles leave room for, up to four in fp32 (784 rows of 256
+    // channels, tail: 43 us with two, 33 with four).
+    static constexpr int ahead(int tr) { return kSteps < 2 ? 1 : sizeof(T) == 4 && NB == 2 && tr < 3 && kSteps >= 4 ? 4 : 2; }
     static constexpr int kParts = sizeof(T) == 2 ? 1 : 3;   // pieces of an activation fragment a lane has
     static constexpr int kRaw = (int)sizeof(T) / 2;         // pieces of a weight fragment a lane reads
     static_assert(C % (16 * NB) == 0, "whole waves");
@@ -68,10 +73,10 @@ __device__ __forceinline__ void split(const float (&x)[8], Piece (&part)[3]) {
     }
 }
 
-__device__ __forceinline__ void split_piece(const Piece (&raw)[2], Piece (&part)[3]) {
+__device__ __forceinline__ void split_piece(const Piece (&raw)[2], Piece (&part)[3], bool minus) {
     float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = __uint_as_float(raw[e >> 2][e & 3]);
+    for (int e = 0; e < 8; ++e) v[e] = minus ? -__uint_as_float(raw[e >> 2][e & 3]) : __uint_as_float(raw[e >> 2][e & 3]);
     split(v, part);
 }
 
@@ -121,7 +126,7 @@ __device__ __forceinline__ void gemm_pass(const Piece* __restrict__ w, const Pie
         for (int p = 0; p < P; ++p) a[0][t][p] = act[(t * P + p) * 64];
     }
     Piece part[2][3];                      // fp32: of the weight fragment at hand and of the next
-    if constexpr (P == 3) split_piece(wb[0][0], part[0]);
+    if constexpr (P == 3) split_piece(wb[0][0], part[0], false);
 #pragma unroll sizeof(T) == 2 ? 4 : 1
     for (int s0 = 0; s0 < KS; s0 += U) {
 #pragma unroll
@@ -142,13 +147,35 @@ __device__ __forceinline__ void gemm_pass(const Piece* __restrict__ w, const Pie
                 } else {
                     constexpr int last = NB - 1;
                     const int at = (d * NB + nb) & 1;
-                    split_piece(wb[(d + (nb == last)) % D][nb == last ? 0 : nb + 1], part[at ^ 1]);
+                    split_piece(wb[(d + (nb == last)) % D][nb == last ? 0 : nb + 1], part[at ^ 1], (d + (nb == last)) % U & 1);
+                    // every other step sums the negated products and is subtracted; a lone step is taken in two halves
 #pragma unroll
-                    for (int sum = 2; sum >= 0; --sum) {       // the smallest products first
+                    for (int half = 0; half < (KS == 1 ? 2 : 1); ++half) {
+                        Piece here[3];
 #pragma unroll
-                        for (int p = sum; p >= 0; --p) {
+                        for (int p = 0; p < 3; ++p) {
+                            here[p] = part[at][p];
+                            if (KS == 1) {
+                                const uint32_t keep = ((threadIdx.x >> 5) & 1) == half ? ~0u : 0u, minus = half ? 0x80008000u : 0u;
 #pragma unroll
-                            for (int t = 0; t < TR; ++t) acc[nb][t] = tile_mfma<bf16_t>(part[at][p], a[d & 1][t][sum - p], acc[nb][t]);
+                                for (int e = 0; e < 4; ++e) here[p][e] = (here[p][e] & keep) ^ minus;
+                            }
+                        }
+                        F32x4 sum[TR];
+#pragma unroll
+                        for (int t = 0; t < TR; ++t) sum[t] = F32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int order = 2; order >= 0; --order) {       // the smallest products first
+#pragma unroll
+                            for (int p = order; p >= 0; --p) {
+#pragma unroll
+                                for (int t = 0; t < TR; ++t) sum[t] = tile_mfma<bf16_t>(here[p], a[d & 1][t][order - p], sum[t]);
+                            }
+                        }
+#pragma unroll
+                        for (int t = 0; t < TR; ++t) {
+                            if ((d + half) & 1) acc[nb][t] -= sum[t];
+                            else acc[nb][t] += sum[t];
                         }
                     }
                     // the next fragment is split in the shadow of this one's products

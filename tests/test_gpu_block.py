@@ -86,7 +86,7 @@ def test_against_the_layers(device, dt, stream, c, hidden, rows):
 def test_fp32_against_float64(device, c, hidden, rows):
     """fp32 products are sums over three bf16 parts of every operand, over 1 to 4 row tiles a workgroup, the outputs shared
     among 1 to 3 of them: the parts hold all 24 bits, so what is left is the rounding of fp32 sums.  Relative 2-norm from
-    float64: fp32 instructions 4.6e-7 at 512 channels (the root of 512 + 1536 terms at some 2^-27 each), the parts 3.9e-7."""
+    float64: fp32 instructions 4.6e-7 at 512 channels, the parts 1.1e-7 (64 sums of 32 terms, each rounded to nearest)."""
     block = Block(c, hidden, torch.float32, device, c + rows)
     gen = torch.Generator().manual_seed(rows)
     x = (torch.randn(1, rows, c, generator=gen) * 2 + 0.5).to(device)
@@ -96,11 +96,11 @@ def test_fp32_against_float64(device, c, hidden, rows):
     w, b, norm = ([t.double() for t in ts] for ts in (block.w, block.b, block.norm))
     got, ref = block.run_head(x), F.layer_norm(x.double(), (c,), norm[0], norm[1])
     ref = torch.cat([F.linear(ref, w[0], b[0]), F.linear(ref, w[1], b[1])], -1)
-    assert (got.double() - ref).norm() <= 5e-7 * ref.norm()
+    assert (got.double() - ref).norm() <= 1.5e-7 * ref.norm()
     got, x1 = block.run_tail(attn, x), x.double() + F.linear(attn.double(), w[2], b[2])
     ref = F.gelu(F.linear(F.layer_norm(x1, (c,), norm[2], norm[3]), w[3], b[3]))
     ref = x1 + F.linear(ref, w[4], b[4])
-    assert ((got.double() - ref).norm(dim=-1) <= 8e-7 * ref.norm(dim=-1)).all()
+    assert ((got.double() - ref).norm(dim=-1) <= 3e-7 * ref.norm(dim=-1)).all()
 
 
 @pytest.mark.parametrize("dt,stream", CASES)
