@@ -689,6 +689,27 @@ size_t clusten_weight_grad_workspace_bytes(const clusten_weight_grad_item* items
 int clusten_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, void* workspace, size_t workspace_bytes,
                         int dtype, clusten_stream stream);
 
+/* The backward of the two forwards above over their rows, which the reference leaves to autograd.  Weights are packed transposes
+ * (clusten_block_pack, transposed = 1): wp_t of Wp (C,C), w1_t of W1 as a (C,H) matrix, w2_t of W2 as (H,C); of W, w0_t of the
+ * first C outputs' rows (C,C) and w1_t of the others' as a (C,N-C) matrix (may be NULL when N == C).
+ *   tail: with d_f = s2 d_out:  d_h = (d_f W2) gelu'(hidden), g = gelu(hidden), d_x = d_out + the gradient through the norm of
+ *     d_h W1, branch = s1 d_x, d_attn = branch Wp; x1, stats and hidden as the forward kept them, d_out and d_x of x_dtype, the others
+ *     of dtype; branch and d_f may be NULL (when there is no scale and x_dtype is dtype they are d_x and d_out).
+ *   linear: d_x = d_res + the gradient through the norm of d_y W; d_res (of x_dtype) may be NULL.
+ *   d_norm_w, d_norm_b (C): the norm's parameter gradients, fp32 sums in a fixed order.  What the products' results pass through on
+ *   their way to the next product is rounded to dtype there and nowhere else.
+ *   workspace: clusten_block_backward_workspace_bytes(rows, C) bytes. */
+size_t clusten_block_backward_workspace_bytes(int64_t rows, int C);
+int clusten_block_tail_backward(const void* d_out, const void* x1, int x_dtype, const float* stats, const float* norm_w,
+                                const void* hidden, const void* wp_t, const void* w1_t, const void* w2_t, const float* scale,
+                                int rows_per_image, void* d_x, void* branch, void* d_f, void* g, void* d_h, void* d_attn,
+                                float* d_norm_w, float* d_norm_b, void* workspace, size_t workspace_bytes, int64_t rows, int C,
+                                int H, int dtype, clusten_stream stream);
+int clusten_norm_linear_backward(const void* d_y, const void* x, int x_dtype, const float* stats, const float* norm_w,
+                                 const void* w0_t, const void* w1_t, const void* d_res, void* d_x, float* d_norm_w, float* d_norm_b,
+                                 void* workspace, size_t workspace_bytes, int64_t rows, int C, int N, int dtype,
+                                 clusten_stream stream);
+
 /* The backward of a block between its products, which the reference leaves to autograd.  Tensors are dense rows of C channels
  * (C in {32,64,128,256,512}) of dtype F32, F16 or BF16 unless said otherwise, on 16-byte boundaries; sums are fp32 in a fixed
  * order; workspace: clusten_row_sums_workspace_bytes(rows, C) bytes.

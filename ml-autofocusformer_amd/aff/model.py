@@ -67,7 +67,7 @@ def default_ops():
                            block_stands_for=(("linear", _native.linear), ("layer_norm", _native.layer_norm),
                                              ("add_layer_norm", _native.add_layer_norm)),
                            weight_grad=_native.weight_grad, weight_grad_supported=_native.weight_grad_supported,
-                           gelu_backward=_native.gelu_backward, norm_backward=_native.norm_backward,
+                           block_tail_backward=_native.block_tail_backward, norm_linear_backward=_native.norm_linear_backward,
                            attention_columns_backward=_native.attention_columns_backward,
                            table_linear_grad=_native.table_linear_grad,
                            blocks_forward=_native.blocks_forward, block_params=_native.BlockParams,
@@ -450,17 +450,17 @@ class _NormLinearRows(torch.autograd.Function):
     def forward(ctx, x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, eps, dt, ops):
         c = x.shape[-1]
         # packed in every forward, not kept: the weights of a training step are new ones
-        packed, at = ops.block_pack(c, dt, [(w_q, False), (w_kv, False)])
+        packed, at = ops.block_pack(c, dt, [(w_q, False), (w_kv, False), (w_q, True), (w_kv, True)])
         qkv, normed, stats = ops.norm_linear(x, norm_w, norm_b, eps, packed, at[0], b_q, b_kv, 3 * c, keep=True)
-        ctx.save_for_backward(x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, normed, stats, torch.cat([w_q, w_kv]).to(dt))
-        ctx.meta = (eps, dt, ops)
+        ctx.save_for_backward(x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, normed, stats, packed)
+        ctx.meta = (eps, dt, ops, at[2:])
         return qkv, x
 
     @staticmethod
     @_types_of_forward
     def backward(ctx, d_qkv, d_res):
-        x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, normed, stats, w = ctx.saved_tensors
-        eps, dt, ops = ctx.meta
+        x, norm_w, norm_b, w_q, b_q, w_kv, b_kv, normed, stats, packed = ctx.saved_tensors
+        eps, dt, ops, at = ctx.meta
         c = x.shape[-1]
         if not _by_kernels(d_qkv, d_res):
             def layers(x, norm_w, norm_b, w_q, b_q, w_kv, b_kv):
@@ -472,7 +472,7 @@ class _NormLinearRows(torch.autograd.Function):
         flat = normed.view(-1, c)
         grads = [None] * 7
         if need[0] or need[1] or need[2]:
-            grads[0], _, grads[1], grads[2] = ops.norm_backward((rows @ w).view(x.shape), x, stats, norm_w, _dense(d_res))
+            grads[0], grads[1], grads[2] = ops.norm_linear_backward(rows, x, stats, norm_w, packed, at, _dense(d_res))
         wanted = [(i, rows[:, cols], need[i + 1]) for i, cols in ((3, slice(0, c)), (5, slice(c, 3 * c))) if need[i] or need[i + 1]]
         if wanted:
             for (i, _, _), (grads[i], grads[i + 1]) in zip(wanted, ops.weight_grad([(d, flat, bias) for _, d, bias in wanted])):
@@ -487,18 +487,17 @@ class _BlockTail(torch.autograd.Function):
     @staticmethod
     def forward(ctx, attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, eps, dt, ops):
         weights = (w_p, w_1, w_2)
-        packed, at = ops.block_pack(x.shape[-1], dt, [(w, False) for w in weights])
+        packed, at = ops.block_pack(x.shape[-1], dt, [(w, False) for w in weights] + [(w, True) for w in weights])
         out, x1, normed, hidden, stats = ops.block_tail(attn, x, packed, at, b_p, norm_w, norm_b, eps, b_1, b_2, scale, keep=True)
-        plain = torch.cat([w.reshape(-1) for w in weights]).to(dt)
-        ctx.save_for_backward(attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, x1, normed, hidden, stats, plain)
-        ctx.meta = (eps, dt, ops)
+        ctx.save_for_backward(attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, x1, normed, hidden, stats, packed)
+        ctx.meta = (eps, dt, ops, at[3:])
         return out
 
     @staticmethod
     @_types_of_forward
     def backward(ctx, d_out):
-        attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, x1, normed, hidden, stats, plain = ctx.saved_tensors
-        eps, dt, ops = ctx.meta
+        attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2, scale, x1, normed, hidden, stats, packed = ctx.saved_tensors
+        eps, dt, ops, at = ctx.meta
         b, c, h = x.shape[0], x.shape[-1], hidden.shape[-1]
         if not _by_kernels(d_out):
             def layers(attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2):
@@ -510,20 +509,10 @@ class _BlockTail(torch.autograd.Function):
             return (*_recorded_backward(layers, ctx, (attn, x, w_p, b_p, norm_w, norm_b, w_1, b_1, w_2, b_2), (d_out,)),
                     None, None, None, None)
         need = ctx.needs_input_grad
-        d_out = _dense(d_out)
-        p16, one, two = plain[:c * c].view(c, c), plain[c * c:c * (c + h)].view(h, c), plain[c * (c + h):].view(c, h)
-        d_f = d_out.to(dt)
-        if scale is not None:
-            d_f = d_f * scale[1].to(dt).view(-1, *(1,) * (x.dim() - 1))
-        d_f = d_f.view(-1, c)
-        g, d_h = ops.gelu_backward(hidden.view(-1, h), d_f @ two)
         grads = [None] * 10
-        separate = x.dtype != dt or scale is not None
-        grads[1], branch, grads[4], grads[5] = ops.norm_backward((d_h @ one).view(x.shape), x1, stats, norm_w, d_out, separate,
-                                                                 None if scale is None else scale[0])
-        branch = (branch if separate else grads[1]).view(-1, c)
-        if need[0]:
-            grads[0] = (branch @ p16).view(attn.shape)
+        grads[1], branch, d_f, g, d_h, grads[0], grads[4], grads[5] = ops.block_tail_backward(_dense(d_out), x1, stats, norm_w, hidden,
+                                                                                              packed, at, scale)
+        branch, d_f, g, d_h = branch.view(-1, c), d_f.view(-1, c), g.view(-1, h), d_h.view(-1, h)
         wanted = [(i, d, y, need[i + 1]) for i, d, y in ((2, branch, attn.view(-1, c)), (6, d_h, normed.view(-1, c)), (8, d_f, g))
                   if need[i] or need[i + 1]]
         if wanted:
@@ -811,9 +800,10 @@ class ClusterTransformerBlock(_Module):
         are not built for, with layer scale or an active dropout, with modules of other types or with hooks, and when the
         caller's `ops` has another implementation of a layer they stand for."""
         ops = self.attn.ops
-        if self.layer_scale or not feat.is_cuda or getattr(ops, "block_tail", None) is None or not self.plain():
-            return None
         grad = torch.is_grad_enabled()
+        if (self.layer_scale or not feat.is_cuda or getattr(ops, "block_tail", None) is None
+                or (grad and getattr(ops, "block_tail_backward", None) is None) or not self.plain()):
+            return None
         if _drops(self.mlp.drop) or _drops(self.attn.proj_drop) or (not grad and _drops(self.drop_path)):
             return None
         dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else torch.float32

@@ -138,6 +138,11 @@ _PROTOTYPES = {
                                                               ctypes.c_int]),
     "clusten_weight_grad": (ctypes.c_int, [ctypes.POINTER(WeightGradItem), ctypes.c_int, ctypes.c_int64, _P, ctypes.c_size_t,
                                            ctypes.c_int, _P]),
+    "clusten_block_backward_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
+    "clusten_block_tail_backward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, _P,
+                                                  _P, _P, ctypes.c_size_t, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_norm_linear_backward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, ctypes.c_int64,
+                                                   ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
     "clusten_row_sums_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
     "clusten_gelu_backward": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, _P]),
     "clusten_norm_backward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, ctypes.c_int, _P, _P, _P,
@@ -1779,6 +1784,87 @@ def block_tail(attn: torch.Tensor, x: torch.Tensor, packed: torch.Tensor, at, bi
                                               *map(_ptr, kept), x.numel() // c, c, hidden,
                                               _DTYPE_CODES[packed.dtype], _stream(device)), "clusten_block_tail_forward")
     return (out,) + kept if keep else out
+
+
+def _packed_fit(packed, at, sizes, what):
+    """Raises unless every (elements) matrix of `sizes` lies inside `packed` at its byte offset."""
+    total = packed.numel() * packed.element_size()
+    if any(o < 0 or o % 16 or o + n * packed.element_size() > total for o, n in zip(at, sizes)):
+        raise RuntimeError(what + ": the packed weights do not hold matrices of these sizes")
+
+
+def _block_backward_sums(rows: int, c: int, device):
+    """Workspace of a block's backward kernel and the norm's two (C,) gradients."""
+    nbytes = load().clusten_block_backward_workspace_bytes(rows, c)
+    return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes, torch.empty(2, c, dtype=torch.float32, device=device)
+
+
+def block_tail_backward(d_out: torch.Tensor, x1: torch.Tensor, stats: torch.Tensor, norm_w, hidden: torch.Tensor, packed: torch.Tensor, at,
+                        scale=None):
+    """Backward of `block_tail` over its rows, from what it kept: (d_x, branch, d_f, g, d_h, d_attn, d_norm_w, d_norm_b).  `at`: byte
+    offsets in `packed` of the packed transposes of Wp, W1 and W2.  d_x (x1's dtype) is the gradient of the residual stream, branch and
+    d_f (packed's dtype) that of the output projection's and of fc2's result, g = gelu(hidden) and d_h what their weights'
+    gradients read besides, d_attn the gradient of the attention's output.  No autograd."""
+    dt, c, h = packed.dtype, x1.shape[-1], hidden.shape[-1]
+    if (x1.dtype not in (torch.float32, dt) or dt not in _DTYPE_CODES or c not in _BLOCK_WIDTHS or h % c or not x1.is_cuda
+            or hidden.numel() * c != x1.numel() * h):
+        raise RuntimeError("block_tail_backward: rows of a width of the block kernels, x1 fp32 or of the weights' dtype")
+    _block_rows((x1.dtype,), c, x1, d_out)
+    _block_rows((dt,), h, hidden)
+    rows, device = x1.numel() // c, x1.device
+    if (stats.numel() != 2 * rows or stats.dtype != torch.float32 or not stats.is_contiguous() or norm_w.dtype != torch.float32
+            or not norm_w.is_contiguous() or norm_w.numel() != c or any(t.device != device for t in (hidden, packed, stats, norm_w))):
+        raise RuntimeError("block_tail_backward: fp32 statistics and norm weight of x1's rows, all on one device")
+    _packed_fit(packed, at, (c * c, c * h, c * h), "block_tail_backward")
+    if scale is not None and (scale.dtype != torch.float32 or not scale.is_contiguous() or tuple(scale.shape) != (2, x1.shape[0])
+                              or scale.device != device):
+        raise RuntimeError("scale must be contiguous fp32 of shape (2,B)")
+    separate = scale is not None or x1.dtype != dt
+    d_x, d_attn = torch.empty_like(x1), torch.empty(x1.shape, dtype=dt, device=device)
+    branch = torch.empty_like(d_attn) if separate else d_x
+    d_f = torch.empty_like(d_attn) if separate else d_out
+    g, d_h = torch.empty_like(hidden), torch.empty_like(hidden)
+    if rows == 0:
+        zero = torch.zeros(2, c, device=device)
+        return d_x, branch, d_f, g, d_h, d_attn, zero[0], zero[1]
+    ws, nbytes, sums = _block_backward_sums(rows, c, device)
+    with _on(device):
+        base, to = packed.data_ptr(), sums.data_ptr()
+        _check(load().clusten_block_tail_backward(d_out.data_ptr(), x1.data_ptr(), _DTYPE_CODES[x1.dtype], stats.data_ptr(), norm_w.data_ptr(),
+                                                  hidden.data_ptr(), base + at[0], base + at[1], base + at[2], _ptr(scale), rows // x1.shape[0],
+                                                  d_x.data_ptr(), branch.data_ptr() if separate else None,
+                                                  d_f.data_ptr() if separate else None, g.data_ptr(), d_h.data_ptr(), d_attn.data_ptr(), to,
+                                                  to + 4 * c, ws.data_ptr(), nbytes, rows, c, h, _DTYPE_CODES[dt], _stream(device)),
+               "clusten_block_tail_backward")
+    return d_x, branch, d_f, g, d_h, d_attn, sums[0], sums[1]
+
+
+def norm_linear_backward(d_y: torch.Tensor, x: torch.Tensor, stats: torch.Tensor, norm_w, packed: torch.Tensor, at, d_res=None):
+    """Backward of `norm_linear` over its rows: (d_x, d_norm_w, d_norm_b), d_x = d_res + the gradient through the norm, of x's dtype.
+    `at`: byte offsets in `packed` of the packed transposes of W's first C rows and of the others.  No autograd."""
+    dt, c, n = packed.dtype, x.shape[-1], d_y.shape[-1]
+    if (x.dtype not in (torch.float32, dt) or dt not in _DTYPE_CODES or c not in _BLOCK_WIDTHS or n % c or not x.is_cuda
+            or d_y.numel() * c != x.numel() * n):
+        raise RuntimeError("norm_linear_backward: rows of a width of the block kernels, x fp32 or of the weights' dtype")
+    _block_rows((x.dtype,), c, x, d_res)
+    _block_rows((dt,), n, d_y)
+    rows, device = x.numel() // c, x.device
+    if (stats.numel() != 2 * rows or stats.dtype != torch.float32 or not stats.is_contiguous() or norm_w.dtype != torch.float32
+            or not norm_w.is_contiguous() or norm_w.numel() != c or any(t.device != device for t in (d_y, packed, stats, norm_w))):
+        raise RuntimeError("norm_linear_backward: fp32 statistics and norm weight of x's rows, all on one device")
+    _packed_fit(packed, at, (c * c, c * (n - c)), "norm_linear_backward")
+    d_x = torch.empty_like(x)
+    if rows == 0:
+        zero = torch.zeros(2, c, device=device)
+        return d_x, zero[0], zero[1]
+    ws, nbytes, sums = _block_backward_sums(rows, c, device)
+    with _on(device):
+        to = sums.data_ptr()
+        _check(load().clusten_norm_linear_backward(d_y.data_ptr(), x.data_ptr(), _DTYPE_CODES[x.dtype], stats.data_ptr(), norm_w.data_ptr(),
+                                                   packed.data_ptr() + at[0], packed.data_ptr() + at[1], _ptr(d_res), d_x.data_ptr(), to,
+                                                   to + 4 * c, ws.data_ptr(), nbytes, rows, c, n, _DTYPE_CODES[dt], _stream(device)),
+               "clusten_norm_linear_backward")
+    return d_x, sums[0], sums[1]
 
 
 def _row_sums(rows: int, c: int, device):

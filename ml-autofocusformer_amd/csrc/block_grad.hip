@@ -48,9 +48,9 @@ __global__ __launch_bounds__(256) void gelu_backward_kernel(const T* __restrict_
     load8(d_g + i * 8, d);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        y[e] = gelu_for<T>(v[e]);
-        const float cdf = sizeof(T) == 2 ? normal_cdf(v[e]) : 0.5f * erfcf(-0.70710678118654752440f * v[e]);
-        d[e] *= cdf + v[e] * 0.39894228040143267794f * __expf(-0.5f * v[e] * v[e]);
+        float slope;
+        y[e] = gelu_and_slope<T>(v[e], slope);
+        d[e] *= slope;
     }
     store8(g + i * 8, y);
     store8(d_h + i * 8, d);
@@ -235,7 +235,7 @@ __global__ __launch_bounds__(1024) void table_linear_grad_kernel(const float* __
 // costs a partial row.
 int row_groups(int64_t rows, int C) {
     const int64_t per = kRowThreads / (C / 8);
-    return (int)min((rows + per - 1) / per, (int64_t)1024);
+    return (int)min((rows + per - 1) / per, (int64_t)kRowSumGroups);
 }
 
 template <typename T, typename S>
@@ -264,12 +264,12 @@ int blank_grad_width(const BlankGrad& a, int C, int groups, hipStream_t stream) 
     return launch_status();
 }
 
+}  // namespace
+
 int launch_column_sums(const float* partial, int groups, int C, float scale0, float* out0, float* out1, hipStream_t stream) {
     hipLaunchKernelGGL(column_sums_kernel, dim3(2 * C / 64), dim3(1024), 0, stream, partial, groups, C, scale0, out0, out1);
     return launch_status();
 }
-
-}  // namespace
 
 size_t row_sums_workspace_bytes(int64_t rows, int C) { return (size_t)row_groups(rows, C) * 2 * C * sizeof(float); }
 

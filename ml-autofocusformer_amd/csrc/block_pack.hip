@@ -9,6 +9,12 @@ int launch_norm_linear_f32(const NormLinearArgs& a, int C, hipStream_t stream);
 int launch_block_tail_f16(const BlockTailArgs& a, int x_dtype, int C, hipStream_t stream);
 int launch_block_tail_bf16(const BlockTailArgs& a, int x_dtype, int C, hipStream_t stream);
 int launch_block_tail_f32(const BlockTailArgs& a, int C, hipStream_t stream);
+int launch_block_tail_backward_f16(const BlockTailGrad& a, int x_dtype, int C, hipStream_t stream);
+int launch_block_tail_backward_bf16(const BlockTailGrad& a, int x_dtype, int C, hipStream_t stream);
+int launch_block_tail_backward_f32(const BlockTailGrad& a, int C, hipStream_t stream);
+int launch_norm_linear_backward_f16(const NormLinearGrad& a, int x_dtype, int C, hipStream_t stream);
+int launch_norm_linear_backward_bf16(const NormLinearGrad& a, int x_dtype, int C, hipStream_t stream);
+int launch_norm_linear_backward_f32(const NormLinearGrad& a, int C, hipStream_t stream);
 
 namespace {
 
@@ -103,6 +109,22 @@ int launch_block_tail(const BlockTailArgs& a, int x_dtype, int C, int dtype, hip
     if (dtype == CLUSTEN_F16) return launch_block_tail_f16(a, x_dtype, C, stream);
     if (dtype == CLUSTEN_BF16) return launch_block_tail_bf16(a, x_dtype, C, stream);
     return launch_block_tail_f32(a, C, stream);
+}
+
+size_t block_backward_workspace_bytes(int64_t rows, int C) {
+    return (size_t)min((rows + 15) / 16, (int64_t)kRowSumGroups) * 2 * C * sizeof(float);
+}
+
+int launch_block_tail_backward(const BlockTailGrad& a, int x_dtype, int C, int dtype, hipStream_t stream) {
+    if (dtype == CLUSTEN_F16) return launch_block_tail_backward_f16(a, x_dtype, C, stream);
+    if (dtype == CLUSTEN_BF16) return launch_block_tail_backward_bf16(a, x_dtype, C, stream);
+    return launch_block_tail_backward_f32(a, C, stream);
+}
+
+int launch_norm_linear_backward(const NormLinearGrad& a, int x_dtype, int C, int dtype, hipStream_t stream) {
+    if (dtype == CLUSTEN_F16) return launch_norm_linear_backward_f16(a, x_dtype, C, stream);
+    if (dtype == CLUSTEN_BF16) return launch_norm_linear_backward_bf16(a, x_dtype, C, stream);
+    return launch_norm_linear_backward_f32(a, C, stream);
 }
 
 }  // namespace clusten

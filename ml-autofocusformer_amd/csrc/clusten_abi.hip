@@ -680,6 +680,55 @@ int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x
     return CLUSTEN_OK;
 }
 
+size_t clusten_block_backward_workspace_bytes(int64_t rows, int C) {
+    return rows > 0 && rows < (int64_t)1 << 31 && block_width_supported(C) ? block_backward_workspace_bytes(rows, C) : 0;
+}
+
+int clusten_block_tail_backward(const void* d_out, const void* x1, int x_dtype, const float* stats, const float* norm_w, const void* hidden,
+                                const void* wp_t, const void* w1_t, const void* w2_t, const float* scale, int rows_per_image, void* d_x,
+                                void* branch, void* d_f, void* g, void* d_h, void* d_attn, float* d_norm_w, float* d_norm_b, void* workspace,
+                                size_t workspace_bytes, int64_t rows, int C, int H, int dtype, clusten_stream stream) {
+    if (!d_out || !x1 || !stats || !norm_w || !hidden || !wp_t || !w1_t || !w2_t || !d_x || !g || !d_h || !d_attn || !d_norm_w || !d_norm_b ||
+        !workspace) {
+        return CLUSTEN_ERR_NULL_POINTER;
+    }
+    if (!block_dtype_ok(dtype) || (x_dtype != dtype && x_dtype != CLUSTEN_F32)) return CLUSTEN_ERR_BAD_DTYPE;
+    const size_t need = clusten_block_backward_workspace_bytes(rows, C);
+    if (need == 0 || H <= 0 || H % C != 0) return CLUSTEN_ERR_BAD_DIMS;
+    if (scale && (rows_per_image <= 0 || rows % rows_per_image != 0)) return CLUSTEN_ERR_BAD_DIMS;
+    if (workspace_bytes < need) return CLUSTEN_ERR_WORKSPACE;
+    const void* all[] = {d_out, x1, norm_w, hidden, wp_t, w1_t, w2_t, d_x, branch, d_f, g, d_h, d_attn, workspace};
+    for (const void* p : all) {
+        if (!aligned16(p)) return CLUSTEN_ERR_UNALIGNED;
+    }
+    if (reinterpret_cast<uintptr_t>(stats) & 7) return CLUSTEN_ERR_UNALIGNED;
+    BlockTailGrad a = {};
+    a.d_out = d_out, a.x1 = x1, a.stats = reinterpret_cast<const float2*>(stats), a.norm_w = norm_w, a.hidden = hidden, a.wp = wp_t, a.w1 = w1_t;
+    a.w2 = w2_t, a.scale = scale, a.d_x = d_x, a.branch = branch, a.d_f = d_f, a.g = g, a.d_h = d_h, a.d_attn = d_attn, a.d_norm_w = d_norm_w;
+    a.d_norm_b = d_norm_b, a.partial = static_cast<float*>(workspace), a.rows = rows, a.rows_per_image = scale ? rows_per_image : 1;
+    a.chunks = H / C;
+    return launch_block_tail_backward(a, x_dtype, C, dtype, as_stream(stream));
+}
+
+int clusten_norm_linear_backward(const void* d_y, const void* x, int x_dtype, const float* stats, const float* norm_w, const void* w0_t,
+                                 const void* w1_t, const void* d_res, void* d_x, float* d_norm_w, float* d_norm_b, void* workspace, size_t workspace_bytes,
+                                 int64_t rows, int C, int N, int dtype, clusten_stream stream) {
+    if (!d_y || !x || !stats || !norm_w || !w0_t || (N > C && !w1_t) || !d_x || !d_norm_w || !d_norm_b || !workspace) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype) || (x_dtype != dtype && x_dtype != CLUSTEN_F32)) return CLUSTEN_ERR_BAD_DTYPE;
+    const size_t need = clusten_block_backward_workspace_bytes(rows, C);
+    if (need == 0 || N <= 0 || N % C != 0) return CLUSTEN_ERR_BAD_DIMS;
+    if (workspace_bytes < need) return CLUSTEN_ERR_WORKSPACE;
+    const void* all[] = {d_y, x, norm_w, w0_t, w1_t, d_res, d_x, workspace};
+    for (const void* p : all) {
+        if (!aligned16(p)) return CLUSTEN_ERR_UNALIGNED;
+    }
+    if (reinterpret_cast<uintptr_t>(stats) & 7) return CLUSTEN_ERR_UNALIGNED;
+    NormLinearGrad a = {};
+    a.d_y = d_y, a.x = x, a.stats = reinterpret_cast<const float2*>(stats), a.norm_w = norm_w, a.w0 = w0_t, a.w1 = w1_t, a.d_res = d_res;
+    a.d_x = d_x, a.d_norm_w = d_norm_w, a.d_norm_b = d_norm_b, a.partial = static_cast<float*>(workspace), a.rows = rows, a.chunks = N / C;
+    return launch_norm_linear_backward(a, x_dtype, C, dtype, as_stream(stream));
+}
+
 size_t clusten_row_sums_workspace_bytes(int64_t rows, int C) {
     return rows > 0 && rows < (int64_t)1 << 31 && block_width_supported(C) ? row_sums_workspace_bytes(rows, C) : 0;
 }

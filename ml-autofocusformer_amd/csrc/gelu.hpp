@@ -65,4 +65,12 @@ __device__ __forceinline__ float gelu_for(float v) {
     else return gelu_erf(v);
 }
 
+// gelu(v) of results of type T, and gelu'(v) = Phi(v) + v phi(v).
+template <typename T>
+__device__ __forceinline__ float gelu_and_slope(float v, float& slope) {
+    const float cdf = sizeof(T) == 2 ? normal_cdf(v) : 0.5f * erfcf(-0.70710678118654752440f * v);
+    slope = cdf + v * 0.39894228040143267794f * __expf(-0.5f * v * v);
+    return gelu_for<T>(v);
+}
+
 }  // namespace clusten

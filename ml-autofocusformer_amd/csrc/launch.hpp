@@ -299,6 +299,51 @@ int launch_block_pack(const clusten_pack_item* items, int count, int C, int dtyp
 int launch_norm_linear(const NormLinearArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);
 int launch_block_tail(const BlockTailArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);
 
+// Backward of the two (block_backward_impl.hpp); the weights are packed transposes.
+struct BlockTailGrad {
+    const void* d_out;     // (rows, C) of S
+    const void* x1;        // (rows, C) of S
+    const float2* stats;
+    const float* norm_w;
+    const void* hidden;    // (rows, H) of T
+    const void* wp;        // Wp^T (C, C)
+    const void* w1;        // W1^T (C, H)
+    const void* w2;        // W2^T (H, C)
+    const float* scale;    // as in BlockTailArgs
+    void* d_x;             // (rows, C) of S
+    void* branch;          // (rows, C) of T: d_x times the image's first factor, or null
+    void* d_f;             // (rows, C) of T: d_out times the image's second factor, or null
+    void* g;               // (rows, H) of T
+    void* d_h;             // (rows, H) of T
+    void* d_attn;          // (rows, C) of T
+    float* d_norm_w;
+    float* d_norm_b;
+    float* partial;
+    int64_t rows;
+    int rows_per_image, chunks;
+};
+struct NormLinearGrad {
+    const void* d_y;       // (rows, N) of T
+    const void* x;         // (rows, C) of S
+    const float2* stats;
+    const float* norm_w;
+    const void* w0;        // W^T of the first C outputs (C, C)
+    const void* w1;        // W^T of the others (C, N - C)
+    const void* d_res;     // (rows, C) of S, or null
+    void* d_x;             // (rows, C) of S
+    float* d_norm_w;
+    float* d_norm_b;
+    float* partial;
+    int64_t rows;
+    int chunks;
+};
+constexpr int kRowSumGroups = 1024;     // partial rows of a sum over all rows, at most
+size_t block_backward_workspace_bytes(int64_t rows, int C);
+int launch_block_tail_backward(const BlockTailGrad& a, int x_dtype, int C, int dtype, hipStream_t stream);
+int launch_norm_linear_backward(const NormLinearGrad& a, int x_dtype, int C, int dtype, hipStream_t stream);
+// Sums of `groups` partial rows of 2 C values: the first C times scale0 to out0, the others to out1.
+int launch_column_sums(const float* partial, int groups, int C, float scale0, float* out0, float* out1, hipStream_t stream);
+
 // Parameter gradients of Linear layers over the same rows (weight_grad.hip).
 size_t weight_grad_workspace_bytes(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype);
 int launch_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, float* workspace, int dtype, hipStream_t stream);

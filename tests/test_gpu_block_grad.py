@@ -80,6 +80,63 @@ def test_norm_backward(device, dt, stream, c, b, n):
     assert branch is None
 
 
+# a row tile, two of them, more tiles than workgroups (1024), last ones partly filled
+ROWS = [(32, 64, 1, 1), (32, 96, 3, 11), (64, 192, 2, 16 * 1024 + 5), (128, 384, 1, 4097), (128, 256, 3, 33), (256, 768, 1, 49),
+        (256, 512, 2, 2100), (512, 1536, 1, 15), (512, 512, 3, 1400)]
+# relative 2-norm: one rounding of a result (a third of the bar in the mean) and what d_h rounded on its way does to a sum
+NORM_BAR = {torch.float16: 5e-4, torch.bfloat16: 4e-3, torch.float32: 6e-7}
+
+
+@pytest.mark.parametrize("dt,stream", [(torch.float16, torch.float16), (torch.float16, torch.float32),
+                                       (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("c,hidden,b,n", ROWS)
+@pytest.mark.parametrize("scaled", [False, True])
+def test_block_backward_over_rows(device, dt, stream, c, hidden, b, n, scaled):
+    """The two kernels of a block's backward against float64 on the same stored operands."""
+    gen = torch.Generator(device).manual_seed(c + n)
+
+    def draw(*shape, scale=1.0):
+        return torch.randn(*shape, generator=gen, device=device) * scale
+
+    w_p, w_1, w_2 = draw(c, c, scale=c ** -0.5), draw(hidden, c, scale=c ** -0.5), draw(c, hidden, scale=hidden ** -0.5)
+    w_q, w_kv = draw(c, c, scale=c ** -0.5), draw(2 * c, c, scale=c ** -0.5)
+    packed, at = _native.block_pack(c, dt, [(w, True) for w in (w_p, w_1, w_2, w_q, w_kv)])
+    x, d_out, d_y = (draw(b, n, c) + 0.5).to(stream), draw(b, n, c).to(stream), draw(b, n, 3 * c).to(dt)
+    h, norm_w = draw(b, n, hidden).to(dt), 1 + 0.2 * draw(c)
+    scale = draw(2, b).abs().to(dt).float() if scaled else None
+    x64, w64, zero = x.double().requires_grad_(True), norm_w.double().requires_grad_(True), torch.zeros(c, device=device).double()
+    b64 = zero.clone().requires_grad_(True)
+    norm = F.layer_norm(x64, (c,), w64, b64)
+    mean = x.double().mean(-1)
+    stats = torch.stack([mean, (x.double().var(-1, unbiased=False) + 1e-5).rsqrt()], -1).float().reshape(-1, 2).contiguous()
+
+    def as_stored(t):
+        return t.to(dt).double()
+
+    def near(got, ref, bar=NORM_BAR[dt]):
+        assert got.shape == ref.shape and (got.double() - ref).norm() <= bar * ref.norm()
+
+    got = _native.block_tail_backward(d_out, x, stats, norm_w, h, packed, at[:3], scale)
+    d_f = as_stored(as_stored(d_out) * (1.0 if scale is None else scale[1].double().view(b, 1, 1)))
+    h64 = h.double().requires_grad_(True)
+    g = F.gelu(h64)
+    d_h = as_stored(torch.autograd.grad(g, h64, d_f @ as_stored(w_2))[0])
+    grads = torch.autograd.grad(norm, (x64, w64, b64), d_h @ as_stored(w_1), retain_graph=True)
+    d_x = (d_out.double() + grads[0]).to(stream).double()
+    branch = as_stored(d_x * (1.0 if scale is None else scale[0].double().view(b, 1, 1)))
+    for t, ref in zip(got, (d_x, branch, d_f, g.detach(), d_h, branch @ as_stored(w_p))):
+        near(t, ref)
+    for t, ref in zip(got[6:], grads[1:]):
+        near(t, ref, max(NORM_BAR[dt], 2e-6))
+
+    for d_res in (None, d_out):
+        got = _native.norm_linear_backward(d_y, x, stats, norm_w, packed, at[3:], d_res)
+        grads = torch.autograd.grad(norm, (x64, w64, b64), d_y.double() @ as_stored(torch.cat([w_q, w_kv])), retain_graph=True)
+        near(got[0], grads[0] if d_res is None else grads[0] + d_res.double(), NORM_BAR[stream])
+        for t, ref in zip(got[1:], grads[1:]):
+            near(t, ref, 2e-6)
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("b,h,n,ch", [(1, 1, 1, 32), (2, 2, 777, 32), (3, 4, 100, 8), (2, 16, 259, 32)])
 def test_attention_columns(device, dt, b, h, n, ch):
