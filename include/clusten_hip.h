@@ -710,6 +710,37 @@ int clusten_norm_linear_backward(const void* d_y, const void* x, int x_dtype, co
                                  void* workspace, size_t workspace_bytes, int64_t rows, int C, int N, int dtype,
                                  clusten_stream stream);
 
+/* The training pass of an attention layer beside its attention kernels (models/aff_transformer.py:103-155 under autograd), dtype F32,
+ * F16 or BF16.
+ *   position_bias: bias (rows,n) = table weight^T + bias_param (may be NULL) for a fp32 table (rows,k), k <= 8, every operand rounded to
+ *     dtype; padded (rows,8) of dtype, when not NULL: the table's rows, zeros behind the k columns.
+ *   position_grad: d_weight (H,k) = sum d_logit[b,h,i,j] table[pe_idx[b,i,j]], d_bias (H) = sum d_logit, for d_logit (B,H,N,M) of dtype,
+ *     pe_idx (B,N,M) inside the table, M a multiple of 4, k <= 5; sums in fp64 in a fixed order.
+ *   dense_attention_train: attention of N <= 64 tokens over all of them, heads of 32 channels: qkv (B,N,3C), C = 32 H, a row holding q, then
+ *     per head k and v; out (B,N,C); bias and padded of position_bias, pe_idx (B,N,N); fp32 inside.  The backward writes all of d_qkv and
+ *     the gradients of the blank token (C) and of the position bias layer.
+ *   scatter_attention_pair: d_key = scale * scatter(d_logit, query) and d_value = scatter(probs, d_out) over pair_lists
+ *     (clusten_cluster_pairs_from_numbers) in one launch; d_key and d_value have out_strides. */
+int clusten_position_bias(const float* table, const float* weight, const float* bias_param, void* bias, void* padded, int rows,
+                          int n, int k, int dtype, clusten_stream stream);
+size_t clusten_position_grad_workspace_bytes(int B, int H, int N, int M);
+int clusten_position_grad(const void* d_logit, const int64_t* pe_idx, const void* padded, float* d_weight, float* d_bias,
+                          void* workspace, size_t workspace_bytes, int B, int H, int N, int M, int rows, int k, int dtype,
+                          clusten_stream stream);
+int clusten_dense_attention_train_forward(const void* qkv, const void* bias, const int64_t* pe_idx, const float* blank_k,
+                                          const float* blank_v, void* out, float scale, int B, int H, int N, int rows, int dtype,
+                                          clusten_stream stream);
+size_t clusten_dense_attention_train_workspace_bytes(int B, int H);
+int clusten_dense_attention_train_backward(const void* qkv, const void* bias, const void* padded, const int64_t* pe_idx,
+                                           const float* blank_k, const float* blank_v, const void* d_out, void* d_qkv,
+                                           float* d_blank_k, float* d_blank_v, float* d_weight, float* d_bias, void* workspace,
+                                           size_t workspace_bytes, float scale, int B, int H, int N, int rows, int k, int dtype,
+                                           clusten_stream stream);
+int clusten_scatter_attention_pair(const void* d_logit, const void* query, clusten_strides query_strides, void* d_key,
+                                   const void* probs, const void* d_out, clusten_strides d_out_strides, void* d_value,
+                                   clusten_strides out_strides, float scale, const void* pair_lists, clusten_attn_shape shape,
+                                   int dtype, clusten_stream stream);
+
 /* The backward of a block between its products, which the reference leaves to autograd.  Tensors are dense rows of C channels
  * (C in {32,64,128,256,512}) of dtype F32, F16 or BF16 unless said otherwise, on 16-byte boundaries; sums are fp32 in a fixed
  * order; workspace: clusten_row_sums_workspace_bytes(rows, C) bytes.

@@ -68,8 +68,11 @@ def default_ops():
                                              ("add_layer_norm", _native.add_layer_norm)),
                            weight_grad=_native.weight_grad, weight_grad_supported=_native.weight_grad_supported,
                            block_tail_backward=_native.block_tail_backward, norm_linear_backward=_native.norm_linear_backward,
-                           attention_columns_backward=_native.attention_columns_backward,
-                           table_linear_grad=_native.table_linear_grad,
+                           attention_rows_backward=_native.attention_rows_backward, position_bias=_native.position_bias,
+                           position_grad=_native.position_grad, cluster_pairs_from_numbers=_native.cluster_pairs_from_numbers,
+                           dense_attention_train=_native.dense_attention_train,
+                           dense_attention_train_backward=_native.dense_attention_train_backward,
+                           dense_attention_train_supported=_native.dense_attention_train_supported,
                            blocks_forward=_native.blocks_forward, block_params=_native.BlockParams,
                            blocks_stand_for=(("cluster_attention", _native.cluster_attention),
                                              ("dense_attention", _native.dense_attention),
@@ -527,24 +530,22 @@ class _ClusterAttentionRows(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, qkv, pe_w, pe_b, blank_k, blank_v, table, plan, pairs, pe_idx, member_idx, mask, heads, scale, ops):
-        dt = qkv.dtype
-        table = table.to(dt)
-        bias = F.linear(table, pe_w.to(dt), pe_b.to(dt))
+        bias, padded = ops.position_bias(table, pe_w, pe_b, qkv.dtype)
         q, key, v = _columns(qkv, heads)
         out, lse = ops.cluster_attention(q, key, v, None, bias, None, None, blank_k, blank_v, scale=scale, plan=plan,
                                          return_lse=True)
-        ctx.save_for_backward(qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, table, plan, pairs, pe_idx, member_idx, mask)
-        ctx.meta = (heads, scale, ops)
+        ctx.save_for_backward(qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, padded, plan, pairs, pe_idx, member_idx, mask)
+        ctx.meta = (table.shape[1], heads, scale, ops)
         return out
 
     @staticmethod
     @_types_of_forward
     def backward(ctx, d_out):
-        qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, table, plan, pairs, pe_idx, member_idx, mask = ctx.saved_tensors
-        heads, scale, ops = ctx.meta
+        qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, padded, plan, pairs, pe_idx, member_idx, mask = ctx.saved_tensors
+        k, heads, scale, ops = ctx.meta
         if not _by_kernels(d_out):
             def layers(qkv, pe_w, pe_b, blank_k, blank_v):
-                bias = F.linear(table, pe_w.to(table.dtype), pe_b.to(table.dtype))
+                bias = F.linear(padded[:, :k], pe_w.to(padded.dtype), pe_b.to(padded.dtype))
                 return _local_attention(*_columns(qkv, heads), bias, blank_k, blank_v, mask, pe_idx, member_idx, scale)
             return (*_recorded_backward(layers, ctx, (qkv, pe_w, pe_b, blank_k, blank_v), (d_out,)), *(None,) * 9)
         q, key, v = _columns(qkv, heads)
@@ -552,13 +553,38 @@ class _ClusterAttentionRows(torch.autograd.Function):
         d_qkv = torch.empty_like(qkv)
         _, probs, d_logit, blank_prob, d_blank = ops.cluster_attention_backward(
             q, key, v, d_out, out, lse, plan, bias, blank_k, blank_v, scale=scale, d_query=_columns(d_qkv, heads)[0])
-        b, h, n, ch = q.shape
-        d_v = ops.scatter_rows(probs, d_out.view(b, n, h, ch).permute(0, 2, 1, 3), member_idx, pairs)
-        d_k = ops.scatter_rows(d_logit, q, member_idx, pairs)
-        d_bk, d_bv = ops.attention_columns_backward(qkv, d_qkv, d_k, d_v, d_out, d_blank, blank_prob, scale)
-        d_w, d_b = ops.table_linear_grad(ops.bias_table_grad(d_logit, pe_idx, bias.shape[0]), table)
+        d_bk, d_bv = ops.attention_rows_backward(qkv, d_qkv, probs, d_logit, d_out, d_blank, blank_prob, pairs, scale)
+        d_w, d_b = ops.position_grad(d_logit, pe_idx, padded, k)
         return (d_qkv, d_w.to(pe_w.dtype), d_b.to(pe_b.dtype), d_bk.reshape(blank_k.shape).to(blank_k.dtype),
                 d_bv.reshape(blank_v.shape).to(blank_v.dtype), *(None,) * 9)
+
+
+class _DenseAttentionRows(torch.autograd.Function):
+    """The attention of every token over all, as `_ClusterAttentionRows`: one kernel forward, one kernel and a sum backward."""
+
+    @staticmethod
+    def forward(ctx, qkv, pe_w, pe_b, blank_k, blank_v, table, pe_idx, heads, scale, ops):
+        bias, padded = ops.position_bias(table, pe_w, pe_b, qkv.dtype)
+        ctx.save_for_backward(qkv, pe_w, pe_b, blank_k, blank_v, bias, padded, pe_idx)
+        ctx.meta = (table.shape[1], heads, scale, ops)
+        return ops.dense_attention_train(qkv, bias, pe_idx, blank_k, blank_v, heads, scale)
+
+    @staticmethod
+    @_types_of_forward
+    def backward(ctx, d_out):
+        qkv, pe_w, pe_b, blank_k, blank_v, bias, padded, pe_idx = ctx.saved_tensors
+        k, heads, scale, ops = ctx.meta
+        if not _by_kernels(d_out):
+            def layers(qkv, pe_w, pe_b, blank_k, blank_v):
+                bias = F.linear(padded[:, :k], pe_w.to(padded.dtype), pe_b.to(padded.dtype))
+                b, n, _ = qkv.shape
+                everyone = torch.arange(n, device=qkv.device).expand(b, n, n)
+                return _local_attention(*_columns(qkv, heads), bias, blank_k, blank_v, None, pe_idx, everyone, scale)
+            return (*_recorded_backward(layers, ctx, (qkv, pe_w, pe_b, blank_k, blank_v), (d_out,)), *(None,) * 5)
+        d_qkv, d_bk, d_bv, d_w, d_b = ops.dense_attention_train_backward(qkv, bias, padded, pe_idx, blank_k, blank_v, _dense(d_out.to(qkv.dtype)),
+                                                                         k, heads, scale)
+        return (d_qkv, d_w.to(pe_w.dtype), d_b.to(pe_b.dtype), d_bk.reshape(blank_k.shape).to(blank_k.dtype),
+                d_bv.reshape(blank_v.shape).to(blank_v.dtype), *(None,) * 5)
 
 
 def _columns(qkv, heads):
@@ -695,9 +721,16 @@ class ClusterAttention(_Module):
         """`attend` of a training pass on the (b,n,3c) rows of the stacked projections."""
         c = self.dim
         pe = self.pos_embed
-        if self._trains_in_one_kernel(qkv[..., :c], global_attn, cluster_idx, grid_lists) and not table.requires_grad:
-            return _ClusterAttentionRows.apply(qkv, pe.weight, pe.bias, self.blank_k, self.blank_v, table, grid_lists[3],
-                                               grid_lists[4], pe_idx, member_idx, cluster_mask, self.num_heads, self.scale, self.ops)
+        # the kernels take a fp32 table of five columns and the parameters of the layer in place
+        if (table.dtype == torch.float32 and table.is_contiguous() and table.shape[1] <= 5 and not table.requires_grad
+                and getattr(self.ops, "position_bias", None) is not None):
+            params = (pe.weight, pe.bias, self.blank_k, self.blank_v)
+            if self._trains_in_one_kernel(qkv[..., :c], global_attn, cluster_idx, grid_lists):
+                return _ClusterAttentionRows.apply(qkv, *params, table, grid_lists[3], grid_lists[4], pe_idx, member_idx, cluster_mask,
+                                                   self.num_heads, self.scale, self.ops)
+            if (global_attn and not _drops(self.attn_drop) and pe_idx.is_contiguous()
+                    and self.ops.dense_attention_train_supported(qkv, self.num_heads)):
+                return _DenseAttentionRows.apply(qkv, *params, table, pe_idx, self.num_heads, self.scale, self.ops)
         q, kv = qkv.split([c, 2 * c], dim=-1)
         return self.attend(q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
 
@@ -1221,7 +1254,9 @@ class BasicLayer(_Module):
                 and (torch.is_autocast_enabled("cuda") or feat.dtype == torch.float32)):
             # training (fp32, or mixed precision): the plan of the one-kernel attention and the sorted pair lists of its
             # backward's scatters, built once for all blocks of the stage (a grid stage hands over one image's lists)
-            pairs = self.ops.cluster_pairs(member_idx)
+            # from the numbers, which the forward reads: lists of whole clusters by construction
+            from_numbers = getattr(self.ops, "cluster_pairs_from_numbers", None)
+            pairs = self.ops.cluster_pairs(member_idx) if from_numbers is None else from_numbers(cluster_idx)
             if pairs is not None:
                 lists = grid_lists if grid_lists is not None else (cluster_idx, pe_idx, mask)
                 grid_lists = tuple(lists) + (planner(lists[0], lists[1], lists[2]), pairs)

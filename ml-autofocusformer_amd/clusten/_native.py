@@ -143,6 +143,18 @@ _PROTOTYPES = {
                                                   _P, _P, ctypes.c_size_t, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
     "clusten_norm_linear_backward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, ctypes.c_int64,
                                                    ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_position_bias": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_position_grad_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "clusten_position_grad": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, ctypes.c_size_t, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                            ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_dense_attention_train_forward": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, ctypes.c_float, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                                            ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_dense_attention_train_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int]),
+    "clusten_dense_attention_train_backward": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, ctypes.c_float,
+                                                             ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                                             ctypes.c_int, _P]),
+    "clusten_scatter_attention_pair": (ctypes.c_int, [_P, _P, Strides, _P, _P, _P, Strides, _P, Strides, ctypes.c_float, _P, AttnShape,
+                                                     ctypes.c_int, _P]),
     "clusten_row_sums_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
     "clusten_gelu_backward": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, _P]),
     "clusten_norm_backward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, ctypes.c_int, _P, _P, _P,
@@ -1945,6 +1957,121 @@ def attention_columns_backward(qkv: torch.Tensor, d_qkv: torch.Tensor, d_k: torc
         at, stream = sums.data_ptr(), _stream(qkv.device)
         _check(lib.clusten_kv_columns(d_k.data_ptr(), d_v.data_ptr(), d_qkv.data_ptr(), scale, b, h, n, ch, code, stream),
                "clusten_kv_columns")
+        _check(lib.clusten_blank_grad(qkv.data_ptr(), c3, d_out.data_ptr(), d_blank.data_ptr(), blank_prob.data_ptr(), scale, at,
+                                      at + 4 * c, ws.data_ptr(), nbytes, b, h, n, c, code, stream), "clusten_blank_grad")
+    return sums[0], sums[1]
+
+
+def position_bias(table: torch.Tensor, weight: torch.Tensor, bias, dtype: torch.dtype):
+    """(table @ weight.T + bias of shape (rows, heads), the table's rows padded to 8 values), both in `dtype` and made of operands rounded
+    to it: the position bias of every row of a (rows, k <= 8) relative-position table.  No autograd."""
+    _require_cuda("table", table)
+    rows, k = table.shape
+    heads = weight.shape[0]
+    for t in (table, weight, bias):
+        if t is not None and (t.dtype != torch.float32 or not t.is_contiguous() or t.device != table.device):
+            raise RuntimeError("position_bias: contiguous fp32 table and parameters on one device")
+    if weight.dim() != 2 or weight.shape[1] != k or k > 8 or (bias is not None and bias.numel() != heads) or dtype not in _DTYPE_CODES:
+        raise RuntimeError("position_bias: table (rows,k), weight (heads,k), bias (heads), k <= 8")
+    out = torch.empty(rows, heads, dtype=dtype, device=table.device)
+    padded = torch.empty(rows, 8, dtype=dtype, device=table.device)
+    with _on(table.device):
+        _check(load().clusten_position_bias(table.data_ptr(), weight.data_ptr(), _ptr(bias), out.data_ptr(), padded.data_ptr(), rows, heads, k,
+                                            _DTYPE_CODES[dtype], _stream(table.device)), "clusten_position_bias")
+    return out, padded
+
+
+def position_grad(d_logit: torch.Tensor, pe_idx: torch.Tensor, padded: torch.Tensor, k: int):
+    """The gradients (d_weight (h,k), d_bias (h)) of `position_bias` from d_logit (b,h,n,m), m a multiple of 4, k <= 5."""
+    b, h, n, m = d_logit.shape
+    _require_cuda("d_logit", d_logit)
+    if (pe_idx.shape != (b, n, m) or pe_idx.dtype != torch.int64 or not pe_idx.is_contiguous() or not d_logit.is_contiguous()
+            or padded.dtype != d_logit.dtype or padded.dim() != 2 or padded.shape[1] != 8 or not padded.is_contiguous()
+            or any(t.device != d_logit.device for t in (pe_idx, padded))):
+        raise RuntimeError("position_grad: contiguous d_logit (b,h,n,m), pe_idx int64 (b,n,m) and padded (rows,8) of d_logit's dtype")
+    d_w, d_b = torch.empty(h, k, device=d_logit.device), torch.empty(h, device=d_logit.device)
+    nbytes = load().clusten_position_grad_workspace_bytes(b, h, n, m)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=d_logit.device)
+    with _on(d_logit.device):
+        _check(load().clusten_position_grad(d_logit.data_ptr(), pe_idx.data_ptr(), padded.data_ptr(), d_w.data_ptr(), d_b.data_ptr(), ws.data_ptr(),
+                                            nbytes, b, h, n, m, padded.shape[0], k, _DTYPE_CODES[d_logit.dtype], _stream(d_logit.device)),
+               "clusten_position_grad")
+    return d_w, d_b
+
+
+def dense_attention_train_supported(qkv: torch.Tensor, heads: int) -> bool:
+    """True when `dense_attention_train` takes (b,n,3c) rows: at most 64 tokens, heads of 32 channels."""
+    return (qkv.is_cuda and qkv.dim() == 3 and qkv.dtype in _DTYPE_CODES and qkv.is_contiguous() and qkv.data_ptr() % 16 == 0
+            and 0 < qkv.shape[1] <= 64 and qkv.shape[2] == 96 * heads and qkv.shape[0] > 0)
+
+
+def _dense_train(qkv, bias, pe_idx, blank_k, blank_v, heads):
+    b, n, _ = qkv.shape
+    if (not dense_attention_train_supported(qkv, heads) or pe_idx.shape != (b, n, n) or pe_idx.dtype != torch.int64 or not pe_idx.is_contiguous()
+            or bias.dtype != qkv.dtype or bias.dim() != 2 or bias.shape[1] != heads or not bias.is_contiguous()
+            or any(t.dtype != torch.float32 or not t.is_contiguous() or t.numel() != 32 * heads for t in (blank_k, blank_v))
+            or any(t.device != qkv.device for t in (bias, pe_idx, blank_k, blank_v))):
+        raise RuntimeError("dense_attention_train: rows, position bias, indices and blank token of one layer of heads of 32 channels")
+    return b, n
+
+
+def dense_attention_train(qkv: torch.Tensor, bias: torch.Tensor, pe_idx: torch.Tensor, blank_k, blank_v, heads: int, scale: float):
+    """Attention of every token over all n <= 64 on the (b,n,3c) rows of the stacked projections: (b,n,c).  `bias` from
+    `position_bias`.  fp32 inside, any of the three types.  No autograd."""
+    b, n = _dense_train(qkv, bias, pe_idx, blank_k, blank_v, heads)
+    out = torch.empty(b, n, 32 * heads, dtype=qkv.dtype, device=qkv.device)
+    with _on(qkv.device):
+        _check(load().clusten_dense_attention_train_forward(qkv.data_ptr(), bias.data_ptr(), pe_idx.data_ptr(), blank_k.data_ptr(), blank_v.data_ptr(),
+                                                            out.data_ptr(), scale, b, heads, n, bias.shape[0], _DTYPE_CODES[qkv.dtype],
+                                                            _stream(qkv.device)), "clusten_dense_attention_train_forward")
+    return out
+
+
+def dense_attention_train_backward(qkv: torch.Tensor, bias: torch.Tensor, padded: torch.Tensor, pe_idx: torch.Tensor, blank_k, blank_v,
+                                   d_out: torch.Tensor, k: int, heads: int, scale: float):
+    """(d_qkv, d_blank_k, d_blank_v, d_weight, d_bias) of `dense_attention_train`; the last two are `position_bias`' gradients."""
+    b, n = _dense_train(qkv, bias, pe_idx, blank_k, blank_v, heads)
+    _block_rows((qkv.dtype,), 32 * heads, d_out)
+    if d_out.numel() != b * n * 32 * heads or padded.dtype != qkv.dtype or tuple(padded.shape) != (bias.shape[0], 8) or not padded.is_contiguous():
+        raise RuntimeError("dense_attention_train_backward: d_out (b,n,c) and padded (rows,8) of the rows' dtype")
+    device = qkv.device
+    d_qkv = torch.empty_like(qkv)
+    d_blank, d_w, d_b = torch.empty(2, 32 * heads, device=device), torch.empty(heads, k, device=device), torch.empty(heads, device=device)
+    nbytes = load().clusten_dense_attention_train_workspace_bytes(b, heads)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    with _on(device):
+        _check(load().clusten_dense_attention_train_backward(qkv.data_ptr(), bias.data_ptr(), padded.data_ptr(), pe_idx.data_ptr(), blank_k.data_ptr(),
+                                                             blank_v.data_ptr(), d_out.data_ptr(), d_qkv.data_ptr(), d_blank[0].data_ptr(),
+                                                             d_blank[1].data_ptr(), d_w.data_ptr(), d_b.data_ptr(), ws.data_ptr(), nbytes, scale, b,
+                                                             heads, n, bias.shape[0], k, _DTYPE_CODES[qkv.dtype], _stream(device)),
+               "clusten_dense_attention_train_backward")
+    return d_qkv, d_blank[0], d_blank[1], d_w, d_b
+
+
+def attention_rows_backward(qkv: torch.Tensor, d_qkv: torch.Tensor, probs: torch.Tensor, d_logit: torch.Tensor, d_out: torch.Tensor,
+                            d_blank: torch.Tensor, blank_prob: torch.Tensor, pair_lists: torch.Tensor, scale: float):
+    """What is left of a local attention's backward behind its kernel: the key and value columns of d_qkv (b,n,3c) - scatters over
+    `pair_lists` (`cluster_pairs_from_numbers`), both in one launch - and the blank token's gradients, each (c,) fp32."""
+    lib = load()
+    b, n, c3 = qkv.shape
+    c, h, m = c3 // 3, probs.shape[1], probs.shape[3]
+    ch = c // h
+    _block_rows((qkv.dtype,), c3, qkv, d_qkv)
+    _block_rows((qkv.dtype,), c, d_out)
+    if (c not in _BLOCK_WIDTHS or ch % 8 or d_out.numel() != b * n * c or tuple(probs.shape) != (b, h, n, m)
+            or any(t.dtype != qkv.dtype or not t.is_contiguous() or t.shape != probs.shape for t in (probs, d_logit))
+            or any(t.dtype != torch.float32 or not t.is_contiguous() or tuple(t.shape) != (b, h, n) for t in (d_blank, blank_prob))):
+        raise RuntimeError("attention_rows_backward: tensors do not belong to one attention layer")
+    if pair_lists.dtype != torch.uint8 or pair_lists.numel() != lib.clusten_cluster_pairs_bytes(b, n, m, n):
+        raise RuntimeError("attention_rows_backward: pair lists of these lists (cluster_pairs_from_numbers)")
+    ws, nbytes, sums = _row_sums(b * n, c, qkv.device)
+    code, size = _DTYPE_CODES[qkv.dtype], qkv.element_size()
+    q, kv, rows = Strides(n * c3, ch, c3), Strides(n * c3, 2 * ch, c3), Strides(n * c, ch, c)
+    with _on(qkv.device):
+        at, key, stream = sums.data_ptr(), d_qkv.data_ptr() + c * size, _stream(qkv.device)
+        _check(lib.clusten_scatter_attention_pair(d_logit.data_ptr(), qkv.data_ptr(), q, key, probs.data_ptr(), d_out.data_ptr(), rows,
+                                                  key + ch * size, kv, scale, pair_lists.data_ptr(), AttnShape(b, h, n, ch, m), code, stream),
+               "clusten_scatter_attention_pair")
         _check(lib.clusten_blank_grad(qkv.data_ptr(), c3, d_out.data_ptr(), d_blank.data_ptr(), blank_prob.data_ptr(), scale, at,
                                       at + 4 * c, ws.data_ptr(), nbytes, b, h, n, c, code, stream), "clusten_blank_grad")
     return sums[0], sums[1]

@@ -789,6 +789,80 @@ int clusten_table_linear_grad(const float* d, const void* x, float* d_weight, fl
     return launch_table_linear_grad(d, x, d_weight, d_bias, rows, n, k, dtype, as_stream(stream));
 }
 
+int clusten_position_bias(const float* table, const float* weight, const float* bias_param, void* bias, void* padded, int rows, int n, int k,
+                          int dtype, clusten_stream stream) {
+    if (!table || !weight || !bias) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (rows <= 0 || n <= 0 || k <= 0 || k > 8 || (int64_t)rows * n >= (int64_t)1 << 31) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(bias) || !aligned16(padded)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_position_bias(table, weight, bias_param, bias, padded, rows, n, k, dtype, as_stream(stream));
+}
+
+size_t clusten_position_grad_workspace_bytes(int B, int H, int N, int M) {
+    return B > 0 && H > 0 && N > 0 && M > 0 ? position_grad_workspace_bytes((int64_t)B * N * M, H) : 0;
+}
+
+int clusten_position_grad(const void* d_logit, const int64_t* pe_idx, const void* padded, float* d_weight, float* d_bias, void* workspace,
+                          size_t workspace_bytes, int B, int H, int N, int M, int rows, int k, int dtype, clusten_stream stream) {
+    if (!d_logit || !pe_idx || !padded || !d_weight || !d_bias || !workspace) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (B <= 0 || H <= 0 || H > 65535 || N <= 0 || M <= 0 || M % 4 != 0 || rows <= 0 || k <= 0 || k > 5) return CLUSTEN_ERR_BAD_DIMS;
+    if (workspace_bytes < clusten_position_grad_workspace_bytes(B, H, N, M)) return CLUSTEN_ERR_WORKSPACE;
+    if (!aligned16(d_logit) || !aligned16(padded) || !aligned16(workspace)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_position_grad(d_logit, pe_idx, padded, d_weight, d_bias, workspace, B, H, N, M, rows, k, dtype, as_stream(stream));
+}
+
+static int dense_train_args(DenseTrain& a, const void* qkv, const void* bias, const int64_t* pe_idx, const float* blank_k, const float* blank_v,
+                            float scale, int B, int H, int N, int rows, int dtype) {
+    if (!qkv || !bias || !pe_idx || !blank_k || !blank_v) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (B <= 0 || H <= 0 || N <= 0 || N > 64 || rows <= 0 || (int64_t)B * H >= (int64_t)1 << 31 || H > 1 << 16) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(qkv)) return CLUSTEN_ERR_UNALIGNED;
+    a = {};
+    a.qkv = qkv, a.bias = bias, a.pe_idx = pe_idx, a.blank_k = blank_k, a.blank_v = blank_v, a.scale = scale, a.B = B, a.H = H, a.N = N;
+    a.rows = rows;
+    return CLUSTEN_OK;
+}
+
+int clusten_dense_attention_train_forward(const void* qkv, const void* bias, const int64_t* pe_idx, const float* blank_k, const float* blank_v,
+                                          void* out, float scale, int B, int H, int N, int rows, int dtype, clusten_stream stream) {
+    DenseTrain a;
+    if (int st = dense_train_args(a, qkv, bias, pe_idx, blank_k, blank_v, scale, B, H, N, rows, dtype)) return st;
+    if (!out) return CLUSTEN_ERR_NULL_POINTER;
+    if (!aligned16(out)) return CLUSTEN_ERR_UNALIGNED;
+    a.out = out;
+    return launch_dense_train(a, dtype, as_stream(stream));
+}
+
+size_t clusten_dense_attention_train_workspace_bytes(int B, int H) { return B > 0 && H > 0 ? dense_train_workspace_bytes(B, H) : 0; }
+
+int clusten_dense_attention_train_backward(const void* qkv, const void* bias, const void* padded, const int64_t* pe_idx, const float* blank_k,
+                                           const float* blank_v, const void* d_out, void* d_qkv, float* d_blank_k, float* d_blank_v,
+                                           float* d_weight, float* d_bias, void* workspace, size_t workspace_bytes, float scale, int B, int H,
+                                           int N, int rows, int k, int dtype, clusten_stream stream) {
+    DenseTrain a;
+    if (int st = dense_train_args(a, qkv, bias, pe_idx, blank_k, blank_v, scale, B, H, N, rows, dtype)) return st;
+    if (!padded || !d_out || !d_qkv || !d_blank_k || !d_blank_v || !d_weight || !d_bias || !workspace) return CLUSTEN_ERR_NULL_POINTER;
+    if (k <= 0 || k > 5) return CLUSTEN_ERR_BAD_DIMS;
+    if (workspace_bytes < clusten_dense_attention_train_workspace_bytes(B, H)) return CLUSTEN_ERR_WORKSPACE;
+    if (!aligned16(padded) || !aligned16(d_out) || !aligned16(d_qkv) || !aligned16(workspace)) return CLUSTEN_ERR_UNALIGNED;
+    a.padded = padded, a.d_out = d_out, a.d_qkv = d_qkv, a.partial = static_cast<float*>(workspace), a.k = k;
+    return launch_dense_train_backward(a, d_blank_k, d_blank_v, d_weight, d_bias, dtype, as_stream(stream));
+}
+
+int clusten_scatter_attention_pair(const void* d_logit, const void* query, clusten_strides query_strides, void* d_key, const void* probs,
+                                   const void* d_out, clusten_strides d_out_strides, void* d_value, clusten_strides out_strides, float scale,
+                                   const void* pair_lists, clusten_attn_shape shape, int dtype, clusten_stream stream) {
+    if (!d_logit || !query || !d_key || !probs || !d_out || !d_value || !pair_lists) return CLUSTEN_ERR_NULL_POINTER;
+    if (dtype != CLUSTEN_F32 && dtype != CLUSTEN_F16 && dtype != CLUSTEN_BF16) return CLUSTEN_ERR_BAD_DTYPE;
+    if (int st = check_attn_shape(shape)) return st;
+    if (!strides_ok(query_strides, shape.C) || !strides_ok(d_out_strides, shape.C) || !strides_ok(out_strides, shape.C)) return CLUSTEN_ERR_BAD_STRIDE;
+    if (!cluster_pairs_supported(shape.B, shape.N, shape.M, shape.N)) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(pair_lists)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_scatter_pair(d_logit, query, query_strides, d_key, probs, d_out, d_out_strides, d_value, out_strides, scale, pair_lists, shape,
+                               dtype, as_stream(stream));
+}
+
 static int check_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype) {
     if (!items) return CLUSTEN_ERR_NULL_POINTER;
     if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;

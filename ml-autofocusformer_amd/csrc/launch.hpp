@@ -344,6 +344,36 @@ int launch_norm_linear_backward(const NormLinearGrad& a, int x_dtype, int C, int
 // Sums of `groups` partial rows of 2 C values: the first C times scale0 to out0, the others to out1.
 int launch_column_sums(const float* partial, int groups, int C, float scale0, float* out0, float* out1, hipStream_t stream);
 
+// Training pass of an attention layer beside its attention kernels (attention_train.hip).
+int launch_position_bias(const float* table, const float* w, const float* b, void* bias, void* padded, int rows, int heads, int k, int dtype,
+                         hipStream_t stream);
+size_t position_grad_workspace_bytes(int64_t total, int heads);
+int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void* padded, float* d_w, float* d_b, void* workspace, int B, int H, int N,
+                         int M, int rows, int k, int dtype, hipStream_t stream);
+struct DenseTrain {
+    const void* qkv;       // (B, N, 3 C): [q | head 0: k v | head 1: k v ...]
+    const void* bias;      // (rows, H)
+    const void* padded;    // (rows, 8)
+    const int64_t* pe_idx; // (B, N, N)
+    const float* blank_k;
+    const float* blank_v;
+    const void* d_out;     // (B, N, C)
+    void* out;             // (B, N, C)
+    void* d_qkv;           // (B, N, 3 C)
+    float* partial;
+    float scale;
+    int B, H, N, rows, k;
+};
+size_t dense_train_workspace_bytes(int B, int H);
+int launch_dense_train(const DenseTrain& a, int dtype, hipStream_t stream);
+int launch_dense_train_backward(const DenseTrain& a, float* d_bk, float* d_bv, float* d_w, float* d_b, int dtype, hipStream_t stream);
+// d_key and d_value of a local attention from its pair lists in one launch: scale * scatter(d_logit, query) and scatter(probs, d_out)
+//   into strided rows (scatter_by_cluster.hip).
+bool scatter_pair_supported(const clusten_attn_shape& s, int dtype);
+int launch_scatter_pair(const void* d_logit, const void* query, clusten_strides qs, void* d_key, const void* probs, const void* d_out,
+                        clusten_strides gs, void* d_value, clusten_strides ys, float scale, const void* pair_lists, clusten_attn_shape s,
+                        int dtype, hipStream_t stream);
+
 // Parameter gradients of Linear layers over the same rows (weight_grad.hip).
 size_t weight_grad_workspace_bytes(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype);
 int launch_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, float* workspace, int dtype, hipStream_t stream);

@@ -1,0 +1,98 @@
+"""GPU parity of what an attention layer's training pass has beside its attention kernels, against float64 on the same stored
+operands (models/aff_transformer.py:103-155 under autograd).
+
+Bars, relative 2-norm: a result stored in 16 bits one rounding of it, 4e-4 fp16 and 3e-3 bf16; fp32 arithmetic on sums of up to 64
+terms and an exponential 1e-6; position gradients, summed in double, 1e-6 of the sum of the terms' magnitudes.
+"""
+import pytest
+import torch
+
+from clusten import _native
+
+pytestmark = pytest.mark.gpu
+
+BAR = {torch.float16: 4e-4, torch.bfloat16: 3e-3, torch.float32: 1e-6}
+DTYPES = list(BAR)
+
+
+def near(got, ref, bar):
+    assert got.shape == ref.shape and (got.double() - ref.double()).norm() <= bar * ref.double().norm()
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("b,h,n,m,rows,k", [(1, 1, 1, 4, 1, 1), (2, 3, 37, 48, 225, 5), (3, 16, 100, 48, 12321, 5), (1, 5, 1030, 12, 961, 3)])
+def test_position_bias(device, dt, b, h, n, m, rows, k):
+    gen = torch.Generator(device).manual_seed(n)
+    table, w, bias = (torch.randn(*s, generator=gen, device=device) for s in ((rows, k), (h, k), (h,)))
+    t64, w64 = table.to(dt).double(), w.to(dt).double()
+    got, padded = _native.position_bias(table, w, bias, dt)
+    near(got, t64 @ w64.t() + bias.to(dt).double(), BAR[dt])
+    assert torch.equal(padded[:, :k], table.to(dt)) and not padded[:, k:].any()
+    near(_native.position_bias(table, w, None, dt)[0], t64 @ w64.t(), BAR[dt])
+    d = torch.randn(b, h, n, m, generator=gen, device=device).to(dt)
+    pe = torch.randint(rows, (b, n, m), generator=gen, device=device)
+    d_w, d_b = _native.position_grad(d, pe, padded, k)
+    terms = d.double().unsqueeze(-1) * t64[pe].unsqueeze(1)
+    assert ((d_w.double() - terms.sum((0, 2, 3))).abs() <= 1e-6 * terms.abs().sum((0, 2, 3)) / (b * n * m) ** 0.5).all()
+    assert ((d_b.double() - d.double().sum((0, 2, 3))).abs() <= 1e-6 * d.double().abs().sum((0, 2, 3)) / (b * n * m) ** 0.5).all()
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("b,h,n", [(1, 1, 1), (3, 2, 7), (2, 16, 49), (5, 3, 64), (1, 4, 63)])
+def test_dense_attention(device, dt, b, h, n):
+    gen = torch.Generator(device).manual_seed(n)
+    c, rows, scale = 32 * h, 169, 32 ** -0.5
+
+    def draw(*shape):
+        return torch.randn(*shape, generator=gen, device=device)
+
+    qkv, d_out = draw(b, n, 3 * c).to(dt), draw(b, n, c).to(dt)
+    table, w, pe_b, bk, bv = draw(rows, 5), 0.3 * draw(h, 5), draw(h), draw(c), draw(c)
+    pe = torch.randint(rows, (b, n, n), generator=gen, device=device)
+    bias, padded = _native.position_bias(table, w, pe_b, dt)
+
+    rows64, bias64, bk64, bv64 = (t.double().requires_grad_(True) for t in (qkv, bias, bk, bv))
+    q = rows64[..., :c].view(b, n, h, 32).permute(0, 2, 1, 3)
+    kv = rows64[..., c:].view(b, n, h, 2, 32).permute(3, 0, 2, 1, 4)
+    logits = q @ kv[0].transpose(-1, -2) * scale + bias64[pe].permute(0, 3, 1, 2)
+    blank = (q * bk64.view(1, h, 1, 32)).sum(-1, keepdim=True) * scale
+    p = torch.softmax(torch.cat([logits, blank], -1), -1)
+    ref = (p[..., :-1] @ kv[1] + p[..., -1:] * bv64.view(1, h, 1, 32)).permute(0, 2, 1, 3).reshape(b, n, c)
+    d_ref = torch.autograd.grad(ref, (rows64, bk64, bv64, bias64), d_out.double())
+
+    near(_native.dense_attention_train(qkv, bias, pe, bk, bv, h, scale), ref.detach(), BAR[dt])
+    got = _native.dense_attention_train_backward(qkv, bias, padded, pe, bk, bv, d_out, 5, h, scale)
+    near(got[0], d_ref[0], BAR[dt])
+    # of the keys' part too, which is the smallest
+    near(got[0][..., c:], d_ref[0][..., c:], 2 * BAR[dt])
+    if n > 1:                                                # with one token d_logit of a row is minus that of its blank token
+        near(got[1], d_ref[1], 3e-6)
+    near(got[2], d_ref[2], 3e-6)
+    d_w, d_b = d_ref[3].t() @ padded[:, :5].double(), d_ref[3].sum(0)
+    size = d_ref[3].abs().sum(0)
+    assert ((got[3].double() - d_w).abs() <= 2e-6 * d_ref[3].abs().t() @ padded[:, :5].double().abs()).all()
+    assert ((got[4].double() - d_b).abs() <= 2e-6 * size).all()
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("b,h,n,ch", [(1, 1, 8, 32), (2, 4, 100, 32), (3, 2, 203, 16), (1, 8, 777, 32), (2, 2, 64, 64)])
+def test_rows_of_an_attention_layer(device, dt, b, h, n, ch):
+    """Both scatters in one launch into the columns of d_qkv, against the scatters one by one."""
+    gen = torch.Generator(device).manual_seed(n)
+    c, m = h * ch, 8 * min(6, n // 8)
+    qkv = torch.randn(b, n, 3 * c, generator=gen, device=device).to(dt)
+    d_out = torch.randn(b, n, c, generator=gen, device=device).to(dt)
+    probs, d_logit = (torch.randn(b, h, n, m, generator=gen, device=device).to(dt) for _ in range(2))
+    d_blank, blank = torch.randn(b, h, n, generator=gen, device=device), torch.rand(b, h, n, generator=gen, device=device)
+    numbers = torch.rand(b, n, (n + 7) // 8, generator=gen, device=device).argsort(-1)[..., :m // 8].int().contiguous()
+    pairs = _native.cluster_pairs_from_numbers(numbers)
+    d_qkv = torch.full_like(qkv, 7.0)
+    d_bk, d_bv = _native.attention_rows_backward(qkv, d_qkv, probs, d_logit, d_out, d_blank, blank, pairs, 0.3)
+    assert (d_qkv[..., :c] == 7.0).all()
+    q, g = qkv[..., :c].view(b, n, h, ch).permute(0, 2, 1, 3), d_out.view(b, n, h, ch).permute(0, 2, 1, 3)
+    d_k, d_v = _native.scatter_rows_by_cluster(d_logit, q, pairs), _native.scatter_rows_by_cluster(probs, g, pairs)
+    kv = d_qkv[..., c:].view(b, n, h, 2, ch).permute(3, 0, 2, 1, 4)
+    near(kv[0], 0.3 * d_k.double(), 2 * BAR[dt])
+    assert torch.equal(kv[1], d_v)
+    near(d_bk, 0.3 * (d_blank.double().unsqueeze(-1) * q.double()).sum((0, 2)).reshape(-1), 5e-6)
+    near(d_bv, (blank.double().unsqueeze(-1) * g.double()).sum((0, 2)).reshape(-1), 5e-6)
