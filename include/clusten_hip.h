@@ -741,6 +741,37 @@ int clusten_scatter_attention_pair(const void* d_logit, const void* query, clust
                                    clusten_strides out_strides, float scale, const void* pair_lists, clusten_attn_shape shape,
                                    int dtype, clusten_stream stream);
 
+/* The training pass of a whole block (models/aff_transformer.py:181-232) by one call a direction: the launches of the entry points
+ * above and of clusten_cluster_attention_forward_train / _backward, clusten_weight_grad and clusten_blank_grad, in order.
+ *   shape: B images of N tokens, H heads of C = 32 channels (H * C a built width), M = 48 with a plan.  Local attention with `plan`
+ *     (clusten_cluster_attention_plan) and, backward, `pair_lists`; with plan = NULL every token attends to all N <= 64.
+ *   param: norm1 weight, bias; norm2 weight, bias; biases of q, kv, proj, fc1, fc2; blank key, blank value; weights of q, kv, proj, fc1,
+ *     fc2; position bias layer's weight, bias: fp32, on 16-byte boundaries.  grad: the same order (backward), fp32; the five weights and
+ *     their biases may be NULL, the bias with its weight.
+ *   x (B*N,C) of x_dtype (F32 or dtype); table (table_rows, table_cols <= 5) fp32; pe_idx (B,N,M) or (B,N,N) int64; factors as `scale` of
+ *     clusten_block_tail_forward, (2,B) or NULL; kept: clusten_block_train_kept_bytes(), written forward and read backward.
+ *   out and d_x (B*N,C) of x_dtype; workspace: clusten_block_train_workspace_bytes() with the gradients' pointers set. */
+typedef struct {
+    const float* param[18];
+    float* grad[18];
+    const void* x;
+    const void* plan;
+    const void* pair_lists;
+    const int64_t* pe_idx;
+    const float* table;
+    const float* factors;
+    void* kept;
+    size_t kept_bytes;
+    clusten_attn_shape shape;
+    int32_t hidden, table_rows, table_cols, lists_shared, x_dtype, dtype;
+    float eps1, eps2, attn_scale;
+} clusten_block_train;
+size_t clusten_block_train_kept_bytes(const clusten_block_train* args);
+size_t clusten_block_train_workspace_bytes(const clusten_block_train* args);
+int clusten_block_train_forward(const clusten_block_train* args, void* out, clusten_stream stream);
+int clusten_block_train_backward(const clusten_block_train* args, const void* d_out, void* d_x, void* workspace,
+                                 size_t workspace_bytes, clusten_stream stream);
+
 /* The backward of a block between its products, which the reference leaves to autograd.  Tensors are dense rows of C channels
  * (C in {32,64,128,256,512}) of dtype F32, F16 or BF16 unless said otherwise, on 16-byte boundaries; sums are fp32 in a fixed
  * order; workspace: clusten_row_sums_workspace_bytes(rows, C) bytes.

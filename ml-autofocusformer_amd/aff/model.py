@@ -68,11 +68,15 @@ def default_ops():
                                              ("add_layer_norm", _native.add_layer_norm)),
                            weight_grad=_native.weight_grad, weight_grad_supported=_native.weight_grad_supported,
                            block_tail_backward=_native.block_tail_backward, norm_linear_backward=_native.norm_linear_backward,
-                           attention_rows_backward=_native.attention_rows_backward, position_bias=_native.position_bias,
-                           position_grad=_native.position_grad, cluster_pairs_from_numbers=_native.cluster_pairs_from_numbers,
-                           dense_attention_train=_native.dense_attention_train,
-                           dense_attention_train_backward=_native.dense_attention_train_backward,
-                           dense_attention_train_supported=_native.dense_attention_train_supported,
+                           cluster_pairs_from_numbers=_native.cluster_pairs_from_numbers,
+                           block_train_forward=_native.block_train_forward, block_train_backward=_native.block_train_backward,
+                           block_train_supported=_native.block_train_supported,
+                           block_train_stands_for=(("norm_linear", _native.norm_linear), ("block_tail", _native.block_tail),
+                                                   ("cluster_attention", _native.cluster_attention),
+                                                   ("cluster_attention_backward", _native.cluster_attention_backward),
+                                                   ("norm_linear_backward", _native.norm_linear_backward),
+                                                   ("block_tail_backward", _native.block_tail_backward),
+                                                   ("scatter_rows", _native.scatter_rows), ("weight_grad", _native.weight_grad)),
                            blocks_forward=_native.blocks_forward, block_params=_native.BlockParams,
                            blocks_stand_for=(("cluster_attention", _native.cluster_attention),
                                              ("dense_attention", _native.dense_attention),
@@ -380,9 +384,10 @@ class _AttnSoftmax(torch.autograd.Function):
         return d_logit, d_bias, None, None, d_blank.to(blank_dtype), None
 
 
-def _recorded_backward(fn, ctx, tensors, grads):
-    """The gradients of `fn(*tensors)` by recorded operations, for a backward pass that is itself differentiated or batched."""
-    needs = ctx.needs_input_grad[:len(tensors)]
+def _recorded_backward(fn, ctx, tensors, grads, needs=None):
+    """The gradients of `fn(*tensors)` by recorded operations, for a backward pass that is itself differentiated or batched.  `needs`: of
+    `tensors`, when they are not the first inputs."""
+    needs = ctx.needs_input_grad[:len(tensors)] if needs is None else needs
     with torch.enable_grad(), torch.autocast("cuda", enabled=False):
         out = fn(*tensors)
         out, grads = zip(*((o, g) for o, g in zip(out if isinstance(out, tuple) else (out,), grads) if o.requires_grad))
@@ -524,67 +529,53 @@ class _BlockTail(torch.autograd.Function):
         return (*(t if n else None for t, n in zip(grads, need)), None, None, None, None)
 
 
-class _ClusterAttentionRows(torch.autograd.Function):
-    """`_ClusterAttention` on the (b,n,3c) rows of the stacked projections, with the position bias' layer inside: the gradients
-    of q, k and v go into one tensor of that form, the blank token's and the bias layer's come from kernels of their own."""
+class _BlockRows(torch.autograd.Function):
+    """A whole block in training by one native call a direction: norm and projections, attention with the position bias' layer inside, and
+    everything behind it, as the inference kernels compute them; what the backward reads is one block of memory.  `params`: as
+    `ClusterTransformerBlock.tensors` gives them.  `plan` and `pairs` of a local attention, else None; `member_idx` and `mask` are read only
+    by a backward that is itself recorded."""
 
     @staticmethod
-    def forward(ctx, qkv, pe_w, pe_b, blank_k, blank_v, table, plan, pairs, pe_idx, member_idx, mask, heads, scale, ops):
-        bias, padded = ops.position_bias(table, pe_w, pe_b, qkv.dtype)
-        q, key, v = _columns(qkv, heads)
-        out, lse = ops.cluster_attention(q, key, v, None, bias, None, None, blank_k, blank_v, scale=scale, plan=plan,
-                                         return_lse=True)
-        ctx.save_for_backward(qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, padded, plan, pairs, pe_idx, member_idx, mask)
-        ctx.meta = (table.shape[1], heads, scale, ops)
+    def forward(ctx, x, table, pe_idx, plan, pairs, factors, member_idx, mask, dt, heads, hidden, eps, scale, ops, *params):
+        out, kept = ops.block_train_forward(x, params, table, pe_idx, plan, pairs, factors, dt, heads, hidden, eps, scale)
+        ctx.save_for_backward(x, table, pe_idx, plan, pairs, factors, member_idx, mask, kept, *params)
+        ctx.meta = (dt, heads, hidden, eps, scale, ops)
         return out
 
     @staticmethod
     @_types_of_forward
     def backward(ctx, d_out):
-        qkv, pe_w, pe_b, blank_k, blank_v, out, lse, bias, padded, plan, pairs, pe_idx, member_idx, mask = ctx.saved_tensors
-        k, heads, scale, ops = ctx.meta
+        x, table, pe_idx, plan, pairs, factors, member_idx, mask, kept, *params = ctx.saved_tensors
+        dt, heads, hidden, eps, scale, ops = ctx.meta
+        need = ctx.needs_input_grad
         if not _by_kernels(d_out):
-            def layers(qkv, pe_w, pe_b, blank_k, blank_v):
-                bias = F.linear(padded[:, :k], pe_w.to(padded.dtype), pe_b.to(padded.dtype))
-                return _local_attention(*_columns(qkv, heads), bias, blank_k, blank_v, mask, pe_idx, member_idx, scale)
-            return (*_recorded_backward(layers, ctx, (qkv, pe_w, pe_b, blank_k, blank_v), (d_out,)), *(None,) * 9)
-        q, key, v = _columns(qkv, heads)
-        d_out = _dense(d_out.to(qkv.dtype))
-        d_qkv = torch.empty_like(qkv)
-        _, probs, d_logit, blank_prob, d_blank = ops.cluster_attention_backward(
-            q, key, v, d_out, out, lse, plan, bias, blank_k, blank_v, scale=scale, d_query=_columns(d_qkv, heads)[0])
-        d_bk, d_bv = ops.attention_rows_backward(qkv, d_qkv, probs, d_logit, d_out, d_blank, blank_prob, pairs, scale)
-        d_w, d_b = ops.position_grad(d_logit, pe_idx, padded, k)
-        return (d_qkv, d_w.to(pe_w.dtype), d_b.to(pe_b.dtype), d_bk.reshape(blank_k.shape).to(blank_k.dtype),
-                d_bv.reshape(blank_v.shape).to(blank_v.dtype), *(None,) * 9)
+            b, n, c = x.shape
+            everyone = torch.arange(n, device=x.device).expand(b, n, n) if plan is None else member_idx
+            t = table.to(dt)
+
+            def layers(x, n1_w, n1_b, n2_w, n2_b, b_q, b_kv, b_p, b_1, b_2, blank_k, blank_v, w_q, w_kv, w_p, w_1, w_2, pe_w, pe_b):
+                s = (1.0, 1.0) if factors is None else factors.to(dt).view(2, b, 1, 1)
+                y = F.layer_norm(x.float(), (c,), n1_w, n1_b, eps[0]).to(dt)
+                qkv = F.linear(y, torch.cat([w_q, w_kv]).to(dt), torch.cat([b_q, b_kv]).to(dt))
+                a = _local_attention(*_columns(qkv, heads), F.linear(t, pe_w.to(dt), pe_b.to(dt)), blank_k, blank_v,
+                                     None if plan is None else mask, pe_idx, everyone, scale)
+                x1 = x + (F.linear(a, w_p.to(dt), b_p.to(dt)) * s[0]).to(x.dtype)
+                y = F.gelu(F.linear(F.layer_norm(x1.float(), (c,), n2_w, n2_b, eps[1]).to(dt), w_1.to(dt), b_1.to(dt)))
+                return x1 + (F.linear(y, w_2.to(dt), b_2.to(dt)) * s[1]).to(x.dtype)
+
+            d_x, *grads = _recorded_backward(layers, ctx, (x, *params), (d_out,), need[:1] + need[14:])
+        else:
+            d_x, grads = ops.block_train_backward(_dense(d_out), kept, need[14:], x, params, table, pe_idx, plan, pairs, factors, dt, heads, hidden,
+                                                  eps, scale)
+        return (d_x if need[0] else None, *(None,) * 13, *(g if n else None for g, n in zip(grads, need[14:])))
 
 
-class _DenseAttentionRows(torch.autograd.Function):
-    """The attention of every token over all, as `_ClusterAttentionRows`: one kernel forward, one kernel and a sum backward."""
+class _ClusterAttentionRows(_BlockRows):
+    """A block whose tokens attend to the members of their nearest clusters."""
 
-    @staticmethod
-    def forward(ctx, qkv, pe_w, pe_b, blank_k, blank_v, table, pe_idx, heads, scale, ops):
-        bias, padded = ops.position_bias(table, pe_w, pe_b, qkv.dtype)
-        ctx.save_for_backward(qkv, pe_w, pe_b, blank_k, blank_v, bias, padded, pe_idx)
-        ctx.meta = (table.shape[1], heads, scale, ops)
-        return ops.dense_attention_train(qkv, bias, pe_idx, blank_k, blank_v, heads, scale)
 
-    @staticmethod
-    @_types_of_forward
-    def backward(ctx, d_out):
-        qkv, pe_w, pe_b, blank_k, blank_v, bias, padded, pe_idx = ctx.saved_tensors
-        k, heads, scale, ops = ctx.meta
-        if not _by_kernels(d_out):
-            def layers(qkv, pe_w, pe_b, blank_k, blank_v):
-                bias = F.linear(padded[:, :k], pe_w.to(padded.dtype), pe_b.to(padded.dtype))
-                b, n, _ = qkv.shape
-                everyone = torch.arange(n, device=qkv.device).expand(b, n, n)
-                return _local_attention(*_columns(qkv, heads), bias, blank_k, blank_v, None, pe_idx, everyone, scale)
-            return (*_recorded_backward(layers, ctx, (qkv, pe_w, pe_b, blank_k, blank_v), (d_out,)), *(None,) * 5)
-        d_qkv, d_bk, d_bv, d_w, d_b = ops.dense_attention_train_backward(qkv, bias, padded, pe_idx, blank_k, blank_v, _dense(d_out.to(qkv.dtype)),
-                                                                         k, heads, scale)
-        return (d_qkv, d_w.to(pe_w.dtype), d_b.to(pe_b.dtype), d_bk.reshape(blank_k.shape).to(blank_k.dtype),
-                d_bv.reshape(blank_v.shape).to(blank_v.dtype), *(None,) * 5)
+class _DenseAttentionRows(_BlockRows):
+    """A block whose tokens attend to all."""
 
 
 def _columns(qkv, heads):
@@ -716,23 +707,6 @@ class ClusterAttention(_Module):
                 and cluster_idx is not None and not global_attn and self.cluster_size == 8 and grid_lists is not None
                 and len(grid_lists) > 4 and not _drops(self.attn_drop)
                 and self.ops.cluster_attention_backward_supported(q.view(b, n, h, c // h).permute(0, 2, 1, 3), cluster_idx.shape[2]))
-
-    def attend_rows(self, qkv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None):
-        """`attend` of a training pass on the (b,n,3c) rows of the stacked projections."""
-        c = self.dim
-        pe = self.pos_embed
-        # the kernels take a fp32 table of five columns and the parameters of the layer in place
-        if (table.dtype == torch.float32 and table.is_contiguous() and table.shape[1] <= 5 and not table.requires_grad
-                and getattr(self.ops, "position_bias", None) is not None):
-            params = (pe.weight, pe.bias, self.blank_k, self.blank_v)
-            if self._trains_in_one_kernel(qkv[..., :c], global_attn, cluster_idx, grid_lists):
-                return _ClusterAttentionRows.apply(qkv, *params, table, grid_lists[3], grid_lists[4], pe_idx, member_idx, cluster_mask,
-                                                   self.num_heads, self.scale, self.ops)
-            if (global_attn and not _drops(self.attn_drop) and pe_idx.is_contiguous()
-                    and self.ops.dense_attention_train_supported(qkv, self.num_heads)):
-                return _DenseAttentionRows.apply(qkv, *params, table, pe_idx, self.num_heads, self.scale, self.ops)
-        q, kv = qkv.split([c, 2 * c], dim=-1)
-        return self.attend(q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
 
     def attend(self, q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None):
         """The attention between its projections: q (b,n,c) and kv (b,n,2c) in, what the output projection reads (b,n,c)
@@ -917,11 +891,34 @@ class ClusterTransformerBlock(_Module):
 
         return _kept(self.__dict__, "_pack_cache", key, make).value
 
-    def fits(self, c, hidden, heads):
+    def fits(self, c, hidden, heads, table_cols=5):
         """True when every parameter has the shape of a block of c channels with `hidden` hidden ones and `heads` heads."""
         want = 5 * [(c,)] + [(2 * c,), (c,), (hidden,)] + 3 * [(c,)] + [(c, c), (2 * c, c), (c, c), (hidden, c), (c, hidden),
-                                                                     (heads, 5), (heads,)]
+                                                                     (heads, table_cols), (heads,)]
         return [tuple(t.shape) for t in self.tensors()] == want
+
+    def _factors(self, feat, dt):
+        """The images' factors of both branches under stochastic depth (fp32), or None."""
+        if not _drops(self.drop_path):
+            return None
+        return torch.stack([self.drop_path.factors(feat.shape[0], dt, feat.device) for _ in range(2)]).float()
+
+    def _train_whole(self, feat, dt, global_attn, table, pe_idx, cluster_idx, grid_lists):
+        """(plan, pairs) when a training pass of the block is one native call - local attention of clusters of 8 by its kernel, or, as (None,
+        None), global attention of a short sequence - else None."""
+        attn, ops = self.attn, self.attn.ops
+        if (getattr(ops, "block_train_forward", None) is None or _drops(attn.attn_drop) or table.requires_grad
+                or any(getattr(ops, name, None) is not fn for name, fn in ops.block_train_stands_for)):
+            return None
+        plan = pairs = None
+        if not global_attn:
+            if cluster_idx is None or cluster_idx.shape[2] != 6 or attn.cluster_size != 8 or grid_lists is None or len(grid_lists) < 5:
+                return None
+            plan, pairs = grid_lists[3:5]
+        if not (ops.block_train_supported(feat, dt, attn.num_heads, self.mlp.fc1.out_features, table, pe_idx, plan, pairs)
+                and self.fits(feat.shape[2], self.mlp.fc1.out_features, attn.num_heads, table.shape[1])):
+            return None
+        return plan, pairs
 
     def forward(self, feat, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None,
                 carry=None):
@@ -934,12 +931,17 @@ class ClusterTransformerBlock(_Module):
         if dt is not None and torch.is_grad_enabled():
             # training: the same kernels, keeping what their backward reads
             attn, mlp, norm1, norm2 = self.attn, self.mlp, self.norm1, self.norm2
+            whole = self._train_whole(feat, dt, global_attn, table, pe_idx, cluster_idx, grid_lists)
+            if whole is not None:
+                plan, pairs = whole
+                return (_DenseAttentionRows if plan is None else _ClusterAttentionRows).apply(
+                    feat, table, pe_idx, plan, pairs, self._factors(feat, dt), member_idx, cluster_mask, dt, attn.num_heads,
+                    mlp.fc1.out_features, (norm1.eps, norm2.eps), attn.scale, ops, *self.tensors()), None
             qkv, feat = _NormLinearRows.apply(feat, norm1.weight, norm1.bias, attn.q.weight, attn.q.bias, attn.kv.weight,
                                               attn.kv.bias, norm1.eps, dt, ops)
-            a = attn.attend_rows(qkv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
-            scale = None
-            if _drops(self.drop_path):
-                scale = torch.stack([self.drop_path.factors(feat.shape[0], dt, feat.device) for _ in range(2)]).float()
+            c = attn.dim
+            a = attn.attend(qkv[..., :c], qkv[..., c:], member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx, grid_lists)
+            scale = self._factors(feat, dt)
             return _BlockTail.apply(a.to(dt).contiguous(), feat, attn.proj.weight, attn.proj.bias, norm2.weight, norm2.bias,
                                     mlp.fc1.weight, mlp.fc1.bias, mlp.fc2.weight, mlp.fc2.bias, scale, norm2.eps, dt, ops), None
         if dt is not None:

@@ -49,6 +49,15 @@ class BlockParams(ctypes.Structure):
                 + [("eps1", ctypes.c_float), ("eps2", ctypes.c_float)])
 
 
+class BlockTrain(ctypes.Structure):
+    """clusten_block_train: a block's training pass (device pointers)."""
+    _fields_ = ([("param", ctypes.c_void_p * 18), ("grad", ctypes.c_void_p * 18)]
+                + [(n, ctypes.c_void_p) for n in ("x", "plan", "pair_lists", "pe_idx", "table", "factors", "kept")]
+                + [("kept_bytes", ctypes.c_size_t), ("shape", AttnShape)]
+                + [(n, ctypes.c_int32) for n in ("hidden", "table_rows", "table_cols", "lists_shared", "x_dtype", "dtype")]
+                + [(n, ctypes.c_float) for n in ("eps1", "eps2", "attn_scale")])
+
+
 _P = ctypes.c_void_p
 _PROTOTYPES = {
     # name: (restype, argtypes)  — one entry per declaration in include/clusten_hip.h
@@ -155,6 +164,10 @@ _PROTOTYPES = {
                                                              ctypes.c_int, _P]),
     "clusten_scatter_attention_pair": (ctypes.c_int, [_P, _P, Strides, _P, _P, _P, Strides, _P, Strides, ctypes.c_float, _P, AttnShape,
                                                      ctypes.c_int, _P]),
+    "clusten_block_train_kept_bytes": (ctypes.c_size_t, [ctypes.POINTER(BlockTrain)]),
+    "clusten_block_train_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(BlockTrain)]),
+    "clusten_block_train_forward": (ctypes.c_int, [ctypes.POINTER(BlockTrain), _P, _P]),
+    "clusten_block_train_backward": (ctypes.c_int, [ctypes.POINTER(BlockTrain), _P, _P, _P, ctypes.c_size_t, _P]),
     "clusten_row_sums_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
     "clusten_gelu_backward": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, _P]),
     "clusten_norm_backward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, ctypes.c_int, _P, _P, _P,
@@ -2126,6 +2139,77 @@ def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torc
                                           _ptr(pe_idx), AttnShape(b, heads, n, 32, m), hidden, scale, _DTYPE_CODES[dtype],
                                           _stream(device)), "clusten_blocks_forward")
     return out
+
+
+def block_train_supported(x: torch.Tensor, dtype: torch.dtype, heads: int, hidden: int, table: torch.Tensor, pe_idx, plan=None, pairs=None) -> bool:
+    """True when `block_train_forward` takes the rows x (B,N,C): what `block_supported` says, heads of 32 channels, a contiguous fp32
+    table of at most five columns; with `plan` (and the pair lists of its numbers) six clusters of 8 a token, else at most 64 tokens."""
+    if x.dim() != 3 or not block_supported(x, dtype, hidden):
+        return False
+    b, n, c = x.shape
+    if (c != 32 * heads or b * n == 0 or b * n >= 1 << 31 or table.dtype != torch.float32 or not table.is_contiguous() or table.dim() != 2
+            or table.shape[1] > 5 or table.device != x.device or pe_idx.dtype != torch.int64 or not pe_idx.is_contiguous()
+            or pe_idx.device != x.device):
+        return False
+    if plan is None:
+        return n <= 64 and pe_idx.shape == (b, n, n)
+    lib = load()
+    return (pairs is not None and pe_idx.shape == (b, n, 48) and plan.dtype == torch.uint8 and pairs.dtype == torch.uint8
+            and plan.numel() in (lib.clusten_cluster_attention_plan_bytes(b, n, 48), lib.clusten_cluster_attention_plan_bytes(1, n, 48))
+            and pairs.numel() == lib.clusten_cluster_pairs_bytes(b, n, 48, n) > 0 and plan.device == pairs.device == x.device)
+
+
+def _block_train(x, params, table, pe_idx, plan, pairs, factors, dtype, heads, hidden, eps, scale):
+    """The argument of a block's training pass, all but what it keeps.  `params`: what `block_train_forward` says."""
+    b, n, _ = x.shape
+    a = BlockTrain()
+    a.param[:] = [t.data_ptr() for t in params]
+    a.x, a.pe_idx, a.table = x.data_ptr(), pe_idx.data_ptr(), table.data_ptr()
+    a.plan, a.pair_lists, a.factors = _ptr(plan), _ptr(pairs), _ptr(factors)
+    a.shape = AttnShape(b, heads, n, 32, n if plan is None else 48)
+    a.hidden, a.x_dtype, a.dtype = hidden, _DTYPE_CODES[x.dtype], _DTYPE_CODES[dtype]
+    a.table_rows, a.table_cols = table.shape
+    a.lists_shared = int(plan is not None and b != 1 and plan.numel() == load().clusten_cluster_attention_plan_bytes(1, n, 48))
+    a.eps1, a.eps2, a.attn_scale = eps[0], eps[1], scale
+    return a
+
+
+def block_train_forward(x: torch.Tensor, params, table: torch.Tensor, pe_idx, plan, pairs, factors, dtype: torch.dtype, heads: int, hidden: int,
+                        eps, scale: float):
+    """A transformer block in training by one call: (out, one uint8 tensor of all the backward reads).  As `block_train_supported`
+    says.  `params`: 18 fp32 tensors in place, in the order of `clusten_block_train`; `factors`: fp32 (2,B) of stochastic depth, or None;
+    `eps`: of the two norms.  No autograd."""
+    lib = load()
+    a = _block_train(x, params, table, pe_idx, plan, pairs, factors, dtype, heads, hidden, eps, scale)
+    a.kept_bytes = lib.clusten_block_train_kept_bytes(a)
+    kept = torch.empty(a.kept_bytes, dtype=torch.uint8, device=x.device)
+    out = torch.empty_like(x)
+    a.kept = kept.data_ptr()
+    with _on(x.device):
+        _check(lib.clusten_block_train_forward(a, out.data_ptr(), _stream(x.device)), "clusten_block_train_forward")
+    return out, kept
+
+
+def block_train_backward(d_out: torch.Tensor, kept: torch.Tensor, needs, x: torch.Tensor, params, table: torch.Tensor, pe_idx, plan, pairs, factors,
+                         dtype: torch.dtype, heads: int, hidden: int, eps, scale: float):
+    """(d_x, the 18 parameters' gradients, fp32) of `block_train_forward`, called with the same arguments and what it kept.  `needs`: 18
+    truth values; the gradients of a Linear layer neither of whose parameters is needed are not formed (None)."""
+    lib = load()
+    _block_rows((x.dtype,), x.shape[-1], x, d_out)
+    a = _block_train(x, params, table, pe_idx, plan, pairs, factors, dtype, heads, hidden, eps, scale)
+    a.kept, a.kept_bytes = kept.data_ptr(), kept.numel()
+    grads = [torch.empty_like(t) for t in params]
+    for bias, weight in ((4, 11), (5, 12), (6, 13), (7, 14), (8, 15)):
+        if not (needs[bias] or needs[weight]):
+            grads[bias] = grads[weight] = None
+    a.grad[:] = [None if g is None else g.data_ptr() for g in grads]
+    d_x = torch.empty_like(x)
+    nbytes = lib.clusten_block_train_workspace_bytes(a)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    with _on(x.device):
+        _check(lib.clusten_block_train_backward(a, d_out.data_ptr(), d_x.data_ptr(), work.data_ptr(), nbytes, _stream(x.device)),
+               "clusten_block_train_backward")
+    return d_x, grads
 
 
 _GRAD_DTYPES = (torch.float32, torch.float16, torch.bfloat16)

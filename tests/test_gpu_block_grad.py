@@ -438,3 +438,23 @@ def walk(node):
             seen.add(f)
             todo += [g for g, _ in f.next_functions]
     return seen
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("local", [True, False])
+def test_frozen_parameters(device, dt, local):
+    """Gradients of a block some of whose parameters take none: those of the others are the same numbers."""
+    grads = []
+    for frozen in ((), ("attn.q.weight", "attn.q.bias", "mlp.fc1.bias", "norm1.weight", "attn.blank_k", "attn.pos_embed.weight")):
+        mod, feat, call = local_stage(device, default_ops()) if local else dense_block(device)
+        names = dict(mod.named_parameters())
+        for name in names:
+            names[name].requires_grad_(not name.endswith(frozen) if frozen else True)
+        x = feat.clone().requires_grad_(True)
+        with torch.autocast("cuda", dtype=torch.float16 if dt == torch.float32 else dt, enabled=dt != torch.float32):
+            out = call(x) if local else call(x)[0]
+        out.float().square().sum().backward()
+        grads.append({"x": x.grad, **{n: p.grad for n, p in names.items()}})
+    for name, ref in grads[0].items():
+        got = grads[1][name]
+        assert (got is None) if name != "x" and name.endswith(frozen) else torch.equal(got, ref), name
