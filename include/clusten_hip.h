@@ -772,6 +772,22 @@ int clusten_block_train_forward(const clusten_block_train* args, void* out, clus
 int clusten_block_train_backward(const clusten_block_train* args, const void* d_out, void* d_x, void* workspace,
                                  size_t workspace_bytes, clusten_stream stream);
 
+/* Training passes around a merge (models/aff_transformer.py:340-358, 496-500 under autograd).
+ *   merge_weights_backward, of clusten_merge_weights_forward: d_rows (B,4,Nout,M) = d_weights (B,Nout,M,4) * prob * mask, which
+ *     clusten_bias_table_grad (H = 4, the same pe_idx) sums into the table's rows, and, with prob, d_prob (B,N), written in full (fp32
+ *     atomics).
+ *   row_score: score (rows) of dtype = sigmoid(x w + bias), operands, the sum and the result rounded to dtype; x (rows,C) of x_dtype (F32
+ *     or dtype), C in {32,64,128,256,512}, w (C) and bias (1, may be NULL) fp32.  The backward: d_x of x_dtype, d_weight (C), d_bias (C floats,
+ *     the first is the bias' gradient); workspace: clusten_row_sums_workspace_bytes(rows, C). */
+int clusten_merge_weights_backward(const float* d_weights, const float* table_weights, const int64_t* pe_idx,
+                                   const int64_t* nbhd_idx, const float* prob, const int64_t* mask, float* d_rows, float* d_prob,
+                                   int B, int N, int Nout, int M, clusten_stream stream);
+int clusten_row_score_forward(const void* x, int x_dtype, const float* weight, const float* bias, void* score, int64_t rows, int C,
+                              int dtype, clusten_stream stream);
+int clusten_row_score_backward(const void* x, int x_dtype, const float* weight, const void* score, const void* d_score, void* d_x,
+                               float* d_weight, float* d_bias, void* workspace, size_t workspace_bytes, int64_t rows, int C,
+                               int dtype, clusten_stream stream);
+
 /* The backward of a block between its products, which the reference leaves to autograd.  Tensors are dense rows of C channels
  * (C in {32,64,128,256,512}) of dtype F32, F16 or BF16 unless said otherwise, on 16-byte boundaries; sums are fp32 in a fixed
  * order; workspace: clusten_row_sums_workspace_bytes(rows, C) bytes.

@@ -52,6 +52,9 @@ def default_ops():
                            linear=_native.linear, linear_supported=_native.linear_supported,
                            add_layer_norm=_native.add_layer_norm, add_layer_norm_supported=_native.add_layer_norm_supported,
                            merge_weights=_native.merge_weights, merge_weights_supported=_native.merge_weights_supported,
+                           merge_weights_backward=_native.merge_weights_backward,
+                           row_score=_native.row_score, row_score_backward=_native.row_score_backward,
+                           row_score_supported=_native.row_score_supported,
                            channel_affine_gelu=_native.channel_affine_gelu,
                            channel_affine_gelu_supported=_native.channel_affine_gelu_supported,
                            add_row_score=_native.add_row_score, add_row_score_supported=_native.add_row_score_supported,
@@ -578,6 +581,64 @@ class _DenseAttentionRows(_BlockRows):
     """A block whose tokens attend to all."""
 
 
+class _MergeWeights(torch.autograd.Function):
+    """The weights a merge's WF operator takes - table rows by position, times importance, times mask - with both gradients from
+    the library's kernels; fp32."""
+
+    @staticmethod
+    def forward(ctx, table_w, prob, pe_idx, member_idx, mask, ops):
+        ctx.save_for_backward(table_w, prob, pe_idx, member_idx, mask)
+        ctx.ops = ops
+        return ops.merge_weights(table_w, pe_idx, member_idx, prob, mask)
+
+    @staticmethod
+    @_types_of_forward
+    def backward(ctx, d_w):
+        table_w, prob, pe_idx, member_idx, mask = ctx.saved_tensors
+        if not _by_kernels(d_w):
+            b, n_out, m = pe_idx.shape
+
+            def layers(table_w, prob):
+                weights = _table_rows(table_w, pe_idx) * prob.gather(1, member_idx.reshape(b, -1)).reshape(b, n_out, m, 1)
+                return weights if mask is None else weights * mask.unsqueeze(3)
+            return (*_recorded_backward(layers, ctx, (table_w, prob), (d_w,)), None, None, None, None)
+        d_table, d_prob = ctx.ops.merge_weights_backward(d_w, table_w, pe_idx, member_idx, prob, mask)
+        return d_table, d_prob, None, None, None, None
+
+
+class _RowScore(torch.autograd.Function):
+    """`sigmoid(linear(x))` of a layer of one output, one pass over the rows a direction."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, dt, ops):
+        score = ops.row_score(x, weight, bias, dt)
+        ctx.save_for_backward(x, weight, bias, score)
+        ctx.meta = (dt, ops)
+        return score
+
+    @staticmethod
+    @_types_of_forward
+    def backward(ctx, d_score):
+        x, weight, bias, score = ctx.saved_tensors
+        dt, ops = ctx.meta
+        if not _by_kernels(d_score):
+            return (*_recorded_backward(lambda x, w, b: F.linear(x.to(dt), w.to(dt), b.to(dt)).sigmoid(), ctx, (x, weight, bias), (d_score,)),
+                    None, None)
+        d_x, d_w, d_b = ops.row_score_backward(x, weight, score, d_score.contiguous())
+        return (*(g if need else None for g, need in zip((d_x, d_w.view(weight.shape), d_b.view(bias.shape)), ctx.needs_input_grad)), None, None)
+
+
+def _score(lin, x, ops):
+    """`lin(x).sigmoid()` for a layer of one output."""
+    if torch.is_grad_enabled() and getattr(ops, "row_score_backward", None) is not None and x.is_cuda:
+        w, b = lin.weight, lin.bias
+        dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else torch.float32
+        if (type(lin) is nn.Linear and w is not None and w.shape[0] == 1 and b is not None and b.dtype == torch.float32 and not _hooked(lin)
+                and not _transformed() and b.device == x.device and ops.row_score_supported(x, w, dt)):
+            return _RowScore.apply(x, w, b, dt, ops)
+    return _linear(lin, x).sigmoid()
+
+
 def _columns(qkv, heads):
     """(q, key, v), each (b,h,n,ch), of (b,n,3c) rows of stacked projections (views)."""
     b, n, c3 = qkv.shape
@@ -1046,6 +1107,10 @@ class ClusterMerging(_Module):
         if one_pass is not None and not torch.is_grad_enabled() and self.ops.merge_weights_supported(table_w):
             # inference: lookup, importance of each neighbour and mask in one kernel
             weights = one_pass(table_w, pe_idx, member_idx, learned_prob, mask_rows)
+        elif (one_pass is not None and getattr(self.ops, "merge_weights_backward", None) is not None and torch.is_grad_enabled()
+              and learned_prob is not None and table_w.is_cuda and table_w.dtype == torch.float32 and table_w.is_contiguous()
+              and self.ops.merge_weights_supported(table_w) and not _transformed()):
+            weights = _MergeWeights.apply(table_w, learned_prob.float().reshape(b, n), pe_idx, member_idx, mask_rows, self.ops)
         else:
             weights = _table_rows(table_w, pe_idx)                                       # (b, n', m, 4)
             if learned_prob is not None:
@@ -1284,7 +1349,7 @@ class BasicLayer(_Module):
             if global_attn:   # merging after a dense stage: every token is every token's neighbour
                 member_idx = torch.arange(n, device=feat.device).expand(b, n, n).contiguous()
             if learned_prob is None:
-                learned_prob = _linear(self.prob_net, feat).sigmoid()
+                learned_prob = _score(self.prob_net, feat, self.ops)
             reserve_num = math.ceil(h / (stride * 2)) * math.ceil(w / (stride * 2))
             pos, feat = self.downsample(pos, feat, member_idx, mask, learned_prob, stride, pe_idx, reserve_num, table)
         return pos, feat

@@ -168,6 +168,10 @@ _PROTOTYPES = {
     "clusten_block_train_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(BlockTrain)]),
     "clusten_block_train_forward": (ctypes.c_int, [ctypes.POINTER(BlockTrain), _P, _P]),
     "clusten_block_train_backward": (ctypes.c_int, [ctypes.POINTER(BlockTrain), _P, _P, _P, ctypes.c_size_t, _P]),
+    "clusten_merge_weights_backward": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_row_score_forward": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_row_score_backward": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, ctypes.c_int64, ctypes.c_int,
+                                                 ctypes.c_int, _P]),
     "clusten_row_sums_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
     "clusten_gelu_backward": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, _P]),
     "clusten_norm_backward": (ctypes.c_int, [_P, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, ctypes.c_int, _P, _P, _P,
@@ -1483,6 +1487,70 @@ def merge_weights(table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: t
                                                  n_out, m, table_weights.shape[1], _stream(device)),
                "clusten_merge_weights_forward")
     return out
+
+
+def merge_weights_backward(d_weights: torch.Tensor, table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: torch.Tensor, prob, mask):
+    """(d_table (rows,4), d_prob (B,N) or None) of `merge_weights` for fp32 d_weights (B,N',M,4), table_weights and prob (B,N)."""
+    lib = load()
+    device = d_weights.device
+    _require_cuda("d_weights", d_weights)
+    b, n_out, m, ic = d_weights.shape
+    if (ic != 4 or d_weights.dtype != torch.float32 or table_weights.dtype != torch.float32 or not table_weights.is_contiguous()
+            or table_weights.dim() != 2 or table_weights.shape[1] != 4 or table_weights.data_ptr() % 16
+            or any(t.shape != (b, n_out, m) or t.dtype != torch.int64 for t in (pe_idx, nbhd_idx))
+            or (prob is not None and (prob.dtype != torch.float32 or not prob.is_contiguous() or prob.dim() != 2 or prob.shape[0] != b))
+            or (mask is not None and mask.shape != pe_idx.shape)
+            or any(t is not None and t.device != device for t in (table_weights, pe_idx, nbhd_idx, prob, mask))):
+        raise RuntimeError("merge_weights_backward: fp32 d_weights (B,N',M,4), table (rows,4), prob (B,N); int64 indices (B,N',M)")
+    d_weights, pe_idx, nbhd_idx = d_weights.contiguous(), pe_idx.contiguous(), nbhd_idx.contiguous()
+    d_weights = d_weights if d_weights.data_ptr() % 16 == 0 else d_weights.clone()
+    mask = None if mask is None else mask.to(torch.int64).contiguous()
+    d_prob = None if prob is None else torch.empty_like(prob)
+    rows = torch.empty(b, 4, n_out, m, dtype=torch.float32, device=device)
+    if rows.numel() == 0:
+        return torch.zeros_like(table_weights), None if prob is None else d_prob.zero_()
+    with _on(device):
+        _check(lib.clusten_merge_weights_backward(d_weights.data_ptr(), table_weights.data_ptr(), pe_idx.data_ptr(), nbhd_idx.data_ptr(), _ptr(prob),
+                                                  _ptr(mask), rows.data_ptr(), _ptr(d_prob), b, 1 if prob is None else prob.shape[1], n_out, m,
+                                                  _stream(device)), "clusten_merge_weights_backward")
+    return bias_table_grad(rows, pe_idx, table_weights.shape[0]), d_prob
+
+
+def row_score_supported(x: torch.Tensor, weight: torch.Tensor, dtype: torch.dtype) -> bool:
+    """True when `row_score` takes rows x (..., C): a width of the block kernels, x fp32 or of `dtype`, a fp32 weight in place."""
+    return (x.is_cuda and x.dim() > 1 and x.shape[-1] in _BLOCK_WIDTHS and dtype in _DTYPE_CODES and x.dtype in (torch.float32, dtype)
+            and x.is_contiguous() and x.data_ptr() % 16 == 0 and 0 < x.numel() // x.shape[-1] < 1 << 31 and weight.dtype == torch.float32
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0 and weight.numel() == x.shape[-1] and weight.device == x.device)
+
+
+def row_score(x: torch.Tensor, weight: torch.Tensor, bias, dtype: torch.dtype) -> torch.Tensor:
+    """sigmoid(x @ weight + bias) of shape (..., 1) in `dtype`, as a Linear layer of one output rounds it.  No autograd."""
+    if not row_score_supported(x, weight, dtype) or (bias is not None and (bias.dtype != torch.float32 or bias.numel() != 1 or bias.device != x.device)):
+        raise RuntimeError("row_score: rows of a width of the block kernels, fp32 weight (C) and bias (1)")
+    out = torch.empty(x.shape[:-1] + (1,), dtype=dtype, device=x.device)
+    c = x.shape[-1]
+    with _on(x.device):
+        _check(load().clusten_row_score_forward(x.data_ptr(), _DTYPE_CODES[x.dtype], weight.data_ptr(), _ptr(bias), out.data_ptr(), x.numel() // c, c,
+                                                _DTYPE_CODES[dtype], _stream(x.device)), "clusten_row_score_forward")
+    return out
+
+
+def row_score_backward(x: torch.Tensor, weight: torch.Tensor, score: torch.Tensor, d_score: torch.Tensor):
+    """(d_x, d_weight (C,), d_bias (1,)) of `row_score`."""
+    if (not row_score_supported(x, weight, score.dtype) or score.numel() * x.shape[-1] != x.numel() or not score.is_contiguous()
+            or d_score.dtype != score.dtype or d_score.numel() != score.numel() or not d_score.is_contiguous()
+            or score.device != x.device or d_score.device != x.device):
+        raise RuntimeError("row_score_backward: rows and weight as row_score takes them, contiguous scores of one dtype")
+    c = x.shape[-1]
+    rows = x.numel() // c
+    d_x = torch.empty_like(x)
+    ws, nbytes, sums = _row_sums(rows, c, x.device)
+    with _on(x.device):
+        at = sums.data_ptr()
+        _check(load().clusten_row_score_backward(x.data_ptr(), _DTYPE_CODES[x.dtype], weight.data_ptr(), score.data_ptr(), d_score.data_ptr(),
+                                                 d_x.data_ptr(), at, at + 4 * c, ws.data_ptr(), nbytes, rows, c, _DTYPE_CODES[score.dtype],
+                                                 _stream(x.device)), "clusten_row_score_backward")
+    return d_x, sums[0], sums[1, :1]
 
 
 def scanline_rank_supported(pos: torch.Tensor, rows: int, cols: int) -> bool:

@@ -863,6 +863,46 @@ int clusten_scatter_attention_pair(const void* d_logit, const void* query, clust
                                dtype, as_stream(stream));
 }
 
+int clusten_merge_weights_backward(const float* d_weights, const float* table_weights, const int64_t* pe_idx, const int64_t* nbhd_idx,
+                                   const float* prob, const int64_t* mask, float* d_rows, float* d_prob, int B, int N, int Nout, int M,
+                                   clusten_stream stream) {
+    if (!d_weights || !pe_idx || !d_rows || (prob && (!table_weights || !nbhd_idx || !d_prob))) return CLUSTEN_ERR_NULL_POINTER;
+    if (B <= 0 || N <= 0 || Nout <= 0 || M <= 0 || ((int64_t)B * Nout * M + 255) / 256 >= (int64_t)1 << 31) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(d_weights) || !aligned16(table_weights) || !aligned16(d_prob)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_merge_weights_backward(d_weights, table_weights, pe_idx, nbhd_idx, prob, mask, d_rows, prob ? d_prob : nullptr, B, N, Nout, M,
+                                         as_stream(stream));
+}
+
+static int row_score_args(RowScore& a, const void* x, int x_dtype, const float* weight, void* score, int64_t rows, int C, int dtype) {
+    if (!x || !weight || !score) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype) || (x_dtype != dtype && x_dtype != CLUSTEN_F32)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (rows <= 0 || rows >= (int64_t)1 << 31 || !block_width_supported(C)) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(x) || !aligned16(weight)) return CLUSTEN_ERR_UNALIGNED;
+    a = {};
+    a.x = x, a.weight = weight, a.score = score, a.rows = rows;
+    return CLUSTEN_OK;
+}
+
+int clusten_row_score_forward(const void* x, int x_dtype, const float* weight, const float* bias, void* score, int64_t rows, int C, int dtype,
+                              clusten_stream stream) {
+    RowScore a;
+    if (int st = row_score_args(a, x, x_dtype, weight, score, rows, C, dtype)) return st;
+    a.bias = bias;
+    return launch_row_score(a, x_dtype, C, dtype, as_stream(stream));
+}
+
+int clusten_row_score_backward(const void* x, int x_dtype, const float* weight, const void* score, const void* d_score, void* d_x,
+                               float* d_weight, float* d_bias, void* workspace, size_t workspace_bytes, int64_t rows, int C, int dtype,
+                               clusten_stream stream) {
+    RowScore a;
+    if (int st = row_score_args(a, x, x_dtype, weight, const_cast<void*>(score), rows, C, dtype)) return st;
+    if (!d_score || !d_x || !d_weight || !d_bias || !workspace) return CLUSTEN_ERR_NULL_POINTER;
+    if (workspace_bytes < row_sums_workspace_bytes(rows, C)) return CLUSTEN_ERR_WORKSPACE;
+    if (!aligned16(d_x) || !aligned16(workspace)) return CLUSTEN_ERR_UNALIGNED;
+    a.d_score = d_score, a.d_x = d_x, a.d_weight = d_weight, a.d_bias = d_bias, a.partial = static_cast<float*>(workspace);
+    return launch_row_score(a, x_dtype, C, dtype, as_stream(stream));
+}
+
 static int check_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype) {
     if (!items) return CLUSTEN_ERR_NULL_POINTER;
     if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;

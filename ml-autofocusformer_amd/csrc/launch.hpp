@@ -374,6 +374,23 @@ int launch_scatter_pair(const void* d_logit, const void* query, clusten_strides 
                         clusten_strides gs, void* d_value, clusten_strides ys, float scale, const void* pair_lists, clusten_attn_shape s,
                         int dtype, hipStream_t stream);
 
+// Training passes of a merge's weights and of the importance score (merge_grad.hip).
+int launch_merge_weights_backward(const float* d_w, const float* table_w, const int64_t* pe_idx, const int64_t* nbhd_idx, const float* prob,
+                                  const int64_t* mask, float* t, float* d_prob, int B, int N, int Nout, int M, hipStream_t stream);
+struct RowScore {
+    const void* x;         // (rows, C) of S
+    const float* weight;   // (C)
+    const float* bias;     // (1), or null
+    void* score;           // (rows) of T
+    const void* d_score;   // (rows) of T
+    void* d_x;             // (rows, C) of S: the backward; null: the forward
+    float* d_weight;       // (C)
+    float* d_bias;         // (C): the first value
+    float* partial;
+    int64_t rows;
+};
+int launch_row_score(const RowScore& a, int x_dtype, int C, int dtype, hipStream_t stream);
+
 // Parameter gradients of Linear layers over the same rows (weight_grad.hip).
 size_t weight_grad_workspace_bytes(const clusten_weight_grad_item* items, int count, int64_t rows, int dtype);
 int launch_weight_grad(const clusten_weight_grad_item* items, int count, int64_t rows, float* workspace, int dtype, hipStream_t stream);

@@ -96,3 +96,36 @@ def test_rows_of_an_attention_layer(device, dt, b, h, n, ch):
     assert torch.equal(kv[1], d_v)
     near(d_bk, 0.3 * (d_blank.double().unsqueeze(-1) * q.double()).sum((0, 2)).reshape(-1), 5e-6)
     near(d_bv, (blank.double().unsqueeze(-1) * g.double()).sum((0, 2)).reshape(-1), 5e-6)
+
+
+@pytest.mark.parametrize("b,n,n_out,m,rows,masked", [(1, 1, 1, 1, 1, False), (2, 50, 12, 48, 225, True), (3, 777, 194, 49, 12321, False)])
+def test_merge_weights(device, b, n, n_out, m, rows, masked):
+    gen = torch.Generator(device).manual_seed(n)
+    table, prob = torch.randn(rows, 4, generator=gen, device=device), torch.rand(b, n, generator=gen, device=device)
+    pe, idx = (torch.randint(k, (b, n_out, m), generator=gen, device=device) for k in (rows, n))
+    mask = torch.randint(2, (b, n_out, m), generator=gen, device=device) if masked else None
+    d = torch.randn(b, n_out, m, 4, generator=gen, device=device)
+    d_table, d_prob = _native.merge_weights_backward(d, table, pe, idx, prob, mask)
+    t64, p64 = table.double().requires_grad_(True), prob.double().requires_grad_(True)
+    w = t64[pe] * p64.gather(1, idx.reshape(b, -1)).reshape(b, n_out, m, 1)
+    w = w if mask is None else w * mask.unsqueeze(3)
+    ref = torch.autograd.grad(w, (t64, p64), d.double())
+    near(d_table, ref[0], 5e-7)
+    near(d_prob, ref[1], 5e-7)
+
+
+@pytest.mark.parametrize("dt,stream", [(torch.float16, torch.float16), (torch.float16, torch.float32), (torch.bfloat16, torch.float32),
+                                       (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("c,b,n", [(32, 1, 1), (64, 2, 16 * 1024 + 1), (128, 3, 99), (256, 1, 7), (512, 2, 2049)])
+def test_row_score(device, dt, stream, c, b, n):
+    gen = torch.Generator(device).manual_seed(n)
+    x, w = torch.randn(b, n, c, generator=gen, device=device).to(stream), torch.randn(1, c, generator=gen, device=device) * c ** -0.5
+    bias, d = torch.randn(1, generator=gen, device=device), torch.randn(b, n, 1, generator=gen, device=device).to(dt)
+    score = _native.row_score(x, w, bias, dt)
+    x64, w64 = x.to(dt).double(), w.to(dt).double()
+    near(score, torch.sigmoid((x64 @ w64.t() + bias.to(dt).double()).to(dt).double()), 2 * BAR[dt])
+    d_x, d_w, d_b = _native.row_score_backward(x, w, score, d)
+    d_z = d.double() * score.double() * (1 - score.double())
+    near(d_x, d_z * w64, BAR[stream])
+    near(d_w, (d_z * x64).sum((0, 1)), 2e-6)
+    assert (d_b.double() - d_z.sum()).abs() <= 2e-6 * d_z.norm()           # what a sum of such terms comes to, not this one
