@@ -137,7 +137,7 @@ __global__ __launch_bounds__(kWave) void cluster_attention_kernel(
 
     __shared__ __attribute__((aligned(1024))) char stage[LDS_BYTES];
 
-    // a workgroup serves the heads [h0, h0 + H) of its tile (see head_groups_for())
+    // a workgroup serves the heads [h0, h0 + H) of its tile (see attention_head_groups())
     const int unit = xcd_tile(blockIdx.x, total_tiles * head_groups);
     if (unit < 0) return;
     const int tile = unit / head_groups;
@@ -439,7 +439,7 @@ int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strid
                  hipStream_t stream) {
     const int tiles_per_batch = (s.N + kTileTokens - 1) / kTileTokens;
     const int total = s.B * tiles_per_batch;
-    const int groups = head_groups_for(total, s.H);  // 196 tokens x 8 heads, B = 128: 69.6 -> 63.9 us
+    const int groups = attention_head_groups(total, s.H, CS == 24 ? 8192 : 3072);
     hipLaunchKernelGGL((cluster_attention_kernel<T, CS>), dim3(xcd_grid(total * groups)), dim3(kWave), 0, stream,
                        static_cast<const T*>(q), qs, static_cast<const T*>(k), ks, static_cast<const T*>(v), vs,
                        cluster_idx, static_cast<const T*>(table), pe_idx, mask, blank_k, blank_v, static_cast<T*>(out),

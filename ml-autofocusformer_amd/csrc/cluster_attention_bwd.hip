@@ -414,7 +414,7 @@ int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strid
                  const clusten_attn_shape& s, hipStream_t stream) {
     const int tiles_per_batch = (s.N + kTileTokens - 1) / kTileTokens;
     const int total = s.B * tiles_per_batch;
-    const int groups = head_groups_for(total, s.H);
+    const int groups = attention_head_groups(total, s.H, 3072);
     hipLaunchKernelGGL((cluster_attention_bwd_kernel<T>), dim3(xcd_grid(total * groups)), dim3(kWave), 0, stream,
                        static_cast<const T*>(q), qs, static_cast<const T*>(k), ks, static_cast<const T*>(v), vs,
                        static_cast<const T*>(d_out), gs, static_cast<const T*>(out), os, lse, cluster_idx,

@@ -353,7 +353,7 @@ int launch_cluster_attention_backward_f32(const void* q, clusten_strides qs, con
                                           hipStream_t stream) {
     const int tiles_per_batch = (s.N + kTileTokens - 1) / kTileTokens;
     const int total = s.B * tiles_per_batch;
-    const int groups = head_groups_for(total, s.H);
+    const int groups = attention_head_groups(total, s.H, 3072);
     hipLaunchKernelGGL(cluster_attention_bwd_f32_kernel, dim3(xcd_grid(total * groups)), dim3(kWave), 0, stream,
                        static_cast<const float*>(q), qs, static_cast<const float*>(k), ks, static_cast<const float*>(v), vs,
                        static_cast<const float*>(d_out), gs, static_cast<const float*>(out), os, lse, cluster_idx,

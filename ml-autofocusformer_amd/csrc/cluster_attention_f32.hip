@@ -53,7 +53,7 @@ __global__ __launch_bounds__(kWave) void cluster_attention_f32_kernel(
     const char* __restrict__ plan, float* __restrict__ lse) {
     __shared__ __attribute__((aligned(1024))) char stage[LDS_BYTES];
 
-    // a workgroup serves the heads [h0, h0 + H) of its tile (see head_groups_for())
+    // a workgroup serves the heads [h0, h0 + H) of its tile (see attention_head_groups())
     const int unit = xcd_tile(blockIdx.x, total_tiles * head_groups);
     if (unit < 0) return;
     const int tile = unit / head_groups;
@@ -338,7 +338,7 @@ int launch_cluster_attention_f32(const void* q, clusten_strides qs, const void* 
                                  const clusten_attn_shape& s, hipStream_t stream) {
     const int tiles_per_batch = (s.N + kTileTokens - 1) / kTileTokens;
     const int total = s.B * tiles_per_batch;
-    const int groups = head_groups_for(total, s.H);
+    const int groups = attention_head_groups(total, s.H, 3072);
     hipLaunchKernelGGL(cluster_attention_f32_kernel, dim3(xcd_grid(total * groups)), dim3(kWave), 0, stream,
                        static_cast<const float*>(q), qs, static_cast<const float*>(k), ks, static_cast<const float*>(v), vs,
                        cluster_idx, static_cast<const float*>(table), pe_idx, mask, blank_k, blank_v,

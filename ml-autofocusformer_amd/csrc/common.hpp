@@ -218,6 +218,18 @@ inline int xcd_grid(int total) { return ((total + kXcds - 1) / kXcds) * kXcds; }
 // tiles) two groups cost AV 3 %.
 inline int head_groups_for(int total_tiles, int H) { return (total_tiles < 8192 && H >= 4) ? 2 : 1; }
 
+// The same for the one-kernel attention, whose heads are longer chains: groups until there are `waves` one-wave workgroups.  Clusters of
+// 24 (two waves fit a SIMD), us with 1 / 2 / 4 / 8 / 16 groups, 16 images: 4608 tiles x 8 heads 152 / 140 / 143 / 158 / -, 1152 x 16 119 / 101 /
+// 79 / 74 / 81, 288 x 32 142 / 80 / 48 / 48 / 41: 8192 waves.  Clusters of 8: fp32 forward 1250 x 8 45 / 40 / 35 / 35, backward 1600 x 8
+// fp16 50 / 35 / 37 / 43, 200 x 8 fp32 58 / 31 / 30 / 30: 3072 waves.  Every group has at least one head.
+inline int attention_head_groups(int total_tiles, int H, int waves) {
+    int groups = head_groups_for(total_tiles, H);
+    while (groups < H && (int64_t)total_tiles * groups < waves) groups *= 2;
+    groups = groups < H ? groups : H;
+    const int heads = (H + groups - 1) / groups;
+    return (H + heads - 1) / heads;
+}
+
 // ---- host-side argument checks ------------------------------------------------------------------
 
 inline bool dtype_ok(int dtype) { return dtype >= CLUSTEN_F32 && dtype <= CLUSTEN_F64; }
