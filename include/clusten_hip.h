@@ -674,6 +674,12 @@ int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x
                            const void* plan, int lists_shared, const int64_t* pe_idx, clusten_attn_shape shape, int hidden,
                            float scale, int dtype, clusten_stream stream);
 
+/* The same with the local attention's bias tables as (H, table_rows): the bias of neighbouring positions then lies side by side.  table_rows = 0:
+ * as above. */
+int clusten_blocks_forward_tables(const clusten_block* blocks, int count, const void* x, int x_dtype, void* out, void* qkv,
+                                  void* attn, const void* plan, int lists_shared, const int64_t* pe_idx, int table_rows,
+                                  clusten_attn_shape shape, int hidden, float scale, int dtype, clusten_stream stream);
+
 /* Parameter gradients of Linear layers over the same `rows` token rows: d_weight (n,k) = d_y^T x and d_bias (n) = the column
  * sums of d_y (d_bias NULL: none), fp32, written in full.  d_y (rows,n) and x (rows,k) of dtype (F32, F16, BF16) with row
  * strides in elements; rows, bases and fp32 results on 16-byte boundaries; n and k multiples of 8; 1 <= count <= 8.  Sums are
@@ -712,7 +718,7 @@ int clusten_norm_linear_backward(const void* d_y, const void* x, int x_dtype, co
 
 /* The training pass of an attention layer beside its attention kernels (models/aff_transformer.py:103-155 under autograd), dtype F32,
  * F16 or BF16.
- *   position_bias: bias (rows,n) = table weight^T + bias_param (may be NULL) for a fp32 table (rows,k), k <= 8, every operand rounded to
+ *   position_bias: bias (n,rows) = weight table^T + bias_param (may be NULL) for a fp32 table (rows,k), k <= 8, every operand rounded to
  *     dtype; padded (rows,8) of dtype, when not NULL: the table's rows, zeros behind the k columns.
  *   position_grad: d_weight (H,k) = sum d_logit[b,h,i,j] table[pe_idx[b,i,j]], d_bias (H) = sum d_logit, for d_logit (B,H,N,M) of dtype,
  *     pe_idx (B,N,M) inside the table, M a multiple of 4, k <= 5; sums in fp64 in a fixed order.

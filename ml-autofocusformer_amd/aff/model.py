@@ -1231,7 +1231,7 @@ class BasicLayer(_Module):
         tensors = [blk.tensors() for blk in self.blocks]
         hidden, scale = first.mlp.fc1.out_features, first.attn.scale
         try:
-            key = (dt, table.data_ptr(), table._version, table.dtype, c, h, hidden,
+            key = (dt, table.data_ptr(), table._version, table.dtype, c, h, hidden, plan is None,
                    [[(t._version, t.data_ptr()) for t in ts] for ts in tensors],
                    [(m["norm1"].eps, m["norm2"].eps, m["attn"].scale, m["attn"].num_heads) for m in map(_modules_of, self.blocks)])
         except AttributeError:                                     # a parameter is None, say the bias of a layer without one
@@ -1246,7 +1246,8 @@ class BasicLayer(_Module):
             params = (ops.block_params * len(tensors))()
             for p, blk, ts in zip(params, self.blocks, tensors):
                 bias = blk.attn.bias_table(table)
-                bias = bias.detach().to(dt).contiguous()
+                bias = bias.detach().to(dt)
+                bias = (bias if plan is None else bias.t()).contiguous()       # by heads for the local attention
                 made.append(bias)
                 if dt != torch.float32:
                     packed, at = blk._packed(dt)
@@ -1269,7 +1270,8 @@ class BasicLayer(_Module):
             params = type(params).from_buffer_copy(params)
             for i, p in enumerate(params):
                 p.w_qkv, _, p.w_proj, p.w1, p.w2 = (base + o for o in at[5 * i:5 * i + 5])
-        return ops.blocks_forward(params, feat, h, hidden, dt, scale, plan, pe_idx if plan is None else None)
+        return ops.blocks_forward(params, feat, h, hidden, dt, scale, plan, pe_idx if plan is None else None,
+                                  0 if plan is None else table.shape[0])
 
     def forward(self, pos, feat, h, w, on_grid, stride, table, radius, feat_ordered=False):
         """`feat_ordered`: the tokens already stand in the order `grid_order` gave (first stage only)."""

@@ -186,6 +186,8 @@ _PROTOTYPES = {
                                                  ctypes.c_int, ctypes.c_int, _P]),
     "clusten_blocks_forward": (ctypes.c_int, [ctypes.POINTER(BlockParams), ctypes.c_int, _P, ctypes.c_int, _P, _P, _P, _P,
                                              ctypes.c_int, _P, AttnShape, ctypes.c_int, ctypes.c_float, ctypes.c_int, _P]),
+    "clusten_blocks_forward_tables": (ctypes.c_int, [ctypes.POINTER(BlockParams), ctypes.c_int, _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_int,
+                                                    _P, ctypes.c_int, AttnShape, ctypes.c_int, ctypes.c_float, ctypes.c_int, _P]),
     "clusten_knn2d": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
 }
 
@@ -2044,7 +2046,7 @@ def attention_columns_backward(qkv: torch.Tensor, d_qkv: torch.Tensor, d_k: torc
 
 
 def position_bias(table: torch.Tensor, weight: torch.Tensor, bias, dtype: torch.dtype):
-    """(table @ weight.T + bias of shape (rows, heads), the table's rows padded to 8 values), both in `dtype` and made of operands rounded
+    """((table @ weight.T + bias).T of shape (heads, rows), the table's rows padded to 8 values), both in `dtype` and made of operands rounded
     to it: the position bias of every row of a (rows, k <= 8) relative-position table.  No autograd."""
     _require_cuda("table", table)
     rows, k = table.shape
@@ -2054,7 +2056,7 @@ def position_bias(table: torch.Tensor, weight: torch.Tensor, bias, dtype: torch.
             raise RuntimeError("position_bias: contiguous fp32 table and parameters on one device")
     if weight.dim() != 2 or weight.shape[1] != k or k > 8 or (bias is not None and bias.numel() != heads) or dtype not in _DTYPE_CODES:
         raise RuntimeError("position_bias: table (rows,k), weight (heads,k), bias (heads), k <= 8")
-    out = torch.empty(rows, heads, dtype=dtype, device=table.device)
+    out = torch.empty(heads, rows, dtype=dtype, device=table.device)
     padded = torch.empty(rows, 8, dtype=dtype, device=table.device)
     with _on(table.device):
         _check(load().clusten_position_bias(table.data_ptr(), weight.data_ptr(), _ptr(bias), out.data_ptr(), padded.data_ptr(), rows, heads, k,
@@ -2089,7 +2091,7 @@ def dense_attention_train_supported(qkv: torch.Tensor, heads: int) -> bool:
 def _dense_train(qkv, bias, pe_idx, blank_k, blank_v, heads):
     b, n, _ = qkv.shape
     if (not dense_attention_train_supported(qkv, heads) or pe_idx.shape != (b, n, n) or pe_idx.dtype != torch.int64 or not pe_idx.is_contiguous()
-            or bias.dtype != qkv.dtype or bias.dim() != 2 or bias.shape[1] != heads or not bias.is_contiguous()
+            or bias.dtype != qkv.dtype or bias.dim() != 2 or bias.shape[0] != heads or not bias.is_contiguous()
             or any(t.dtype != torch.float32 or not t.is_contiguous() or t.numel() != 32 * heads for t in (blank_k, blank_v))
             or any(t.device != qkv.device for t in (bias, pe_idx, blank_k, blank_v))):
         raise RuntimeError("dense_attention_train: rows, position bias, indices and blank token of one layer of heads of 32 channels")
@@ -2103,7 +2105,7 @@ def dense_attention_train(qkv: torch.Tensor, bias: torch.Tensor, pe_idx: torch.T
     out = torch.empty(b, n, 32 * heads, dtype=qkv.dtype, device=qkv.device)
     with _on(qkv.device):
         _check(load().clusten_dense_attention_train_forward(qkv.data_ptr(), bias.data_ptr(), pe_idx.data_ptr(), blank_k.data_ptr(), blank_v.data_ptr(),
-                                                            out.data_ptr(), scale, b, heads, n, bias.shape[0], _DTYPE_CODES[qkv.dtype],
+                                                            out.data_ptr(), scale, b, heads, n, bias.shape[1], _DTYPE_CODES[qkv.dtype],
                                                             _stream(qkv.device)), "clusten_dense_attention_train_forward")
     return out
 
@@ -2113,7 +2115,7 @@ def dense_attention_train_backward(qkv: torch.Tensor, bias: torch.Tensor, padded
     """(d_qkv, d_blank_k, d_blank_v, d_weight, d_bias) of `dense_attention_train`; the last two are `position_bias`' gradients."""
     b, n = _dense_train(qkv, bias, pe_idx, blank_k, blank_v, heads)
     _block_rows((qkv.dtype,), 32 * heads, d_out)
-    if d_out.numel() != b * n * 32 * heads or padded.dtype != qkv.dtype or tuple(padded.shape) != (bias.shape[0], 8) or not padded.is_contiguous():
+    if d_out.numel() != b * n * 32 * heads or padded.dtype != qkv.dtype or tuple(padded.shape) != (bias.shape[1], 8) or not padded.is_contiguous():
         raise RuntimeError("dense_attention_train_backward: d_out (b,n,c) and padded (rows,8) of the rows' dtype")
     device = qkv.device
     d_qkv = torch.empty_like(qkv)
@@ -2124,7 +2126,7 @@ def dense_attention_train_backward(qkv: torch.Tensor, bias: torch.Tensor, padded
         _check(load().clusten_dense_attention_train_backward(qkv.data_ptr(), bias.data_ptr(), padded.data_ptr(), pe_idx.data_ptr(), blank_k.data_ptr(),
                                                              blank_v.data_ptr(), d_out.data_ptr(), d_qkv.data_ptr(), d_blank[0].data_ptr(),
                                                              d_blank[1].data_ptr(), d_w.data_ptr(), d_b.data_ptr(), ws.data_ptr(), nbytes, scale, b,
-                                                             heads, n, bias.shape[0], k, _DTYPE_CODES[qkv.dtype], _stream(device)),
+                                                             heads, n, bias.shape[1], k, _DTYPE_CODES[qkv.dtype], _stream(device)),
                "clusten_dense_attention_train_backward")
     return d_qkv, d_blank[0], d_blank[1], d_w, d_b
 
@@ -2171,11 +2173,13 @@ def table_linear_grad(d: torch.Tensor, x: torch.Tensor):
     return d_w, d_b
 
 
-def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torch.dtype, scale: float, plan=None, pe_idx=None):
+def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torch.dtype, scale: float, plan=None, pe_idx=None,
+                   table_rows=0):
     """The transformer blocks of a stage one after the other, issued by one call: `params` is a ctypes array of BlockParams
     (what it points at is the caller's to keep), x (B,N,C) the token rows with C = 32 * heads.  Local attention with the
     lists `plan` was built from (`cluster_attention_plan`), or, with `pe_idx` (B,N,N) instead, attention over all N <= 64
-    tokens.  The same kernels as `norm_linear`, `cluster_attention` / `dense_attention` and `block_tail` block by block.  No
+    tokens.  `table_rows`: of bias tables laid out (heads, table_rows), local attention only; 0 when they are (rows, heads).  The same
+    kernels as `norm_linear`, `cluster_attention` / `dense_attention` and `block_tail` block by block.  No
     autograd: for inference."""
     lib = load()
     _require_cuda("x", x)
@@ -2202,10 +2206,10 @@ def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torc
     scratch = torch.empty(b * n * 4 * c, dtype=dtype, device=device)         # q | k, v rows and the attention's output
     with _on(device):
         at = scratch.data_ptr()
-        _check(lib.clusten_blocks_forward(params, len(params), x.data_ptr(), _DTYPE_CODES[x.dtype], out.data_ptr(), at,
-                                          at + b * n * 3 * c * scratch.element_size(), _ptr(plan), int(b != 1 and lb == 1),
-                                          _ptr(pe_idx), AttnShape(b, heads, n, 32, m), hidden, scale, _DTYPE_CODES[dtype],
-                                          _stream(device)), "clusten_blocks_forward")
+        _check(lib.clusten_blocks_forward_tables(params, len(params), x.data_ptr(), _DTYPE_CODES[x.dtype], out.data_ptr(), at,
+                                                 at + b * n * 3 * c * scratch.element_size(), _ptr(plan), int(b != 1 and lb == 1),
+                                                 _ptr(pe_idx), table_rows, AttnShape(b, heads, n, 32, m), hidden, scale,
+                                                 _DTYPE_CODES[dtype], _stream(device)), "clusten_blocks_forward_tables")
     return out
 
 

@@ -2,7 +2,7 @@
 // relative-position table, the gradients of the small Linear layer that makes it, and the global attention of a short sequence
 // (models/aff_transformer.py:108-155 with every token attending to every token) forward and backward.
 //
-// position_bias: bias = table W^T + b for the (rows, k <= 8) table, W and b rounded to the layer's type as autocast rounds them, and
+// position_bias: bias (heads, rows) = W table^T + b for the (rows, k <= 8) table, W and b rounded to the layer's type as autocast rounds them, and
 // the table's rows in that type padded to 8 values, a piece that position_grad gathers.  One launch; the casts and the product were four.
 //
 // position_grad: d_W (heads, k) = sum d_logit[b,h,i,j] table[pe_idx[b,i,j]], d_b = sum d_logit.  The gradient of the bias of every table row
@@ -28,11 +28,11 @@ __global__ __launch_bounds__(256) void position_bias_kernel(const float* __restr
                                                             int heads, int k) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= rows * heads) return;
-    const int row = i / heads, head = i - row * heads;
+    const int head = i / rows, row = i - head * rows;
     float s = 0.f;
     for (int j = 0; j < k; ++j) s += to_acc(from_acc<T>(table[(int64_t)row * k + j])) * to_acc(from_acc<T>(w[head * k + j]));
     if (b) s += to_acc(from_acc<T>(b[head]));
-    bias[i] = from_acc<T>(s);
+    bias[(int64_t)head * rows + row] = from_acc<T>(s);
     if (padded && head == 0) {
         for (int j = 0; j < kTableCols; ++j) padded[(int64_t)row * kTableCols + j] = from_acc<T>(j < k ? table[(int64_t)row * k + j] : 0.f);
     }
@@ -186,7 +186,7 @@ __device__ __forceinline__ void probabilities(const DenseTrain& a, int image, in
     const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
     float s[4][4];
     row_products(q, k, ty, tx, s);
-    const T* bias = static_cast<const T*>(a.bias);
+    const T* bias = static_cast<const T*>(a.bias) + (int64_t)head * a.rows;
     const int64_t* pe = a.pe_idx + (int64_t)image * a.N * a.N;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -194,7 +194,7 @@ __device__ __forceinline__ void probabilities(const DenseTrain& a, int image, in
         for (int j = 0; j < 4; ++j) {
             const int row = 4 * ty + i, col = tx + 16 * j;
             float v = -INFINITY;
-            if (row < a.N && col < a.N) v = s[i][j] * a.scale + to_acc(bias[min((uint64_t)pe[row * a.N + col], (uint64_t)(a.rows - 1)) * a.H + head]);
+            if (row < a.N && col < a.N) v = s[i][j] * a.scale + to_acc(bias[min((uint64_t)pe[row * a.N + col], (uint64_t)(a.rows - 1))]);
             p[row * kSPitch + col] = v;
         }
     }

@@ -207,7 +207,7 @@ int clusten_block_train_forward(const clusten_block_train* args, void* out, clus
         clusten_strides q, kv, rows;
         strides_of(z, q, kv, rows);
         const char* key = kept + k.qkv + (size_t)z.C * z.e;
-        if (int st = launch_cluster_attention(kept + k.qkv, q, key, kv, key + 32 * z.e, kv, nullptr, kept + k.bias, nullptr, nullptr,
+        if (int st = launch_cluster_attention(kept + k.qkv, q, key, kv, key + 32 * z.e, kv, nullptr, table_by_heads(kept + k.bias, z.table_rows), nullptr, nullptr,
                                               a.param[kBlankK], a.param[kBlankV], kept + k.attn, rows, a.attn_scale, a.lists_shared != 0, a.plan,
                                               reinterpret_cast<float*>(kept + k.lse), z.shape, a.dtype, stream)) {
             return st;
@@ -267,7 +267,7 @@ int clusten_block_train_backward(const clusten_block_train* args, const void* d_
         const char* key = query + (size_t)z.C * z.e;
         char* d_key = work + s.d_qkv + (size_t)z.C * z.e;
         if (int st = launch_cluster_attention_backward(query, q, key, kv, key + 32 * z.e, kv, work + s.d_attn, rows, kept + k.attn, rows,
-                                                       reinterpret_cast<const float*>(kept + k.lse), nullptr, kept + k.bias, nullptr, nullptr,
+                                                       reinterpret_cast<const float*>(kept + k.lse), nullptr, table_by_heads(kept + k.bias, z.table_rows), nullptr, nullptr,
                                                        a.param[kBlankK], a.param[kBlankV], work + s.d_qkv, q, work + s.probs, work + s.d_logit,
                                                        reinterpret_cast<float*>(work + s.blank_prob), reinterpret_cast<float*>(work + s.d_blank),
                                                        a.attn_scale, a.lists_shared != 0, a.plan, z.shape, a.dtype, stream)) {

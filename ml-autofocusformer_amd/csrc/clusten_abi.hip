@@ -206,7 +206,7 @@ int clusten_cluster_attention_forward(const void* query, clusten_strides query_s
         !strides_ok(out_strides, shape.C)) {
         return CLUSTEN_ERR_BAD_STRIDE;
     }
-    return launch_cluster_attention(query, query_strides, key, key_strides, value, value_strides, cluster_idx, bias_table,
+    return launch_cluster_attention(query, query_strides, key, key_strides, value, value_strides, cluster_idx, table_by_rows(bias_table, shape.H),
                                     pe_idx, mask, blank_key, blank_value, out, out_strides, scale, lists_shared != 0, nullptr,
                                     nullptr, shape, dtype, as_stream(stream));
 }
@@ -241,7 +241,7 @@ int clusten_cluster_attention_forward_planned(const void* query, clusten_strides
         return CLUSTEN_ERR_BAD_STRIDE;
     }
     if (!aligned16(plan)) return CLUSTEN_ERR_UNALIGNED;
-    return launch_cluster_attention(query, query_strides, key, key_strides, value, value_strides, nullptr, bias_table,
+    return launch_cluster_attention(query, query_strides, key, key_strides, value, value_strides, nullptr, table_by_rows(bias_table, shape.H),
                                     nullptr, nullptr, blank_key, blank_value, out, out_strides, scale, lists_shared != 0, plan,
                                     nullptr, shape, dtype, as_stream(stream));
 }
@@ -262,7 +262,7 @@ int clusten_cluster_attention_forward_train(const void* query, clusten_strides q
         return CLUSTEN_ERR_BAD_STRIDE;
     }
     if (!aligned16(plan)) return CLUSTEN_ERR_UNALIGNED;
-    return launch_cluster_attention(query, query_strides, key, key_strides, value, value_strides, nullptr, bias_table,
+    return launch_cluster_attention(query, query_strides, key, key_strides, value, value_strides, nullptr, table_by_rows(bias_table, shape.H),
                                     nullptr, nullptr, blank_key, blank_value, out, out_strides, scale, lists_shared != 0, plan,
                                     lse, shape, dtype, as_stream(stream));
 }
@@ -287,7 +287,7 @@ int clusten_cluster_attention_backward(const void* query, clusten_strides query_
     }
     if (!aligned16(plan)) return CLUSTEN_ERR_UNALIGNED;
     return launch_cluster_attention_backward(query, query_strides, key, key_strides, value, value_strides, d_out,
-                                             d_out_strides, out, out_strides, lse, nullptr, bias_table, nullptr, nullptr,
+                                             d_out_strides, out, out_strides, lse, nullptr, table_by_rows(bias_table, shape.H), nullptr, nullptr,
                                              blank_key, blank_value, d_query, d_query_strides, probs, d_logit, blank_prob,
                                              d_blank_logit, scale, lists_shared != 0, plan, shape, dtype, as_stream(stream));
 }
@@ -643,6 +643,15 @@ int clusten_block_tail_forward(const void* attn, const void* x, int x_dtype, con
 int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x, int x_dtype, void* out, void* qkv, void* attn,
                            const void* plan, int lists_shared, const int64_t* pe_idx, clusten_attn_shape shape, int hidden,
                            float scale, int dtype, clusten_stream stream) {
+    return clusten_blocks_forward_tables(blocks, count, x, x_dtype, out, qkv, attn, plan, lists_shared, pe_idx, 0, shape, hidden, scale, dtype,
+                                         stream);
+}
+
+int clusten_blocks_forward_tables(const clusten_block* blocks, int count, const void* x, int x_dtype, void* out, void* qkv, void* attn,
+                                  const void* plan, int lists_shared, const int64_t* pe_idx, int table_rows, clusten_attn_shape shape,
+                                  int hidden, float scale, int dtype, clusten_stream stream) {
+    if (table_rows < 0 || (table_rows > 0 && !plan)) return CLUSTEN_ERR_BAD_DIMS;
+    if (plan && !aligned16(plan)) return CLUSTEN_ERR_UNALIGNED;
     if (!blocks || !x || !out || !qkv || !attn || (!plan && !pe_idx)) return CLUSTEN_ERR_NULL_POINTER;
     if (count <= 0) return CLUSTEN_ERR_BAD_DIMS;
     if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
@@ -665,8 +674,11 @@ int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x
                                                  nullptr, rows, C, 3 * C, dtype, stream)) {
             return st;
         }
-        const int st = plan ? clusten_cluster_attention_forward_planned(q, qs, k, kv, v, kv, plan, b.bias_table, lists_shared,
-                                                                        b.blank_k, b.blank_v, attn, os, scale, shape, dtype, stream)
+        if (!b.bias_table || !b.blank_k || !b.blank_v) return CLUSTEN_ERR_NULL_POINTER;
+        const int st = plan ? launch_cluster_attention(q, qs, k, kv, v, kv, nullptr,
+                                                       table_rows ? table_by_heads(b.bias_table, table_rows) : table_by_rows(b.bias_table, shape.H),
+                                                       nullptr, nullptr, b.blank_k, b.blank_v, attn, os, scale, lists_shared != 0, plan, nullptr,
+                                                       shape, dtype, as_stream(stream))
                             : clusten_dense_attention_forward(q, qs, k, kv, v, kv, b.bias_table, pe_idx, b.blank_k, b.blank_v,
                                                               attn, os, scale, shape, dtype, stream);
         if (st) return st;

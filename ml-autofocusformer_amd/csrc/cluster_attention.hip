@@ -38,14 +38,14 @@
 namespace clusten {
 
 int launch_cluster_attention_f32(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
-                                 clusten_strides vs, const int32_t* cluster_idx, const void* table, const int64_t* pe_idx,
+                                 clusten_strides vs, const int32_t* cluster_idx, BiasTable table, const int64_t* pe_idx,
                                  const int64_t* mask, const float* blank_k, const float* blank_v, void* out,
                                  clusten_strides os, float scale, int lists_shared, const void* plan, float* lse,
                                  const clusten_attn_shape& s, hipStream_t stream);   // cluster_attention_f32.hip
 // cluster_attention_resident.hip: short sequences, the K and V rows of an (image, head) resident in LDS
 bool cluster_attention_resident_takes(const clusten_attn_shape& s, int dtype);
 int launch_cluster_attention_resident(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
-                                      clusten_strides vs, const int32_t* cluster_idx, const void* table,
+                                      clusten_strides vs, const int32_t* cluster_idx, BiasTable table,
                                       const int64_t* pe_idx, const int64_t* mask, const float* blank_k,
                                       const float* blank_v, void* out, clusten_strides os, float scale, int lists_shared,
                                       const void* plan, float* lse, const clusten_attn_shape& s, int dtype,
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kWave) void cluster_attention_plan_kernel(const int
 template <typename T, int CS>
 __global__ __launch_bounds__(kWave) void cluster_attention_kernel(
     const T* __restrict__ q, clusten_strides qs, const T* __restrict__ k, clusten_strides ks, const T* __restrict__ v,
-    clusten_strides vs, const int32_t* __restrict__ cluster_idx, const T* __restrict__ table,
+    clusten_strides vs, const int32_t* __restrict__ cluster_idx, BiasTable table,
     const int64_t* __restrict__ pe_idx, const int64_t* __restrict__ mask, const float* __restrict__ blank_k,
     const float* __restrict__ blank_v, T* __restrict__ out, clusten_strides os, int H_all, int N, float scale,
     int tiles_per_batch, int total_tiles, int lists_shared, int head_groups, const char* __restrict__ plan,
@@ -264,11 +264,12 @@ __global__ __launch_bounds__(kWave) void cluster_attention_kernel(
         }
 
         // small per-head operands: their latency passes under the score computation
+        const char* table_h = static_cast<const char*>(table.cells) + (int64_t)(h0 + h) * table.per_head * 2;
         float bias[kRuns];
 #pragma unroll
         for (int r = 0; r < kRuns; ++r) {
-            const uint32_t cell = lane_offset(((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)H_all + (uint32_t)(h0 + h)) * 2);
-            bias[r] = to_acc(*reinterpret_cast<const T*>(reinterpret_cast<const char*>(table) + cell)) +
+            const uint32_t cell = lane_offset((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)table.per_row * 2);
+            bias[r] = to_acc(*reinterpret_cast<const T*>(table_h + cell)) +
                       (pe[r] < 0 ? -100.f : 0.f);
         }
         const float4 bk = *reinterpret_cast<const float4*>(blank_k + (h0 + h) * kC + 4 * i);
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(kWave) void cluster_attention_kernel(
 
 template <typename T, int CS>
 int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
-                 clusten_strides vs, const int32_t* cluster_idx, const void* table, const int64_t* pe_idx,
+                 clusten_strides vs, const int32_t* cluster_idx, BiasTable table, const int64_t* pe_idx,
                  const int64_t* mask, const float* blank_k, const float* blank_v, void* out, clusten_strides os,
                  float scale, int lists_shared, const void* plan, float* lse, const clusten_attn_shape& s,
                  hipStream_t stream) {
@@ -442,7 +443,7 @@ int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strid
     const int groups = attention_head_groups(total, s.H, CS == 24 ? 8192 : 3072);
     hipLaunchKernelGGL((cluster_attention_kernel<T, CS>), dim3(xcd_grid(total * groups)), dim3(kWave), 0, stream,
                        static_cast<const T*>(q), qs, static_cast<const T*>(k), ks, static_cast<const T*>(v), vs,
-                       cluster_idx, static_cast<const T*>(table), pe_idx, mask, blank_k, blank_v, static_cast<T*>(out),
+                       cluster_idx, table, pe_idx, mask, blank_k, blank_v, static_cast<T*>(out),
                        os, s.H, s.N, scale, tiles_per_batch, total, lists_shared, groups, static_cast<const char*>(plan), lse);
     return launch_status();
 }
@@ -474,7 +475,7 @@ int launch_cluster_attention_plan(const int32_t* cluster_idx, const int64_t* pe_
 }
 
 int launch_cluster_attention(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
-                             clusten_strides vs, const int32_t* cluster_idx, const void* table, const int64_t* pe_idx,
+                             clusten_strides vs, const int32_t* cluster_idx, BiasTable table, const int64_t* pe_idx,
                              const int64_t* mask, const float* blank_k, const float* blank_v, void* out,
                              clusten_strides os, float scale, int lists_shared, const void* plan, float* lse,
                              clusten_attn_shape s, int dtype, hipStream_t stream) {

@@ -29,7 +29,7 @@ namespace clusten {
 int launch_cluster_attention_backward_f32(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
                                           clusten_strides vs, const void* d_out, clusten_strides gs, const void* out,
                                           clusten_strides os, const float* lse, const int32_t* cluster_idx,
-                                          const void* table, const int64_t* pe_idx, const int64_t* mask,
+                                          BiasTable table, const int64_t* pe_idx, const int64_t* mask,
                                           const float* blank_k, const float* blank_v, void* d_q, clusten_strides dqs,
                                           void* probs, void* d_logit, float* p_blank, float* ds_blank, float scale,
                                           int lists_shared, const void* plan, const clusten_attn_shape& s,
@@ -70,7 +70,7 @@ template <typename T>
 __global__ __launch_bounds__(kWave) void cluster_attention_bwd_kernel(
     const T* __restrict__ q, clusten_strides qs, const T* __restrict__ k, clusten_strides ks, const T* __restrict__ v,
     clusten_strides vs, const T* __restrict__ d_out, clusten_strides gs, const T* __restrict__ out, clusten_strides os,
-    const float* __restrict__ lse, const int32_t* __restrict__ cluster_idx, const T* __restrict__ table,
+    const float* __restrict__ lse, const int32_t* __restrict__ cluster_idx, BiasTable table,
     const int64_t* __restrict__ pe_idx, const int64_t* __restrict__ mask, const float* __restrict__ blank_k,
     const float* __restrict__ blank_v, T* __restrict__ d_q, clusten_strides dqs, T* __restrict__ probs,
     T* __restrict__ d_logit, float* __restrict__ p_blank, float* __restrict__ ds_blank, int H_all, int N, float scale,
@@ -173,11 +173,12 @@ __global__ __launch_bounds__(kWave) void cluster_attention_bwd_kernel(
         const char* g_lds = stage + G_BASE + (h & 1) * Q_SLOT;
 
         // small per-head operands of the lane's token, requested before the wait for the rows
+        const char* table_h = static_cast<const char*>(table.cells) + (int64_t)(hh) * table.per_head * 2;
         float bias[kR];
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            const uint32_t cell = lane_offset(((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)H_all + (uint32_t)hh) * 2);
-            bias[r] = to_acc(*reinterpret_cast<const T*>(reinterpret_cast<const char*>(table) + cell)) +
+            const uint32_t cell = lane_offset((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)table.per_row * 2);
+            bias[r] = to_acc(*reinterpret_cast<const T*>(table_h + cell)) +
                       (pe[r] < 0 ? -100.f : 0.f);
         }
         const float4 bk = *reinterpret_cast<const float4*>(blank_k + hh * kC + 4 * i);
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(kWave) void cluster_attention_bwd_kernel(
 template <typename T>
 int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v, clusten_strides vs,
                  const void* d_out, clusten_strides gs, const void* out, clusten_strides os, const float* lse,
-                 const int32_t* cluster_idx, const void* table, const int64_t* pe_idx, const int64_t* mask,
+                 const int32_t* cluster_idx, BiasTable table, const int64_t* pe_idx, const int64_t* mask,
                  const float* blank_k, const float* blank_v, void* d_q, clusten_strides dqs, void* probs, void* d_logit,
                  float* p_blank, float* ds_blank, float scale, int lists_shared, const void* plan,
                  const clusten_attn_shape& s, hipStream_t stream) {
@@ -418,7 +419,7 @@ int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strid
     hipLaunchKernelGGL((cluster_attention_bwd_kernel<T>), dim3(xcd_grid(total * groups)), dim3(kWave), 0, stream,
                        static_cast<const T*>(q), qs, static_cast<const T*>(k), ks, static_cast<const T*>(v), vs,
                        static_cast<const T*>(d_out), gs, static_cast<const T*>(out), os, lse, cluster_idx,
-                       static_cast<const T*>(table), pe_idx, mask, blank_k, blank_v, static_cast<T*>(d_q), dqs,
+                       table, pe_idx, mask, blank_k, blank_v, static_cast<T*>(d_q), dqs,
                        static_cast<T*>(probs), static_cast<T*>(d_logit), p_blank, ds_blank, s.H, s.N, scale,
                        tiles_per_batch, total, lists_shared, groups, static_cast<const char*>(plan));
     return launch_status();
@@ -428,7 +429,7 @@ int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strid
 
 int launch_cluster_attention_backward(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
                                       clusten_strides vs, const void* d_out, clusten_strides gs, const void* out,
-                                      clusten_strides os, const float* lse, const int32_t* cluster_idx, const void* table,
+                                      clusten_strides os, const float* lse, const int32_t* cluster_idx, BiasTable table,
                                       const int64_t* pe_idx, const int64_t* mask, const float* blank_k,
                                       const float* blank_v, void* d_q, clusten_strides dqs, void* probs, void* d_logit,
                                       float* p_blank, float* ds_blank, float scale, int lists_shared, const void* plan,

@@ -51,7 +51,7 @@ __global__ __launch_bounds__(kWave) void cluster_attention_bwd_f32_kernel(
     const float* __restrict__ q, clusten_strides qs, const float* __restrict__ k, clusten_strides ks,
     const float* __restrict__ v, clusten_strides vs, const float* __restrict__ d_out, clusten_strides gs,
     const float* __restrict__ out, clusten_strides os, const float* __restrict__ lse,
-    const int32_t* __restrict__ cluster_idx, const float* __restrict__ table, const int64_t* __restrict__ pe_idx,
+    const int32_t* __restrict__ cluster_idx, BiasTable table, const int64_t* __restrict__ pe_idx,
     const int64_t* __restrict__ mask, const float* __restrict__ blank_k, const float* __restrict__ blank_v,
     float* __restrict__ d_q, clusten_strides dqs, float* __restrict__ probs, float* __restrict__ d_logit,
     float* __restrict__ p_blank, float* __restrict__ ds_blank, int H_all, int N, float scale, int tiles_per_batch,
@@ -146,11 +146,12 @@ __global__ __launch_bounds__(kWave) void cluster_attention_bwd_f32_kernel(
         const char* g_lds = stage + G_BASE + (h & 1) * Q_SLOT;
 
         // small per-head operands of the lane's token, requested before the wait for the rows
+        const char* table_h = static_cast<const char*>(table.cells) + (int64_t)(hh) * table.per_head * 4;
         float bias[kR];
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            const uint32_t cell = lane_offset(((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)H_all + (uint32_t)hh) * 4);
-            bias[r] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(table) + cell) + (pe[r] < 0 ? -100.f : 0.f);
+            const uint32_t cell = lane_offset((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)table.per_row * 4);
+            bias[r] = *reinterpret_cast<const float*>(table_h + cell) + (pe[r] < 0 ? -100.f : 0.f);
         }
         const float4 bk = *reinterpret_cast<const float4*>(blank_k + hh * kC + 4 * i);
         const float4 bv4 = *reinterpret_cast<const float4*>(blank_v + hh * kC + 4 * i);
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(kWave) void cluster_attention_bwd_f32_kernel(
 int launch_cluster_attention_backward_f32(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
                                           clusten_strides vs, const void* d_out, clusten_strides gs, const void* out,
                                           clusten_strides os, const float* lse, const int32_t* cluster_idx,
-                                          const void* table, const int64_t* pe_idx, const int64_t* mask,
+                                          BiasTable table, const int64_t* pe_idx, const int64_t* mask,
                                           const float* blank_k, const float* blank_v, void* d_q, clusten_strides dqs,
                                           void* probs, void* d_logit, float* p_blank, float* ds_blank, float scale,
                                           int lists_shared, const void* plan, const clusten_attn_shape& s,
@@ -357,7 +358,7 @@ int launch_cluster_attention_backward_f32(const void* q, clusten_strides qs, con
     hipLaunchKernelGGL(cluster_attention_bwd_f32_kernel, dim3(xcd_grid(total * groups)), dim3(kWave), 0, stream,
                        static_cast<const float*>(q), qs, static_cast<const float*>(k), ks, static_cast<const float*>(v), vs,
                        static_cast<const float*>(d_out), gs, static_cast<const float*>(out), os, lse, cluster_idx,
-                       static_cast<const float*>(table), pe_idx, mask, blank_k, blank_v, static_cast<float*>(d_q), dqs,
+                       table, pe_idx, mask, blank_k, blank_v, static_cast<float*>(d_q), dqs,
                        static_cast<float*>(probs), static_cast<float*>(d_logit), p_blank, ds_blank, s.H, s.N, scale,
                        tiles_per_batch, total, lists_shared, groups, static_cast<const char*>(plan));
     return launch_status();

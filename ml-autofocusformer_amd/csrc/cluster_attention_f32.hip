@@ -47,7 +47,7 @@ static_assert(kTileTokens * fSRow * 4 <= fPassRows * fRB, "the scores fit the K 
 __global__ __launch_bounds__(kWave) void cluster_attention_f32_kernel(
     const float* __restrict__ q, clusten_strides qs, const float* __restrict__ k, clusten_strides ks,
     const float* __restrict__ v, clusten_strides vs, const int32_t* __restrict__ cluster_idx,
-    const float* __restrict__ table, const int64_t* __restrict__ pe_idx, const int64_t* __restrict__ mask,
+    BiasTable table, const int64_t* __restrict__ pe_idx, const int64_t* __restrict__ mask,
     const float* __restrict__ blank_k, const float* __restrict__ blank_v, float* __restrict__ out, clusten_strides os,
     int H_all, int N, float scale, int tiles_per_batch, int total_tiles, int lists_shared, int head_groups,
     const char* __restrict__ plan, float* __restrict__ lse) {
@@ -150,11 +150,12 @@ __global__ __launch_bounds__(kWave) void cluster_attention_f32_kernel(
         }
 
         // small per-head operands: their latency passes under the score computation
+        const char* table_h = static_cast<const char*>(table.cells) + (int64_t)(h0 + h) * table.per_head * 4;
         float bias[kR];
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            const uint32_t cell = lane_offset(((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)H_all + (uint32_t)(h0 + h)) * 4);
-            bias[r] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(table) + cell) + (pe[r] < 0 ? -100.f : 0.f);
+            const uint32_t cell = lane_offset((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)table.per_row * 4);
+            bias[r] = *reinterpret_cast<const float*>(table_h + cell) + (pe[r] < 0 ? -100.f : 0.f);
         }
         const float4 bk = *reinterpret_cast<const float4*>(blank_k + (h0 + h) * kC + 4 * i);
         const float bv[2] = {blank_v[(h0 + h) * kC + r16], blank_v[(h0 + h) * kC + 16 + r16]};
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(kWave) void cluster_attention_f32_kernel(
 }  // namespace
 
 int launch_cluster_attention_f32(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
-                                 clusten_strides vs, const int32_t* cluster_idx, const void* table, const int64_t* pe_idx,
+                                 clusten_strides vs, const int32_t* cluster_idx, BiasTable table, const int64_t* pe_idx,
                                  const int64_t* mask, const float* blank_k, const float* blank_v, void* out,
                                  clusten_strides os, float scale, int lists_shared, const void* plan, float* lse,
                                  const clusten_attn_shape& s, hipStream_t stream) {
@@ -341,7 +342,7 @@ int launch_cluster_attention_f32(const void* q, clusten_strides qs, const void* 
     const int groups = attention_head_groups(total, s.H, 3072);
     hipLaunchKernelGGL(cluster_attention_f32_kernel, dim3(xcd_grid(total * groups)), dim3(kWave), 0, stream,
                        static_cast<const float*>(q), qs, static_cast<const float*>(k), ks, static_cast<const float*>(v), vs,
-                       cluster_idx, static_cast<const float*>(table), pe_idx, mask, blank_k, blank_v,
+                       cluster_idx, table, pe_idx, mask, blank_k, blank_v,
                        static_cast<float*>(out), os, s.H, s.N, scale, tiles_per_batch, total, lists_shared, groups,
                        static_cast<const char*>(plan), lse);
     return launch_status();

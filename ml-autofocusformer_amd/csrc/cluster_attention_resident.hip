@@ -53,7 +53,7 @@ inline int resident_lds_bytes(int N) { return 2 * resident_rows_bytes(N) + kResW
 template <typename T>
 __global__ __launch_bounds__(kResWaves* kWave) void cluster_attention_resident_kernel(
     const T* __restrict__ q, clusten_strides qs, const T* __restrict__ k, clusten_strides ks, const T* __restrict__ v,
-    clusten_strides vs, const int32_t* __restrict__ cluster_idx, const T* __restrict__ table,
+    clusten_strides vs, const int32_t* __restrict__ cluster_idx, BiasTable table,
     const int64_t* __restrict__ pe_idx, const int64_t* __restrict__ mask, const float* __restrict__ blank_k,
     const float* __restrict__ blank_v, T* __restrict__ out, clusten_strides os, int H_all, int N, float scale,
     int tiles_per_batch, int total_units, int lists_shared, const char* __restrict__ plan, float* __restrict__ lse) {
@@ -164,11 +164,12 @@ __global__ __launch_bounds__(kResWaves* kWave) void cluster_attention_resident_k
         }
         const bool twice = __any(repeats) != 0;
         // the bias of the lane's slots, then the next tile's plan and q rows: requested before the wait for this tile's
+        const char* table_h = static_cast<const char*>(table.cells) + (int64_t)(h) * table.per_head * 2;
         float bias[kR];
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-            const uint32_t cell = lane_offset(((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)H_all + (uint32_t)h) * 2);
-            bias[r] = to_acc(*reinterpret_cast<const T*>(reinterpret_cast<const char*>(table) + cell)) +
+            const uint32_t cell = lane_offset((uint32_t)(pe[r] & 0x7fffffff) * (uint32_t)table.per_row * 2);
+            bias[r] = to_acc(*reinterpret_cast<const T*>(table_h + cell)) +
                       (pe[r] < 0 ? -100.f : 0.f);
         }
         if (more) {
@@ -326,7 +327,7 @@ __global__ __launch_bounds__(kResWaves* kWave) void cluster_attention_resident_k
 
 template <typename T>
 int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v, clusten_strides vs,
-                 const int32_t* cluster_idx, const void* table, const int64_t* pe_idx, const int64_t* mask,
+                 const int32_t* cluster_idx, BiasTable table, const int64_t* pe_idx, const int64_t* mask,
                  const float* blank_k, const float* blank_v, void* out, clusten_strides os, float scale, int lists_shared,
                  const void* plan, float* lse, const clusten_attn_shape& s, hipStream_t stream) {
     const int tiles_per_batch = (s.N + kTileTokens - 1) / kTileTokens;
@@ -340,7 +341,7 @@ int launch_typed(const void* q, clusten_strides qs, const void* k, clusten_strid
     }
     hipLaunchKernelGGL((cluster_attention_resident_kernel<T>), dim3(xcd_grid(total)), dim3(kResWaves * kWave), lds, stream,
                        static_cast<const T*>(q), qs, static_cast<const T*>(k), ks, static_cast<const T*>(v), vs,
-                       cluster_idx, static_cast<const T*>(table), pe_idx, mask, blank_k, blank_v, static_cast<T*>(out), os,
+                       cluster_idx, table, pe_idx, mask, blank_k, blank_v, static_cast<T*>(out), os,
                        s.H, s.N, scale, tiles_per_batch, total, lists_shared, static_cast<const char*>(plan), lse);
     return launch_status();
 }
@@ -363,7 +364,7 @@ bool cluster_attention_resident_takes(const clusten_attn_shape& s, int dtype) {
 }
 
 int launch_cluster_attention_resident(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
-                                      clusten_strides vs, const int32_t* cluster_idx, const void* table,
+                                      clusten_strides vs, const int32_t* cluster_idx, BiasTable table,
                                       const int64_t* pe_idx, const int64_t* mask, const float* blank_k,
                                       const float* blank_v, void* out, clusten_strides os, float scale, int lists_shared,
                                       const void* plan, float* lse, const clusten_attn_shape& s, int dtype,

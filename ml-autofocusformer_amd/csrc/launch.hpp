@@ -77,13 +77,23 @@ int launch_attn_softmax(const void* attn, const void* table, const int64_t* pe_i
                         const float* blank, const void* q, clusten_strides qs, const float* blank_k, float* probs,
                         float* blank_prob, clusten_attn_shape s, int dtype, hipStream_t stream);
 
+// Position bias of (row of the relative-position table, head): element row * per_row + head * per_head.  Neighbours of a token are
+// neighbouring rows of the table: by heads, the bias of a run of eight neighbours lies in a line or two, by rows in eight.
+struct BiasTable {
+    const void* cells;
+    int32_t per_row, per_head;
+};
+inline BiasTable table_by_rows(const void* cells, int heads) { return {cells, heads, 1}; }     // (rows, heads)
+inline BiasTable table_by_heads(const void* cells, int rows) { return {cells, 1, rows}; }      // (heads, rows)
+
+
 // Local attention of a cluster-ordered sequence in one kernel (QK, position bias, mask, blank token, softmax, AV,
 // blank value): see cluster_attention.hip.  q, k, v, out : strided (B,H,N,C) of T in {F16, BF16, F32}, C = 32;
 //   cluster_idx (B,N,6) int32; table (rows,H) of T; pe_idx, mask (may be null) : int64 (B,N,M) — or (1,N,.) each
 //   when lists_shared; M = 48 (clusters of 8) or, for 16-bit data, 144 (clusters of 24);
 //   blank_k, blank_v : fp32 (H,C);  lse (may be null): fp32 (B,H,N), the logarithm of each softmax's denominator.
 int launch_cluster_attention(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
-                             clusten_strides vs, const int32_t* cluster_idx, const void* table, const int64_t* pe_idx,
+                             clusten_strides vs, const int32_t* cluster_idx, BiasTable table, const int64_t* pe_idx,
                              const int64_t* mask, const float* blank_k, const float* blank_v, void* out,
                              clusten_strides os, float scale, int lists_shared, const void* plan, float* lse,
                              clusten_attn_shape s, int dtype, hipStream_t stream);
@@ -92,7 +102,7 @@ int launch_cluster_attention(const void* q, clusten_strides qs, const void* k, c
 // cluster_attention_bwd.hip.  d_out, out: strided (B,H,N,C) like q; lse: what the forward wrote.
 int launch_cluster_attention_backward(const void* q, clusten_strides qs, const void* k, clusten_strides ks, const void* v,
                                       clusten_strides vs, const void* d_out, clusten_strides gs, const void* out,
-                                      clusten_strides os, const float* lse, const int32_t* cluster_idx, const void* table,
+                                      clusten_strides os, const float* lse, const int32_t* cluster_idx, BiasTable table,
                                       const int64_t* pe_idx, const int64_t* mask, const float* blank_k,
                                       const float* blank_v, void* d_q, clusten_strides dqs, void* probs, void* d_logit,
                                       float* p_blank, float* ds_blank, float scale, int lists_shared, const void* plan,
@@ -352,7 +362,7 @@ int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void*
                          int M, int rows, int k, int dtype, hipStream_t stream);
 struct DenseTrain {
     const void* qkv;       // (B, N, 3 C): [q | head 0: k v | head 1: k v ...]
-    const void* bias;      // (rows, H)
+    const void* bias;      // (H, rows)
     const void* padded;    // (rows, 8)
     const int64_t* pe_idx; // (B, N, N)
     const float* blank_k;

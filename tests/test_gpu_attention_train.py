@@ -26,9 +26,9 @@ def test_position_bias(device, dt, b, h, n, m, rows, k):
     table, w, bias = (torch.randn(*s, generator=gen, device=device) for s in ((rows, k), (h, k), (h,)))
     t64, w64 = table.to(dt).double(), w.to(dt).double()
     got, padded = _native.position_bias(table, w, bias, dt)
-    near(got, t64 @ w64.t() + bias.to(dt).double(), BAR[dt])
+    near(got, (t64 @ w64.t() + bias.to(dt).double()).t(), BAR[dt])
     assert torch.equal(padded[:, :k], table.to(dt)) and not padded[:, k:].any()
-    near(_native.position_bias(table, w, None, dt)[0], t64 @ w64.t(), BAR[dt])
+    near(_native.position_bias(table, w, None, dt)[0], (t64 @ w64.t()).t(), BAR[dt])
     d = torch.randn(b, h, n, m, generator=gen, device=device).to(dt)
     pe = torch.randint(rows, (b, n, m), generator=gen, device=device)
     d_w, d_b = _native.position_grad(d, pe, padded, k)
@@ -54,7 +54,7 @@ def test_dense_attention(device, dt, b, h, n):
     rows64, bias64, bk64, bv64 = (t.double().requires_grad_(True) for t in (qkv, bias, bk, bv))
     q = rows64[..., :c].view(b, n, h, 32).permute(0, 2, 1, 3)
     kv = rows64[..., c:].view(b, n, h, 2, 32).permute(3, 0, 2, 1, 4)
-    logits = q @ kv[0].transpose(-1, -2) * scale + bias64[pe].permute(0, 3, 1, 2)
+    logits = q @ kv[0].transpose(-1, -2) * scale + bias64.t()[pe].permute(0, 3, 1, 2)
     blank = (q * bk64.view(1, h, 1, 32)).sum(-1, keepdim=True) * scale
     p = torch.softmax(torch.cat([logits, blank], -1), -1)
     ref = (p[..., :-1] @ kv[1] + p[..., -1:] * bv64.view(1, h, 1, 32)).permute(0, 2, 1, 3).reshape(b, n, c)
@@ -68,9 +68,9 @@ def test_dense_attention(device, dt, b, h, n):
     if n > 1:                                                # with one token d_logit of a row is minus that of its blank token
         near(got[1], d_ref[1], 3e-6)
     near(got[2], d_ref[2], 3e-6)
-    d_w, d_b = d_ref[3].t() @ padded[:, :5].double(), d_ref[3].sum(0)
-    size = d_ref[3].abs().sum(0)
-    assert ((got[3].double() - d_w).abs() <= 2e-6 * d_ref[3].abs().t() @ padded[:, :5].double().abs()).all()
+    d_w, d_b = d_ref[3] @ padded[:, :5].double(), d_ref[3].sum(1)
+    size = d_ref[3].abs().sum(1)
+    assert ((got[3].double() - d_w).abs() <= 2e-6 * d_ref[3].abs() @ padded[:, :5].double().abs()).all()
     assert ((got[4].double() - d_b).abs() <= 2e-6 * size).all()
 
 
