@@ -315,7 +315,7 @@ template <typename T, typename S, int C, typename Args>
 int launch_backward_width(const Args& a, hipStream_t stream) {
     // Two tiles at most: four 16-bit ones of 256 channels, or three fp32 ones, do not fit the registers.
     constexpr int MOST = sizeof(T) == 4 && (C == 32 || C == 512) ? 1 : 2;
-    const int tiles = sizeof(T) == 4 ? block_split_f32(MOST, a.rows, 1, false).tiles : block_row_tiles(MOST, a.rows);
+    const int tiles = block_split((int)sizeof(T), C, MOST, a.rows, 1, false).tiles;
     if constexpr (MOST >= 2) {
         if (tiles == 2) return launch_backward_tiles<T, S, C, 2>(a, stream);
     }

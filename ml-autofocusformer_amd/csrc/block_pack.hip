@@ -49,29 +49,24 @@ __global__ __launch_bounds__(256) void block_pack_kernel(PackItems items, int NB
 
 bool block_width_supported(int C) { return C == 32 || C == 64 || C == 128 || C == 256 || C == 512; }
 
-// 16-bit products are bound by the weights every workgroup streams from the L2 (0.9 MB at C = 256, H = 768): as many rows as
-// `most` allows, as long as half of the 256 compute units have a workgroup (tail, us with 4 / 2 / 1 tiles: 25 088 rows of 256
-// channels 44 / 54 / -, 9216 rows of 512 48 / 68 / 76, 6272 rows of 512 60 / 48 / 67, 1003 rows of 256 21 / 15 / 13).
-int block_row_tiles(int most, int64_t rows) {
-    int tiles = most;
-    while (tiles > 1 && (rows + 16 * tiles - 1) / (16 * tiles) < 128) tiles /= 2;
-    return tiles;
-}
-
-// fp32 weights are twice the bytes and are split next to the products: a workgroup's time is some w for the weights of a chunk of C
-// outputs and m a row tile for its products, w : m = 5 : 3 (784 rows of 256 channels: tail 33 / 44 / 57 us with 1 / 2 / 3 tiles,
-// norm_linear 16 / 20 / 24 / 30 with 1 .. 4), and a round of 256 workgroups, one a compute unit, takes as long as one.  What gives
-// the fewest rounds' time is taken.  Tail, us with 1 / 2 / 3 tiles: 9800 rows of 256 channels 99 / 93 / 61, 3136 rows 34 / 44 / 57;
-// norm_linear at 9800 rows 41 / 39 / 28 / 33 unsplit, 45 / 38 / 39 / 33 in three; 3136 rows 17 / 21 / 25 / 30 and 19 / 19 / 14 / 16;
-// 2450 rows of 512 50 / 64 / 88 and 42 / 30 / 39.
-BlockSplit block_split_f32(int most, int64_t rows, int chunks, bool may_split) {
+// A workgroup's time is some w for a chunk of C outputs, whose weights every workgroup streams from the L2, m for its products of each
+// row tile and n for what lies ahead of the chunks; the compute unit with the most workgroups decides, and with weights on their
+// way and products going on in all of them at once it takes as long as they do one by one.  What gives the least is taken.
+// w : m : n = 5 : 3 : 5 in fp32 (784 rows of 256 channels: tail 33 / 44 / 57 us with 1 / 2 / 3 tiles, norm_linear 16 / 20 / 24 / 30 with
+// 1 .. 4), 5 : 3 : 8 in 16 bits, 9 : 2 : 12 with 512 channels (49 rows: tail 34 / 40 / 46 / 54, norm_linear 16 / 19 / 21 / 23).
+// fp32, us with 1 / 2 / 3 tiles: tail 9800 rows of 256 channels 99 / 93 / 61, 3136 rows 34 / 44 / 57; norm_linear 9800 rows 41 / 39 / 28 / 33
+// unsplit, 45 / 38 / 39 / 33 in three, 2450 rows of 512 50 / 64 and 42 / 30.
+// fp16, us with 1 / 2 / 3 / 4 tiles: tail 25 088 rows of 256 channels 68 / 54 / 56 / 44, 36 864 89 / 65 / 60 / 70, 9216 of 512 105 / 94 / 55 / 64,
+// 6272 66 / 47 / 52 / 61; norm_linear 9216 rows of 512 47 / 38 / 27 / 31 unsplit, 44 / 32 / 36 / 30 in three, 49 rows 16 and 10.
+BlockSplit block_split(int elem_size, int C, int most, int64_t rows, int chunks, bool may_split) {
+    const bool wide = elem_size == 2 && C == 512;
+    const int w = wide ? 9 : 5, m = wide ? 2 : 3, n = wide ? 12 : elem_size == 2 ? 8 : 5;
     BlockSplit best = {1, 1};
     int64_t cost = 0;
     for (int tiles = 1; tiles <= most; ++tiles) {
         const int64_t groups = (rows + 16 * tiles - 1) / (16 * tiles);
         for (int split = 1; split <= (may_split && groups <= 256 ? chunks : 1); ++split) {
-            // the norm ahead of the products is about as long as the weights of a chunk
-            const int64_t here = (groups * split + 255) / 256 * ((chunks + split - 1) / split * (5 + 3 * tiles) + 5);
+            const int64_t here = (groups * split + 255) / 256 * ((chunks + split - 1) / split * (w + m * tiles) + (may_split ? n : 0));
             if (cost == 0 || here < cost) cost = here, best = {tiles, split};
         }
     }

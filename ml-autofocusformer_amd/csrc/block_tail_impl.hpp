@@ -182,11 +182,11 @@ int launch_block_tail_width(const BlockTailArgs& a, hipStream_t stream) {
     // fp32 with three bf16 parts a value, against fp32 instructions: 9800 rows of 256 channels 111 -> 68 us, 39 200 of 128 115 -> 74,
     // 156 800 of 64 110 -> 86, 2450 of 512 136 -> 118, bound by the weights from the L2 (20 us of the 68) and the products (40).
     constexpr int MOST = sizeof(T) == 4 ? (C == 256 ? 3 : C == 64 || C == 128 ? 2 : 1) : (C > 128 ? 4 : 2);
-    const int tiles = sizeof(T) == 4 ? block_split_f32(MOST, a.rows, 1, false).tiles : block_row_tiles(MOST, a.rows);
+    const int tiles = block_split((int)sizeof(T), C, MOST, a.rows, 1, false).tiles;
     if constexpr (MOST >= 4) {
         if (tiles == 4) return launch_block_tail_tiles<T, S, C, 4>(a, stream);
     }
-    if constexpr (MOST >= 3 && sizeof(T) == 4) {
+    if constexpr (MOST >= 3) {
         if (tiles == 3) return launch_block_tail_tiles<T, S, C, 3>(a, stream);
     }
     if constexpr (MOST >= 2) {

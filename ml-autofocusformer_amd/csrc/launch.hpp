@@ -296,13 +296,11 @@ struct BlockTailArgs {
     float2* stats;         // (rows)
 };
 bool block_width_supported(int C);
-// Tiles of 16 rows a workgroup takes (4, 2 or 1, at most `most`): 16-bit products.
-int block_row_tiles(int most, int64_t rows);
-// The same for fp32 products (1 .. most), and over how many workgroups the chunks of C outputs are shared.
+// Tiles of 16 rows a workgroup takes (1 .. most), and, when they may be shared, over how many workgroups the chunks of C outputs are.
 struct BlockSplit {
     int tiles, split;
 };
-BlockSplit block_split_f32(int most, int64_t rows, int chunks, bool may_split);
+BlockSplit block_split(int elem_size, int C, int most, int64_t rows, int chunks, bool may_split);
 // dst = a weight matrix of fp32 in the order the block kernels of width C read it in, as dtype.  src is (n,k), or (k,n)
 //   when transposed (dst is then that of its transpose); n and k multiples of C.
 int launch_block_pack(const clusten_pack_item* items, int count, int C, int dtype, hipStream_t stream);

@@ -87,19 +87,11 @@ int launch_norm_linear_width(const NormLinearArgs& a, hipStream_t stream) {
     // Up to 64 channels two fp32 tiles (25 088 rows of 64: 11 us, 13 with four).  fp32 with three bf16 parts a value, against fp32
     // instructions: 9800 rows of 256 channels 51 -> 34 us, 39 200 of 128 48 -> 35, 156 800 of 64 58 -> 38, 2450 of 512 45 -> 31.
     constexpr int MOST = sizeof(T) == 4 ? (C > 256 || C <= 64 ? 2 : 4) : 4;
-    BlockSplit cut;
-    if constexpr (sizeof(T) == 4) {
-        cut = block_split_f32(MOST, a.rows, a.chunks, true);
-    } else {
-        // Few workgroups share the output chunks among them, each normalising its rows again: 17 -> 7 us for the 49 rows of 512
-        // channels of one image, 29 -> 27 us at 9216 rows of 512; at 25 088 rows of 256 (392 workgroups) 21.7 -> 23.5.
-        cut.tiles = block_row_tiles(MOST, a.rows);
-        cut.split = (a.rows + 16 * cut.tiles - 1) / (16 * cut.tiles) < 256 ? a.chunks : 1;
-    }
+    const BlockSplit cut = block_split((int)sizeof(T), C, MOST, a.rows, a.chunks, true);
     if constexpr (MOST >= 4) {
         if (cut.tiles == 4) return launch_norm_linear_tiles<T, S, C, 4>(a, cut.split, stream);
     }
-    if constexpr (MOST >= 3 && sizeof(T) == 4) {
+    if constexpr (MOST >= 3) {
         if (cut.tiles == 3) return launch_norm_linear_tiles<T, S, C, 3>(a, cut.split, stream);
     }
     if (cut.tiles == 2) return launch_norm_linear_tiles<T, S, C, 2>(a, cut.split, stream);

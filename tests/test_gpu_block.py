@@ -16,11 +16,12 @@ from oracle import clusten_oracle as oracle
 pytestmark = pytest.mark.gpu
 
 BAR = {torch.float16: 2e-3, torch.bfloat16: 1e-2, torch.float32: 1e-5}
-# fp32 and 16-bit token streams; row counts below a tile, across tiles, and enough for 2 and 4 tiles a workgroup
+# fp32 and 16-bit token streams; row counts below a tile, across tiles, and enough for 2, 3 and 4 tiles a workgroup
 CASES = [(torch.float16, torch.float16), (torch.float16, torch.float32), (torch.bfloat16, torch.bfloat16),
          (torch.float32, torch.float32)]
 SHAPES = [(32, 64, 1), (32, 96, 70), (64, 192, 16), (64, 128, 16 * 1024 + 3), (128, 384, 33), (128, 128, 8192 + 17),
-          (256, 768, 49), (256, 512, 16 * 1024 + 1), (512, 1536, 15), (512, 1024, 8192 - 5)]
+          (256, 768, 49), (256, 512, 16 * 1024 + 1), (512, 1536, 15), (512, 1024, 8192 - 5), (512, 512, 4096 + 1),
+          (512, 512, 9217), (256, 256, 33 * 1024 + 7)]
 
 
 class Block:
