@@ -236,7 +236,7 @@ __global__ __launch_bounds__(kThreads, 2) void weight_grad_kernel(GradArgs a) {
     }
 }
 
-// dst[i] = the sum of src[s * stride + i] over the splits, in a fixed order: 16 float4 columns per workgroup, 16 threads each.
+// dst[i] = the sum of src[s * stride + i] over the splits, in a fixed order: 256 / GROUPS float4 columns per workgroup, GROUPS threads each.
 struct Segment {
     float* dst;
     int64_t at, count;         // floats, multiples of 4
@@ -247,27 +247,40 @@ struct SumArgs {
     int64_t stride;
     int segments, splits;
 };
-constexpr int kSumColumns = 16;
 
+template <int GROUPS>
 __global__ __launch_bounds__(kThreads) void sum_splits_kernel(SumArgs a) {
-    __shared__ F32x4 part[kThreads];
-    const int col = threadIdx.x % kSumColumns, group = threadIdx.x / kSumColumns;
-    int64_t at = ((int64_t)blockIdx.x * kSumColumns + col) * 4;
+    constexpr int COLUMNS = kThreads / GROUPS;
+    const int col = threadIdx.x % COLUMNS, group = threadIdx.x / COLUMNS;
+    int64_t at = ((int64_t)blockIdx.x * COLUMNS + col) * 4;
     int which = 0;
     while (which < a.segments && at >= a.segment[which].count) at -= a.segment[which++].count;
     F32x4 v = F32x4{0.f, 0.f, 0.f, 0.f};
     if (which < a.segments) {
         const float* src = a.src + a.segment[which].at + at;
-#pragma unroll 4
-        for (int s = group; s < a.splits; s += kThreads / kSumColumns) v += *reinterpret_cast<const F32x4*>(src + s * a.stride);
+#pragma unroll 8
+        for (int s = group; s < a.splits; s += GROUPS) v += *reinterpret_cast<const F32x4*>(src + s * a.stride);
     }
-    part[threadIdx.x] = v;
-    __syncthreads();
-    if (group == 0 && which < a.segments) {
+    if constexpr (GROUPS > 1) {
+        __shared__ F32x4 part[kThreads];
+        part[threadIdx.x] = v;
+        __syncthreads();
+        if (group == 0) {
 #pragma unroll
-        for (int g = 1; g < kThreads / kSumColumns; ++g) v += part[g * kSumColumns + col];
-        *reinterpret_cast<F32x4*>(a.segment[which].dst + at) = v;
+            for (int g = 1; g < GROUPS; ++g) v += part[g * COLUMNS + col];
+        }
     }
+    if (group == 0 && which < a.segments) *reinterpret_cast<F32x4*>(a.segment[which].dst + at) = v;
+}
+
+// Threads of a column: as many as leave each about a dozen splits, eight of which it requests together.  With 16 for any number of
+// splits, the two of a block of 512 channels (12.6 MB each; 64 images of 49 tokens) left 14 of 16 threads without one: 44.2 -> 8.8 us; ten of
+// 256 channels 14.1 -> 7.1 us.  Where there are more, the 42 of 128 channels take 9.2 us with four threads (9.1 with 16).
+void launch_sum_splits(const SumArgs& a, int64_t columns, hipStream_t stream) {
+    auto grid = [&](int per) { return dim3((unsigned)((columns + per - 1) / per)); };
+    if (a.splits <= 12) hipLaunchKernelGGL((sum_splits_kernel<1>), grid(kThreads), dim3(kThreads), 0, stream, a);
+    else if (a.splits <= 48) hipLaunchKernelGGL((sum_splits_kernel<4>), grid(kThreads / 4), dim3(kThreads), 0, stream, a);
+    else hipLaunchKernelGGL((sum_splits_kernel<16>), grid(kThreads / 16), dim3(kThreads), 0, stream, a);
 }
 
 struct Split {
@@ -334,8 +347,7 @@ int launch_weight_grad(const clusten_weight_grad_item* items, int count, int64_t
     else if (dtype == CLUSTEN_BF16) launch_tiles<bf16_t>(g, s.tile, stream);
     else launch_tiles<float>(g, s.tile, stream);
     if (int st = launch_status()) return st;
-    const int64_t columns = s.per_split / 4;
-    hipLaunchKernelGGL(sum_splits_kernel, dim3((unsigned)((columns + kSumColumns - 1) / kSumColumns)), dim3(kThreads), 0, stream, sum);
+    launch_sum_splits(sum, s.per_split / 4, stream);
     return launch_status();
 }
 

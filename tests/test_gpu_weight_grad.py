@@ -42,6 +42,18 @@ def test_weight_grad_against_float64(dtype, rows):
         assert all(torch.equal(a[0], b[0]) for a, b in zip(again, first))
 
 
+# ranges of 512 rows: 1 to 12 of them are added up by one thread, 13 to 48 by four, more by sixteen
+@pytest.mark.parametrize("splits", [1, 12, 13, 48, 49, 65])
+def test_sums_of_the_splits(splits):
+    nat = _native()
+    gen = torch.Generator(device="cuda").manual_seed(splits)
+    d_y, x = (torch.randn(512 * splits, 64, generator=gen, device="cuda").half() for _ in range(2))
+    (d_w, d_b), = nat.weight_grad([(d_y, x, True)])
+    assert bool(((d_w.double() - d_y.double().t() @ x.double()).abs() <= _bound(d_y, x)).all())
+    one = torch.ones(512 * splits, 1, device="cuda").half()
+    assert bool(((d_b.double() - d_y.double().sum(0)).abs() <= _bound(d_y, one)[:, 0]).all())
+
+
 def test_an_infinity_stays_in_its_row_and_column():
     nat = _native()
     d_y, x = torch.ones(130, 64, device="cuda").half(), torch.ones(130, 64, device="cuda").half()
