@@ -6,7 +6,7 @@
 // the table's rows in that type padded to 8 values, a piece that position_grad gathers.  One launch; the casts and the product were four.
 //
 // position_grad: d_W (heads, k) = sum d_logit[b,h,i,j] table[pe_idx[b,i,j]], d_b = sum d_logit.  The gradient of the bias of every table row
-// need not be formed (a scatter into 12 000 rows, then a product over them: 23 + 20 us a layer of AFF-Tiny at 64 images, now 25 + 5): a
+// need not be formed (a scatter into 12 000 rows, then a product over them: 23 + 20 us a layer of AFF-Tiny at 64 images, now 14 + 5): a
 // value meets its row of the table directly.  Every lane sums in double, so that nothing is lost where positive and negative values cancel;
 // partial sums are added in a fixed order.
 //
@@ -53,6 +53,8 @@ __device__ __forceinline__ void table_row(const T* __restrict__ padded, int64_t 
 constexpr int kGradHeads = 4;      // heads a workgroup of position_grad sums for
 constexpr int kGradSums = 6;       // of a head: five columns and the bias
 
+// Bound by the trips to memory of an index and its table row, and in a small launch by the exchanges at the end.  Mean of a layer of AFF-Tiny at 64
+// images: 24.2 -> 14.0 us with the next indices requested ahead, fewer exchanges and four workgroups a compute unit instead of two.
 // Workgroup (x, y): values x, x + gridDim.x, ... (in 256 quads) of heads 4 y ..; partial: (gridDim.x, heads, 6) doubles.
 template <typename T>
 __global__ __launch_bounds__(256) void position_grad_kernel(const T* __restrict__ d_logit, const int64_t* __restrict__ pe_idx,
@@ -61,15 +63,17 @@ __global__ __launch_bounds__(256) void position_grad_kernel(const T* __restrict_
     __shared__ double sums[4][kGradHeads * kGradSums];
     const int h0 = blockIdx.y * kGradHeads, here = min(kGradHeads, heads - h0);
     double acc[kGradHeads][kGradSums] = {};
-    for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < total / 4; q += (int64_t)gridDim.x * 256) {
-        const int64_t at = q * 4, image = at / per_image, place = at - image * per_image;
-        const int64_t* idx = pe_idx + at;
-        int64_t row[4];
+    const int64_t quads = total / 4, step = (int64_t)gridDim.x * 256;
+    int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x, row[4];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) row[e] = idx[e];
+    for (int e = 0; e < 4; ++e) row[e] = pe_idx[min(q, quads - 1) * 4 + e];
+    for (; q < quads; q += step) {
+        const int64_t at = q * 4, image = at / per_image, place = at - image * per_image;
         float t[4][kTableCols];
 #pragma unroll
         for (int e = 0; e < 4; ++e) table_row(padded, min((uint64_t)row[e], (uint64_t)(rows - 1)), t[e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) row[e] = pe_idx[min(q + step, quads - 1) * 4 + e];      // the next quad's, while this one's rows travel
 #pragma unroll
         for (int h = 0; h < kGradHeads; ++h) {
             if (h < here) {
@@ -84,16 +88,23 @@ __global__ __launch_bounds__(256) void position_grad_kernel(const T* __restrict_
             }
         }
     }
+    // sums over the wave: at each exchange a lane keeps half of its values and gives the other half away, value i ends in lanes 2 i and 2 i + 1
+    // (32 exchanges of a double; 144 when every lane keeps all 24, which took longer than the values of a deep layer)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double v[32];
 #pragma unroll
-    for (int h = 0; h < kGradHeads; ++h) {
+    for (int j = 0; j < 32; ++j) v[j] = j < kGradHeads * kGradSums ? acc[j / kGradSums % kGradHeads][j % kGradSums] : 0.;
 #pragma unroll
-        for (int j = 0; j < kGradSums; ++j) {
-            double s = acc[h][j];
-            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-            if (lane == 0) sums[wave][h * kGradSums + j] = s;
+    for (int half = 16; half > 0; half >>= 1) {
+        const bool upper = (lane & 2 * half) != 0;
+#pragma unroll
+        for (int j = 0; j < half; ++j) {
+            const double kept = upper ? v[j + half] : v[j], given = upper ? v[j] : v[j + half];
+            v[j] = kept + __shfl_xor(given, 2 * half);
         }
     }
+    v[0] += __shfl_xor(v[0], 1);
+    if ((lane & 1) == 0 && lane / 2 < kGradHeads * kGradSums) sums[wave][lane / 2] = v[0];
     __syncthreads();
     if ((int)threadIdx.x < here * kGradSums) {
         double s = 0.;
@@ -369,7 +380,9 @@ __global__ __launch_bounds__(256) void dense_sums_kernel(const float* __restrict
     }
 }
 
-int position_groups(int64_t total) { return (int)min((total / 4 + 255) / 256, (int64_t)512); }
+// Workgroups of position_grad: four fit a compute unit, and a thread takes at least two quads of values, else its last exchanges are the
+// larger part.
+int position_groups(int64_t total) { return (int)max((int64_t)1, min((total / 4 + 511) / 512, (int64_t)1024)); }
 
 template <typename F>
 int on_type(int dtype, F&& f) {

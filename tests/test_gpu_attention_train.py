@@ -37,6 +37,21 @@ def test_position_bias(device, dt, b, h, n, m, rows, k):
     assert ((d_b.double() - d.double().sum((0, 2, 3))).abs() <= 1e-6 * d.double().abs().sum((0, 2, 3)) / (b * n * m) ** 0.5).all()
 
 
+# one workgroup, two, the most and the most with values to spare; whole and partial groups of four heads
+@pytest.mark.parametrize("b,h,n,m", [(1, 1, 128, 16), (1, 4, 129, 16), (2, 7, 21845, 48), (2, 5, 21900, 48)])
+def test_position_gradient_workgroups(device, b, h, n, m):
+    gen = torch.Generator(device).manual_seed(n)
+    table = torch.randn(225, 5, generator=gen, device=device)
+    _, padded = _native.position_bias(table, torch.randn(h, 5, device=device), None, torch.float16)
+    d = torch.randn(b, h, n, m, generator=gen, device=device).half()
+    pe = torch.randint(225, (b, n, m), generator=gen, device=device)
+    d_w, d_b = _native.position_grad(d, pe, padded, 5)
+    for head in range(h):
+        terms = d[:, head].double().unsqueeze(-1) * padded.double()[pe][..., :5]
+        assert ((d_w[head].double() - terms.sum((0, 1, 2))).abs() <= 1e-6 * terms.abs().sum((0, 1, 2)) / (b * n * m) ** 0.5).all()
+        assert (d_b[head].double() - d[:, head].double().sum()).abs() <= 1e-6 * d[:, head].double().abs().sum() / (b * n * m) ** 0.5
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("b,h,n", [(1, 1, 1), (3, 2, 7), (2, 16, 49), (5, 3, 64), (1, 4, 63)])
 def test_dense_attention(device, dt, b, h, n):
