@@ -113,25 +113,6 @@ __global__ __launch_bounds__(256) void position_grad_kernel(const T* __restrict_
     }
 }
 
-// One wave a head.
-__global__ __launch_bounds__(64) void position_sums_kernel(const double* __restrict__ partial, int groups, int heads, int k,
-                                                           float* __restrict__ d_w, float* __restrict__ d_b) {
-    const int head = blockIdx.x;
-    double s[kGradSums] = {};
-    for (int g = threadIdx.x; g < groups; g += 64) {
-#pragma unroll
-        for (int j = 0; j < kGradSums; ++j) s[j] += partial[((int64_t)g * heads + head) * kGradSums + j];
-    }
-#pragma unroll
-    for (int j = 0; j < kGradSums; ++j) {
-        for (int o = 32; o > 0; o >>= 1) s[j] += __shfl_xor(s[j], o);
-    }
-    if (threadIdx.x == 0) {
-        for (int j = 0; j < k; ++j) d_w[head * k + j] = (float)s[j];
-        d_b[head] = (float)s[kGradSums - 1];
-    }
-}
-
 // ---- global attention of up to 64 tokens ----------------------------------------------------------------------------------
 
 constexpr int kTokens = 64, kCh = 32, kPitch = kCh + 4, kSPitch = kTokens + 4;     // pitches in floats: 16-byte rows, spread over the banks
@@ -408,8 +389,8 @@ int launch_position_bias(const float* table, const float* w, const float* b, voi
 
 size_t position_grad_workspace_bytes(int64_t total, int heads) { return (size_t)position_groups(total) * heads * kGradSums * sizeof(double); }
 
-int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void* padded, float* d_w, float* d_b, void* workspace, int B, int H, int N,
-                         int M, int rows, int k, int dtype, hipStream_t stream) {
+int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void* padded, float* d_w, float* d_b, void* workspace, GradSums* later, int B,
+                         int H, int N, int M, int rows, int k, int dtype, hipStream_t stream) {
     const int64_t per_image = (int64_t)N * M, total = B * per_image;
     const int groups = position_groups(total);
     double* partial = static_cast<double*>(workspace);
@@ -418,9 +399,7 @@ int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void*
         hipLaunchKernelGGL((position_grad_kernel<T>), dim3(groups, (H + kGradHeads - 1) / kGradHeads), dim3(256), 0, stream,
                            static_cast<const T*>(d_logit), pe_idx, static_cast<const T*>(padded), partial, H, per_image, total, rows);
     });
-    if (st) return st;
-    hipLaunchKernelGGL(position_sums_kernel, dim3(H), dim3(64), 0, stream, partial, groups, H, k, d_w, d_b);
-    return launch_status();
+    return st ? st : add_up(PositionSums{partial, d_w, d_b, groups, H, k}, later, stream);
 }
 
 size_t dense_train_workspace_bytes(int B, int H) { return (size_t)B * H * kDenseSums * sizeof(float); }

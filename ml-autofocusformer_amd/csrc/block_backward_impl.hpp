@@ -308,7 +308,7 @@ int launch_backward_tiles(const Args& a, hipStream_t stream) {
         hipLaunchKernelGGL((norm_linear_backward_kernel<T, S, C, TR>), dim3(groups), threads, 0, stream, a);
     }
     if (int st = launch_status()) return st;
-    return launch_column_sums(a.partial, (int)groups, C, 1.f, a.d_norm_w, a.d_norm_b, stream);
+    return add_up(ColumnSums{a.partial, a.d_norm_w, a.d_norm_b, 1.f, (int)groups, C}, a.later, stream);
 }
 
 template <typename T, typename S, int C, typename Args>

@@ -67,8 +67,8 @@ size_t packed_at(const Sizes& z, int i) {
 }
 
 struct Scratch {
-    size_t d_x1, branch, d_f, g, d_h, d_attn, d_qkv, probs, d_logit, blank_prob, d_blank, sums, weights, bytes;
-    size_t sums_bytes, weights_bytes;
+    size_t d_x1, branch, d_f, g, d_h, d_attn, d_qkv, probs, d_logit, blank_prob, d_blank, sums_tail, sums_blank, sums_attn, sums_head, weights, bytes;
+    size_t weights_bytes;
 };
 Scratch scratch_layout(const clusten_block_train& a, const Sizes& z, const clusten_weight_grad_item* items, int count) {
     Layout l;
@@ -86,11 +86,11 @@ Scratch scratch_layout(const clusten_block_train& a, const Sizes& z, const clust
     s.d_logit = l.take(pairs * z.e);
     s.blank_prob = l.take(z.local ? (size_t)z.rows * z.heads * 4 : 0);
     s.d_blank = l.take(z.local ? (size_t)z.rows * z.heads * 4 : 0);
-    // partial sums of one kernel at a time
-    s.sums_bytes = std::max(block_backward_workspace_bytes(z.rows, z.C), row_sums_workspace_bytes(z.rows, z.C));
-    s.sums_bytes = std::max(s.sums_bytes, z.local ? position_grad_workspace_bytes((int64_t)z.rows * z.shape.M, z.heads)
-                                                  : dense_train_workspace_bytes(z.shape.B, z.heads));
-    s.sums = l.take(s.sums_bytes);
+    // partial sums, all of them added up at the end
+    s.sums_tail = l.take(block_backward_workspace_bytes(z.rows, z.C));
+    s.sums_blank = l.take(z.local ? row_sums_workspace_bytes(z.rows, z.C) : 0);
+    s.sums_attn = l.take(z.local ? position_grad_workspace_bytes((int64_t)z.rows * z.shape.M, z.heads) : dense_train_workspace_bytes(z.shape.B, z.heads));
+    s.sums_head = l.take(block_backward_workspace_bytes(z.rows, z.C));
     s.weights_bytes = count ? weight_grad_workspace_bytes(items, count, z.rows, a.dtype) : 0;
     s.weights = l.take(s.weights_bytes);
     s.bytes = l.bytes;
@@ -249,14 +249,15 @@ int clusten_block_train_backward(const clusten_block_train* args, const void* d_
     if (workspace_bytes < s.bytes) return CLUSTEN_ERR_WORKSPACE;
     const bool separate = a.factors != nullptr || a.x_dtype != a.dtype;
     const char* packed_t = kept + k.packed + packed_at(z, 5) * z.e;
-    float* sums = reinterpret_cast<float*>(work + s.sums);
+    GradSums sums = {};
+    auto partial = [&](size_t at) { return reinterpret_cast<float*>(work + at); };
 
     BlockTailGrad tail = {};
     tail.d_out = d_out, tail.x1 = kept + k.x1, tail.stats = reinterpret_cast<const float2*>(kept + k.stats2), tail.norm_w = a.param[kNorm2W];
     tail.hidden = kept + k.hidden, tail.wp = packed_t + packed_at(z, 2) * z.e, tail.w1 = packed_t + packed_at(z, 3) * z.e;
     tail.w2 = packed_t + packed_at(z, 4) * z.e, tail.scale = a.factors, tail.d_x = work + s.d_x1, tail.branch = separate ? work + s.branch : nullptr;
     tail.d_f = separate ? work + s.d_f : nullptr, tail.g = work + s.g, tail.d_h = work + s.d_h, tail.d_attn = work + s.d_attn;
-    tail.d_norm_w = a.grad[kNorm2W], tail.d_norm_b = a.grad[kNorm2B], tail.partial = sums, tail.rows = z.rows;
+    tail.d_norm_w = a.grad[kNorm2W], tail.d_norm_b = a.grad[kNorm2B], tail.partial = partial(s.sums_tail), tail.later = &sums, tail.rows = z.rows;
     tail.rows_per_image = a.factors ? a.shape.N : 1, tail.chunks = z.H / z.C;
     if (int st = launch_block_tail_backward(tail, a.x_dtype, z.C, a.dtype, stream)) return st;
 
@@ -278,25 +279,26 @@ int clusten_block_train_backward(const clusten_block_train* args, const void* d_
             return st;
         }
         if (int st = launch_blank_grad(query, 3 * z.C, work + s.d_attn, reinterpret_cast<const float*>(work + s.d_blank),
-                                       reinterpret_cast<const float*>(work + s.blank_prob), a.attn_scale, a.grad[kBlankK], a.grad[kBlankV], sums,
-                                       z.shape.B, z.heads, z.shape.N, z.C, a.dtype, stream)) {
+                                       reinterpret_cast<const float*>(work + s.blank_prob), a.attn_scale, a.grad[kBlankK], a.grad[kBlankV],
+                                       partial(s.sums_blank), &sums, z.shape.B, z.heads, z.shape.N, z.C, a.dtype, stream)) {
             return st;
         }
-        if (int st = launch_position_grad(work + s.d_logit, a.pe_idx, kept + k.padded, a.grad[kPeW], a.grad[kPeB], sums, z.shape.B, z.heads,
-                                          z.shape.N, z.shape.M, z.table_rows, a.table_cols, a.dtype, stream)) {
+        if (int st = launch_position_grad(work + s.d_logit, a.pe_idx, kept + k.padded, a.grad[kPeW], a.grad[kPeB], work + s.sums_attn,
+                                          &sums, z.shape.B, z.heads, z.shape.N, z.shape.M, z.table_rows, a.table_cols, a.dtype, stream)) {
             return st;
         }
     } else {
         DenseTrain d = dense_args(a, z, kept, k);
-        d.d_out = work + s.d_attn, d.d_qkv = work + s.d_qkv, d.partial = sums;
+        d.d_out = work + s.d_attn, d.d_qkv = work + s.d_qkv, d.partial = partial(s.sums_attn);
         if (int st = launch_dense_train_backward(d, a.grad[kBlankK], a.grad[kBlankV], a.grad[kPeW], a.grad[kPeB], a.dtype, stream)) return st;
     }
 
     NormLinearGrad head = {};
     head.d_y = work + s.d_qkv, head.x = a.x, head.stats = reinterpret_cast<const float2*>(kept + k.stats1), head.norm_w = a.param[kNorm1W];
     head.w0 = packed_t, head.w1 = packed_t + packed_at(z, 1) * z.e, head.d_res = work + s.d_x1, head.d_x = d_x, head.d_norm_w = a.grad[kNorm1W];
-    head.d_norm_b = a.grad[kNorm1B], head.partial = sums, head.rows = z.rows, head.chunks = 3;
+    head.d_norm_b = a.grad[kNorm1B], head.partial = partial(s.sums_head), head.later = &sums, head.rows = z.rows, head.chunks = 3;
     if (int st = launch_norm_linear_backward(head, a.x_dtype, z.C, a.dtype, stream)) return st;
+    if (int st = launch_grad_sums(sums, stream)) return st;
 
     const char* branch = separate ? work + s.branch : work + s.d_x1;
     const char* d_f = separate ? work + s.d_f : static_cast<const char*>(d_out);

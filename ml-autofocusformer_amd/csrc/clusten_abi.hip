@@ -780,8 +780,8 @@ int clusten_blank_grad(const void* q, int q_stride, const void* d_out, const flo
     if (need == 0) return CLUSTEN_ERR_BAD_DIMS;
     if (workspace_bytes < need) return CLUSTEN_ERR_TOO_LARGE;
     if (!aligned16(q) || !aligned16(d_out) || !aligned16(workspace)) return CLUSTEN_ERR_UNALIGNED;
-    return launch_blank_grad(q, q_stride, d_out, d_logit, prob, scale, d_blank_k, d_blank_v, static_cast<float*>(workspace), B, H, N, C, dtype,
-                             as_stream(stream));
+    return launch_blank_grad(q, q_stride, d_out, d_logit, prob, scale, d_blank_k, d_blank_v, static_cast<float*>(workspace), nullptr, B, H, N, C,
+                             dtype, as_stream(stream));
 }
 
 int clusten_kv_columns(const void* d_k, const void* d_v, void* d_qkv, float scale, int B, int H, int N, int ch, int dtype,
@@ -821,7 +821,7 @@ int clusten_position_grad(const void* d_logit, const int64_t* pe_idx, const void
     if (B <= 0 || H <= 0 || H > 65535 || N <= 0 || M <= 0 || M % 4 != 0 || rows <= 0 || k <= 0 || k > 5) return CLUSTEN_ERR_BAD_DIMS;
     if (workspace_bytes < clusten_position_grad_workspace_bytes(B, H, N, M)) return CLUSTEN_ERR_WORKSPACE;
     if (!aligned16(d_logit) || !aligned16(padded) || !aligned16(workspace)) return CLUSTEN_ERR_UNALIGNED;
-    return launch_position_grad(d_logit, pe_idx, padded, d_weight, d_bias, workspace, B, H, N, M, rows, k, dtype, as_stream(stream));
+    return launch_position_grad(d_logit, pe_idx, padded, d_weight, d_bias, workspace, nullptr, B, H, N, M, rows, k, dtype, as_stream(stream));
 }
 
 static int dense_train_args(DenseTrain& a, const void* qkv, const void* bias, const int64_t* pe_idx, const float* blank_k, const float* blank_v,

@@ -308,6 +308,30 @@ int launch_norm_linear(const NormLinearArgs& a, int x_dtype, int C, int dtype, h
 int launch_block_tail(const BlockTailArgs& a, int x_dtype, int C, int dtype, hipStream_t stream);
 
 // Backward of the two (block_backward_impl.hpp); the weights are packed transposes.
+// Partial rows that kernels left, added up in one launch: up to three of 2 C columns (the first C times scale0 to out0, the others to out1) and
+// a position bias layer's.  Kernels that are given one leave their sums to it, and launch them themselves otherwise.
+struct ColumnSums {
+    const float* partial;      // (groups, 2 C)
+    float* out0;
+    float* out1;
+    float scale0;
+    int groups, C;
+};
+struct PositionSums {
+    const double* partial;     // (groups, heads, 6): five columns and the bias
+    float* d_w;                // (heads, k)
+    float* d_b;
+    int groups, heads, k;
+};
+struct GradSums {
+    ColumnSums column[3];
+    PositionSums position;     // heads 0: none
+    int columns;
+};
+int launch_grad_sums(const GradSums& sums, hipStream_t stream);
+int add_up(const ColumnSums& sums, GradSums* later, hipStream_t stream);
+int add_up(const PositionSums& sums, GradSums* later, hipStream_t stream);
+
 struct BlockTailGrad {
     const void* d_out;     // (rows, C) of S
     const void* x1;        // (rows, C) of S
@@ -327,6 +351,7 @@ struct BlockTailGrad {
     float* d_norm_w;
     float* d_norm_b;
     float* partial;
+    GradSums* later;       // or null
     int64_t rows;
     int rows_per_image, chunks;
 };
@@ -342,6 +367,7 @@ struct NormLinearGrad {
     float* d_norm_w;
     float* d_norm_b;
     float* partial;
+    GradSums* later;       // or null
     int64_t rows;
     int chunks;
 };
@@ -349,15 +375,13 @@ constexpr int kRowSumGroups = 1024;     // partial rows of a sum over all rows, 
 size_t block_backward_workspace_bytes(int64_t rows, int C);
 int launch_block_tail_backward(const BlockTailGrad& a, int x_dtype, int C, int dtype, hipStream_t stream);
 int launch_norm_linear_backward(const NormLinearGrad& a, int x_dtype, int C, int dtype, hipStream_t stream);
-// Sums of `groups` partial rows of 2 C values: the first C times scale0 to out0, the others to out1.
-int launch_column_sums(const float* partial, int groups, int C, float scale0, float* out0, float* out1, hipStream_t stream);
 
 // Training pass of an attention layer beside its attention kernels (attention_train.hip).
 int launch_position_bias(const float* table, const float* w, const float* b, void* bias, void* padded, int rows, int heads, int k, int dtype,
                          hipStream_t stream);
 size_t position_grad_workspace_bytes(int64_t total, int heads);
-int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void* padded, float* d_w, float* d_b, void* workspace, int B, int H, int N,
-                         int M, int rows, int k, int dtype, hipStream_t stream);
+int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void* padded, float* d_w, float* d_b, void* workspace, GradSums* later, int B,
+                         int H, int N, int M, int rows, int k, int dtype, hipStream_t stream);
 struct DenseTrain {
     const void* qkv;       // (B, N, 3 C): [q | head 0: k v | head 1: k v ...]
     const void* bias;      // (H, rows)
@@ -410,7 +434,7 @@ int launch_norm_backward(const void* d_y, const void* x, int x_dtype, const floa
                          void* branch, const float* scale, int rows_per_image, float* d_weight, float* d_bias, float* workspace, int64_t rows, int C,
                          int dtype, hipStream_t stream);
 int launch_blank_grad(const void* q, int q_stride, const void* d_out, const float* d_logit, const float* prob, float scale, float* d_blank_k,
-                      float* d_blank_v, float* workspace, int B, int H, int N, int C, int dtype, hipStream_t stream);
+                      float* d_blank_v, float* workspace, GradSums* later, int B, int H, int N, int C, int dtype, hipStream_t stream);
 int launch_kv_columns(const void* d_k, const void* d_v, void* d_qkv, float scale, int B, int H, int N, int ch, int dtype, hipStream_t stream);
 int launch_table_linear_grad(const float* d, const void* x, float* d_w, float* d_b, int64_t rows, int heads, int k, int dtype, hipStream_t stream);
 

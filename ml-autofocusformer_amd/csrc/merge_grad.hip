@@ -123,7 +123,7 @@ int launch_width(const RowScore& a, hipStream_t stream) {
     const int most = (int)min(groups, (int64_t)kRowSumGroups);
     hipLaunchKernelGGL((row_score_backward_kernel<T, S, C>), dim3(most), dim3(kThreads), 0, stream, a);
     if (int st = launch_status()) return st;
-    return launch_column_sums(a.partial, most, C, 1.f, a.d_weight, a.d_bias, stream);
+    return add_up(ColumnSums{a.partial, a.d_weight, a.d_bias, 1.f, most, C}, nullptr, stream);
 }
 
 template <typename T, typename S>
