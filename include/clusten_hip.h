@@ -674,8 +674,8 @@ int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x
                            const void* plan, int lists_shared, const int64_t* pe_idx, clusten_attn_shape shape, int hidden,
                            float scale, int dtype, clusten_stream stream);
 
-/* The same with the local attention's bias tables as (H, table_rows): the bias of neighbouring positions then lies side by side.  table_rows = 0:
- * as above. */
+/* The same with the bias tables as (H, table_rows), for local attention - the bias of neighbouring positions then lies side by side - and for
+ * fp32 blocks over all N <= 64 tokens, heads of 32 channels, which take no other.  table_rows = 0: as above. */
 int clusten_blocks_forward_tables(const clusten_block* blocks, int count, const void* x, int x_dtype, void* out, void* qkv,
                                   void* attn, const void* plan, int lists_shared, const int64_t* pe_idx, int table_rows,
                                   clusten_attn_shape shape, int hidden, float scale, int dtype, clusten_stream stream);

@@ -46,6 +46,7 @@ def default_ops():
                            cluster_attention_backward=_native.cluster_attention_backward,
                            cluster_attention_backward_supported=_native.cluster_attention_backward_supported,
                            cluster_pairs=_native.cluster_pairs, scatter_rows=_native.scatter_rows,
+                           dense_attention_train=_native.dense_attention_train,
                            dense_attention=_native.dense_attention,
                            dense_attention_supported=_native.dense_attention_supported,
                            layer_norm=_native.layer_norm, layer_norm_supported=_native.layer_norm_supported,
@@ -83,6 +84,7 @@ def default_ops():
                            blocks_forward=_native.blocks_forward, block_params=_native.BlockParams,
                            blocks_stand_for=(("cluster_attention", _native.cluster_attention),
                                              ("dense_attention", _native.dense_attention),
+                                             ("dense_attention_train", _native.dense_attention_train),
                                              ("norm_linear", _native.norm_linear), ("block_tail", _native.block_tail)))
 
 
@@ -769,6 +771,22 @@ class ClusterAttention(_Module):
                 and len(grid_lists) > 4 and not _drops(self.attn_drop)
                 and self.ops.cluster_attention_backward_supported(q.view(b, n, h, c // h).permute(0, 2, 1, 3), cluster_idx.shape[2]))
 
+    def _attend_to_all(self, q, kv, pe_idx, table):
+        """`attend` of an fp32 inference pass over all tokens by one kernel, or None where it is not built for the call."""
+        rows_op = getattr(self.ops, "dense_attention_train", None)
+        b, n, c = q.shape
+        if (rows_op is None or _drops(self.attn_drop) or _transformed() or c != 32 * self.num_heads or not 0 < n <= 64 or b == 0
+                or kv.dtype != q.dtype or pe_idx.shape != (b, n, n) or pe_idx.dtype != torch.int64
+                or not all(_kernel_parameter(t, q) and t.numel() == c for t in (self.blank_k, self.blank_v))):
+            return None
+        bias = self.bias_table(table)
+        if bias.dtype != torch.float32:
+            return None
+        one = q.stride() == kv.stride() == (n * 3 * c, 3 * c, 1) and kv.data_ptr() == q.data_ptr() + 4 * c and q.data_ptr() % 16 == 0
+        qkv = q.as_strided((b, n, 3 * c), (n * 3 * c, 3 * c, 1)) if one else torch.cat([q, kv], dim=2)
+        return rows_op(qkv.detach(), bias.detach().t().contiguous(), pe_idx.contiguous(), self.blank_k.detach(), self.blank_v.detach(),
+                       self.num_heads, self.scale)
+
     def attend(self, q, kv, member_idx, cluster_mask, pe_idx, global_attn, table, cluster_idx=None, grid_lists=None):
         """The attention between its projections: q (b,n,c) and kv (b,n,2c) in, what the output projection reads (b,n,c)
         out.  The query is not scaled yet; q and kv may be column ranges of one matrix."""
@@ -807,6 +825,10 @@ class ClusterAttention(_Module):
             out = dense(q.view(b, n, h, ch).permute(0, 2, 1, 3), key, v, self.bias_table(table), pe_idx,
                         self.blank_k, self.blank_v, scale=self.scale)
             return out
+        if global_attn and q.dtype == torch.float32 and not torch.is_grad_enabled() and q.is_cuda:
+            out = self._attend_to_all(q, kv, pe_idx, table)
+            if out is not None:
+                return out
         q = (q * self.scale).reshape(b, n, h, ch).permute(0, 2, 1, 3)                    # (b,h,n,ch) view
         if global_attn:
             attn = q @ key.transpose(-1, -2)                                             # (b,h,n,n)
@@ -1221,13 +1243,14 @@ class BasicLayer(_Module):
                 dt == torch.float32 and getattr(ops, "block_layout", None) is None):
             return None
         if global_attn:
-            if n > 64 or dt == torch.float32:
+            if n > 64:
                 return None
             plan = None
         else:
             plan = lists[3] if lists is not None and len(lists) > 3 else None
             if plan is None or not (self.cluster_size == 8 or (self.cluster_size == 24 and dt != torch.float32)):
                 return None
+        by_heads = plan is not None or dt == torch.float32         # bias tables (heads, rows); else (rows, heads)
         tensors = [blk.tensors() for blk in self.blocks]
         hidden, scale = first.mlp.fc1.out_features, first.attn.scale
         try:
@@ -1247,7 +1270,7 @@ class BasicLayer(_Module):
             for p, blk, ts in zip(params, self.blocks, tensors):
                 bias = blk.attn.bias_table(table)
                 bias = bias.detach().to(dt)
-                bias = (bias if plan is None else bias.t()).contiguous()       # by heads for the local attention
+                bias = (bias.t() if by_heads else bias).contiguous()
                 made.append(bias)
                 if dt != torch.float32:
                     packed, at = blk._packed(dt)
@@ -1271,7 +1294,7 @@ class BasicLayer(_Module):
             for i, p in enumerate(params):
                 p.w_qkv, _, p.w_proj, p.w1, p.w2 = (base + o for o in at[5 * i:5 * i + 5])
         return ops.blocks_forward(params, feat, h, hidden, dt, scale, plan, pe_idx if plan is None else None,
-                                  0 if plan is None else table.shape[0])
+                                  table.shape[0] if by_heads else 0)
 
     def forward(self, pos, feat, h, w, on_grid, stride, table, radius, feat_ordered=False):
         """`feat_ordered`: the tokens already stand in the order `grid_order` gave (first stage only)."""

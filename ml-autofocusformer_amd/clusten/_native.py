@@ -2178,9 +2178,9 @@ def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torc
     """The transformer blocks of a stage one after the other, issued by one call: `params` is a ctypes array of BlockParams
     (what it points at is the caller's to keep), x (B,N,C) the token rows with C = 32 * heads.  Local attention with the
     lists `plan` was built from (`cluster_attention_plan`), or, with `pe_idx` (B,N,N) instead, attention over all N <= 64
-    tokens.  `table_rows`: of bias tables laid out (heads, table_rows), local attention only; 0 when they are (rows, heads).  The same
-    kernels as `norm_linear`, `cluster_attention` / `dense_attention` and `block_tail` block by block.  No
-    autograd: for inference."""
+    tokens.  `table_rows`: of bias tables laid out (heads, table_rows) - local attention, or fp32 blocks over all tokens, which
+    have no other - and 0 when they are (rows, heads).  The same kernels as `norm_linear`, `cluster_attention` / `dense_attention`
+    (fp32: `dense_attention_train`) and `block_tail` block by block.  No autograd: for inference."""
     lib = load()
     _require_cuda("x", x)
     device = x.device
@@ -2196,8 +2196,8 @@ def blocks_forward(params, x: torch.Tensor, heads: int, hidden: int, dtype: torc
         lb, m = fits[0]
     else:
         _require_cuda("pe_idx", pe_idx, device)
-        if pe_idx.shape != (b, n, n) or pe_idx.dtype != torch.int64 or n > 64 or dtype == torch.float32:
-            raise RuntimeError("pe_idx must be int64 of shape (B,N,N), N <= 64, and the blocks fp16 / bf16")
+        if pe_idx.shape != (b, n, n) or pe_idx.dtype != torch.int64 or n > 64 or (dtype == torch.float32) != (table_rows > 0):
+            raise RuntimeError("pe_idx must be int64 of shape (B,N,N), N <= 64, and the tables of fp32 blocks, and of these only, by heads")
         pe_idx = pe_idx.contiguous()
         lb, m = b, n
     out = torch.empty_like(x)

@@ -650,7 +650,12 @@ int clusten_blocks_forward(const clusten_block* blocks, int count, const void* x
 int clusten_blocks_forward_tables(const clusten_block* blocks, int count, const void* x, int x_dtype, void* out, void* qkv, void* attn,
                                   const void* plan, int lists_shared, const int64_t* pe_idx, int table_rows, clusten_attn_shape shape,
                                   int hidden, float scale, int dtype, clusten_stream stream) {
-    if (table_rows < 0 || (table_rows > 0 && !plan)) return CLUSTEN_ERR_BAD_DIMS;
+    // attention over all tokens: 16-bit data by matrix instructions with (rows, heads) tables, fp32 by the training pass' forward kernel,
+    // which takes them by heads.  A forward of 50 images in fp32, five such layers of 49 tokens and 16 heads: 6334 us with an
+    // fp32 layer's library products, gather, copies and softmax (20 launches between norm_linear and block_tail), 5690 with the kernel.
+    const bool by_heads = plan ? table_rows > 0 : dtype == CLUSTEN_F32;
+    if (table_rows < 0 || (!plan && by_heads != (table_rows > 0))) return CLUSTEN_ERR_BAD_DIMS;
+    if (!plan && by_heads && (shape.C != 32 || shape.N > 64 || (int64_t)shape.B * shape.H >= (int64_t)1 << 31)) return CLUSTEN_ERR_BAD_DIMS;
     if (plan && !aligned16(plan)) return CLUSTEN_ERR_UNALIGNED;
     if (!blocks || !x || !out || !qkv || !attn || (!plan && !pe_idx)) return CLUSTEN_ERR_NULL_POINTER;
     if (count <= 0) return CLUSTEN_ERR_BAD_DIMS;
@@ -675,12 +680,19 @@ int clusten_blocks_forward_tables(const clusten_block* blocks, int count, const 
             return st;
         }
         if (!b.bias_table || !b.blank_k || !b.blank_v) return CLUSTEN_ERR_NULL_POINTER;
-        const int st = plan ? launch_cluster_attention(q, qs, k, kv, v, kv, nullptr,
-                                                       table_rows ? table_by_heads(b.bias_table, table_rows) : table_by_rows(b.bias_table, shape.H),
-                                                       nullptr, nullptr, b.blank_k, b.blank_v, attn, os, scale, lists_shared != 0, plan, nullptr,
-                                                       shape, dtype, as_stream(stream))
-                            : clusten_dense_attention_forward(q, qs, k, kv, v, kv, b.bias_table, pe_idx, b.blank_k, b.blank_v,
-                                                              attn, os, scale, shape, dtype, stream);
+        int st;
+        if (plan) {
+            st = launch_cluster_attention(q, qs, k, kv, v, kv, nullptr,
+                                          by_heads ? table_by_heads(b.bias_table, table_rows) : table_by_rows(b.bias_table, shape.H), nullptr,
+                                          nullptr, b.blank_k, b.blank_v, attn, os, scale, lists_shared != 0, plan, nullptr, shape, dtype,
+                                          as_stream(stream));
+        } else if (by_heads) {
+            st = clusten_dense_attention_train_forward(qkv, b.bias_table, pe_idx, b.blank_k, b.blank_v, attn, scale, shape.B, shape.H, shape.N,
+                                                       table_rows, dtype, stream);
+        } else {
+            st = clusten_dense_attention_forward(q, qs, k, kv, v, kv, b.bias_table, pe_idx, b.blank_k, b.blank_v, attn, os, scale, shape, dtype,
+                                                 stream);
+        }
         if (st) return st;
         // a workgroup of the tail reads its own rows only, all of them before it writes the first: in place from block 1 on
         if (int st2 = clusten_block_tail_forward(attn, in, x_dtype, b.w_proj, b.b_proj, b.norm2_w, b.norm2_b, b.eps2, b.w1, b.b1,

@@ -144,3 +144,24 @@ def test_row_score(device, dt, stream, c, b, n):
     near(d_x, d_z * w64, BAR[stream])
     near(d_w, (d_z * x64).sum((0, 1)), 2e-6)
     assert (d_b.double() - d_z.sum()).abs() <= 2e-6 * d_z.norm()           # what a sum of such terms comes to, not this one
+
+
+@pytest.mark.parametrize("columns", [True, False])
+@pytest.mark.parametrize("b,n", [(1, 1), (3, 49), (2, 63), (2, 64), (2, 65)])
+def test_global_attention_of_an_fp32_forward(device, b, n, columns):
+    """q and kv as columns of one matrix, as the block kernels leave them, and as tensors of their own; up to 64 tokens are one kernel."""
+    import copy
+    from aff.model import ClusterAttention
+    torch.manual_seed(n)
+    attn = ClusterAttention(64, 2).to(device)
+    with torch.no_grad():
+        for p in attn.parameters():
+            p.copy_(torch.randn_like(p) * 0.5)
+    table, pe = torch.randn(169, 5, device=device), torch.randint(169, (b, n, n), device=device)
+    qkv = torch.randn(b, n, 192, device=device)
+    q, kv = (qkv[..., :64], qkv[..., 64:]) if columns else (qkv[..., :64].contiguous(), qkv[..., 64:].contiguous())
+    everyone = torch.arange(n, device=device).expand(b, n, n)
+    with torch.no_grad():
+        got = attn.attend(q, kv, everyone, None, pe, True, table)
+        ref = copy.deepcopy(attn).double().attend(q.double(), kv.double(), everyone, None, pe, True, table.double())
+    near(got, ref, BAR[torch.float32])
