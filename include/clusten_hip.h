@@ -449,10 +449,20 @@ int clusten_linear_forward(const void* x, int64_t x_row_stride, const void* weig
  * input of the normalisation) done in the same pass.  x (rows,C) of in_dtype, out (rows,C) of out_dtype (F32,
  * F16 or BF16 each); weight, bias (C) fp32; all contiguous and 16-byte aligned (else CLUSTEN_ERR_UNALIGNED);
  * C in {64,128,256,384,512,768,1024} (else CLUSTEN_ERR_BAD_DIMS).
- * Inference only (no statistics are kept for a backward pass).  No counterpart in the reference's extension
- * modules. */
+ * Inference (the next keeps (mean, 1 / deviation) of every row in stats (rows,2), on a 16-byte boundary, for the backward).  No
+ * counterpart in the reference's extension modules. */
 int clusten_layer_norm_forward(const void* x, int in_dtype, const float* weight, const float* bias, void* out,
                                int64_t rows, int C, float eps, int out_dtype, clusten_stream stream);
+int clusten_layer_norm_forward_train(const void* x, int in_dtype, const float* weight, const float* bias, void* out, float* stats,
+                                     int64_t rows, int C, float eps, int out_dtype, clusten_stream stream);
+
+/* Its backward: d_x (rows,C) of x's type, d_weight and d_bias (C) fp32 from d_y (rows,C) of dy_dtype, F32 or, for x of the same type or
+ * F32, F16 / BF16.  fp32 inside, sums over the rows in a fixed order.  rows < 2^31, C as above; workspace:
+ * clusten_layer_norm_backward_workspace_bytes(rows, C) bytes (0: not supported); 16-byte aligned as above. */
+size_t clusten_layer_norm_backward_workspace_bytes(int64_t rows, int C);
+int clusten_layer_norm_backward(const void* d_y, int dy_dtype, const void* x, int x_dtype, const float* stats, const float* weight, void* d_x,
+                                float* d_weight, float* d_bias, void* workspace, size_t workspace_bytes, int64_t rows, int C,
+                                clusten_stream stream);
 
 /* Layer normalisation (as clusten_layer_norm_forward) of rows read in a given order, with a per-channel bias added
  * first:

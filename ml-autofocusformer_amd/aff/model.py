@@ -49,6 +49,7 @@ def default_ops():
                            dense_attention_train=_native.dense_attention_train,
                            dense_attention=_native.dense_attention,
                            dense_attention_supported=_native.dense_attention_supported,
+                           layer_norm_train=_native.layer_norm_train, layer_norm_backward=_native.layer_norm_backward,
                            layer_norm=_native.layer_norm, layer_norm_supported=_native.layer_norm_supported,
                            linear=_native.linear, linear_supported=_native.linear_supported,
                            add_layer_norm=_native.add_layer_norm, add_layer_norm_supported=_native.add_layer_norm_supported,
@@ -309,12 +310,55 @@ def _linear_pair(first, second, x, ops=None):
     return y[..., :n_first], y[..., n_first:]
 
 
-def _layer_norm(norm, x, ops, feeds_linear=False):
-    """`norm(x)` for an nn.LayerNorm; in inference on the GPU through the library's one-pass kernel when `ops` has it.
+class _LayerNormRows(torch.autograd.Function):
+    """`F.layer_norm(x.float(), ...)` returned as `out_dtype`, one pass over the rows a direction."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias, eps, out_dtype, ops):
+        out, stats = ops.layer_norm_train(x, weight, bias, eps, out_dtype)
+        ctx.save_for_backward(x, weight, bias, stats)
+        ctx.meta = (eps, out_dtype, ops)
+        return out
+
+    @staticmethod
+    @_types_of_forward
+    def backward(ctx, d_y):
+        x, weight, bias, stats = ctx.saved_tensors
+        eps, out_dtype, ops = ctx.meta
+        if not _by_kernels(d_y):
+            return (*_recorded_backward(lambda x, w, b: F.layer_norm(x.float(), (x.shape[-1],), w, b, eps).to(out_dtype), ctx, (x, weight, bias),
+                                        (d_y,)), None, None, None)
+        grads = ops.layer_norm_backward(_dense(d_y), x, stats, weight)
+        return (*(g if need else None for g, need in zip(grads, ctx.needs_input_grad)), None, None, None)
+
+
+def _train_layer_norm(norm, x, ops, linear):
+    """`norm(x)` of a training step by the library's kernels, or None where they do not stand for it."""
+    w, b = norm.weight, norm.bias
+    amp = torch.is_autocast_enabled("cuda")
+    if (getattr(ops, "layer_norm_backward", None) is None or not x.is_cuda or type(norm) is not nn.LayerNorm or _hooked(norm) or _transformed()
+            or not ops.layer_norm_supported(x) or not (x.dtype == torch.float32 or amp) or not 0 < x.numel() // x.shape[-1] < 1 << 31
+            or tuple(norm.normalized_shape) != x.shape[-1:] or not (_kernel_parameter(w, x) and _kernel_parameter(b, x))):
+        return None
+    narrow = amp and type(linear) is nn.Linear and not _hooked(linear)
+    out_dtype = torch.get_autocast_dtype("cuda") if narrow else torch.float32
+    x = x.contiguous()
+    if out_dtype not in (torch.float32, torch.float16, torch.bfloat16) or x.data_ptr() % 16 or (
+            narrow and x.dtype not in (torch.float32, out_dtype)):
+        return None
+    return _LayerNormRows.apply(x, w, b, norm.eps, out_dtype, ops)
+
+
+def _layer_norm(norm, x, ops, feeds_linear=False, linear=None):
+    """`norm(x)` for an nn.LayerNorm; on the GPU through the library's one-pass kernels when `ops` has them.
 
     `feeds_linear`: the result is only read by Linear layers, so under mixed precision it is produced in the
-    autocast dtype directly (the rounding those layers would apply to their input, done once)."""
+    autocast dtype directly (the rounding those layers would apply to their input, done once); in training only for the one layer
+    `linear` that reads it."""
     fn = getattr(ops, "layer_norm", None)
+    if torch.is_grad_enabled():
+        out = _train_layer_norm(norm, x, ops, linear)
+        return norm(x) if out is None else out
     if fn is None or torch.is_grad_enabled() or not ops.layer_norm_supported(x):
         return norm(x)
     out_dtype = torch.get_autocast_dtype("cuda") if (feeds_linear and torch.is_autocast_enabled("cuda")) else None
@@ -1140,7 +1184,7 @@ class ClusterMerging(_Module):
             if cluster_mask is not None:
                 weights = weights * mask_rows.unsqueeze(3)
         merged = self.ops.wf(weights, feat, member_idx).reshape(b, n_out, -1)            # channel = ic * c + c'
-        return pos, _linear(self.linear, _layer_norm(self.norm, merged, self.ops, True), self.ops)
+        return pos, _linear(self.linear, _layer_norm(self.norm, merged, self.ops, True, self.linear), self.ops)
 
 
 class BasicLayer(_Module):

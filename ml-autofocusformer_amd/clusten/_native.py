@@ -114,6 +114,11 @@ _PROTOTYPES = {
                                              ctypes.c_int, ctypes.c_int, _P]),
     "clusten_layer_norm_forward": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, ctypes.c_int64, ctypes.c_int,
                                                  ctypes.c_float, ctypes.c_int, _P]),
+    "clusten_layer_norm_forward_train": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, ctypes.c_float,
+                                                        ctypes.c_int, _P]),
+    "clusten_layer_norm_backward_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
+    "clusten_layer_norm_backward": (ctypes.c_int, [_P, ctypes.c_int, _P, ctypes.c_int, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, ctypes.c_int64,
+                                                   ctypes.c_int, _P]),
     "clusten_layer_norm_rows_forward": (ctypes.c_int, [_P, ctypes.c_int, _P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_int64,
                                                       ctypes.c_int, ctypes.c_float, ctypes.c_int, _P]),
     "clusten_channel_affine_gelu_forward": (ctypes.c_int, [_P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, ctypes.c_int,
@@ -1269,6 +1274,46 @@ def layer_norm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: f
                                                    ctypes.c_float(eps), _DTYPE_CODES[out_dtype], _stream(device)),
                "clusten_layer_norm_rows_forward")
     return out
+
+
+def _norm_rows(x, *vectors):
+    c = x.shape[-1] if x.dim() else 0
+    if (not layer_norm_supported(x) or not x.is_contiguous() or x.data_ptr() % 16 or not 0 < x.numel() // c < 1 << 31
+            or any(t.dtype != torch.float32 or not t.is_contiguous() or t.numel() != c or t.data_ptr() % 16 or t.device != x.device
+                   for t in vectors)):
+        raise RuntimeError("layer_norm in training: contiguous rows of a built width, fp32 weight and bias, on 16-byte boundaries of one device")
+    return c, x.numel() // c
+
+
+def layer_norm_train(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor, eps: float, out_dtype: torch.dtype):
+    """(`layer_norm(x, weight, bias, eps, out_dtype)`, fp32 (rows,2) statistics for `layer_norm_backward`).  No autograd."""
+    c, rows = _norm_rows(x, weight, bias)
+    out = torch.empty(x.shape, dtype=out_dtype, device=x.device)
+    stats = torch.empty(rows, 2, dtype=torch.float32, device=x.device)
+    with _on(x.device):
+        _check(load().clusten_layer_norm_forward_train(x.data_ptr(), _DTYPE_CODES[x.dtype], weight.data_ptr(), bias.data_ptr(), out.data_ptr(),
+                                                       stats.data_ptr(), rows, c, eps, _DTYPE_CODES[out_dtype], _stream(x.device)),
+               "clusten_layer_norm_forward_train")
+    return out, stats
+
+
+def layer_norm_backward(d_y: torch.Tensor, x: torch.Tensor, stats: torch.Tensor, weight: torch.Tensor):
+    """(d_x of x's dtype, d_weight, d_bias fp32) of `layer_norm_train`."""
+    c, rows = _norm_rows(x, weight)
+    if (d_y.shape != x.shape or not d_y.is_contiguous() or d_y.data_ptr() % 16 or d_y.device != x.device
+            or not (d_y.dtype in (torch.float32, x.dtype) or (x.dtype == torch.float32 and d_y.dtype in _DTYPE_CODES))
+            or stats.shape != (rows, 2) or stats.dtype != torch.float32 or not stats.is_contiguous() or stats.device != x.device):
+        raise RuntimeError("layer_norm_backward: contiguous gradients of x's shape, fp32 or of x's dtype, and the forward's statistics")
+    d_x, sums = torch.empty_like(x), torch.empty(2, c, dtype=torch.float32, device=x.device)
+    lib = load()
+    nbytes = lib.clusten_layer_norm_backward_workspace_bytes(rows, c)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    with _on(x.device):
+        at = sums.data_ptr()
+        _check(lib.clusten_layer_norm_backward(d_y.data_ptr(), _DTYPE_CODES[d_y.dtype], x.data_ptr(), _DTYPE_CODES[x.dtype], stats.data_ptr(),
+                                               weight.data_ptr(), d_x.data_ptr(), at, at + 4 * c, ws.data_ptr(), nbytes, rows, c,
+                                               _stream(x.device)), "clusten_layer_norm_backward")
+    return d_x, sums[0], sums[1]
 
 
 def channel_affine_gelu_supported(x: torch.Tensor) -> bool:

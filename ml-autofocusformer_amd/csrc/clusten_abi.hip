@@ -414,14 +414,41 @@ int clusten_linear_forward(const void* x, int64_t x_row_stride, const void* weig
     return launch_skinny_linear(x, x_row_stride, weight, bias, out, rows, K, Nout, act, dtype, as_stream(stream));
 }
 
-int clusten_layer_norm_forward(const void* x, int in_dtype, const float* weight, const float* bias, void* out,
-                               int64_t rows, int C, float eps, int out_dtype, clusten_stream stream) {
+static int layer_norm_call(const void* x, int in_dtype, const float* weight, const float* bias, void* out, float* stats, int64_t rows, int C,
+                           float eps, int out_dtype, clusten_stream stream) {
     if (!x || !weight || !bias || !out) return CLUSTEN_ERR_NULL_POINTER;
     if (out_dtype != CLUSTEN_F32 && out_dtype != CLUSTEN_F16 && out_dtype != CLUSTEN_BF16) return CLUSTEN_ERR_BAD_DTYPE;
     if (in_dtype != CLUSTEN_F32 && in_dtype != CLUSTEN_F16 && in_dtype != CLUSTEN_BF16) return CLUSTEN_ERR_BAD_DTYPE;
     if (rows <= 0 || C <= 0 || (rows + 3) / 4 >= ((int64_t)1 << 31)) return CLUSTEN_ERR_BAD_DIMS;
-    if (!aligned16(x) || !aligned16(weight) || !aligned16(bias) || !aligned16(out)) return CLUSTEN_ERR_UNALIGNED;
-    return launch_layer_norm(x, in_dtype, weight, bias, out, rows, C, eps, out_dtype, as_stream(stream));
+    if (!aligned16(x) || !aligned16(weight) || !aligned16(bias) || !aligned16(out) || !aligned16(stats)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_layer_norm(x, in_dtype, weight, bias, out, stats, rows, C, eps, out_dtype, as_stream(stream));
+}
+
+int clusten_layer_norm_forward(const void* x, int in_dtype, const float* weight, const float* bias, void* out,
+                               int64_t rows, int C, float eps, int out_dtype, clusten_stream stream) {
+    return layer_norm_call(x, in_dtype, weight, bias, out, nullptr, rows, C, eps, out_dtype, stream);
+}
+
+int clusten_layer_norm_forward_train(const void* x, int in_dtype, const float* weight, const float* bias, void* out, float* stats,
+                                     int64_t rows, int C, float eps, int out_dtype, clusten_stream stream) {
+    if (!stats) return CLUSTEN_ERR_NULL_POINTER;
+    return layer_norm_call(x, in_dtype, weight, bias, out, stats, rows, C, eps, out_dtype, stream);
+}
+
+size_t clusten_layer_norm_backward_workspace_bytes(int64_t rows, int C) { return layer_norm_backward_workspace_bytes(rows, C); }
+
+int clusten_layer_norm_backward(const void* d_y, int dy_dtype, const void* x, int x_dtype, const float* stats, const float* weight, void* d_x,
+                                float* d_weight, float* d_bias, void* workspace, size_t workspace_bytes, int64_t rows, int C,
+                                clusten_stream stream) {
+    if (!d_y || !x || !stats || !weight || !d_x || !d_weight || !d_bias || !workspace) return CLUSTEN_ERR_NULL_POINTER;
+    const size_t need = layer_norm_backward_workspace_bytes(rows, C);
+    if (need == 0) return CLUSTEN_ERR_BAD_DIMS;
+    if (workspace_bytes < need) return CLUSTEN_ERR_WORKSPACE;
+    if (!aligned16(d_y) || !aligned16(x) || !aligned16(stats) || !aligned16(weight) || !aligned16(d_x) || !aligned16(workspace)) {
+        return CLUSTEN_ERR_UNALIGNED;
+    }
+    return launch_layer_norm_backward(d_y, dy_dtype, x, x_dtype, stats, weight, d_x, d_weight, d_bias, static_cast<float*>(workspace), rows, C,
+                                      as_stream(stream));
 }
 
 int clusten_layer_norm_rows_forward(const void* x, int in_dtype, const int64_t* order, int group, const void* pre_bias,

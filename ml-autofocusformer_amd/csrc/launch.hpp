@@ -175,8 +175,12 @@ int launch_skinny_linear(const void* x, int64_t ldx, const void* w, const void* 
 
 // out[r,:] = (x[r,:] - mean) * rsqrt(var + eps) * weight + bias for `rows` rows of C channels
 //   (C in {64,128,256,384,512,768,1024}); x and out of dtype F32, F16 or BF16 each, arithmetic in fp32.
-int launch_layer_norm(const void* x, int in_dtype, const float* weight, const float* bias, void* out, int64_t rows, int C,
+int launch_layer_norm(const void* x, int in_dtype, const float* weight, const float* bias, void* out, float* stats, int64_t rows, int C,
                       float eps, int out_dtype, hipStream_t stream);
+// Its backward (layer_norm_grad.hip); stats (rows, 2) as the forward left them, partial of the bytes below (0: not supported).
+size_t layer_norm_backward_workspace_bytes(int64_t rows, int C);
+int launch_layer_norm_backward(const void* d_y, int dy_dtype, const void* x, int x_dtype, const float* stats, const float* weight, void* d_x,
+                               float* d_weight, float* d_bias, float* partial, int64_t rows, int C, hipStream_t stream);
 
 // layer norm of rows read in a given order (order may be null) with a per-channel bias (may be null) added first.
 int launch_layer_norm_rows(const void* x, int in_dtype, const int64_t* order, int group, const void* pre_bias,

@@ -17,7 +17,7 @@
 // A row is held by L lanes, W consecutive channels per lane and step (W = 8 when a 16-bit tensor is among the
 // operands, so that their accesses are 16 bytes per lane, else 4), C / (W L) steps; mean and variance are two reductions over registers (the
 // variance from the centred values, as a two-pass computation gives it), across the lanes of the row with xor
-// shuffles.  All arithmetic is fp32.
+// shuffles.  All arithmetic is fp32.  In training (mean, 1 / deviation) of every row is kept for layer_norm_grad.hip.
 #include <type_traits>
 
 #include "launch.hpp"
@@ -69,7 +69,8 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const InT* __restrict__
                                                          InT* __restrict__ sum_out, const float* __restrict__ weight,
                                                          const float* __restrict__ bias, OutT* __restrict__ out,
                                                          int64_t rows, float eps, const int64_t* __restrict__ order,
-                                                         int group, const InT* __restrict__ pre_bias) {
+                                                         int group, const InT* __restrict__ pre_bias,
+                                                         float2* __restrict__ stats) {
     constexpr int C = W * L * V;
     constexpr int ROWS_PER_WG = 256 / L;
     const int sub = threadIdx.x % L;
@@ -119,6 +120,7 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const InT* __restrict__
     }
     const float rstd = rsqrtf(row_sum<L>(sq) * (1.f / C) + eps);
     if (!live) return;
+    if (stats && sub == 0) stats[row] = make_float2(mean, rstd);
     OutT* orow = out + row * C;
 #pragma unroll
     for (int s = 0; s < V; ++s) {
@@ -140,22 +142,22 @@ __global__ __launch_bounds__(256) void layer_norm_kernel(const InT* __restrict__
 template <typename InT, typename ResT, typename OutT, int L, int V, int W = 4>
 int launch_lv(const void* x, const void* branch, void* sum_out, const float* weight, const float* bias, void* out,
               int64_t rows, float eps, hipStream_t stream, const int64_t* order = nullptr, int group = 1,
-              const void* pre_bias = nullptr) {
+              const void* pre_bias = nullptr, float2* stats = nullptr) {
     constexpr int ROWS_PER_WG = 256 / L;
     const int64_t blocks = (rows + ROWS_PER_WG - 1) / ROWS_PER_WG;
     hipLaunchKernelGGL((layer_norm_kernel<InT, ResT, OutT, L, V, W>), dim3((unsigned)blocks), dim3(256), 0, stream,
                        static_cast<const InT*>(x), static_cast<const ResT*>(branch), static_cast<InT*>(sum_out), weight,
-                       bias, static_cast<OutT*>(out), rows, eps, order, group, static_cast<const InT*>(pre_bias));
+                       bias, static_cast<OutT*>(out), rows, eps, order, group, static_cast<const InT*>(pre_bias), stats);
     return launch_status();
 }
 
 template <typename InT, typename ResT, typename OutT>
 int launch_typed(const void* x, const void* branch, void* sum_out, const float* weight, const float* bias, void* out,
                  int64_t rows, int C, float eps, hipStream_t stream, const int64_t* order = nullptr, int group = 1,
-                 const void* pre_bias = nullptr) {
+                 const void* pre_bias = nullptr, float2* stats = nullptr) {
     // eight channels per lane (16-byte accesses to 16-bit rows) when a 16-bit tensor is among the operands
     constexpr bool wide = sizeof(InT) == 2 || sizeof(OutT) == 2;
-#define CLUSTEN_LN_ARGS x, branch, sum_out, weight, bias, out, rows, eps, stream, order, group, pre_bias
+#define CLUSTEN_LN_ARGS x, branch, sum_out, weight, bias, out, rows, eps, stream, order, group, pre_bias, stats
     if constexpr (wide) {
         switch (C) {
             case 64: return launch_lv<InT, ResT, OutT, 8, 1, 8>(CLUSTEN_LN_ARGS);
@@ -184,17 +186,17 @@ int launch_typed(const void* x, const void* branch, void* sum_out, const float* 
 template <typename InT>
 int launch_in(const void* x, const float* weight, const float* bias, void* out, int64_t rows, int C, float eps,
               int out_dtype, hipStream_t stream, const int64_t* order = nullptr, int group = 1,
-              const void* pre_bias = nullptr) {
+              const void* pre_bias = nullptr, float2* stats = nullptr) {
     switch (out_dtype) {
         case CLUSTEN_F32:
             return launch_typed<InT, void, float>(x, nullptr, nullptr, weight, bias, out, rows, C, eps, stream, order, group,
-                                                  pre_bias);
+                                                  pre_bias, stats);
         case CLUSTEN_F16:
             return launch_typed<InT, void, f16_t>(x, nullptr, nullptr, weight, bias, out, rows, C, eps, stream, order, group,
-                                                  pre_bias);
+                                                  pre_bias, stats);
         case CLUSTEN_BF16:
             return launch_typed<InT, void, bf16_t>(x, nullptr, nullptr, weight, bias, out, rows, C, eps, stream, order,
-                                                   group, pre_bias);
+                                                   group, pre_bias, stats);
         default: return CLUSTEN_ERR_BAD_DTYPE;
     }
 }
@@ -210,12 +212,13 @@ int launch_add(const void* x, int x_dtype, const void* branch, void* sum_out, co
 
 }  // namespace
 
-int launch_layer_norm(const void* x, int in_dtype, const float* weight, const float* bias, void* out, int64_t rows, int C,
+int launch_layer_norm(const void* x, int in_dtype, const float* weight, const float* bias, void* out, float* stats_, int64_t rows, int C,
                       float eps, int out_dtype, hipStream_t stream) {
+    float2* stats = reinterpret_cast<float2*>(stats_);
     switch (in_dtype) {
-        case CLUSTEN_F32: return launch_in<float>(x, weight, bias, out, rows, C, eps, out_dtype, stream);
-        case CLUSTEN_F16: return launch_in<f16_t>(x, weight, bias, out, rows, C, eps, out_dtype, stream);
-        case CLUSTEN_BF16: return launch_in<bf16_t>(x, weight, bias, out, rows, C, eps, out_dtype, stream);
+        case CLUSTEN_F32: return launch_in<float>(x, weight, bias, out, rows, C, eps, out_dtype, stream, nullptr, 1, nullptr, stats);
+        case CLUSTEN_F16: return launch_in<f16_t>(x, weight, bias, out, rows, C, eps, out_dtype, stream, nullptr, 1, nullptr, stats);
+        case CLUSTEN_BF16: return launch_in<bf16_t>(x, weight, bias, out, rows, C, eps, out_dtype, stream, nullptr, 1, nullptr, stats);
         default: return CLUSTEN_ERR_BAD_DTYPE;
     }
 }

@@ -458,3 +458,46 @@ def test_frozen_parameters(device, dt, local):
     for name, ref in grads[0].items():
         got = grads[1][name]
         assert (got is None) if name != "x" and name.endswith(frozen) else torch.equal(got, ref), name
+
+
+# every width; a row, a workgroup's rows and one more, and more rows than all workgroups take at once
+@pytest.mark.parametrize("c,rows", [(64, 1), (64, 33), (64, 40000), (128, 17), (256, 9), (384, 1025), (512, 4101), (768, 8), (1024, 5000)])
+@pytest.mark.parametrize("dt,dy", [(torch.float32, torch.float32), (torch.float32, torch.float16), (torch.float32, torch.bfloat16),
+                                   (torch.float16, torch.float32), (torch.float16, torch.float16), (torch.bfloat16, torch.float32),
+                                   (torch.bfloat16, torch.bfloat16)])
+def test_layer_norm_in_training(device, c, rows, dt, dy):
+    """Against float64.  A result stored in 16 bits: one rounding, 4e-4 / 3e-3; fp32: 1e-6 (a row's two sums); column sums: 2e-6 of the
+    root of the sum of the squared terms, which is what roundings of 2^-24 of running sums over up to 40 rows a lane add up to."""
+    gen = torch.Generator(device).manual_seed(rows + c)
+    x, d = (torch.randn(1, rows, c, generator=gen, device=device).to(t) for t in (dt, dy))
+    w, b = 1 + 0.2 * torch.randn(c, generator=gen, device=device), torch.randn(c, generator=gen, device=device)
+    ref = [t.double().requires_grad_() for t in (x, w, b)]
+    y = torch.nn.functional.layer_norm(ref[0], (c,), ref[1], ref[2], 1e-5)
+    d_x, d_w, d_b = torch.autograd.grad(y, ref, d.double())
+    bar = {torch.float32: 1e-6, torch.float16: 4e-4, torch.bfloat16: 3e-3}
+    out, stats = _native.layer_norm_train(x, w, b, 1e-5, dy)
+    got = _native.layer_norm_backward(d, x, stats, w)
+    assert (out.double() - y).norm() <= bar[dy] * y.norm() and (got[0].double() - d_x).norm() <= bar[dt] * d_x.norm() + 1e-12
+    h = ((y - ref[2]) / ref[1]).detach()
+    for g, want, terms in ((got[1], d_w, d.double() * h), (got[2], d_b, d.double())):
+        assert ((g.double() - want).abs() <= 2e-6 * terms.square().sum((0, 1)).sqrt() + 1e-12).all()
+
+
+@pytest.mark.parametrize("amp", [torch.float16, torch.bfloat16, None])
+def test_layer_norm_module_in_training(device, amp):
+    """The module through the kernels: strided rows, a gradient that is an expanded view, a backward that is itself differentiated."""
+    from aff.model import _layer_norm, default_ops
+    norm = torch.nn.LayerNorm(64).to(device)
+    base = torch.randn(3, 64, 50, device=device, generator=torch.Generator(device).manual_seed(3)).to(amp or torch.float32).requires_grad_()
+
+    def grads(fn, create):
+        with torch.autocast("cuda", dtype=amp or torch.float16, enabled=amp is not None):
+            y = fn(base.transpose(1, 2))
+        assert y.dtype == torch.float32
+        return torch.autograd.grad(y.mean(1).pow(3).sum(), (base, norm.weight, norm.bias), create_graph=create)
+
+    mine, theirs = grads(lambda x: _layer_norm(norm, x, default_ops()), False), grads(norm, False)
+    twice = grads(lambda x: _layer_norm(norm, x, default_ops()), True)
+    for a, b, c in zip(mine, theirs, twice):
+        bar = 2e-5 if a.dtype == torch.float32 else 2 * BAR[a.dtype]
+        assert a.dtype == b.dtype == c.dtype and (a - b).norm() <= bar * b.norm() and (c - b).norm() <= bar * b.norm() and c.requires_grad
