@@ -788,6 +788,15 @@ int clusten_block_train_forward(const clusten_block_train* args, void* out, clus
 int clusten_block_train_backward(const clusten_block_train* args, const void* d_out, void* d_x, void* workspace,
                                  size_t workspace_bytes, clusten_stream stream);
 
+/* The table of merge weights in training (models/aff_transformer.py:343-350): out (rows,4) = gelu(layer_norm(table W^T + b)) of table
+ * (rows,5), W (4,5), b, norm_w, norm_b (4), all fp32; the operands and the result of the product rounded to dtype (F32, F16, BF16).
+ * backward: d_params (32) = the gradients of W, b, norm_w and norm_b one behind the other, in fp32, in a fixed order.  out and d_out on
+ * 16-byte boundaries; rows < 2^31. */
+int clusten_merge_table_forward(const float* table, const float* weight, const float* bias, const float* norm_w, const float* norm_b, float eps,
+                                float* out, int64_t rows, int dtype, clusten_stream stream);
+int clusten_merge_table_backward(const float* d_out, const float* table, const float* weight, const float* bias, const float* norm_w,
+                                 const float* norm_b, float eps, float* d_params, int64_t rows, int dtype, clusten_stream stream);
+
 /* Training passes around a merge (models/aff_transformer.py:340-358, 496-500 under autograd).
  *   merge_weights_backward, of clusten_merge_weights_forward: d_rows (B,4,Nout,M) = d_weights (B,Nout,M,4) * prob * mask, which
  *     clusten_bias_table_grad (H = 4, the same pe_idx) sums into the table's rows, and, with prob, d_prob (B,N), written in full (fp32

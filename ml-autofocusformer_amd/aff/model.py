@@ -54,6 +54,8 @@ def default_ops():
                            linear=_native.linear, linear_supported=_native.linear_supported,
                            add_layer_norm=_native.add_layer_norm, add_layer_norm_supported=_native.add_layer_norm_supported,
                            merge_weights=_native.merge_weights, merge_weights_supported=_native.merge_weights_supported,
+                           merge_table=_native.merge_table, merge_table_backward=_native.merge_table_backward,
+                           merge_table_supported=_native.merge_table_supported,
                            merge_weights_backward=_native.merge_weights_backward,
                            row_score=_native.row_score, row_score_backward=_native.row_score_backward,
                            row_score_supported=_native.row_score_supported,
@@ -627,6 +629,40 @@ class _DenseAttentionRows(_BlockRows):
     """A block whose tokens attend to all."""
 
 
+class _MergeTable(torch.autograd.Function):
+    """A merge's weight of every relative position - Linear, norm and GELU over the table - by one kernel a direction."""
+
+    @staticmethod
+    def forward(ctx, table, weight, bias, norm_w, norm_b, eps, dt, ops):
+        ctx.save_for_backward(table, weight, bias, norm_w, norm_b)
+        ctx.meta = (eps, dt, ops)
+        return ops.merge_table(table, weight, bias, norm_w, norm_b, eps, dt)
+
+    @staticmethod
+    @_types_of_forward
+    def backward(ctx, d_out):
+        table, *params = ctx.saved_tensors
+        eps, dt, ops = ctx.meta
+        if not _by_kernels(d_out):
+            def layers(w, b, norm_w, norm_b):
+                return F.gelu(F.layer_norm(F.linear(table.to(dt), w.to(dt), b.to(dt)).float(), (4,), norm_w, norm_b, eps))
+            return (None, *_recorded_backward(layers, ctx, params, (d_out,), ctx.needs_input_grad[1:5]), None, None, None)
+        grads = ops.merge_table_backward(_dense(d_out), table, *params, eps, dt)
+        return (None, *(g if need else None for g, need in zip(grads, ctx.needs_input_grad[1:5])), None, None, None)
+
+
+def _weight_table(net, table, ops):
+    """`net(table)` for a merge's weight net."""
+    if (torch.is_grad_enabled() and getattr(ops, "merge_table_backward", None) is not None and table.is_cuda and not table.requires_grad
+            and type(net) is nn.Sequential and tuple(map(type, net)) == (nn.Linear, nn.LayerNorm, nn.GELU) and net[2].approximate == "none"
+            and not any(map(_hooked, (net, *net))) and not _transformed()):
+        params = (net[0].weight, net[0].bias, net[1].weight, net[1].bias)
+        dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled("cuda") else torch.float32
+        if all(p is not None for p in params) and tuple(net[1].normalized_shape) == (4,) and ops.merge_table_supported(table, *params, dt):
+            return _MergeTable.apply(table, *params, net[1].eps, dt, ops)
+    return net(table)
+
+
 class _MergeWeights(torch.autograd.Function):
     """The weights a merge's WF operator takes - table rows by position, times importance, times mask - with both gradients from
     the library's kernels; fp32."""
@@ -1168,7 +1204,7 @@ class ClusterMerging(_Module):
         if cluster_mask is not None and mask_rows is None:
             mask_rows = cluster_mask.gather(1, rows)
         table_w = _table_function(self, "_weight_table_cache", self.weight_net, table,
-                                  lambda: self.weight_net(table))                         # (rows, 4)
+                                  lambda: _weight_table(self.weight_net, table, self.ops))  # (rows, 4)
         one_pass = getattr(self.ops, "merge_weights", None)
         if one_pass is not None and not torch.is_grad_enabled() and self.ops.merge_weights_supported(table_w):
             # inference: lookup, importance of each neighbour and mask in one kernel

@@ -114,6 +114,8 @@ _PROTOTYPES = {
                                              ctypes.c_int, ctypes.c_int, _P]),
     "clusten_layer_norm_forward": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, ctypes.c_int64, ctypes.c_int,
                                                  ctypes.c_float, ctypes.c_int, _P]),
+    "clusten_merge_table_forward": (ctypes.c_int, [_P, _P, _P, _P, _P, ctypes.c_float, _P, ctypes.c_int64, ctypes.c_int, _P]),
+    "clusten_merge_table_backward": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, ctypes.c_float, _P, ctypes.c_int64, ctypes.c_int, _P]),
     "clusten_layer_norm_forward_train": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, _P, ctypes.c_int64, ctypes.c_int, ctypes.c_float,
                                                         ctypes.c_int, _P]),
     "clusten_layer_norm_backward_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),
@@ -1534,6 +1536,39 @@ def merge_weights(table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: t
                                                  n_out, m, table_weights.shape[1], _stream(device)),
                "clusten_merge_weights_forward")
     return out
+
+
+def merge_table_supported(table: torch.Tensor, weight, bias, norm_w, norm_b, dtype: torch.dtype) -> bool:
+    """True when `merge_table` takes a (rows,5) table with the parameters of a Linear layer of four outputs and of its norm, fp32 in place."""
+    return (table.is_cuda and table.dim() == 2 and table.shape[1] == 5 and 0 < table.shape[0] < 1 << 31 and dtype in _DTYPE_CODES
+            and tuple(weight.shape) == (4, 5) and all(t.numel() == 4 for t in (bias, norm_w, norm_b))
+            and all(t.dtype == torch.float32 and t.is_contiguous() and t.device == table.device for t in (table, weight, bias, norm_w, norm_b)))
+
+
+def merge_table(table, weight, bias, norm_w, norm_b, eps: float, dtype: torch.dtype) -> torch.Tensor:
+    """F.gelu(F.layer_norm(F.linear(table, weight, bias), (4,), norm_w, norm_b, eps)), the Linear layer's operands and result rounded to
+    dtype: (rows,4) fp32.  No autograd."""
+    if not merge_table_supported(table, weight, bias, norm_w, norm_b, dtype):
+        raise RuntimeError("merge_table: contiguous fp32 table (rows,5), weight (4,5), bias and norm of 4 on one device")
+    out = torch.empty(table.shape[0], 4, dtype=torch.float32, device=table.device)
+    with _on(table.device):
+        _check(load().clusten_merge_table_forward(table.data_ptr(), weight.data_ptr(), bias.data_ptr(), norm_w.data_ptr(), norm_b.data_ptr(), eps,
+                                                  out.data_ptr(), out.shape[0], _DTYPE_CODES[dtype], _stream(table.device)),
+               "clusten_merge_table_forward")
+    return out
+
+
+def merge_table_backward(d_out, table, weight, bias, norm_w, norm_b, eps: float, dtype: torch.dtype):
+    """The gradients (d_weight, d_bias, d_norm_w, d_norm_b) of `merge_table`, fp32."""
+    if (not merge_table_supported(table, weight, bias, norm_w, norm_b, dtype) or tuple(d_out.shape) != (table.shape[0], 4)
+            or d_out.dtype != torch.float32 or not d_out.is_contiguous() or d_out.data_ptr() % 16 or d_out.device != table.device):
+        raise RuntimeError("merge_table_backward: contiguous fp32 gradients (rows,4) and what merge_table takes")
+    d = torch.empty(32, dtype=torch.float32, device=table.device)
+    with _on(table.device):
+        _check(load().clusten_merge_table_backward(d_out.data_ptr(), table.data_ptr(), weight.data_ptr(), bias.data_ptr(), norm_w.data_ptr(),
+                                                   norm_b.data_ptr(), eps, d.data_ptr(), table.shape[0], _DTYPE_CODES[dtype],
+                                                   _stream(table.device)), "clusten_merge_table_backward")
+    return d[:20].view(4, 5), d[20:24], d[24:28], d[28:]
 
 
 def merge_weights_backward(d_weights: torch.Tensor, table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: torch.Tensor, prob, mask):

@@ -914,6 +914,24 @@ int clusten_scatter_attention_pair(const void* d_logit, const void* query, clust
                                dtype, as_stream(stream));
 }
 
+static int merge_table_call(MergeTable a, bool backward, int dtype, clusten_stream stream) {
+    if (!a.table || !a.weight || !a.bias || !a.norm_w || !a.norm_b || (backward ? !a.d_out || !a.d_params : !a.out)) return CLUSTEN_ERR_NULL_POINTER;
+    if (!block_dtype_ok(dtype)) return CLUSTEN_ERR_BAD_DTYPE;
+    if (a.rows <= 0 || a.rows >= (int64_t)1 << 31) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(a.d_out) || !aligned16(a.out)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_merge_table(a, backward, dtype, as_stream(stream));
+}
+
+int clusten_merge_table_forward(const float* table, const float* weight, const float* bias, const float* norm_w, const float* norm_b, float eps,
+                                float* out, int64_t rows, int dtype, clusten_stream stream) {
+    return merge_table_call(MergeTable{table, weight, bias, norm_w, norm_b, nullptr, out, nullptr, rows, eps}, false, dtype, stream);
+}
+
+int clusten_merge_table_backward(const float* d_out, const float* table, const float* weight, const float* bias, const float* norm_w,
+                                 const float* norm_b, float eps, float* d_params, int64_t rows, int dtype, clusten_stream stream) {
+    return merge_table_call(MergeTable{table, weight, bias, norm_w, norm_b, d_out, nullptr, d_params, rows, eps}, true, dtype, stream);
+}
+
 int clusten_merge_weights_backward(const float* d_weights, const float* table_weights, const int64_t* pe_idx, const int64_t* nbhd_idx,
                                    const float* prob, const int64_t* mask, float* d_rows, float* d_prob, int B, int N, int Nout, int M,
                                    clusten_stream stream) {

@@ -386,6 +386,20 @@ int launch_position_bias(const float* table, const float* w, const float* b, voi
 size_t position_grad_workspace_bytes(int64_t total, int heads);
 int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void* padded, float* d_w, float* d_b, void* workspace, GradSums* later, int B,
                          int H, int N, int M, int rows, int k, int dtype, hipStream_t stream);
+// The table of merge weights in training and its 32 parameters' gradients (merge_table.hip).
+struct MergeTable {
+    const float* table;    // (rows, 5)
+    const float* weight;   // (4, 5)
+    const float* bias;
+    const float* norm_w;
+    const float* norm_b;
+    const float* d_out;    // (rows, 4)
+    float* out;            // (rows, 4)
+    float* d_params;       // (32): weight, bias, norm_w, norm_b
+    int64_t rows;
+    float eps;
+};
+int launch_merge_table(const MergeTable& a, bool backward, int dtype, hipStream_t stream);
 struct DenseTrain {
     const void* qkv;       // (B, N, 3 C): [q | head 0: k v | head 1: k v ...]
     const void* bias;      // (H, rows)

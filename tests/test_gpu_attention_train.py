@@ -165,3 +165,32 @@ def test_global_attention_of_an_fp32_forward(device, b, n, columns):
         got = attn.attend(q, kv, everyone, None, pe, True, table)
         ref = copy.deepcopy(attn).double().attend(q.double(), kv.double(), everyone, None, pe, True, table.double())
     near(got, ref, BAR[torch.float32])
+
+
+# one row, a workgroup's, one more, several rows a thread
+@pytest.mark.parametrize("rows", [1, 256, 1025, 12321])
+@pytest.mark.parametrize("dt", DTYPES)
+def test_merge_table(device, dt, rows):
+    """Against float64 from the same rounded Linear layer: where a rounding falls the other way a value moves by one of dt, which the norm
+    of four values can blow up, so that 16-bit bars are those of a rounding times ten.  Through the module besides, and differentiated twice."""
+    from aff.model import _weight_table, default_ops
+    gen = torch.Generator(device).manual_seed(rows)
+    net = torch.nn.Sequential(torch.nn.Linear(5, 4), torch.nn.LayerNorm(4), torch.nn.GELU()).to(device)
+    with torch.no_grad():
+        for p in net.parameters():
+            p.copy_(torch.randn(p.shape, generator=gen, device=device))
+    table, d = torch.randn(rows, 5, generator=gen, device=device), torch.randn(rows, 4, generator=gen, device=device)
+    params = (net[0].weight, net[0].bias, net[1].weight, net[1].bias)
+    ref = [p.detach().to(dt if i < 2 else torch.float32).double().requires_grad_() for i, p in enumerate(params)]
+    y = table.to(dt).double() @ ref[0].t() + ref[1]
+    y = y + (y.to(dt).double() - y).detach()
+    y = torch.nn.functional.gelu(torch.nn.functional.layer_norm(y, (4,), ref[2], ref[3], 1e-5))
+    want = torch.autograd.grad(y, ref, d.double())
+    bar = {torch.float32: 1e-5, torch.float16: 4e-3, torch.bfloat16: 3e-2}[dt]
+    for create in (False, True):
+        with torch.autocast("cuda", dtype=torch.float16 if dt == torch.float32 else dt, enabled=dt != torch.float32):
+            out = _weight_table(net, table, default_ops())
+        assert type(out.grad_fn).__name__ == "_MergeTableBackward"
+        near(out, y.detach(), bar)
+        for got, g in zip(torch.autograd.grad(out, params, d, create_graph=create), want):
+            assert got.shape == g.shape and (got - g).norm() <= bar * max(g.norm(), (d.double().norm() ** 2 / 4) ** 0.5)
