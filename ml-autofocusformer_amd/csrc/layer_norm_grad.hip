@@ -5,7 +5,9 @@
 // Bound by its three streams.  A lane takes 8 consecutive channels a step (16-byte accesses), a row L lanes of V steps, so that both row
 // sums are exchanges inside a wave; column sums stay in registers over all rows a lane takes and every workgroup leaves one partial row,
 // added up in a fixed order.  At most 1024 workgroups, four a compute unit.  The framework ran a copy to fp32 and three kernels over fp32
-// rows, one of them for the column sums alone.
+// rows, one of them for the column sums alone.  Kernel time of a training step with this and the forward that keeps statistics, against
+// the framework's: AFF-Tiny at 64 images, fp16 15.65 -> 14.93 ms (200 704 rows of 64 channels at the patch embedding, 50 176 of 256 and
+// fewer, wider ones behind it), 24 images at 256 x 256 10.86 -> 10.43.
 #include "common.hpp"
 #include "launch.hpp"
 
