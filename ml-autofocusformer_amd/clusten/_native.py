@@ -1580,13 +1580,14 @@ def merge_weights_backward(d_weights: torch.Tensor, table_weights: torch.Tensor,
     if (ic != 4 or d_weights.dtype != torch.float32 or table_weights.dtype != torch.float32 or not table_weights.is_contiguous()
             or table_weights.dim() != 2 or table_weights.shape[1] != 4 or table_weights.data_ptr() % 16
             or any(t.shape != (b, n_out, m) or t.dtype != torch.int64 for t in (pe_idx, nbhd_idx))
-            or (prob is not None and (prob.dtype != torch.float32 or not prob.is_contiguous() or prob.dim() != 2 or prob.shape[0] != b))
+            or (prob is not None and (prob.dtype != torch.float32 or prob.dim() != 2 or prob.shape[0] != b))
             or (mask is not None and mask.shape != pe_idx.shape)
             or any(t is not None and t.device != device for t in (table_weights, pe_idx, nbhd_idx, prob, mask))):
         raise RuntimeError("merge_weights_backward: fp32 d_weights (B,N',M,4), table (rows,4), prob (B,N); int64 indices (B,N',M)")
     d_weights, pe_idx, nbhd_idx = d_weights.contiguous(), pe_idx.contiguous(), nbhd_idx.contiguous()
     d_weights = d_weights if d_weights.data_ptr() % 16 == 0 else d_weights.clone()
     mask = None if mask is None else mask.to(torch.int64).contiguous()
+    prob = None if prob is None else prob.contiguous()           # a column of wider rows, say
     d_prob = None if prob is None else torch.empty_like(prob)
     rows = torch.empty(b, 4, n_out, m, dtype=torch.float32, device=device)
     if rows.numel() == 0:

@@ -194,3 +194,33 @@ def test_merge_table(device, dt, rows):
         near(out, y.detach(), bar)
         for got, g in zip(torch.autograd.grad(out, params, d, create_graph=create), want):
             assert got.shape == g.shape and (got - g).norm() <= bar * max(g.norm(), (d.double().norm() ** 2 / 4) ** 0.5)
+
+
+def merging(device, n=48, c=32):
+    """A merge of n tokens that all see each other: the module, scores, and its forward on given scores and mask."""
+    from aff.model import ClusterMerging, default_ops, relative_position_table
+    gen = torch.Generator(device).manual_seed(n)
+    torch.manual_seed(n)
+    merge = ClusterMerging(c, 2 * c, ops=default_ops()).to(device)
+    table = relative_position_table(64)[0].to(device)
+    at = torch.arange(n, device=device)
+    pos = torch.stack([at % 7, at // 7], 1).float().expand(2, n, 2).contiguous()
+    everyone = at.expand(2, n, n).contiguous()
+    pe = torch.randint(table.shape[0], (2, n, n), generator=gen, device=device)
+    feat, score = torch.randn(2, n, c, generator=gen, device=device), torch.rand(2, n, 1, generator=gen, device=device)
+
+    def call(score, mask=None, module=merge):
+        return module(pos, feat, everyone, mask, score, 4, pe, 0, table)[1]
+    return merge, score, call
+
+
+def test_merge_of_strided_scores(device):
+    """Scores that are a column of wider rows, in training: the gradients of the same scores in rows of their own, but for the order of
+    the atomic additions (48 terms a score, 1e-6 of them)."""
+    merge, score, call = merging(device)
+    results = []
+    for s in (score, torch.cat([score, score + 1, score], 2)[..., :1]):
+        s = s.detach().requires_grad_()
+        results.append(torch.autograd.grad(call(s).square().sum(), [s, *merge.parameters()]))
+    for a, b in zip(*results):
+        near(a, b, 1e-5)
