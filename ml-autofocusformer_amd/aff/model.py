@@ -1191,7 +1191,7 @@ class ClusterMerging(_Module):
         mask_rows = None
         if rows_op is not None and self.ops.merge_rows_supported(pos, member_idx, pe_idx):
             # the rows of the per-token tensors at the centres in one launch
-            if cluster_mask is not None and self.ops.merge_rows_supported(cluster_mask):
+            if cluster_mask is not None and not cluster_mask.requires_grad and self.ops.merge_rows_supported(cluster_mask):
                 pos, member_idx, pe_idx, mask_rows = rows_op(centre, pos, member_idx, pe_idx, cluster_mask)
             else:
                 pos, member_idx, pe_idx = rows_op(centre, pos, member_idx, pe_idx)
@@ -1211,7 +1211,7 @@ class ClusterMerging(_Module):
             weights = one_pass(table_w, pe_idx, member_idx, learned_prob, mask_rows)
         elif (one_pass is not None and getattr(self.ops, "merge_weights_backward", None) is not None and torch.is_grad_enabled()
               and learned_prob is not None and table_w.is_cuda and table_w.dtype == torch.float32 and table_w.is_contiguous()
-              and self.ops.merge_weights_supported(table_w) and not _transformed()):
+              and self.ops.merge_weights_supported(table_w) and not _transformed() and not (mask_rows is not None and mask_rows.requires_grad)):
             weights = _MergeWeights.apply(table_w, learned_prob.float().reshape(b, n), pe_idx, member_idx, mask_rows, self.ops)
         else:
             weights = _table_rows(table_w, pe_idx)                                       # (b, n', m, 4)

@@ -1507,7 +1507,8 @@ def merge_weights_supported(table_weights: torch.Tensor) -> bool:
 def merge_weights(table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: torch.Tensor, prob, mask):
     """table_weights[pe_idx] * prob.gather(nbhd_idx) * mask as one (B,N',M,4) fp32 tensor: the weights the WF
     operator takes (models/aff_transformer.py:340-358).  table_weights (rows,4); pe_idx, nbhd_idx (B,N',M) int64;
-    prob (B,N) or (B,N,1) or None; mask (B,N',M) of 0/1 or None.  No autograd: for inference."""
+    prob (B,N) or (B,N,1) or None; mask (B,N',M) of whole numbers, which the kernel reads, or of fractions, or None.  No autograd:
+    for inference."""
     lib = load()
     _require_cuda("table_weights", table_weights)
     device = table_weights.device
@@ -1526,7 +1527,8 @@ def merge_weights(table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: t
         _require_cuda("mask", mask, device)
         if mask.shape != pe_idx.shape:
             raise RuntimeError("mask must have the shape of pe_idx")
-        mask = mask.to(torch.int64).contiguous()
+    fractions = mask.detach() if mask is not None and mask.is_floating_point() else None
+    mask = None if mask is None or fractions is not None else mask.to(torch.int64).contiguous()
     out = torch.empty(b, n_out, m, table_weights.shape[1], dtype=torch.float32, device=device)
     if out.numel() == 0:
         return out
@@ -1535,7 +1537,7 @@ def merge_weights(table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: t
                                                  _ptr(nbhd_idx.contiguous()), _ptr(prob), _ptr(mask), _ptr(out), b, n,
                                                  n_out, m, table_weights.shape[1], _stream(device)),
                "clusten_merge_weights_forward")
-    return out
+    return out if fractions is None else out.mul_(fractions.unsqueeze(3))
 
 
 def merge_table_supported(table: torch.Tensor, weight, bias, norm_w, norm_b, dtype: torch.dtype) -> bool:
@@ -1584,6 +1586,8 @@ def merge_weights_backward(d_weights: torch.Tensor, table_weights: torch.Tensor,
             or (mask is not None and mask.shape != pe_idx.shape)
             or any(t is not None and t.device != device for t in (table_weights, pe_idx, nbhd_idx, prob, mask))):
         raise RuntimeError("merge_weights_backward: fp32 d_weights (B,N',M,4), table (rows,4), prob (B,N); int64 indices (B,N',M)")
+    if mask is not None and mask.is_floating_point():            # fractions: the kernel reads whole numbers
+        d_weights, mask = (d_weights * mask.unsqueeze(3)).float(), None
     d_weights, pe_idx, nbhd_idx = d_weights.contiguous(), pe_idx.contiguous(), nbhd_idx.contiguous()
     d_weights = d_weights if d_weights.data_ptr() % 16 == 0 else d_weights.clone()
     mask = None if mask is None else mask.to(torch.int64).contiguous()

@@ -224,3 +224,28 @@ def test_merge_of_strided_scores(device):
         results.append(torch.autograd.grad(call(s).square().sum(), [s, *merge.parameters()]))
     for a, b in zip(*results):
         near(a, b, 1e-5)
+
+
+def layered(merge):
+    """The same merge, its weights by recorded operations."""
+    import copy
+    other = copy.deepcopy(merge)
+    other.ops = type(other.ops)(**{**vars(other.ops), "merge_weights": None})
+    return other
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.float64])
+def test_merge_with_a_mask_of_fractions(device, dt):
+    """A mask that is no table of 0 and 1, in inference and in training, as a constant and as what takes a gradient itself."""
+    merge, score, call = merging(device)
+    mask = torch.rand(2, 48, 48, generator=torch.Generator(device).manual_seed(1), device=device).to(dt)
+    with torch.no_grad():
+        near(call(score, mask), call(score, mask.float(), layered(merge)), 1e-5)
+    results = []
+    for module in (merge, layered(merge)):
+        s, m = score.clone().requires_grad_(), mask.float().requires_grad_()
+        constant = mask if module is merge else mask.float()
+        results.append(torch.autograd.grad(call(s, constant, module).square().sum(), [s, *module.parameters()])
+                       + torch.autograd.grad(call(s, m, module).square().sum(), [m, s]))
+    for a, b in zip(*results):
+        near(a, b, 1e-5)
