@@ -249,3 +249,30 @@ def test_merge_with_a_mask_of_fractions(device, dt):
                        + torch.autograd.grad(call(s, m, module).square().sum(), [m, s]))
     for a, b in zip(*results):
         near(a, b, 1e-5)
+
+
+def test_merge_under_deterministic_algorithms(device):
+    """The scores' gradient is made of atomic additions: not where the caller asked for the same bits every time."""
+    merge, score, call = merging(device)
+    s, routes, grads = score.clone().requires_grad_(), [], []
+    for _ in range(2):
+        torch.use_deterministic_algorithms(True, warn_only=True)
+        try:
+            out = call(s)
+            grads.append(torch.autograd.grad(out.square().sum(), s, retain_graph=True)[0])
+        finally:
+            torch.use_deterministic_algorithms(False)
+        routes.append([f for f in walk(out.grad_fn) if type(f).__name__ == "_MergeWeightsBackward"])
+    assert not any(routes) and torch.equal(*grads)
+    out = call(s)
+    assert any(type(f).__name__ == "_MergeWeightsBackward" for f in walk(out.grad_fn))
+
+
+def walk(node):
+    seen, todo = set(), [node]
+    while todo:
+        f = todo.pop()
+        if f is not None and f not in seen:
+            seen.add(f)
+            todo += [g for g, _ in f.next_functions]
+    return seen
