@@ -553,7 +553,7 @@ int clusten_bias_table_grad(const void* d_logit, const int64_t* pe_idx, float* d
  * (models/aff_transformer.py:340-358), in one pass instead of a row lookup, a gather and two multiplications:
  *   weights[b,i,j,:] = table_weights[pe_idx[b,i,j], :] * prob[b, nbhd_idx[b,i,j]] * mask[b,i,j]
  * table_weights (rows,IC), prob (B,N) or NULL, weights (B,Nout,M,IC): fp32, contiguous; pe_idx (values in
- * [0,rows) — unchecked), nbhd_idx (values in [0,N) — unchecked; may be NULL when prob is), mask (0/1, or NULL):
+ * [0,rows) — unchecked), nbhd_idx (values in [0,N), others give NaN; may be NULL when prob is), mask (0/1, or NULL):
  * int64 (B,Nout,M).  IC = 4 (else CLUSTEN_ERR_BAD_DIMS); table_weights and weights 16-byte aligned (else
  * CLUSTEN_ERR_UNALIGNED).  Inference only.  No counterpart in the reference's extension modules. */
 int clusten_merge_weights_forward(const float* table_weights, const int64_t* pe_idx, const int64_t* nbhd_idx,
@@ -800,7 +800,7 @@ int clusten_merge_table_backward(const float* d_out, const float* table, const f
 /* Training passes around a merge (models/aff_transformer.py:340-358, 496-500 under autograd).
  *   merge_weights_backward, of clusten_merge_weights_forward: d_rows (B,4,Nout,M) = d_weights (B,Nout,M,4) * prob * mask, which
  *     clusten_bias_table_grad (H = 4, the same pe_idx) sums into the table's rows, and, with prob, d_prob (B,N), written in full (fp32
- *     atomics).
+ *     atomics).  A neighbour outside [0,N) gives NaN in d_rows and nothing to d_prob.
  *   row_score: score (rows) of dtype = sigmoid(x w + bias), operands, the sum and the result rounded to dtype; x (rows,C) of x_dtype (F32
  *     or dtype), C in {32,64,128,256,512}, w (C) and bias (1, may be NULL) fp32.  The backward: d_x of x_dtype, d_weight (C), d_bias (C floats,
  *     the first is the bias' gradient); workspace: clusten_row_sums_workspace_bytes(rows, C). */

@@ -25,10 +25,12 @@ __global__ __launch_bounds__(256) void merge_weights_backward_kernel(const float
     const float m = mask ? (float)mask[e] : 1.f;
     float s = m;
     if (prob) {
-        const int64_t row = image * N + nbhd_idx[e];
-        s *= prob[row];
+        const int64_t nb = nbhd_idx[e];
+        const bool inside = (uint64_t)nb < (uint64_t)N;      // a neighbour outside the image has no score: NaN, as in the forward
+        const int64_t row = image * N + nb;
+        s *= inside ? prob[row] : NAN;
         const float4 w = *reinterpret_cast<const float4*>(table_w + pe_idx[e] * 4);
-        if (m != 0.f) unsafeAtomicAdd(d_prob + row, m * ((d.x * w.x + d.y * w.y) + (d.z * w.z + d.w * w.w)));
+        if (inside && m != 0.f) unsafeAtomicAdd(d_prob + row, m * ((d.x * w.x + d.y * w.y) + (d.z * w.z + d.w * w.w)));
     }
     float* to = t + image * 4 * per_image + place;
     to[0] = d.x * s, to[per_image] = d.y * s, to[2 * per_image] = d.z * s, to[3 * per_image] = d.w * s;

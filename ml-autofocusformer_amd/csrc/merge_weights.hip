@@ -22,7 +22,10 @@ __global__ __launch_bounds__(256) void merge_weights_kernel(const float* __restr
     if (e >= pairs) return;
     float4 w = *reinterpret_cast<const float4*>(table_w + pe_idx[e] * 4);
     float s = 1.f;
-    if (prob) s = prob[(e / pairs_per_batch) * N + nbhd_idx[e]];
+    if (prob) {
+        const int64_t nb = nbhd_idx[e];
+        s = (uint64_t)nb < (uint64_t)N ? prob[(e / pairs_per_batch) * N + nb] : NAN;
+    }
     if (mask) s *= (float)mask[e];
     w.x *= s, w.y *= s, w.z *= s, w.w *= s;
     *reinterpret_cast<float4*>(out + e * 4) = w;   // plain: the merge kernel reads it next

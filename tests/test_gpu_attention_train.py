@@ -196,6 +196,26 @@ def test_merge_table(device, dt, rows):
             assert got.shape == g.shape and (got - g).norm() <= bar * max(g.norm(), (d.double().norm() ** 2 / 4) ** 0.5)
 
 
+def test_merge_weights_of_neighbours_outside(device):
+    """Neighbours that are no token: NaN where they stand, nothing read or written there, every other value as without them."""
+    gen = torch.Generator(device).manual_seed(2)
+    b, n, n_out, m, rows = 2, 50, 12, 48, 225
+    table, prob = torch.randn(rows, 4, generator=gen, device=device), torch.rand(b, n, generator=gen, device=device)
+    pe, idx = (torch.randint(k, (b, n_out, m), generator=gen, device=device) for k in (rows - 1, n))
+    d = torch.randn(b, n_out, m, 4, generator=gen, device=device)
+    bad = idx.clone()
+    bad[0, 3, 5], bad[1, 11, 47], bad[1, 0, 0] = n, -1, 1 << 40
+    out, pe_bad = bad != idx, pe.clone()
+    pe_bad[out] = rows - 1                                       # a row of the table of their own
+    got, want = _native.merge_weights(table, pe_bad, bad, prob, None), _native.merge_weights(table, pe_bad, idx, prob, None)
+    assert got[out].isnan().all() and torch.equal(got[~out], want[~out])
+    d_table, d_prob = _native.merge_weights_backward(d, table, pe_bad, bad, prob, None)
+    masked = _native.merge_weights_backward(d, table, pe_bad, idx, prob, (~out).long())
+    assert d_table[-1].isnan().all()
+    near(d_table[:-1], masked[0][:-1], 5e-7)
+    near(d_prob, masked[1], 5e-7)
+
+
 def merging(device, n=48, c=32):
     """A merge of n tokens that all see each other: the module, scores, and its forward on given scores and mask."""
     from aff.model import ClusterMerging, default_ops, relative_position_table
