@@ -736,7 +736,8 @@ int clusten_norm_linear_backward(const void* d_y, const void* x, int x_dtype, co
  *     per head k and v; out (B,N,C); bias and padded of position_bias, pe_idx (B,N,N); fp32 inside.  The backward writes all of d_qkv and
  *     the gradients of the blank token (C) and of the position bias layer.
  *   scatter_attention_pair: d_key = scale * scatter(d_logit, query) and d_value = scatter(probs, d_out) over pair_lists
- *     (clusten_cluster_pairs_from_numbers) in one launch; d_key and d_value have out_strides. */
+ *     (clusten_cluster_pairs_from_numbers) in one launch; d_key and d_value have out_strides.  Lists that are not whole clusters (their
+ *     flag is set: a number outside the sequence, or clusten_cluster_pairs of other lists) make both NaN. */
 int clusten_position_bias(const float* table, const float* weight, const float* bias_param, void* bias, void* padded, int rows,
                           int n, int k, int dtype, clusten_stream stream);
 size_t clusten_position_grad_workspace_bytes(int B, int H, int N, int M);
@@ -760,7 +761,8 @@ int clusten_scatter_attention_pair(const void* d_logit, const void* query, clust
 /* The training pass of a whole block (models/aff_transformer.py:181-232) by one call a direction: the launches of the entry points
  * above and of clusten_cluster_attention_forward_train / _backward, clusten_weight_grad and clusten_blank_grad, in order.
  *   shape: B images of N tokens, H heads of C = 32 channels (H * C a built width), M = 48 with a plan.  Local attention with `plan`
- *     (clusten_cluster_attention_plan) and, backward, `pair_lists`; with plan = NULL every token attends to all N <= 64.
+ *     (clusten_cluster_attention_plan) and, backward, `pair_lists` of the same cluster numbers, every one of them inside the sequence (lists
+ *     that are not whole clusters make the keys' and values' gradients NaN); with plan = NULL every token attends to all N <= 64.
  *   param: norm1 weight, bias; norm2 weight, bias; biases of q, kv, proj, fc1, fc2; blank key, blank value; weights of q, kv, proj, fc1,
  *     fc2; position bias layer's weight, bias: fp32, on 16-byte boundaries.  grad: the same order (backward), fp32; the five weights and
  *     their biases may be NULL, the bias with its weight.

@@ -44,7 +44,7 @@ struct Scatters {
     Scatter job[2];
 };
 
-template <typename T, int C>
+template <typename T, int C, bool PAIR>
 __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs, const int32_t* __restrict__ starts,
                                                                    const int32_t* __restrict__ ends,
                                                                    const int32_t* __restrict__ pairs,
@@ -80,10 +80,21 @@ __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs
     const int flagged = not_whole != nullptr ? *not_whole : 0;
     const int first = starts[unit];
     const int last = ends[unit];
-    if (flagged != 0) return;   // not lists of whole clusters: the atomic kernels run instead
     const int b = unit / clusters_per_image;
     const int g = unit - b * clusters_per_image;
     const int lane = threadIdx.x;
+    if (flagged != 0) {         // not lists of whole clusters
+        if constexpr (PAIR) {   // nothing else writes these rows: NaN, so that it shows
+            const float v[4] = {NAN, NAN, NAN, NAN};
+            const int quads = min(8, N - 8 * g) * (C / 4);
+            for (int i = h_first * quads + lane; i < h_last * quads; i += kWave) {
+                const int h = i / quads, q = i - h * quads;
+                T* row = y + (int64_t)b * ys.b + (int64_t)h * ys.h + (int64_t)(g * 8 + q / (C / 4)) * ys.n;
+                *reinterpret_cast<typename Quad<T>::raw*>(row + q % (C / 4) * 4) = Quad<T>::pack(v);
+            }
+        }
+        return;                 // a single scatter: the atomic kernels run instead
+    }
     const int r16 = lane & 15, kq = lane >> 4;
     const int count = last - first;
     int* list = reinterpret_cast<int*>(stage + L_BASE);
@@ -190,8 +201,14 @@ int launch_typed_c(const Scatters& jobs, int count, const int32_t* starts, const
     const int per_image = (s.N + 7) / 8;
     const int64_t total = (int64_t)s.B * per_image;
     if (total >= ((int64_t)1 << 30)) return CLUSTEN_ERR_BAD_DIMS;
-    hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C>), dim3(xcd_grid((int)total), head_shares(total * count, s.H), count), dim3(kWave), 0, stream,
-                       jobs, starts, ends, pairs, not_whole, s.H, s.N, s.M, per_image, (int)total);
+    const dim3 grid(xcd_grid((int)total), head_shares(total * count, s.H), count);
+    if (count == 2) {
+        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, true>), grid, dim3(kWave), 0, stream, jobs, starts, ends, pairs, not_whole, s.H, s.N, s.M,
+                           per_image, (int)total);
+    } else {
+        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, false>), grid, dim3(kWave), 0, stream, jobs, starts, ends, pairs, not_whole, s.H, s.N,
+                           s.M, per_image, (int)total);
+    }
     return launch_status();
 }
 

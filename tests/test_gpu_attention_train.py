@@ -113,6 +113,25 @@ def test_rows_of_an_attention_layer(device, dt, b, h, n, ch):
     near(d_bv, (blank.double().unsqueeze(-1) * g.double()).sum((0, 2)).reshape(-1), 5e-6)
 
 
+# head shares of a cluster: all heads to one workgroup, and one each
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("b,h,n,ch", [(2, 2, 101, 32), (1, 8, 8, 16), (40, 2, 3999, 32)])
+def test_rows_of_lists_that_are_not_whole_clusters(device, dt, b, h, n, ch):
+    """A cluster number outside the sequence, and lists of any rows: NaN in every key and value column, nothing left as it was."""
+    gen = torch.Generator(device).manual_seed(1)
+    c, m = h * ch, 8
+    qkv, d_out = torch.randn(b, n, 3 * c, generator=gen, device=device).to(dt), torch.randn(b, n, c, generator=gen, device=device).to(dt)
+    probs, d_logit = (torch.randn(b, h, n, m, generator=gen, device=device).to(dt) for _ in range(2))
+    blank = torch.rand(b, h, n, generator=gen, device=device)
+    numbers = torch.randint((n + 7) // 8, (b, n, 1), generator=gen, device=device).int()
+    numbers[-1, n // 2, 0] = (n + 7) // 8
+    lists = torch.randint(n, (b, n, m), generator=gen, device=device)
+    for pairs in (_native.cluster_pairs_from_numbers(numbers), _native.cluster_pairs(lists)):
+        d_qkv = torch.full_like(qkv, 7.0)
+        _native.attention_rows_backward(qkv, d_qkv, probs, d_logit, d_out, blank, blank, pairs, 0.3)
+        assert (d_qkv[..., :c] == 7.0).all() and d_qkv[..., c:].isnan().all()
+
+
 @pytest.mark.parametrize("b,n,n_out,m,rows,masked", [(1, 1, 1, 1, 1, False), (2, 50, 12, 48, 225, True), (3, 777, 194, 49, 12321, False)])
 def test_merge_weights(device, b, n, n_out, m, rows, masked):
     gen = torch.Generator(device).manual_seed(n)
