@@ -76,6 +76,7 @@ def default_ops():
                            weight_grad=_native.weight_grad, weight_grad_supported=_native.weight_grad_supported,
                            block_tail_backward=_native.block_tail_backward, norm_linear_backward=_native.norm_linear_backward,
                            cluster_pairs_from_numbers=_native.cluster_pairs_from_numbers,
+                           cluster_pairs_from_numbers_stands_for=(("cluster_pairs", _native.cluster_pairs),),
                            block_train_forward=_native.block_train_forward, block_train_backward=_native.block_train_backward,
                            block_train_supported=_native.block_train_supported,
                            block_train_stands_for=(("norm_linear", _native.norm_linear), ("block_tail", _native.block_tail),
@@ -83,7 +84,8 @@ def default_ops():
                                                    ("cluster_attention_backward", _native.cluster_attention_backward),
                                                    ("norm_linear_backward", _native.norm_linear_backward),
                                                    ("block_tail_backward", _native.block_tail_backward),
-                                                   ("scatter_rows", _native.scatter_rows), ("weight_grad", _native.weight_grad)),
+                                                   ("scatter_rows", _native.scatter_rows), ("weight_grad", _native.weight_grad),
+                                                   ("block_pack", _native.block_pack), ("bias_table_grad", _native.bias_table_grad)),
                            blocks_forward=_native.blocks_forward, block_params=_native.BlockParams,
                            blocks_stand_for=(("cluster_attention", _native.cluster_attention),
                                              ("dense_attention", _native.dense_attention),
@@ -1429,6 +1431,8 @@ class BasicLayer(_Module):
             # backward's scatters, built once for all blocks of the stage (a grid stage hands over one image's lists)
             # from the numbers, which the forward reads: lists of whole clusters by construction
             from_numbers = getattr(self.ops, "cluster_pairs_from_numbers", None)
+            if any(getattr(self.ops, name, None) is not fn for name, fn in getattr(self.ops, "cluster_pairs_from_numbers_stands_for", ())):
+                from_numbers = None
             pairs = self.ops.cluster_pairs(member_idx) if from_numbers is None else from_numbers(cluster_idx)
             if pairs is not None:
                 lists = grid_lists if grid_lists is not None else (cluster_idx, pe_idx, mask)

@@ -460,6 +460,25 @@ def test_frozen_parameters(device, dt, local):
         assert (got is None) if name != "x" and name.endswith(frozen) else torch.equal(got, ref), name
 
 
+@pytest.mark.parametrize("name", ["block_pack", "bias_table_grad", "cluster_pairs", "cluster_attention_plan", "norm_linear", "scatter_rows"])
+def test_replaced_operations_are_called_in_training(device, name):
+    """What a caller put in the place of an operation that a native call for a whole block stands for, with the same gradients."""
+    calls = []
+
+    def counted(*args, **kwargs):
+        calls.append(name)
+        return getattr(_native, name)(*args, **kwargs)
+
+    results = []
+    for ops in (default_ops(), SimpleNamespace(**{**vars(default_ops()), name: counted})):
+        stage, feat, call = local_stage(device, ops)
+        x = feat.clone().requires_grad_(True)
+        results.append(torch.autograd.grad(call(x).square().sum(), [x, *stage.parameters()]))
+    assert calls
+    for got, ref in zip(*results):
+        assert norm_error(got, ref) < 1e-5
+
+
 # every width; a row, a workgroup's rows and one more, and more rows than all workgroups take at once
 @pytest.mark.parametrize("c,rows", [(64, 1), (64, 33), (64, 40000), (128, 17), (256, 9), (384, 1025), (512, 4101), (768, 8), (1024, 5000)])
 @pytest.mark.parametrize("dt,dy", [(torch.float32, torch.float32), (torch.float32, torch.float16), (torch.float32, torch.bfloat16),
