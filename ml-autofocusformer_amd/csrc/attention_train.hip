@@ -172,6 +172,13 @@ __device__ __forceinline__ void weighted_rows(const float* m, const float* x, in
     }
 }
 
+// exp for results of type T.  The short form rounds its argument times log2 e to fp32: 2e-6 of the result 50 below the maximum, which
+// 16-bit results do not show and fp32 ones do.
+template <typename T>
+__device__ __forceinline__ float exponential(float x) {
+    return sizeof(T) == 4 ? expf(x) : __expf(x);
+}
+
 // Probabilities of the rows and of the blank token (p, blank) from q, k in LDS.
 template <typename T>
 __device__ __forceinline__ void probabilities(const DenseTrain& a, int image, int head, const float* q, const float* k, float* p, float* blank) {
@@ -206,10 +213,10 @@ __device__ __forceinline__ void probabilities(const DenseTrain& a, int image, in
     top = fmaxf(top, __shfl_xor(top, 2));
     float sum = 0.f;
 #pragma unroll
-    for (int c = 0; c < kTokens / 4; ++c) v[c] = __expf(v[c] - top), sum += v[c];
+    for (int c = 0; c < kTokens / 4; ++c) v[c] = exponential<T>(v[c] - top), sum += v[c];
     sum += __shfl_xor(sum, 1);
     sum += __shfl_xor(sum, 2);
-    z = __expf(z - top);
+    z = exponential<T>(z - top);
     const float inv = 1.f / (sum + z);
 #pragma unroll
     for (int c = 0; c < kTokens / 4; ++c) p[row * kSPitch + part + 4 * c] = v[c] * inv;

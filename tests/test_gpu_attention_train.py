@@ -89,6 +89,22 @@ def test_dense_attention(device, dt, b, h, n):
     assert ((got[4].double() - d_b).abs() <= 2e-6 * size).all()
 
 
+def test_exponential_of_fp32_global_attention(device):
+    """Scores far below a row's maximum.  With q = 0 they are the table's values; token i sees the blank token (score 0, value 0) and one
+    other at -40 - 0.789 i, so that its result is that exponential: one of 1 ulp (2^-23), a sum, a reciprocal and two products rounded
+    once each, 2^-23 + 4 * 2^-24.  An exponential whose argument times log2 e is rounded is off by 3.4e-6."""
+    n, h = 48, 2
+    scores = torch.cat([torch.tensor([-1000.0]), -40 - 0.789 * torch.arange(n)]).to(device)
+    pe, at = torch.zeros(1, n, n, dtype=torch.int64, device=device), torch.arange(n, device=device)
+    pe[0, at, at] = at + 1
+    qkv = torch.zeros(1, n, 96 * h, device=device)
+    qkv[..., 32 * h:].view(1, n, h, 2, 32)[..., 1, :] = 1.0
+    blank = torch.zeros(32 * h, device=device)
+    out = _native.dense_attention_train(qkv, scores.expand(h, n + 1).contiguous(), pe, blank, blank, h, 1.0)
+    ref = (scores[1:].double().exp() / (1 + scores[1:].double().exp())).view(1, n, 1)
+    assert ((out.double() - ref).abs() <= 3 * 2 ** -23 * ref).all()
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("b,h,n,ch", [(1, 1, 8, 32), (2, 4, 100, 32), (3, 2, 203, 16), (1, 8, 777, 32), (2, 2, 64, 64)])
 def test_rows_of_an_attention_layer(device, dt, b, h, n, ch):
