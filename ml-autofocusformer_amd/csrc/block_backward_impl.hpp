@@ -203,7 +203,7 @@ __global__ __launch_bounds__((64 * BlockCfg<T, C>::kWaves), 2) void block_tail_b
         // act has been read to the end: its last product lies ahead of the barriers of the hidden layer and the row totals
 #pragma unroll
         for (int t = 0; t < TR; ++t) {
-            const float s = a.scale ? a.scale[(uint32_t)row[t] / (uint32_t)a.rows_per_image] : 1.f;
+            const float s = a.scale ? to_acc(from_acc<T>(a.scale[(uint32_t)row[t] / (uint32_t)a.rows_per_image])) : 1.f;     // as the forward rounds it
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 const int64_t to = row[t] * C + ch0 + f * Cfg::kStep;

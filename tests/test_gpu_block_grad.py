@@ -479,6 +479,29 @@ def test_replaced_operations_are_called_in_training(device, name):
         assert norm_error(got, ref) < 1e-5
 
 
+@pytest.mark.parametrize("dt,stream", [(torch.float16, torch.float16), (torch.float16, torch.float32), (torch.bfloat16, torch.float32),
+                                       (torch.float32, torch.float32)])
+def test_factors_that_are_no_numbers_of_the_type(device, dt, stream):
+    """Factors that fp16 and bf16 do not hold: both branches' are rounded to the type, in the backward as in the forward."""
+    gen = torch.Generator(device).manual_seed(7)
+    b, n, c, hidden = 3, 33, 64, 128
+
+    def draw(*shape):
+        return torch.randn(*shape, generator=gen, device=device)
+
+    w_p, w_1, w_2 = draw(c, c) / 8, draw(hidden, c) / 8, draw(c, hidden) / 11
+    packed, at = _native.block_pack(c, dt, [(w, t) for t in (False, True) for w in (w_p, w_1, w_2)])
+    x, d_out, attn = draw(b, n, c).to(stream), draw(b, n, c).to(stream), draw(b, n, c).to(dt)
+    norm_w, norm_b, zero = 1 + 0.2 * draw(c), draw(c), torch.zeros(hidden, device=device)
+    scale = torch.tensor([[1 / 0.9, 1 / 0.7, 0.0], [1 / 0.6, 0.0, 1 / 0.9]], device=device)
+    results = []
+    for s in (scale, scale.to(dt).float()):
+        out, x1, normed, hid, stats = _native.block_tail(attn, x, packed, at[:3], zero[:c], norm_w, norm_b, 1e-5, zero, zero[:c], s, keep=True)
+        results.append((out, x1) + tuple(_native.block_tail_backward(d_out, x1, stats, norm_w, hid, packed, at[3:], s)))
+    for got, ref in zip(*results):
+        assert torch.equal(got, ref)
+
+
 # every width; a row, a workgroup's rows and one more, and more rows than all workgroups take at once
 @pytest.mark.parametrize("c,rows", [(64, 1), (64, 33), (64, 40000), (128, 17), (256, 9), (384, 1025), (512, 4101), (768, 8), (1024, 5000)])
 @pytest.mark.parametrize("dt,dy", [(torch.float32, torch.float32), (torch.float32, torch.float16), (torch.float32, torch.bfloat16),
