@@ -8,7 +8,7 @@
 // position_grad: d_W (heads, k) = sum d_logit[b,h,i,j] table[pe_idx[b,i,j]], d_b = sum d_logit.  The gradient of the bias of every table row
 // need not be formed (a scatter into 12 000 rows, then a product over them: 23 + 20 us a layer of AFF-Tiny at 64 images, now 14 + 5): a
 // value meets its row of the table directly.  Every lane sums in double, so that nothing is lost where positive and negative values cancel;
-// partial sums are added in a fixed order.
+// partial sums, doubles too, are added in a fixed order.  The same holds for these sums of global attention below.
 //
 // dense_attention_train / _backward: one workgroup per image and head, everything in LDS as fp32, fp32 arithmetic on the vector unit: 49
 // tokens of 32 channels are 0.3 MFLOP a product, and the five products of a backward are bound by the reads of their operands from LDS.
@@ -118,6 +118,8 @@ __global__ __launch_bounds__(256) void position_grad_kernel(const T* __restrict_
 constexpr int kTokens = 64, kCh = 32, kPitch = kCh + 4, kSPitch = kTokens + 4;     // pitches in floats: 16-byte rows, spread over the banks
 constexpr int kDenseThreads = 256;
 constexpr int kDenseSums = 2 * kCh + kGradSums;      // partial sums of an image and head: blank key, blank value, position bias layer
+constexpr int kDensePitch = 2 * kCh + 2 * kGradSums; // their floats: the last kind in double, from which an even place starts
+static_assert(kCh % 2 == 0 && kDensePitch % 2 == 0, "doubles on 8-byte boundaries");
 
 template <typename T>
 __device__ __forceinline__ void rows_to_lds(const T* __restrict__ src, int64_t pitch, int n, float* dst) {
@@ -253,7 +255,7 @@ template <typename T>
 __global__ __launch_bounds__(kDenseThreads) void dense_train_backward_kernel(DenseTrain a) {
     __shared__ __attribute__((aligned(16))) float q[kTokens * kPitch], k[kTokens * kPitch], v[kTokens * kPitch], g[kTokens * kPitch];
     __shared__ __attribute__((aligned(16))) float p[kTokens * kSPitch], ds[kTokens * kSPitch], blank[kTokens], d_blank[kTokens];
-    __shared__ float sums[4][kGradSums];
+    __shared__ double sums[4][kGradSums];
     const int image = blockIdx.x / a.H, head = blockIdx.x - image * a.H, C = a.H * kCh;
     const T* rows = static_cast<const T*>(a.qkv) + (int64_t)image * a.N * 3 * C;
     rows_to_lds(rows + head * kCh, 3 * C, a.N, q);
@@ -308,10 +310,10 @@ __global__ __launch_bounds__(kDenseThreads) void dense_train_backward_kernel(Den
 #pragma unroll
     for (int j = 0; j < kGradSums; ++j) {
         for (int o = 32; o > 0; o >>= 1) pos[j] += __shfl_xor(pos[j], o);
-        if (lane == 0) sums[wave][j] = (float)pos[j];
+        if (lane == 0) sums[wave][j] = pos[j];
     }
     __syncthreads();
-    float* partial = a.partial + (int64_t)blockIdx.x * kDenseSums;
+    float* partial = a.partial + (int64_t)blockIdx.x * kDensePitch;
     const int ty = threadIdx.x >> 3, tx = threadIdx.x & 7;
     T* to = static_cast<T*>(a.d_qkv) + (int64_t)image * a.N * 3 * C;
     const auto store = [&](const float (&x)[2][4], int column, float scale) {
@@ -344,7 +346,7 @@ __global__ __launch_bounds__(kDenseThreads) void dense_train_backward_kernel(Den
         partial[threadIdx.x] = threadIdx.x < kCh ? s * a.scale : s;
     } else if (threadIdx.x < kDenseSums) {
         const int j = threadIdx.x - 2 * kCh;
-        partial[threadIdx.x] = (sums[0][j] + sums[1][j]) + (sums[2][j] + sums[3][j]);
+        reinterpret_cast<double*>(partial + 2 * kCh)[j] = (sums[0][j] + sums[1][j]) + (sums[2][j] + sums[3][j]);
     }
 }
 
@@ -355,7 +357,10 @@ __global__ __launch_bounds__(256) void dense_sums_kernel(const float* __restrict
     const int head = blockIdx.x, col = threadIdx.x & 127, half = threadIdx.x >> 7;
     double s = 0.;
     if (col < kDenseSums) {
-        for (int b = half; b < images; b += 2) s += (double)partial[((int64_t)b * heads + head) * kDenseSums + col];
+        for (int b = half; b < images; b += 2) {
+            const float* row = partial + ((int64_t)b * heads + head) * kDensePitch;
+            s += col < 2 * kCh ? (double)row[col] : reinterpret_cast<const double*>(row + 2 * kCh)[col - 2 * kCh];
+        }
     }
     sums[half][col] = s;
     __syncthreads();
@@ -409,7 +414,7 @@ int launch_position_grad(const void* d_logit, const int64_t* pe_idx, const void*
     return st ? st : add_up(PositionSums{partial, d_w, d_b, groups, H, k}, later, stream);
 }
 
-size_t dense_train_workspace_bytes(int B, int H) { return (size_t)B * H * kDenseSums * sizeof(float); }
+size_t dense_train_workspace_bytes(int B, int H) { return (size_t)B * H * kDensePitch * sizeof(float); }
 
 int launch_dense_train(const DenseTrain& a, int dtype, hipStream_t stream) {
     return on_type(dtype, [&](auto t) {

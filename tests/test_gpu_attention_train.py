@@ -105,6 +105,21 @@ def test_exponential_of_fp32_global_attention(device):
     assert ((out.double() - ref).abs() <= 3 * 2 ** -23 * ref).all()
 
 
+def test_position_gradient_of_global_attention_cancels(device):
+    """Terms that cancel but for 2^-26 of them: uniform probabilities of 1/64 and powers of two, so that every product is exact and a sum in
+    double is too.  Two images of 63 tokens; the large terms stand in rows that different waves add up."""
+    n, table = 63, torch.zeros(64, 5)
+    table[1, :2] = torch.tensor([1.0, 0.5])
+    pe, qkv, d_out = torch.zeros(2, n, n, dtype=torch.int64), torch.zeros(2, n, 96), torch.zeros(2, n, 32)
+    pe[:, :, 0] = 1
+    qkv[:, 0, 64], qkv[:, 1, 64] = 1.0, -1.0
+    d_out[:, 0, 0], d_out[:, 1, 0], d_out[:, 16, 0] = 2.0 ** 26, 1.0, -2.0 ** 26
+    table, pe, qkv, d_out, blank = (t.to(device) for t in (table, pe, qkv, d_out, torch.zeros(32)))
+    bias, padded = _native.position_bias(table, torch.zeros(1, 5, device=device), None, torch.float32)
+    got = _native.dense_attention_train_backward(qkv, bias, padded, pe, blank, blank, d_out, 5, 1, 1.0)
+    assert got[3].tolist() == [[2 / 64, 1 / 64, 0, 0, 0]] and got[4].tolist() == [0]
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("b,h,n,ch", [(1, 1, 8, 32), (2, 4, 100, 32), (3, 2, 203, 16), (1, 8, 777, 32), (2, 2, 64, 64)])
 def test_rows_of_an_attention_layer(device, dt, b, h, n, ch):
