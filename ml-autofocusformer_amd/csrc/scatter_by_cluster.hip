@@ -32,7 +32,8 @@ constexpr int kListMax = 256;    // pairs of a cluster held in LDS at a time
 constexpr int kPadEntry = 1 << 30;   // list entry flag: the pair names the short last cluster; here, for its pad slots
 constexpr int kEntryMask = kPadEntry - 1;
 
-// One scatter: y += scale * ..., the rows of y strided.  A launch takes up to two over the same lists (d_key and d_value).
+// One scatter: y += scale * ..., the rows of y strided.  A launch takes two over the same lists (d_key and d_value: PAIR), or one, whose y
+// is contiguous and whose scale is 1 (with the pair's addressing it was some tenths of a per cent slower).
 struct Scatter {
     const void* p;
     const void* x;
@@ -51,7 +52,7 @@ __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs
                                                                    const int32_t* __restrict__ not_whole,
                                                                    int H, int N, int M, int clusters_per_image,
                                                                    int total_clusters) {
-    const Scatter& job = jobs.job[blockIdx.z];
+    const Scatter& job = jobs.job[PAIR ? blockIdx.z : 0];
     const T* __restrict__ p = static_cast<const T*>(job.p);
     const T* __restrict__ x = static_cast<const T*>(job.x);
     T* __restrict__ y = static_cast<T*>(job.y);
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs
             }
         }
         // rows 4*kq + j of the result (kq < 2: the cluster's 8 rows), channels 16*cb + r16
-        T* y_rows = y + (int64_t)b * ys.b + (int64_t)h * ys.h + (int64_t)g * 8 * ys.n;
+        T* y_rows = PAIR ? y + (int64_t)b * ys.b + (int64_t)h * ys.h + (int64_t)g * 8 * ys.n : y + (((int64_t)b * H + h) * N + (int64_t)g * 8) * C;
         lds_sync();
         if (kq < 2) {
 #pragma unroll
@@ -182,8 +183,13 @@ __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs
             const int q = q0 + lane;
             if (q < 8 * C / 4 && q / (C / 4) < rows_here) {
                 const F32x4 o = *reinterpret_cast<const F32x4*>(stage + O_BASE + q * 16);
-                const float v[4] = {o[0] * job.scale, o[1] * job.scale, o[2] * job.scale, o[3] * job.scale};
-                *reinterpret_cast<typename Quad<T>::raw*>(y_rows + (int64_t)(q / (C / 4)) * ys.n + q % (C / 4) * 4) = Quad<T>::pack(v);
+                if constexpr (PAIR) {
+                    const float v[4] = {o[0] * job.scale, o[1] * job.scale, o[2] * job.scale, o[3] * job.scale};
+                    *reinterpret_cast<typename Quad<T>::raw*>(y_rows + (int64_t)(q / (C / 4)) * ys.n + q % (C / 4) * 4) = Quad<T>::pack(v);
+                } else {
+                    const float v[4] = {o[0], o[1], o[2], o[3]};
+                    *reinterpret_cast<typename Quad<T>::raw*>(y_rows + q * 4) = Quad<T>::pack(v);
+                }
             }
         }
     }
@@ -249,9 +255,7 @@ int launch_scatter_by_cluster(const void* p, const void* x, clusten_strides xs, 
                               hipStream_t stream) {
     if ((s.C != 16 && s.C != 32 && s.C != 64) || s.N < 8 || s.M % 8 != 0 || s.M > kPairMaxSlots || s.M == 0) return CLUSTEN_ERR_BAD_DIMS;
     if (!scatter_by_cluster_supported(p, x, xs, y, s, dtype)) return CLUSTEN_ERR_UNALIGNED;
-    clusten_strides ys;
-    ys.b = (int64_t)s.H * s.N * s.C, ys.h = (int64_t)s.N * s.C, ys.n = s.C;
-    const Scatters jobs = {{{p, x, y, xs, ys, 1.f}, {}}};
+    const Scatters jobs = {{{p, x, y, xs, {}, 1.f}, {}}};
     return launch_jobs(jobs, 1, starts, ends, pairs, not_whole, s, dtype, stream);
 }
 
