@@ -45,8 +45,8 @@ struct Scatters {
     Scatter job[2];
 };
 
-template <typename T, int C, bool PAIR>
-__global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs, const int32_t* __restrict__ starts,
+template <typename T, int C, bool PAIR, int WAVES>
+__global__ __launch_bounds__(kWave * WAVES) void scatter_by_cluster_kernel(Scatters jobs, const int32_t* __restrict__ starts,
                                                                    const int32_t* __restrict__ ends,
                                                                    const int32_t* __restrict__ pairs,
                                                                    const int32_t* __restrict__ not_whole,
@@ -57,7 +57,10 @@ __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs
     const T* __restrict__ x = static_cast<const T*>(job.x);
     T* __restrict__ y = static_cast<T*>(job.y);
     const clusten_strides xs = job.xs, ys = job.ys;
-    const int h_first = (int)((int64_t)H * blockIdx.y / gridDim.y), h_last = (int)((int64_t)H * (blockIdx.y + 1) / gridDim.y);
+    // the waves of a workgroup and the workgroups of a column of the grid share the heads; no wave reads another's LDS
+    const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int share = blockIdx.y * WAVES + wave, shares = gridDim.y * WAVES;
+    const int h_first = (int)((int64_t)H * share / shares), h_last = (int)((int64_t)H * (share + 1) / shares);
     constexpr int EB = (int)sizeof(T);
     constexpr int ROW_B = C * EB;                    // bytes of an x row
     constexpr int PIECE_B = 8 * EB;                  // bytes of the 8 elements of p a pair contributes
@@ -70,9 +73,10 @@ __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs
     constexpr int P_BASE = X_BASE + X_BYTES;
     constexpr int O_BASE = P_BASE + 1024;
     constexpr int L_BASE = O_BASE + 8 * C * 4;
-    constexpr int LDS_BYTES = L_BASE + kListMax * 4;
+    constexpr int LDS_BYTES = (L_BASE + kListMax * 4 + 1023) / 1024 * 1024;
     static_assert(X_BYTES % 1024 == 0 && 1024 % ROW_B == 0, "whole LDS-direct loads, whole rows per load");
-    __shared__ __attribute__((aligned(1024))) char stage[LDS_BYTES];
+    __shared__ __attribute__((aligned(1024))) char stages[WAVES * LDS_BYTES];
+    char* const stage = stages + wave * LDS_BYTES;
 
     const int unit = xcd_tile(blockIdx.x, total_clusters);
     if (unit < 0) return;
@@ -83,7 +87,7 @@ __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs
     const int last = ends[unit];
     const int b = unit / clusters_per_image;
     const int g = unit - b * clusters_per_image;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x % kWave;
     if (flagged != 0) {         // not lists of whole clusters
         if constexpr (PAIR) {   // nothing else writes these rows: NaN, so that it shows
             const float v[4] = {NAN, NAN, NAN, NAN};
@@ -195,27 +199,37 @@ __global__ __launch_bounds__(kWave) void scatter_by_cluster_kernel(Scatters jobs
     }
 }
 
-// Workgroups that share the heads of a cluster: a wave walks its heads one after the other, each a chain of loads, products and stores,
-// so a launch is given enough waves to hide them, the list of a cluster being read again by each.  50 images of 777
-// tokens, 4 heads, fp16: 36.7 -> 31.6 us with two workgroups a cluster; d_key and d_value of a layer of AFF-Tiny at 64 images, mean of 25
-// layers: 2 x 43.6 us in two launches of one workgroup a cluster, 48.9 us in one.
+// Waves that share the heads of a cluster: a wave walks its heads one after the other, each a chain of loads, products and stores, so a
+// launch is given enough waves to hide them, the list of a cluster being read again by each.  Two of them make a workgroup: where the lists
+// are not whole clusters all of them leave, at 0.2 us a thousand workgroups.  us before the heads were shared / with as many one-wave
+// workgroups / now, and the same where they leave: 50 images of 777 tokens, 4 heads, fp16 47.1 / 41.8 / 38.4 (four waves), lists of any rows, with
+// the atomic kernels that take them 106.4 / 108.6 / 107.7; 2 of 1024, 8 heads, fp16 44.9 / 13.7 / 13.7; 8 of 777, 4 heads, fp32, any rows
+// 144.7 / 145.6 / 145.1.  d_key and d_value of a layer of AFF-Tiny at 64 images, mean of 25 layers: 2 x 43.6 us in two launches of one wave
+// a cluster, 48.9 us in one.
 inline int head_shares(int64_t waves, int H) { return (int)min((int64_t)H, max((int64_t)1, (int64_t)16384 / waves)); }
 
-template <typename T, int C>
-int launch_typed_c(const Scatters& jobs, int count, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
+template <typename T, int C, bool PAIR>
+int launch_jobs_of(const Scatters& jobs, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
                    const clusten_attn_shape& s, hipStream_t stream) {
     const int per_image = (s.N + 7) / 8;
     const int64_t total = (int64_t)s.B * per_image;
     if (total >= ((int64_t)1 << 30)) return CLUSTEN_ERR_BAD_DIMS;
-    const dim3 grid(xcd_grid((int)total), head_shares(total * count, s.H), count);
-    if (count == 2) {
-        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, true>), grid, dim3(kWave), 0, stream, jobs, starts, ends, pairs, not_whole, s.H, s.N, s.M,
-                           per_image, (int)total);
+    const int shares = head_shares(total * (PAIR ? 2 : 1), s.H);
+    if (shares == 1) {
+        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, PAIR, 1>), dim3(xcd_grid((int)total), 1, PAIR ? 2 : 1), dim3(kWave), 0, stream, jobs,
+                           starts, ends, pairs, not_whole, s.H, s.N, s.M, per_image, (int)total);
     } else {
-        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, false>), grid, dim3(kWave), 0, stream, jobs, starts, ends, pairs, not_whole, s.H, s.N,
-                           s.M, per_image, (int)total);
+        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, PAIR, 2>), dim3(xcd_grid((int)total), (shares + 1) / 2, PAIR ? 2 : 1), dim3(2 * kWave), 0,
+                           stream, jobs, starts, ends, pairs, not_whole, s.H, s.N, s.M, per_image, (int)total);
     }
     return launch_status();
+}
+
+template <typename T, int C>
+int launch_typed_c(const Scatters& jobs, int count, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
+                   const clusten_attn_shape& s, hipStream_t stream) {
+    return count == 2 ? launch_jobs_of<T, C, true>(jobs, starts, ends, pairs, not_whole, s, stream)
+                      : launch_jobs_of<T, C, false>(jobs, starts, ends, pairs, not_whole, s, stream);
 }
 
 template <typename T>
