@@ -502,6 +502,90 @@ def test_factors_that_are_no_numbers_of_the_type(device, dt, stream):
         assert torch.equal(got, ref)
 
 
+@pytest.mark.parametrize("dt", DTYPES)
+def test_what_a_training_step_is_made_of(device, dt):
+    """A model's graph has a node of its own for every block and merge, and the layers' general form for none of what these stand for.
+    In bf16 with local lists in every stage, as above."""
+    net = build(default_ops(), device, 0.4, (48, 48, 24) if dt == torch.bfloat16 else (48, 48, 48, 48)).train()
+    images = torch.randn(2, 3, 96, 96, generator=torch.Generator(device).manual_seed(1), device=device)
+    with torch.autocast("cuda", dtype=torch.float16 if dt == torch.float32 else dt, enabled=dt != torch.float32):
+        out = net(images)
+    names = [type(f).__name__ for f in walk(out.grad_fn)]
+    stages = [m for m in net.modules() if isinstance(m, BasicLayer)]
+    merges = sum(m.downsample is not None for m in stages)
+    local = names.count("_ClusterAttentionRowsBackward")
+    if dt != torch.bfloat16:
+        assert local + names.count("_DenseAttentionRowsBackward") == sum(len(m.blocks) for m in stages) and 0 < local < sum(len(m.blocks) for m in stages)
+        assert "_NormLinearRowsBackward" not in names and "_BlockTailBackward" not in names
+    else:
+        assert local > 0
+    for name in ("_MergeWeightsBackward", "_MergeTableBackward", "_RowScoreBackward"):
+        assert names.count(name) == merges, name
+    assert names.count("_LayerNormRowsBackward") == merges + 1       # of the merges and at the end; the patch embedding's 32 channels are not built
+
+
+def test_global_attention_of_an_fp32_forward_is_one_kernel(device):
+    """The stage's blocks by one call, and, issued one by one, the attention by its kernel."""
+    calls = []
+
+    def counted(name):
+        def call(*args, **kwargs):
+            calls.append(name)
+            return getattr(_native, name)(*args, **kwargs)
+        return call
+
+    images, counts = torch.randn(2, 3, 96, 96, generator=torch.Generator(device).manual_seed(1), device=device), {}
+    for name in ("blocks_forward", "dense_attention_train"):
+        ops = SimpleNamespace(**{**vars(default_ops()), name: counted(name)})
+        net = build(ops, device, 0.0, (48, 48, 48, 48)).eval()
+        calls.clear()
+        with torch.no_grad():
+            net(images)
+        counts[name] = len(calls)
+    stages = [m for m in net.modules() if isinstance(m, BasicLayer)]
+    assert counts["blocks_forward"] == len(stages)
+    assert counts["dense_attention_train"] == sum(len(m.blocks) for m in stages[-2:])        # 36 and 9 tokens; 576 and 144 ahead of them
+
+
+@pytest.mark.parametrize("masked", [True, False])
+def test_second_derivatives_of_merge_weights(device, masked):
+    """fp32 against the recorded formula: gradients, those of a backward that is itself recorded, and a batch of gradients."""
+    from aff.model import _MergeWeights
+    gen = torch.Generator(device).manual_seed(5)
+    b, n, n_out, m, rows = 2, 50, 12, 48, 225
+    table, prob = torch.randn(rows, 4, generator=gen, device=device), torch.rand(b, n, generator=gen, device=device)
+    pe, idx = (torch.randint(k, (b, n_out, m), generator=gen, device=device) for k in (rows, n))
+    mask = torch.randint(2, (b, n_out, m), generator=gen, device=device) if masked else None
+
+    def recorded(t, p, *_):
+        w = t[pe] * p.gather(1, idx.reshape(b, -1)).reshape(b, n_out, m, 1)
+        return w if mask is None else w * mask.unsqueeze(3)
+
+    derivatives_agree(lambda t, p: _MergeWeights.apply(t, p, pe, idx, mask, default_ops()), recorded, (table, prob), gen)
+
+
+@pytest.mark.parametrize("c", [32, 128])
+def test_second_derivatives_of_row_scores(device, c):
+    from aff.model import _RowScore
+    gen = torch.Generator(device).manual_seed(c)
+    x, w, bias = (torch.randn(*s, generator=gen, device=device) * k for s, k in (((2, 33, c), 1.0), ((1, c), c ** -0.5), ((1,), 1.0)))
+    derivatives_agree(lambda *a: _RowScore.apply(*a, torch.float32, default_ops()), lambda *a: F.linear(*a).sigmoid(), (x, w, bias), gen)
+
+
+def derivatives_agree(fn, recorded, tensors, gen):
+    results, batch = [], None
+    for f in (fn, recorded):
+        wanted = [t.clone().requires_grad_() for t in tensors]
+        out = f(*wanted)
+        batch = torch.randn(3, *out.shape, generator=gen, device=out.device) if batch is None else batch
+        plain = torch.autograd.grad(out, wanted, batch[0], retain_graph=True)
+        first = torch.autograd.grad(out, wanted, batch[0], create_graph=True)
+        second = torch.autograd.grad(sum(g.square().sum() for g in first), wanted, allow_unused=True)
+        results.append(plain + first + second + torch.autograd.grad(f(*wanted), wanted, batch, is_grads_batched=True))
+    for got, ref in zip(*results):
+        assert (got is None and ref is None) or norm_error(got, ref) < 1e-5
+
+
 # every width; a row, a workgroup's rows and one more, and more rows than all workgroups take at once
 @pytest.mark.parametrize("c,rows", [(64, 1), (64, 33), (64, 40000), (128, 17), (256, 9), (384, 1025), (512, 4101), (768, 8), (1024, 5000)])
 @pytest.mark.parametrize("dt,dy", [(torch.float32, torch.float32), (torch.float32, torch.float16), (torch.float32, torch.bfloat16),
