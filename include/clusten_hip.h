@@ -555,7 +555,11 @@ int clusten_bias_table_grad(const void* d_logit, const int64_t* pe_idx, float* d
  * table_weights (rows,IC), prob (B,N) or NULL, weights (B,Nout,M,IC): fp32, contiguous; pe_idx (values in
  * [0,rows) — unchecked), nbhd_idx (values in [0,N), others give NaN; may be NULL when prob is), mask (0/1, or NULL):
  * int64 (B,Nout,M).  IC = 4 (else CLUSTEN_ERR_BAD_DIMS); table_weights and weights 16-byte aligned (else
- * CLUSTEN_ERR_UNALIGNED).  Inference only.  No counterpart in the reference's extension modules. */
+ * CLUSTEN_ERR_UNALIGNED).  With `rows` given, positions outside [0,rows) give NaN and read nothing.  No counterpart in the reference's
+ * extension modules. */
+int clusten_merge_weights_forward_rows(const float* table_weights, int64_t rows, const int64_t* pe_idx, const int64_t* nbhd_idx,
+                                       const float* prob, const int64_t* mask, float* weights,
+                                       int B, int N, int Nout, int M, int IC, clusten_stream stream);
 int clusten_merge_weights_forward(const float* table_weights, const int64_t* pe_idx, const int64_t* nbhd_idx,
                                   const float* prob, const int64_t* mask, float* weights,
                                   int B, int N, int Nout, int M, int IC, clusten_stream stream);
@@ -802,10 +806,14 @@ int clusten_merge_table_backward(const float* d_out, const float* table, const f
 /* Training passes around a merge (models/aff_transformer.py:340-358, 496-500 under autograd).
  *   merge_weights_backward, of clusten_merge_weights_forward: d_rows (B,4,Nout,M) = d_weights (B,Nout,M,4) * prob * mask, which
  *     clusten_bias_table_grad (H = 4, the same pe_idx) sums into the table's rows, and, with prob, d_prob (B,N), written in full (fp32
- *     atomics).  A neighbour outside [0,N) gives NaN in d_rows and nothing to d_prob.
+ *     atomics).  A neighbour outside [0,N) gives NaN in d_rows and nothing to d_prob;
+ *     with `rows` (of table_weights) given, a position outside them gives NaN to its neighbour's d_prob and reads nothing.
  *   row_score: score (rows) of dtype = sigmoid(x w + bias), operands, the sum and the result rounded to dtype; x (rows,C) of x_dtype (F32
  *     or dtype), C in {32,64,128,256,512}, w (C) and bias (1, may be NULL) fp32.  The backward: d_x of x_dtype, d_weight (C), d_bias (C floats,
  *     the first is the bias' gradient); workspace: clusten_row_sums_workspace_bytes(rows, C). */
+int clusten_merge_weights_backward_rows(const float* d_weights, const float* table_weights, int64_t rows, const int64_t* pe_idx,
+                                        const int64_t* nbhd_idx, const float* prob, const int64_t* mask, float* d_rows, float* d_prob,
+                                        int B, int N, int Nout, int M, clusten_stream stream);
 int clusten_merge_weights_backward(const float* d_weights, const float* table_weights, const int64_t* pe_idx,
                                    const int64_t* nbhd_idx, const float* prob, const int64_t* mask, float* d_rows, float* d_prob,
                                    int B, int N, int Nout, int M, clusten_stream stream);

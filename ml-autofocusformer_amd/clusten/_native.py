@@ -135,6 +135,8 @@ _PROTOTYPES = {
                                                     _P]),
     "clusten_bias_table_grad": (ctypes.c_int, [_P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                               ctypes.c_int, ctypes.c_int, _P]),
+    "clusten_merge_weights_forward_rows": (ctypes.c_int, [_P, ctypes.c_int64, _P, _P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                                          ctypes.c_int, ctypes.c_int, _P]),
     "clusten_merge_weights_forward": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                                     ctypes.c_int, ctypes.c_int, _P]),
     "clusten_scanline_rank_max_tokens": (ctypes.c_int, []),
@@ -175,6 +177,8 @@ _PROTOTYPES = {
     "clusten_block_train_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(BlockTrain)]),
     "clusten_block_train_forward": (ctypes.c_int, [ctypes.POINTER(BlockTrain), _P, _P]),
     "clusten_block_train_backward": (ctypes.c_int, [ctypes.POINTER(BlockTrain), _P, _P, _P, ctypes.c_size_t, _P]),
+    "clusten_merge_weights_backward_rows": (ctypes.c_int, [_P, _P, ctypes.c_int64, _P, _P, _P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                                           ctypes.c_int, _P]),
     "clusten_merge_weights_backward": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _P]),
     "clusten_row_score_forward": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, ctypes.c_int64, ctypes.c_int, ctypes.c_int, _P]),
     "clusten_row_score_backward": (ctypes.c_int, [_P, ctypes.c_int, _P, _P, _P, _P, _P, _P, _P, ctypes.c_size_t, ctypes.c_int64, ctypes.c_int,
@@ -1533,10 +1537,10 @@ def merge_weights(table_weights: torch.Tensor, pe_idx: torch.Tensor, nbhd_idx: t
     if out.numel() == 0:
         return out
     with _on(device):
-        _check(lib.clusten_merge_weights_forward(_ptr(table_weights), _ptr(pe_idx.contiguous()),
-                                                 _ptr(nbhd_idx.contiguous()), _ptr(prob), _ptr(mask), _ptr(out), b, n,
-                                                 n_out, m, table_weights.shape[1], _stream(device)),
-               "clusten_merge_weights_forward")
+        _check(lib.clusten_merge_weights_forward_rows(_ptr(table_weights), table_weights.shape[0], _ptr(pe_idx.contiguous()),
+                                                      _ptr(nbhd_idx.contiguous()), _ptr(prob), _ptr(mask), _ptr(out), b, n,
+                                                      n_out, m, table_weights.shape[1], _stream(device)),
+               "clusten_merge_weights_forward_rows")
     return out if fractions is None else out.mul_(fractions.unsqueeze(3))
 
 
@@ -1597,9 +1601,10 @@ def merge_weights_backward(d_weights: torch.Tensor, table_weights: torch.Tensor,
     if rows.numel() == 0:
         return torch.zeros_like(table_weights), None if prob is None else d_prob.zero_()
     with _on(device):
-        _check(lib.clusten_merge_weights_backward(d_weights.data_ptr(), table_weights.data_ptr(), pe_idx.data_ptr(), nbhd_idx.data_ptr(), _ptr(prob),
-                                                  _ptr(mask), rows.data_ptr(), _ptr(d_prob), b, 1 if prob is None else prob.shape[1], n_out, m,
-                                                  _stream(device)), "clusten_merge_weights_backward")
+        _check(lib.clusten_merge_weights_backward_rows(d_weights.data_ptr(), table_weights.data_ptr(), table_weights.shape[0], pe_idx.data_ptr(),
+                                                       nbhd_idx.data_ptr(), _ptr(prob), _ptr(mask), rows.data_ptr(), _ptr(d_prob), b,
+                                                       1 if prob is None else prob.shape[1], n_out, m, _stream(device)),
+               "clusten_merge_weights_backward_rows")
     return bias_table_grad(rows, pe_idx, table_weights.shape[0]), d_prob
 
 

@@ -534,15 +534,21 @@ int clusten_bias_table_grad(const void* d_logit, const int64_t* pe_idx, float* d
     return launch_bias_table_grad(d_logit, pe_idx, d_table, B, H, N, M, rows, dtype, as_stream(stream));
 }
 
+int clusten_merge_weights_forward_rows(const float* table_weights, int64_t rows, const int64_t* pe_idx, const int64_t* nbhd_idx,
+                                       const float* prob, const int64_t* mask, float* weights, int B, int N, int Nout, int M,
+                                       int IC, clusten_stream stream) {
+    if (!table_weights || !pe_idx || !weights) return CLUSTEN_ERR_NULL_POINTER;
+    if (prob && !nbhd_idx) return CLUSTEN_ERR_NULL_POINTER;
+    if (B <= 0 || N <= 0 || Nout <= 0 || M <= 0 || IC != 4 || rows <= 0) return CLUSTEN_ERR_BAD_DIMS;
+    if (((int64_t)B * Nout * M + 255) / 256 >= ((int64_t)1 << 31)) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(table_weights) || !aligned16(weights)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_merge_weights(table_weights, pe_idx, nbhd_idx, prob, mask, weights, B, N, Nout, M, rows, as_stream(stream));
+}
+
 int clusten_merge_weights_forward(const float* table_weights, const int64_t* pe_idx, const int64_t* nbhd_idx,
                                   const float* prob, const int64_t* mask, float* weights, int B, int N, int Nout, int M,
                                   int IC, clusten_stream stream) {
-    if (!table_weights || !pe_idx || !weights) return CLUSTEN_ERR_NULL_POINTER;
-    if (prob && !nbhd_idx) return CLUSTEN_ERR_NULL_POINTER;
-    if (B <= 0 || N <= 0 || Nout <= 0 || M <= 0 || IC != 4) return CLUSTEN_ERR_BAD_DIMS;
-    if (((int64_t)B * Nout * M + 255) / 256 >= ((int64_t)1 << 31)) return CLUSTEN_ERR_BAD_DIMS;
-    if (!aligned16(table_weights) || !aligned16(weights)) return CLUSTEN_ERR_UNALIGNED;
-    return launch_merge_weights(table_weights, pe_idx, nbhd_idx, prob, mask, weights, B, N, Nout, M, as_stream(stream));
+    return clusten_merge_weights_forward_rows(table_weights, INT64_MAX, pe_idx, nbhd_idx, prob, mask, weights, B, N, Nout, M, IC, stream);
 }
 
 size_t clusten_scanline_rank_workspace_bytes(int B, int N) {
@@ -932,14 +938,21 @@ int clusten_merge_table_backward(const float* d_out, const float* table, const f
     return merge_table_call(MergeTable{table, weight, bias, norm_w, norm_b, d_out, nullptr, d_params, rows, eps}, true, dtype, stream);
 }
 
+int clusten_merge_weights_backward_rows(const float* d_weights, const float* table_weights, int64_t rows, const int64_t* pe_idx,
+                                        const int64_t* nbhd_idx, const float* prob, const int64_t* mask, float* d_rows, float* d_prob,
+                                        int B, int N, int Nout, int M, clusten_stream stream) {
+    if (!d_weights || !pe_idx || !d_rows || (prob && (!table_weights || !nbhd_idx || !d_prob))) return CLUSTEN_ERR_NULL_POINTER;
+    if (B <= 0 || N <= 0 || Nout <= 0 || M <= 0 || rows <= 0 || ((int64_t)B * Nout * M + 255) / 256 >= (int64_t)1 << 31) return CLUSTEN_ERR_BAD_DIMS;
+    if (!aligned16(d_weights) || !aligned16(table_weights) || !aligned16(d_prob)) return CLUSTEN_ERR_UNALIGNED;
+    return launch_merge_weights_backward(d_weights, table_weights, pe_idx, nbhd_idx, prob, mask, d_rows, prob ? d_prob : nullptr, B, N, Nout, M,
+                                         rows, as_stream(stream));
+}
+
 int clusten_merge_weights_backward(const float* d_weights, const float* table_weights, const int64_t* pe_idx, const int64_t* nbhd_idx,
                                    const float* prob, const int64_t* mask, float* d_rows, float* d_prob, int B, int N, int Nout, int M,
                                    clusten_stream stream) {
-    if (!d_weights || !pe_idx || !d_rows || (prob && (!table_weights || !nbhd_idx || !d_prob))) return CLUSTEN_ERR_NULL_POINTER;
-    if (B <= 0 || N <= 0 || Nout <= 0 || M <= 0 || ((int64_t)B * Nout * M + 255) / 256 >= (int64_t)1 << 31) return CLUSTEN_ERR_BAD_DIMS;
-    if (!aligned16(d_weights) || !aligned16(table_weights) || !aligned16(d_prob)) return CLUSTEN_ERR_UNALIGNED;
-    return launch_merge_weights_backward(d_weights, table_weights, pe_idx, nbhd_idx, prob, mask, d_rows, prob ? d_prob : nullptr, B, N, Nout, M,
-                                         as_stream(stream));
+    return clusten_merge_weights_backward_rows(d_weights, table_weights, INT64_MAX, pe_idx, nbhd_idx, prob, mask, d_rows, d_prob, B, N, Nout, M,
+                                               stream);
 }
 
 static int row_score_args(RowScore& a, const void* x, int x_dtype, const float* weight, void* score, int64_t rows, int C, int dtype) {

@@ -218,7 +218,7 @@ int launch_bias_table_grad(const void* d_logit, const int64_t* pe_idx, float* d_
 // w[b,i,j,:4] = table_w[pe_idx[b,i,j], :4] * prob[b, nbhd_idx[b,i,j]] * mask[b,i,j]   (prob, mask may be null)
 //   table_w (rows,4), prob (B,N), w (B,Nout,M,4): fp32;  pe_idx, nbhd_idx, mask: int64 (B,Nout,M).
 int launch_merge_weights(const float* table_w, const int64_t* pe_idx, const int64_t* nbhd_idx, const float* prob,
-                         const int64_t* mask, float* out, int B, int N, int Nout, int M, hipStream_t stream);
+                         const int64_t* mask, float* out, int B, int N, int Nout, int M, int64_t rows, hipStream_t stream);
 
 // ranking[b,:] = the order of the tokens of image b along the scan-line walk over a rows x cols anchor grid with
 //   cells of cell_w x cell_h (see scanline_rank.hip).  pos (B,N,2) fp32 as (x, y); ranking (B,N) int64; N <= scanline_rank_max_tokens()
@@ -426,7 +426,7 @@ int launch_scatter_pair(const void* d_logit, const void* query, clusten_strides 
 
 // Training passes of a merge's weights and of the importance score (merge_grad.hip).
 int launch_merge_weights_backward(const float* d_w, const float* table_w, const int64_t* pe_idx, const int64_t* nbhd_idx, const float* prob,
-                                  const int64_t* mask, float* t, float* d_prob, int B, int N, int Nout, int M, hipStream_t stream);
+                                  const int64_t* mask, float* t, float* d_prob, int B, int N, int Nout, int M, int64_t rows, hipStream_t stream);
 struct RowScore {
     const void* x;         // (rows, C) of S
     const float* weight;   // (C)

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256) void merge_weights_backward_kernel(const float
                                                                      const int64_t* __restrict__ pe_idx, const int64_t* __restrict__ nbhd_idx,
                                                                      const float* __restrict__ prob, const int64_t* __restrict__ mask,
                                                                      float* __restrict__ t, float* __restrict__ d_prob, int64_t pairs,
-                                                                     int64_t per_image, int N) {
+                                                                     int64_t per_image, int N, int64_t rows) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= pairs) return;
     const int64_t image = e / per_image, place = e - image * per_image;
@@ -29,7 +29,9 @@ __global__ __launch_bounds__(256) void merge_weights_backward_kernel(const float
         const bool inside = (uint64_t)nb < (uint64_t)N;      // a neighbour outside the image has no score: NaN, as in the forward
         const int64_t row = image * N + nb;
         s *= inside ? prob[row] : NAN;
-        const float4 w = *reinterpret_cast<const float4*>(table_w + pe_idx[e] * 4);
+        const int64_t at = pe_idx[e];
+        float4 w = make_float4(NAN, NAN, NAN, NAN);          // a position outside the table
+        if ((uint64_t)at < (uint64_t)rows) w = *reinterpret_cast<const float4*>(table_w + at * 4);
         if (inside && m != 0.f) unsafeAtomicAdd(d_prob + row, m * ((d.x * w.x + d.y * w.y) + (d.z * w.z + d.w * w.w)));
     }
     float* to = t + image * 4 * per_image + place;
@@ -143,13 +145,13 @@ int launch_typed(const RowScore& a, int C, hipStream_t stream) {
 }  // namespace
 
 int launch_merge_weights_backward(const float* d_w, const float* table_w, const int64_t* pe_idx, const int64_t* nbhd_idx, const float* prob,
-                                  const int64_t* mask, float* t, float* d_prob, int B, int N, int Nout, int M, hipStream_t stream) {
+                                  const int64_t* mask, float* t, float* d_prob, int B, int N, int Nout, int M, int64_t rows, hipStream_t stream) {
     const int64_t per = (int64_t)Nout * M, pairs = per * B;
     if (d_prob) {
         if (int st = launch_zero_f32(d_prob, (size_t)B * N, stream)) return st;
     }
     hipLaunchKernelGGL(merge_weights_backward_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream, d_w, table_w, pe_idx, nbhd_idx, prob,
-                       mask, t, d_prob, pairs, per, N);
+                       mask, t, d_prob, pairs, per, N, rows);
     return launch_status();
 }
 

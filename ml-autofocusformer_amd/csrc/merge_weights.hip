@@ -17,10 +17,13 @@ __global__ __launch_bounds__(256) void merge_weights_kernel(const float* __restr
                                                             const int64_t* __restrict__ nbhd_idx,
                                                             const float* __restrict__ prob,
                                                             const int64_t* __restrict__ mask, float* __restrict__ out,
-                                                            int64_t pairs, int64_t pairs_per_batch, int N) {
+                                                            int64_t pairs, int64_t pairs_per_batch, int N,
+                                                            int64_t rows) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (e >= pairs) return;
-    float4 w = *reinterpret_cast<const float4*>(table_w + pe_idx[e] * 4);
+    const int64_t at = pe_idx[e];
+    float4 w = make_float4(NAN, NAN, NAN, NAN);      // a position outside the table, as of a neighbour outside the image below
+    if ((uint64_t)at < (uint64_t)rows) w = *reinterpret_cast<const float4*>(table_w + at * 4);
     float s = 1.f;
     if (prob) {
         const int64_t nb = nbhd_idx[e];
@@ -34,11 +37,11 @@ __global__ __launch_bounds__(256) void merge_weights_kernel(const float* __restr
 }  // namespace
 
 int launch_merge_weights(const float* table_w, const int64_t* pe_idx, const int64_t* nbhd_idx, const float* prob,
-                         const int64_t* mask, float* out, int B, int N, int Nout, int M, hipStream_t stream) {
+                         const int64_t* mask, float* out, int B, int N, int Nout, int M, int64_t rows, hipStream_t stream) {
     const int64_t per_batch = (int64_t)Nout * M;
     const int64_t pairs = per_batch * B;
     hipLaunchKernelGGL(merge_weights_kernel, dim3((unsigned)((pairs + 255) / 256)), dim3(256), 0, stream, table_w, pe_idx,
-                       nbhd_idx, prob, mask, out, pairs, per_batch, N);
+                       nbhd_idx, prob, mask, out, pairs, per_batch, N, rows);
     return launch_status();
 }
 

@@ -266,6 +266,27 @@ def test_merge_weights_of_neighbours_outside(device):
     near(d_prob, masked[1], 5e-7)
 
 
+def test_merge_weights_of_positions_outside(device):
+    """Positions that are no row of the table: NaN where they stand and in their neighbour's gradient, nothing read there, every other
+    value as without them."""
+    gen = torch.Generator(device).manual_seed(3)
+    b, n, n_out, m, rows = 2, 50, 12, 48, 225
+    table, prob = torch.randn(rows, 4, generator=gen, device=device), torch.rand(b, n, generator=gen, device=device)
+    pe, idx = (torch.randint(k, (b, n_out, m), generator=gen, device=device) for k in (rows, n - 1))
+    d = torch.randn(b, n_out, m, 4, generator=gen, device=device)
+    bad = pe.clone()
+    bad[0, 3, 5], bad[1, 11, 47], bad[1, 0, 0] = rows, -1, 1 << 40
+    out = bad != pe
+    idx[out] = n - 1                                             # a neighbour of their own
+    got, want = _native.merge_weights(table, bad, idx, prob, None), _native.merge_weights(table, pe, idx, prob, None)
+    assert got[out].isnan().all() and torch.equal(got[~out], want[~out])
+    d_table, d_prob = _native.merge_weights_backward(d, table, bad, idx, prob, None)
+    masked = _native.merge_weights_backward(d, table, pe, idx, prob, (~out).long())
+    assert d_prob[:, -1].isnan().all()
+    near(d_prob[:, :-1], masked[1][:, :-1], 5e-7)
+    near(d_table, masked[0], 5e-7)
+
+
 def merging(device, n=48, c=32):
     """A merge of n tokens that all see each other: the module, scores, and its forward on given scores and mask."""
     from aff.model import ClusterMerging, default_ops, relative_position_table
