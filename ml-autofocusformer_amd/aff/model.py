@@ -1212,7 +1212,7 @@ class ClusterMerging(_Module):
             # inference: lookup, importance of each neighbour and mask in one kernel
             weights = one_pass(table_w, pe_idx, member_idx, learned_prob, mask_rows)
         elif (one_pass is not None and getattr(self.ops, "merge_weights_backward", None) is not None and torch.is_grad_enabled()
-              and learned_prob is not None and table_w.is_cuda and table_w.dtype == torch.float32 and table_w.is_contiguous()
+              and learned_prob is not None and table_w.is_cuda and table_w.dtype == torch.float32 and table_w.is_contiguous() and pe_idx.dtype == torch.int64
               and self.ops.merge_weights_supported(table_w) and not _transformed() and not (mask_rows is not None and mask_rows.requires_grad)
               and not torch.are_deterministic_algorithms_enabled()):           # its gradient of the scores is added up by atomics
             weights = _MergeWeights.apply(table_w, learned_prob.float().reshape(b, n), pe_idx, member_idx, mask_rows, self.ops)

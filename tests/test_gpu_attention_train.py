@@ -300,8 +300,8 @@ def merging(device, n=48, c=32):
     pe = torch.randint(table.shape[0], (2, n, n), generator=gen, device=device)
     feat, score = torch.randn(2, n, c, generator=gen, device=device), torch.rand(2, n, 1, generator=gen, device=device)
 
-    def call(score, mask=None, module=merge):
-        return module(pos, feat, everyone, mask, score, 4, pe, 0, table)[1]
+    def call(score, mask=None, module=merge, positions=torch.int64):
+        return module(pos, feat, everyone, mask, score, 4, pe.to(positions), 0, table)[1]
     return merge, score, call
 
 
@@ -313,6 +313,17 @@ def test_merge_of_strided_scores(device):
     for s in (score, torch.cat([score, score + 1, score], 2)[..., :1]):
         s = s.detach().requires_grad_()
         results.append(torch.autograd.grad(call(s).square().sum(), [s, *merge.parameters()]))
+    for a, b in zip(*results):
+        near(a, b, 1e-5)
+
+
+def test_merge_of_narrow_positions(device):
+    """Positions in 32 bits, which the recorded lookup takes and the kernel does not, in training."""
+    merge, score, call = merging(device)
+    results = []
+    for dt in (torch.int64, torch.int32):
+        s = score.clone().requires_grad_()
+        results.append(torch.autograd.grad(call(s, positions=dt).square().sum(), [s, *merge.parameters()]))
     for a, b in zip(*results):
         near(a, b, 1e-5)
 
