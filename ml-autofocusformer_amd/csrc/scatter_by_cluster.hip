@@ -21,6 +21,8 @@
 // the slots past its rows (models/point_utils.py pads member lists with index 0): those slots add to row 0, so
 // such a pair is listed a second time, flagged, under cluster 0, where the sum of its pad slots feeds row 0.
 // It has no counterpart in the reference's extension modules.
+#include <type_traits>
+
 #include "launch.hpp"
 #include "mfma.hpp"
 
@@ -32,35 +34,43 @@ constexpr int kListMax = 256;    // pairs of a cluster held in LDS at a time
 constexpr int kPadEntry = 1 << 30;   // list entry flag: the pair names the short last cluster; here, for its pad slots
 constexpr int kEntryMask = kPadEntry - 1;
 
-// One scatter: y += scale * ..., the rows of y strided.  A launch takes two over the same lists (d_key and d_value: PAIR), or one, whose y
-// is contiguous and whose scale is 1 (with the pair's addressing it was some tenths of a per cent slower).
+// A launch takes one scatter, whose y is contiguous, or two over the same lists (d_key and d_value: PAIR): y += scale * ..., the rows of y
+// strided.  A workgroup of one wave is short enough for what it does ahead of its first load to show: 128 images of 3136 tokens, 2 heads, fp32
+// took 124.7 us with the pair's arguments and the heads' split worked out by a division, 122.9 with its own and the split as an argument.
 struct Scatter {
     const void* p;
     const void* x;
     void* y;
-    clusten_strides xs, ys;
+    clusten_strides xs;
+};
+struct StridedScatter : Scatter {
+    clusten_strides ys;
     float scale;
 };
-struct Scatters {
-    Scatter job[2];
+struct Pair {
+    StridedScatter job[2];
 };
 
-template <typename T, int C, bool PAIR, int WAVES>
-__global__ __launch_bounds__(kWave * WAVES) void scatter_by_cluster_kernel(Scatters jobs, const int32_t* __restrict__ starts,
+// Jobs: Scatter or Pair; `heads` of a wave.
+template <typename T, int C, typename Jobs, int WAVES>
+__global__ __launch_bounds__(kWave * WAVES) void scatter_by_cluster_kernel(Jobs jobs, const int32_t* __restrict__ starts,
                                                                    const int32_t* __restrict__ ends,
                                                                    const int32_t* __restrict__ pairs,
                                                                    const int32_t* __restrict__ not_whole,
-                                                                   int H, int N, int M, int clusters_per_image,
+                                                                   int H, int heads, int N, int M, int clusters_per_image,
                                                                    int total_clusters) {
-    const Scatter& job = jobs.job[PAIR ? blockIdx.z : 0];
+    constexpr bool PAIR = std::is_same<Jobs, Pair>::value;
+    const auto& job = [&]() -> const auto& {
+        if constexpr (PAIR) return jobs.job[blockIdx.z];
+        else return jobs;
+    }();
     const T* __restrict__ p = static_cast<const T*>(job.p);
     const T* __restrict__ x = static_cast<const T*>(job.x);
     T* __restrict__ y = static_cast<T*>(job.y);
-    const clusten_strides xs = job.xs, ys = job.ys;
+    const clusten_strides xs = job.xs;
     // the waves of a workgroup and the workgroups of a column of the grid share the heads; no wave reads another's LDS
     const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int share = blockIdx.y * WAVES + wave, shares = gridDim.y * WAVES;
-    const int h_first = (int)((int64_t)H * share / shares), h_last = (int)((int64_t)H * (share + 1) / shares);
+    const int h_first = WAVES == 1 ? 0 : min(H, (int)(blockIdx.y * WAVES + wave) * heads), h_last = WAVES == 1 ? H : min(H, h_first + heads);
     constexpr int EB = (int)sizeof(T);
     constexpr int ROW_B = C * EB;                    // bytes of an x row
     constexpr int PIECE_B = 8 * EB;                  // bytes of the 8 elements of p a pair contributes
@@ -94,7 +104,7 @@ __global__ __launch_bounds__(kWave * WAVES) void scatter_by_cluster_kernel(Scatt
             const int quads = min(8, N - 8 * g) * (C / 4);
             for (int i = h_first * quads + lane; i < h_last * quads; i += kWave) {
                 const int h = i / quads, q = i - h * quads;
-                T* row = y + (int64_t)b * ys.b + (int64_t)h * ys.h + (int64_t)(g * 8 + q / (C / 4)) * ys.n;
+                T* row = y + (int64_t)b * job.ys.b + (int64_t)h * job.ys.h + (int64_t)(g * 8 + q / (C / 4)) * job.ys.n;
                 *reinterpret_cast<typename Quad<T>::raw*>(row + q % (C / 4) * 4) = Quad<T>::pack(v);
             }
         }
@@ -169,7 +179,9 @@ __global__ __launch_bounds__(kWave * WAVES) void scatter_by_cluster_kernel(Scatt
             }
         }
         // rows 4*kq + j of the result (kq < 2: the cluster's 8 rows), channels 16*cb + r16
-        T* y_rows = PAIR ? y + (int64_t)b * ys.b + (int64_t)h * ys.h + (int64_t)g * 8 * ys.n : y + (((int64_t)b * H + h) * N + (int64_t)g * 8) * C;
+        T* y_rows;
+        if constexpr (PAIR) y_rows = y + (int64_t)b * job.ys.b + (int64_t)h * job.ys.h + (int64_t)g * 8 * job.ys.n;
+        else y_rows = y + (((int64_t)b * H + h) * N + (int64_t)g * 8) * C;
         lds_sync();
         if (kq < 2) {
 #pragma unroll
@@ -189,7 +201,7 @@ __global__ __launch_bounds__(kWave * WAVES) void scatter_by_cluster_kernel(Scatt
                 const F32x4 o = *reinterpret_cast<const F32x4*>(stage + O_BASE + q * 16);
                 if constexpr (PAIR) {
                     const float v[4] = {o[0] * job.scale, o[1] * job.scale, o[2] * job.scale, o[3] * job.scale};
-                    *reinterpret_cast<typename Quad<T>::raw*>(y_rows + (int64_t)(q / (C / 4)) * ys.n + q % (C / 4) * 4) = Quad<T>::pack(v);
+                    *reinterpret_cast<typename Quad<T>::raw*>(y_rows + (int64_t)(q / (C / 4)) * job.ys.n + q % (C / 4) * 4) = Quad<T>::pack(v);
                 } else {
                     const float v[4] = {o[0], o[1], o[2], o[3]};
                     *reinterpret_cast<typename Quad<T>::raw*>(y_rows + q * 4) = Quad<T>::pack(v);
@@ -208,47 +220,44 @@ __global__ __launch_bounds__(kWave * WAVES) void scatter_by_cluster_kernel(Scatt
 // a cluster, 48.9 us in one.
 inline int head_shares(int64_t waves, int H) { return (int)min((int64_t)H, max((int64_t)1, (int64_t)16384 / waves)); }
 
-template <typename T, int C, bool PAIR>
-int launch_jobs_of(const Scatters& jobs, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
+template <typename T, int C, typename Jobs>
+int launch_jobs_of(const Jobs& jobs, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
                    const clusten_attn_shape& s, hipStream_t stream) {
+    constexpr bool PAIR = std::is_same<Jobs, Pair>::value;
     const int per_image = (s.N + 7) / 8;
     const int64_t total = (int64_t)s.B * per_image;
     if (total >= ((int64_t)1 << 30)) return CLUSTEN_ERR_BAD_DIMS;
-    const int shares = head_shares(total * (PAIR ? 2 : 1), s.H);
+    const int shares = head_shares(total * (PAIR ? 2 : 1), s.H), whole = shares == 1 ? 1 : min(s.H, (shares + 1) / 2 * 2);    // of two waves
+    const int heads = (s.H + whole - 1) / whole;
     if (shares == 1) {
-        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, PAIR, 1>), dim3(xcd_grid((int)total), 1, PAIR ? 2 : 1), dim3(kWave), 0, stream, jobs,
-                           starts, ends, pairs, not_whole, s.H, s.N, s.M, per_image, (int)total);
+        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, Jobs, 1>), dim3(xcd_grid((int)total), 1, PAIR ? 2 : 1), dim3(kWave), 0, stream, jobs,
+                           starts, ends, pairs, not_whole, s.H, heads, s.N, s.M, per_image, (int)total);
     } else {
-        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, PAIR, 2>), dim3(xcd_grid((int)total), (shares + 1) / 2, PAIR ? 2 : 1), dim3(2 * kWave), 0,
-                           stream, jobs, starts, ends, pairs, not_whole, s.H, s.N, s.M, per_image, (int)total);
+        const int waves = (s.H + heads - 1) / heads;
+        hipLaunchKernelGGL((scatter_by_cluster_kernel<T, C, Jobs, 2>), dim3(xcd_grid((int)total), (waves + 1) / 2, PAIR ? 2 : 1), dim3(2 * kWave), 0,
+                           stream, jobs, starts, ends, pairs, not_whole, s.H, heads, s.N, s.M, per_image, (int)total);
     }
     return launch_status();
 }
 
-template <typename T, int C>
-int launch_typed_c(const Scatters& jobs, int count, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
-                   const clusten_attn_shape& s, hipStream_t stream) {
-    return count == 2 ? launch_jobs_of<T, C, true>(jobs, starts, ends, pairs, not_whole, s, stream)
-                      : launch_jobs_of<T, C, false>(jobs, starts, ends, pairs, not_whole, s, stream);
-}
-
-template <typename T>
-int launch_typed(const Scatters& jobs, int count, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
+template <typename T, typename Jobs>
+int launch_typed(const Jobs& jobs, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
                  const clusten_attn_shape& s, hipStream_t stream) {
     switch (s.C) {
-        case 16: return launch_typed_c<T, 16>(jobs, count, starts, ends, pairs, not_whole, s, stream);
-        case 32: return launch_typed_c<T, 32>(jobs, count, starts, ends, pairs, not_whole, s, stream);
-        case 64: return launch_typed_c<T, 64>(jobs, count, starts, ends, pairs, not_whole, s, stream);
+        case 16: return launch_jobs_of<T, 16>(jobs, starts, ends, pairs, not_whole, s, stream);
+        case 32: return launch_jobs_of<T, 32>(jobs, starts, ends, pairs, not_whole, s, stream);
+        case 64: return launch_jobs_of<T, 64>(jobs, starts, ends, pairs, not_whole, s, stream);
         default: return CLUSTEN_ERR_BAD_DIMS;
     }
 }
 
-int launch_jobs(const Scatters& jobs, int count, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
+template <typename Jobs>
+int launch_jobs(const Jobs& jobs, const int32_t* starts, const int32_t* ends, const int32_t* pairs, const int32_t* not_whole,
                 const clusten_attn_shape& s, int dtype, hipStream_t stream) {
     switch (dtype) {
-        case CLUSTEN_F32: return launch_typed<float>(jobs, count, starts, ends, pairs, not_whole, s, stream);
-        case CLUSTEN_F16: return launch_typed<f16_t>(jobs, count, starts, ends, pairs, not_whole, s, stream);
-        case CLUSTEN_BF16: return launch_typed<bf16_t>(jobs, count, starts, ends, pairs, not_whole, s, stream);
+        case CLUSTEN_F32: return launch_typed<float>(jobs, starts, ends, pairs, not_whole, s, stream);
+        case CLUSTEN_F16: return launch_typed<f16_t>(jobs, starts, ends, pairs, not_whole, s, stream);
+        case CLUSTEN_BF16: return launch_typed<bf16_t>(jobs, starts, ends, pairs, not_whole, s, stream);
         default: return CLUSTEN_ERR_BAD_DTYPE;
     }
 }
@@ -269,8 +278,7 @@ int launch_scatter_by_cluster(const void* p, const void* x, clusten_strides xs, 
                               hipStream_t stream) {
     if ((s.C != 16 && s.C != 32 && s.C != 64) || s.N < 8 || s.M % 8 != 0 || s.M > kPairMaxSlots || s.M == 0) return CLUSTEN_ERR_BAD_DIMS;
     if (!scatter_by_cluster_supported(p, x, xs, y, s, dtype)) return CLUSTEN_ERR_UNALIGNED;
-    const Scatters jobs = {{{p, x, y, xs, {}, 1.f}, {}}};
-    return launch_jobs(jobs, 1, starts, ends, pairs, not_whole, s, dtype, stream);
+    return launch_jobs(Scatter{p, x, y, xs}, starts, ends, pairs, not_whole, s, dtype, stream);
 }
 
 bool scatter_pair_supported(const clusten_attn_shape& s, int dtype) {
@@ -289,8 +297,8 @@ int launch_scatter_pair(const void* d_logit, const void* query, clusten_strides 
     }
     const ClusterPairsLayout l = cluster_pairs_layout(s.B, s.N, s.M, s.N);
     const char* ws = static_cast<const char*>(pair_lists);
-    const Scatters jobs = {{{d_logit, query, d_key, qs, ys, scale}, {probs, d_out, d_value, gs, ys, 1.f}}};
-    return launch_jobs(jobs, 2, reinterpret_cast<const int32_t*>(ws + l.starts), reinterpret_cast<const int32_t*>(ws + l.ends),
+    const Pair jobs = {{{{d_logit, query, d_key, qs}, ys, scale}, {{probs, d_out, d_value, gs}, ys, 1.f}}};
+    return launch_jobs(jobs, reinterpret_cast<const int32_t*>(ws + l.starts), reinterpret_cast<const int32_t*>(ws + l.ends),
                        reinterpret_cast<const int32_t*>(ws + l.pairs), reinterpret_cast<const int32_t*>(ws + l.flag), s, dtype, stream);
 }
 

@@ -149,6 +149,20 @@ def test_backward_cluster_by_cluster_with_a_short_last_cluster(device, dtype):
     _check_wf_backward(case, device, dtype)
 
 
+# heads by waves that share a cluster: 3 + 2; 2 + 1; 2 + 2 + 1 and a wave without; one each and a wave without
+@pytest.mark.parametrize("B,H", [(15, 5), (15, 3), (12, 5), (12, 3)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_heads_of_a_scatter_that_waves_do_not_divide(device, dtype, B, H):
+    """Every head's rows, against the same head scattered by itself, which one wave a cluster does."""
+    g = torch.Generator(device).manual_seed(B + H)
+    N, M, C = 3199, 16, 32
+    pairs = _native.cluster_pairs_from_numbers(torch.randint(400, (B, N, M // 8), generator=g, device=device).int())
+    p, x = (torch.randn(B, H, N, k, generator=g, device=device).to(dtype) for k in (M, C))
+    got = _native.scatter_rows_by_cluster(p, x, pairs)
+    for h in range(H):
+        assert torch.equal(got[:, h], _native.scatter_rows_by_cluster(p[:, h:h + 1].contiguous(), x[:, h:h + 1], pairs)[:, 0])
+
+
 def test_cluster_by_cluster_scatter_properties(device):
     g = torch.Generator().manual_seed(81)
     B, H, N, C = 2, 3, 200, 32
