@@ -823,7 +823,8 @@ int clusten_row_score_backward(const void* x, int x_dtype, const float* weight, 
                                float* d_weight, float* d_bias, void* workspace, size_t workspace_bytes, int64_t rows, int C,
                                int dtype, clusten_stream stream);
 
-/* The backward of a block between its products, which the reference leaves to autograd.  Tensors are dense rows of C channels
+/* The backward of a block between its products, which the reference leaves to autograd: for callers that take the products from elsewhere.
+ * clusten_block_train_backward uses none of them but blank and the sums.  Tensors are dense rows of C channels
  * (C in {32,64,128,256,512}) of dtype F32, F16 or BF16 unless said otherwise, on 16-byte boundaries; sums are fp32 in a fixed
  * order; workspace: clusten_row_sums_workspace_bytes(rows, C) bytes.
  *   gelu: g = gelu(h), d_h = d_g gelu'(h); count a multiple of 8; d_h may be d_g.

@@ -2067,7 +2067,8 @@ def _block_rows(dtype, c, *tensors):
 
 
 def gelu_backward(hidden: torch.Tensor, d_g: torch.Tensor):
-    """(gelu(hidden), d_g * gelu'(hidden)), the exact GELU; d_g is overwritten with the second.  No autograd."""
+    """(gelu(hidden), d_g * gelu'(hidden)), the exact GELU; d_g is overwritten with the second.  By itself: `block_tail_backward` has it
+    inside.  No autograd."""
     _block_rows((hidden.dtype,), hidden.shape[-1], hidden, d_g)
     if hidden.dtype not in _DTYPE_CODES or hidden.numel() % 8:
         raise RuntimeError("gelu_backward takes fp32, fp16 or bf16 tensors of a multiple of 8 values")
@@ -2082,7 +2083,8 @@ def gelu_backward(hidden: torch.Tensor, d_g: torch.Tensor):
 def norm_backward(d_y: torch.Tensor, x: torch.Tensor, stats: torch.Tensor, weight: torch.Tensor, d_res=None, branch=False, scale=None):
     """Backward of y = LayerNorm(x) with statistics `stats` (`norm_linear(..., keep=True)`): (d_x, branch, d_weight, d_bias)
     with d_x = d_res + the gradient through the norm, of x's dtype, and, with `branch`, a copy of it in d_y's dtype times the
-    images' factors `scale` (fp32 (B,), B the first axis of x; None: 1).  No autograd."""
+    images' factors `scale` (fp32 (B,), B the first axis of x; None: 1).  By itself: `block_tail_backward` and `norm_linear_backward`
+    have it inside.  No autograd."""
     c = x.shape[-1]
     _block_rows((d_y.dtype,), c, d_y)
     _block_rows((x.dtype,), c, x, d_res)
@@ -2111,7 +2113,8 @@ def norm_backward(d_y: torch.Tensor, x: torch.Tensor, stats: torch.Tensor, weigh
 def attention_columns_backward(qkv: torch.Tensor, d_qkv: torch.Tensor, d_k: torch.Tensor, d_v: torch.Tensor, d_out: torch.Tensor,
                                d_blank: torch.Tensor, blank_prob: torch.Tensor, scale: float):
     """What is left of an attention layer's backward behind its scatters: scale * d_k and d_v (B,H,N,ch) into the key / value
-    columns of d_qkv (B,N,3C), and the blank token's gradients (scale * sum d_blank q, sum blank_prob d_out), each (C,) fp32."""
+    columns of d_qkv (B,N,3C), and the blank token's gradients (scale * sum d_blank q, sum blank_prob d_out), each (C,) fp32.
+    For scatters of one's own; `attention_rows_backward` needs no such step."""
     lib = load()
     b, n, c3 = qkv.shape
     c, h = c3 // 3, d_k.shape[1]
@@ -2155,7 +2158,8 @@ def position_bias(table: torch.Tensor, weight: torch.Tensor, bias, dtype: torch.
 
 
 def position_grad(d_logit: torch.Tensor, pe_idx: torch.Tensor, padded: torch.Tensor, k: int):
-    """The gradients (d_weight (h,k), d_bias (h)) of `position_bias` from d_logit (b,h,n,m), m a multiple of 4, k <= 5."""
+    """The gradients (d_weight (h,k), d_bias (h)) of `position_bias` from d_logit (b,h,n,m), m a multiple of 4, k <= 5; a part of
+    `block_train_backward`, as are `attention_rows_backward` and `dense_attention_train_backward`."""
     b, h, n, m = d_logit.shape
     _require_cuda("d_logit", d_logit)
     if (pe_idx.shape != (b, n, m) or pe_idx.dtype != torch.int64 or not pe_idx.is_contiguous() or not d_logit.is_contiguous()
@@ -2251,7 +2255,8 @@ def attention_rows_backward(qkv: torch.Tensor, d_qkv: torch.Tensor, probs: torch
 
 
 def table_linear_grad(d: torch.Tensor, x: torch.Tensor):
-    """(d^T x, column sums of d) for fp32 d (rows, n) and x (rows, k), k <= 8: the parameter gradients of a position bias layer."""
+    """(d^T x, column sums of d) for fp32 d (rows, n) and x (rows, k), k <= 8: the parameter gradients of a position bias layer
+    from its table's (`bias_table_grad`).  `position_grad` needs no table."""
     if not (d.is_cuda and d.device == x.device and d.dtype == torch.float32 and x.dtype in _DTYPE_CODES and d.is_contiguous()
             and x.is_contiguous() and d.dim() == 2 and x.dim() == 2 and d.shape[0] == x.shape[0] and 0 < x.shape[1] <= 8):
         raise RuntimeError("table_linear_grad: contiguous fp32 d (rows,n) and x (rows,k), k <= 8")

@@ -314,7 +314,8 @@ int launch_backward_tiles(const Args& a, hipStream_t stream) {
 template <typename T, typename S, int C, typename Args>
 int launch_backward_width(const Args& a, hipStream_t stream) {
     // Two tiles at most: four 16-bit ones of 256 channels do not fit the registers, nor do two fp32 ones of 128 and 256 (37 and 10 spilled), which
-    // are faster all the same where there are rows for them.  block_split's weights are the forward's.  us with 1 / 2 tiles, tail and
+    // are faster all the same where there are rows for them.  block_split's weights are the forward's, and its rounds
+    // beyond the 1024 workgroups launched are turns of their loops.  us with 1 / 2 tiles, tail and
     // norm_linear, fp32: 784 rows of 256 channels 46 / 64 and 22 / 27, 6272 rows 91 / 71 and 43 / 32, 50 176 rows 575 / 484 and 258 / 207;
     // 50 176 rows of 128 195 / 174 and 76 / 59; 200 704 rows of 64 283 / 236 and 110 / 94.  fp16: 12 544 rows of 256 58 / 46 and 28 / 20, 6272 rows
     // of 512 96 / 66 and 42 / 29, 200 704 of 64 150 / 125 and 53 / 42.  Where workgroups of narrow rows share a unit the rule takes the second

@@ -1,7 +1,8 @@
-// What the backward pass of a transformer block does between its products: the gradient of the GELU, of a layer norm with the
-// residual addition ahead of it, of the blank token, of the position bias' small Linear layer, and the order of the key and
-// value gradients.  The products with the weights
-// are block_backward_impl.hpp's or the library's.
+// Row kernels of a transformer block's backward.  What a training step runs: the blank token's gradients (`blank_grad`) and the launch that
+// adds up every kernel's partial sums (`grad_sums_kernel`).  The gradients of the GELU, of a layer norm with the residual addition ahead
+// of it and of the position bias' Linear layer, and the order of the key and value gradients, are entry points that stand by themselves,
+// for callers that take the products with the weights from elsewhere: a block's own backward has them inside the kernels of
+// block_backward_impl.hpp, attention_train.hip and scatter_by_cluster.hip.
 //
 // All of them stream rows of C channels once and are bound by that.  A lane takes 8 consecutive channels (16 bytes of 16-bit
 // data), C / 8 lanes a row, so that a wave holds 512 / C whole rows and row sums are a few lane exchanges; column sums stay in
@@ -167,7 +168,8 @@ __global__ __launch_bounds__(kRowThreads) void blank_grad_kernel(BlankGrad a) {
 
 // The sums of partial rows: 16 threads a column, 64 columns a workgroup, then a workgroup per head of a position bias layer.  Bound by the
 // trips to memory of a few workgroups, 5 us however few they are: a block's backward adds its four kinds up in one launch
-// at its end.  A step of AFF-Tiny at 64 images: 113 launches of 585 us, now 33 of 208 us.
+// at its end.  A step of AFF-Tiny at 64 images: 113 launches of 585 us, now 38 of 239 us, the
+// norms that stand by themselves and the merges' scores among them.
 constexpr int kPositionSums = 6;
 __global__ __launch_bounds__(1024) void grad_sums_kernel(GradSums a) {
     __shared__ double shared[16 * 64 / 2];

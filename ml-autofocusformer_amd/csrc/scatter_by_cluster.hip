@@ -217,7 +217,7 @@ __global__ __launch_bounds__(kWave * WAVES) void scatter_by_cluster_kernel(Jobs 
 // workgroups / now, and the same where they leave: 50 images of 777 tokens, 4 heads, fp16 47.1 / 41.8 / 38.4 (four waves), lists of any rows, with
 // the atomic kernels that take them 106.4 / 108.6 / 107.7; 2 of 1024, 8 heads, fp16 44.9 / 13.7 / 13.7; 8 of 777, 4 heads, fp32, any rows
 // 144.7 / 145.6 / 145.1.  d_key and d_value of a layer of AFF-Tiny at 64 images, mean of 25 layers: 2 x 43.6 us in two launches of one wave
-// a cluster, 48.9 us in one.
+// a cluster, 47.8 us in one.
 inline int head_shares(int64_t waves, int H) { return (int)min((int64_t)H, max((int64_t)1, (int64_t)16384 / waves)); }
 
 template <typename T, int C, typename Jobs>

@@ -11,7 +11,7 @@
 //   piece (s, t, lane) = channels s * kStep + kElems * kq .. of row 16 t + r16      (kStep = 32 channels).
 //
 // fp32 products run on the bf16 matrix instructions, every operand as the sum of three bf16 numbers (`split`): 24 bits, so that
-// nothing of an operand is lost.  The six products of parts that reach above 2^-24 of a term are summed in fp32, what is left out is
+// nothing of an operand of ordinary size is lost.  The six products of parts that reach above 2^-24 of a term are summed in fp32, what is left out is
 // below 2^-25 of it.  The instructions round a sum down, by up to 2^-26 of it: six to a step on running sums shifted the mean of 33 000
 // rows' results by 3e-6 of their deviation.  The six of a step therefore start from zero, smallest first, and their sum is
 // added by a fp32 addition, which rounds to nearest; and every other step is summed negated and subtracted, so that what is left of
@@ -20,7 +20,9 @@
 // instructions of all its row tiles, in their shadow.  Against float64 the results are nearer than the fp32 instructions' (relative
 // 2-norm, norm_linear / block_tail, fp32 instructions -> parts): 1.56 / 1.69 -> 0.77 / 0.72e-7 at 64 channels, 2.14 / 2.34 ->
 // 0.83 / 0.79e-7 at 128, 2.93 / 3.30 -> 0.92 / 0.93e-7 at 256, 4.12 / 4.63 -> 1.07 / 1.13e-7 at 512.
-// An operand that is infinite makes its results NaN where fp32 arithmetic may give infinity; finite ones up to 3.38e38 are exact.
+// Where it ends: an operand that is infinite, or finite above 3.38e38 (bf16's largest number), makes its results NaN where fp32 arithmetic
+// may give infinity; of one below 2^-103 the last part falls among bf16's subnormals, below 2^-110 beneath them, so that fewer than 24
+// bits are held, what is lost being some 2^-126 at most.
 #pragma once
 
 #include <type_traits>
